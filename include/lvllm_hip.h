@@ -697,8 +697,8 @@ typedef struct lvllm_moe_routing {
 } lvllm_moe_routing;
 /* the `top` experts of every row and their weights; with a shared one a last assignment, expert number `experts`, weighted by the
  * sigmoid of the last row of w (GATED) or 1 (PLAIN).  bias null: none.  The assignments come grouped by expert: offsets [experts +
- * shared + 1], token and slot [assignments], tiles [max_tiles + 1, 4] of lvllm_moe_tile slots, slot_weight [assignments] (null:
- * not kept).  `packed`: w as lvllm_pack_weight leaves it, rows padded to a multiple of 16 */
+ * shared + 1], token and slot [assignments], tiles [max_tiles + 1, 4] of at least lvllm_moe_tile slots (what max_tiles is
+ * counted with), slot_weight [assignments] (null: not kept).  `packed`: w as lvllm_pack_weight leaves it, rows padded to a multiple of 16 */
 int lvllm_moe_tile(int packed, int rows);
 int64_t lvllm_moe_route_workspace_bytes(const lvllm_moe_routing* routing, int rows, int width, int packed);
 int lvllm_moe_route(int32_t* ids, float* weights, int32_t* offsets, int32_t* token, int32_t* slot, float* slot_weight,

@@ -47,6 +47,13 @@ struct MoeActivation {
   __device__ __forceinline__ float operator()(float g, float u) const {
     return silu ? g / (1.f + expf(-g)) * u : clamped_unit_of(g, u, limit);
   }
+  // ... for a result of 16 bits
+  __device__ __forceinline__ float rounded(float g, float u) const {
+    if (silu) return g * sigmoid_16bit(g) * u;
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return g * sigmoid_16bit(1.702f * g) * (u + 1.f);
+  }
 };
 __device__ __forceinline__ float slot_weight_of(const MoeParams& p, int slot) {
   return p.slot_weight != nullptr ? p.slot_weight[slot] : 1.f;
@@ -244,9 +251,14 @@ __device__ __forceinline__ void moe_count_assignments(const int32_t* ids, int ro
   }
 }
 
-// slots of a tile: of the matrix-core body for prompts, and of those for few rows and for sizes without one
-constexpr int kMoeTile = 128, kMoeSmallTile = 16, kMoeFewRows = 64;
-inline int moe_tile(bool packed, int rows) { return packed && rows > kMoeFewRows ? kMoeTile : kMoeSmallTile; }
+// slots of a tile: of the matrix-core bodies for prompts, and of those for few rows and for sizes without one
+constexpr int kMoeRingTile = 64, kMoeTile = 128, kMoeSmallTile = 16, kMoeFewRows = 64;
+// Below 45 slots an expert the weights' bytes bound the products and the ring is ahead (moe_ring_kernel); from there on tiles of
+// 128 are: 50 slots an expert, up + down, 138 us against 144.  `slots` of all `experts`, the shared one's included.
+inline int moe_tile(bool packed, int rows, int64_t slots, int experts) {
+  if (!packed || rows <= kMoeFewRows) return kMoeSmallTile;
+  return slots < (int64_t)45 * experts ? kMoeRingTile : kMoeTile;
+}
 
 bool moe_takes_mfma(int width, int dtype);
 int launch_moe_mfma(const MoeParams& p, int product, hipStream_t s);

@@ -4,11 +4,10 @@
 //   * few slots per expert (decode steps): bound by the weights' bytes.  A workgroup takes 16 slots of one expert and a share
 //     of its outputs; the slots' rows sit in LDS in fragment order (2048 of K at a time), every wave streams the two W tiles
 //     of its own (1 KiB a load, eight k-steps in flight behind the eight in use) and needs no other wave;
-//   * prompts: 256 W rows x 128 slots a workgroup, a wave 64 x 128.  W goes from memory straight into the operand registers
-//     of the one wave that uses it, the slots' rows straight to LDS, 32 of K a step, three steps in flight behind the one in
-//     use (through LDS, W would take more of its bandwidth than there is).  A slot's 64 bytes are four chunks, exchanged so
-//     that a fragment read is free of bank conflicts.  An XCD gets consecutive work: up to eight tiles of an expert side by
-//     side, W block after W block, so that its L2 serves a W block to all of them and their rows to the next blocks.
+//   * prompts: tiles of 64 or 128 slots x 256 W rows, moe_ring_kernel and moe_tile_kernel (moe.h, moe_tile).  A slot's 64 bytes
+//     of a k-step are four chunks, exchanged so that a fragment read is free of bank conflicts.
+#include <algorithm>
+
 #include "moe.h"
 
 namespace lvllm {
@@ -117,7 +116,7 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
   if constexpr (GATED) {
     const MoeActivation act(p, e);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = act(acc[0][r] * f, acc[1][r] * f);
+    for (int r = 0; r < 4; ++r) v[r] = act.rounded(acc[0][r] * f, acc[1][r] * f);
     store4<BF16>((uint16_t*)p.out + (int64_t)slot * p.ff_max + 16 * u + 4 * g, v);
   } else {
 #pragma unroll
@@ -129,49 +128,304 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
   }
 }
 
-constexpr int kTileW = 16;                                 // W tiles of a workgroup
-constexpr int kStages = 4, kStageBytes = kMoeTile * 64;    // of 32 of K: 16-slot groups of 1 KiB
+constexpr int kTileW = 16;  // W tiles of a workgroup
 
-__device__ __forceinline__ void to_lds(const uint16_t* src, char* dst) {  // 16 bytes a lane, 1 KiB a wave
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                   (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+// A workgroup's turns.  An XCD gets an eighth of the last expert's tiles (the shared expert may be larger: its tiles come first)
+// and of all others', as units: up to 1024 slots of an expert side by side, W block after W block, so that its L2 serves a W
+// block to all of them and their rows to the next blocks.  Its workgroups take units in turn.
+struct TileWork {
+  int e, block, s0, s1, steps, ntiles;  // slots s0 .. s1 - 1, k-steps, W tiles of 16 rows of the expert
+  bool any;
+};
+template <int PRODUCT, int TILE>
+__device__ __forceinline__ TileWork tile_work(const MoeParams& p, const int blocks_first, const int blocks_last, const int turn) {
+  constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
+  constexpr int kSide = 1024 / TILE;
+  TileWork t{};
+  const int xcd = blockIdx.x & 7, cu = blockIdx.x >> 3, cus = gridDim.x >> 3;
+  const int tiles_first = p.tiles[4 * p.max_tiles];
+  const int all_first = tiles_first * blocks_first, all_last = (p.tiles[4 * p.max_tiles + 1] - tiles_first) * blocks_last;
+  const int per_first = (all_first + 7) / 8, per_last = (all_last + 7) / 8;
+  // the first `own` turns are the last expert's, as long as `as_long` of the others (going down, k-steps are its inner size):
+  // workgroups with one turn of them fewer start on the others by so much earlier
+  const int as_long = UP ? 1 : max(1, (p.ff_last + p.ff_first / 2) / p.ff_first);
+  const int full = per_last / cus, rest = per_last % cus;  // (`rest` workgroups have full + 1 of them)
+  const int own = full + (cu < rest);
+  int unit, blocks, tile;
+  if (turn < own) {
+    unit = xcd * per_last + turn * cus + cu;
+    if (unit >= all_last) return t;
+    blocks = blocks_last;
+    tile = tiles_first + unit / blocks;
+    unit += tiles_first * blocks;
+  } else {
+    const int late = cu < rest ? as_long : 0, round = turn - own + late;  // while the others were at their longer turn
+    const int mine = rest == 0 || round >= as_long ? (rest == 0 ? round * cus : as_long * (cus - rest) + (round - as_long) * cus) + cu
+                                                   : round * (cus - rest) + cu - rest;
+    unit = xcd * per_first + mine;
+    if (mine >= per_first || unit >= all_first) return t;
+    blocks = blocks_first;
+    tile = unit / blocks;
+  }
+  t.e = p.tiles[4 * tile];
+  const int tile0 = p.tiles[4 * tile + 2], count = p.tiles[4 * tile + 3];
+  if (t.e < 0 || t.e >= p.experts || count <= 0) return t;
+  unit -= tile0 * blocks;  // of this expert's
+  const int group = unit / (kSide * blocks), side = min(kSide, count - group * kSide);
+  unit -= group * kSide * blocks;
+  t.block = unit / side;
+  tile = tile0 + group * kSide + unit - t.block * side;
+  t.s0 = p.tiles[4 * tile + 1];
+  t.s1 = min(min(p.offsets[t.e + 1], t.s0 + TILE), p.slots);
+  const int ff = p.ff[t.e];
+  t.steps = (UP ? p.width : ff) >> 5;
+  t.ntiles = GATED ? ff >> 3 : (UP ? ff : p.width) >> 4;
+  t.any = t.block * kTileW < t.ntiles && t.s0 < t.s1;
+  return t;
 }
+
+// A wave's results by way of 2 KiB of LDS of its own: W tiles nt0 .. of groups of 16 slots, slot0 + m * next ..; 64 outputs of a
+// group at a time, so that a store is a line of a slot's row (8 bytes a lane as the products leave them took 17 000 clocks of a
+// turn's 110 000).
+template <int PRODUCT, int NT, int MT, typename WEIGHT>
+__device__ __forceinline__ void tile_store(const MoeParams& p, int e, const e_f32x4_t (&acc)[NT][MT], char* lds, int nt0, int ntiles,
+                                           int slot0, int next, int s1, WEIGHT weight) {
+  constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
+  [[maybe_unused]] const MoeActivation act(p, GATED ? e : -1);
+  constexpr int kPart = GATED && NT > 4 ? 8 : 4, kOuts = kPart * (GATED ? 8 : 16), kChunks = kOuts / 8;  // of 8 outputs
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int64_t out_ld = UP ? p.ff_max : p.width;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int slot = slot0 + m * next;
+    if (slot >= s1) break;
+    const float f = UP ? weight(slot + c) : 1.f;
+#pragma unroll
+    for (int n0 = 0; n0 < NT; n0 += kPart) {
+#pragma unroll
+      for (int n = n0; n < n0 + kPart; n += GATED ? 2 : 1) {
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if constexpr (GATED) v[r] = act.rounded(acc[n][m][r] * f, acc[n + 1][m][r] * f);
+          else v[r] = UP ? relu_squared_of(acc[n][m][r] * f) : acc[n][m][r];
+        }
+        const int chunk = (GATED ? n - n0 : 2 * (n - n0)) + (g >> 1);
+        store4<BF16>(reinterpret_cast<uint16_t*>(lds + c * (kOuts * 2) + ((chunk ^ c) & (kChunks - 1)) * 16 + (g & 1) * 8), v);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the wave's own next reads see it)
+      const int first = (nt0 + n0) * (GATED ? 8 : 16), outs = (ntiles - nt0 - n0) * (GATED ? 8 : 16);
+#pragma unroll
+      for (int j = 0; j < kChunks / 4; ++j) {
+        const int r = j * (64 / kChunks) + lane / kChunks, q = lane % kChunks;
+        const e_u32x4_t v = *reinterpret_cast<const e_u32x4_t*>(lds + r * (kOuts * 2) + ((q ^ r) & (kChunks - 1)) * 16);
+        if (slot + r < s1 && q * 8 < outs)
+          *reinterpret_cast<e_u32x4_t*>((uint16_t*)p.out + (slot + r) * out_ld + first + q * 8) = v;
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read before it is written again)
+    }
+  }
+}
+
+// 16 (4) bytes a lane to consecutive LDS; base: the same in all lanes
+#define LV_TO_LDS(NAME, BYTES)                                                                                        \
+  __device__ __forceinline__ void NAME(const char* base, uint32_t offset, void* dst) {                               \
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + offset),                 \
+                                     (__attribute__((address_space(3))) void*)dst, BYTES, 0, 0);                     \
+  }
+LV_TO_LDS(to_lds16, 16)
+LV_TO_LDS(to_lds4, 4)
+#undef LV_TO_LDS
+
+// Few slots an expert, behind more than kMoeFewRows rows: bound by the weights' bytes.  256 W rows x 64 slots a workgroup of 8
+// waves, a wave 128 x 16, one workgroup a CU for up to 64 turns.  Both operands come by way of LDS, a ring of six k-steps of
+// 32 of which four are on their way (80 KiB a CU: 2 us of what HBM gives it), and the first steps of a turn are on their way
+// while the turn before stores: no turn waits for memory by itself, as the shared expert's tiles behind all others did.  A
+// step's fragments are read while the step before multiplies.  All turns are looked up at the start, a lane each.
+// 2048 wide, up + down in us, moe_tile_kernel first: 32 experts of 1408, 2 of them and 2816 shared, 80 rows 137, 119, 300 rows
+// 136, 122; 64 experts of 1408, 6 and 2816 shared, 128 rows 238, 227, 512 rows 253, 250; from 45 slots an expert on slower.
+constexpr int kRingSlots = kMoeRingTile, kRingStages = 6, kRingCopies = 3, kTurns = 64;
+struct alignas(16) Turn {
+  int64_t w;                // bytes to the block's first W tile
+  int s0, s1, steps, left;  // slots s0 .. s1 - 1, k-steps, W tiles from the first one on
+  int block, e;
+};
+constexpr int kRingStep = 16 * 1024 + kRingSlots * 64;       // 1 KiB fragments of W, then of slots
+constexpr int kRingResults = kRingStages * kRingStep;        // 2 KiB a wave
+constexpr int kRingTokens = kRingResults + 8 * 2048;         // its 16 slots' rows, 256 bytes a wave
+constexpr int kRingWeights = kRingTokens + 8 * 256;          // weights of the slots of this turn and of the next one
+constexpr int kRingTable = kRingWeights + 2 * kRingSlots * 4;
+constexpr int kRingLds = kRingTable + kTurns * (int)sizeof(Turn) + 16;
+static_assert(kRingLds <= 160 * 1024, "a CU's LDS");
+
+// Reads of LDS beside copies to it: in one block with their wait (behind an ordinary read the compiler waits for all copies).
+__device__ __forceinline__ uint32_t lds_at(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
+}
+__device__ __forceinline__ uint32_t lds_word(const void* p) {
+  uint32_t v;
+  asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(lds_at(p)) : "memory");
+  return v;
+}
+
+template <int PRODUCT>
+__global__ __launch_bounds__(512, 2) void moe_ring_kernel(const MoeParams p, const int blocks_first, const int blocks_last) {
+  constexpr bool UP = PRODUCT != kMoeDown;
+  constexpr int S = kRingStages;
+  extern __shared__ __attribute__((aligned(16))) char ring[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, c = lane & 15;
+  Turn* const table = reinterpret_cast<Turn*>(ring + kRingTable);
+  int* const found = reinterpret_cast<int*>(ring + kRingTable + kTurns * sizeof(Turn));
+  if (wave == 0) {
+    const TileWork t = tile_work<PRODUCT, kRingSlots>(p, blocks_first, blocks_last, lane);
+    const uint64_t any = __ballot(t.any);
+    if (t.any)
+      table[__popcll(any & ((1ull << lane) - 1))] =
+          Turn{(p.w_offset[t.e] + (int64_t)t.block * kTileW * t.steps * 512) * 2, t.s0, t.s1, t.steps,
+               t.ntiles - t.block * kTileW, t.block, t.e};
+    if (lane == 0) *found = __popcll(any);
+  }
+  __syncthreads();
+  const int turns = __builtin_amdgcn_readfirstlane(*found);
+  if (turns == 0) return;
+  const int64_t ld = (int64_t)(UP ? p.width : p.ff_max) * 2;
+  const int wm = wave & 1, wn = wave >> 1, group = wave & 3;  // (two waves copy a group of slots alike)
+
+  struct Work {           // the same in all lanes, but for x
+    const char *w0, *w1;  // this wave's W tiles of a step
+    int s0, s1, steps, left, block, e;
+    const char* x;        // the lane's piece of a step's slots
+  };
+  auto turn_at = [&](int i) __attribute__((always_inline)) {
+    e_u32x4_t u, v;
+    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:16\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(u), "=&v"(v) : "v"(lds_at(table + i)) : "memory");
+    auto one = [](uint32_t z) { return (int)__builtin_amdgcn_readfirstlane((int)z); };
+    Work t;
+    t.s0 = one(u.z), t.s1 = one(u.w), t.steps = one(v.x), t.left = one(v.y), t.block = one(v.z), t.e = one(v.w);
+    const char* w = (const char*)p.w + ((int64_t)one(u.y) << 32 | (uint32_t)one(u.x));
+    t.w0 = w + (int64_t)min(wave * 2, t.left - 1) * t.steps * 1024;
+    t.w1 = w + (int64_t)min(wave * 2 + 1, t.left - 1) * t.steps * 1024;
+    return t;
+  };
+  char* const tokens = ring + kRingTokens + wave * 256;
+  auto ask = [&](const Work& t, int i) __attribute__((always_inline)) {  // older than the copies after it: there once they are
+    if constexpr (UP) {
+      to_lds4((const char*)p.token, (uint32_t)min(t.s0 + group * 16 + c, t.s1 - 1) * 4, tokens);
+      if (p.slot_weight != nullptr && wave == 0)
+        to_lds4((const char*)p.slot_weight, (uint32_t)min(t.s0 + lane, t.s1 - 1) * 4, ring + kRingWeights + (i & 1) * kRingSlots * 4);
+    }
+  };
+  auto take = [&](Work& t) __attribute__((always_inline)) {
+    const int64_t row = UP ? min(max((int)lds_word(tokens + (lane >> 2) * 4), 0), p.rows - 1)
+                           : min(t.s0 + group * 16 + (lane >> 2), t.s1 - 1);
+    t.x = (const char*)p.x + row * ld + ((lane & 3) ^ ((lane >> 4) & 2)) * 16;  // (chunks trade places against bank conflicts)
+  };
+  const uint32_t lane16 = lane * 16;
+  const char* const wread = ring + wm * 8192 + lane * 16;
+  const char* const xread = ring + 16 * 1024 + wn * 1024 + c * 64 + ((g ^ ((c >> 2) & 2)) * 16);
+  auto arrive = [&]() __attribute__((always_inline)) {
+    // loads retire in order: with only the youngest three steps' outstanding, the next one's have landed ...
+    __builtin_amdgcn_s_waitcnt((S - 3) * kRingCopies | (7 << 4) | (15 << 8));
+    asm volatile("s_barrier" ::: "memory");  // ... for every wave; and everyone has read the stage that is filled next
+  };
+  e_f32x4_t acc[8][1];
+  e_u32x4_t a[2][8], x[2];
+  auto read = [&](int stage, int i, int par) __attribute__((always_inline)) {
+    if (i < 8) a[par][i] = *reinterpret_cast<const e_u32x4_t*>(wread + stage + i * 1024);
+    else x[par] = *reinterpret_cast<const e_u32x4_t*>(xread + stage);
+  };
+
+  Work now = turn_at(0), next;
+  ask(now, 0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  take(now);
+  auto copy = [&](int k, int stage, int j) __attribute__((always_inline)) {  // behind the last step: of the next turn's
+    const bool over = k >= now.steps;
+    if (over) k = min(k - now.steps, next.steps - 1);
+    if (j < 2) to_lds16((over ? j ? next.w1 : next.w0 : j ? now.w1 : now.w0) + k * 1024, lane16, ring + stage + (wave * 2 + j) * 1024);
+    else to_lds16((over ? next.x : now.x) + k * 64, 0, ring + stage + (16 + group) * 1024);
+  };
+  next = now;
+  auto after = [&](int stage) __attribute__((always_inline)) { return stage == (S - 1) * kRingStep ? 0 : stage + kRingStep; };
+  auto before = [&](int stage) __attribute__((always_inline)) { return stage == 0 ? (S - 1) * kRingStep : stage - kRingStep; };
+  int stage = 0;      // of the current step
+  bool alone = true;  // no turn before has copied this one's first steps, or not all of them
+  for (int i = 0;; ++i) {
+    if (alone || now.steps < S) {
+      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+      int to = stage;
+#pragma unroll
+      for (int k = 0; k < S - 1; ++k, to = after(to))
+#pragma unroll
+        for (int j = 0; j < kRingCopies; ++j) copy(k, to, j);
+    }
+    alone = now.steps < S;
+    const bool more = i + 1 < turns;
+    auto step = [&](int k, int par) __attribute__((always_inline)) {
+      arrive();
+      const int ahead = after(stage), fill = before(stage);
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        if ((n & 1) == 0 && n / 2 < kRingCopies) copy(k + S - 1, fill, n / 2);
+        read(ahead, n == 0 ? 8 : n, par ^ 1);
+        acc[n][0] = moe_mfma(a[par][n], x[par], acc[n][0]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      read(ahead, 0, par ^ 1);
+      stage = ahead;
+    };
+    int k = 0;
+    auto run_to = [&](int end) __attribute__((always_inline)) {
+      for (; k + 2 <= end; k += 2) {
+        step(k, 0);
+        step(k + 1, 1);
+      }
+    };
+#pragma unroll
+    for (int n = 0; n < 8; ++n) acc[n][0] = e_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    arrive();
+#pragma unroll
+    for (int j = 0; j < 9; ++j) read(stage, j, 0);
+    if (more) {
+      next = turn_at(i + 1);
+      ask(next, i + 1);
+      run_to(min(2 * S, now.steps - S));
+      if (k < S) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      take(next);
+    } else {  // (none: this one's first steps again, and nobody reads them)
+      next = now;
+    }
+    run_to(now.steps);
+    if (k < now.steps) step(k, 0);
+    tile_store<PRODUCT, 8, 1>(p, now.e, acc, ring + kRingResults + wave * 2048, now.block * kTileW + wm * 8,
+                              now.block * kTileW + now.left, now.s0 + wn * 16, 0, now.s1, [&](int slot) {
+      return p.slot_weight == nullptr ? 1.f
+                                      : __builtin_bit_cast(float, lds_word(ring + kRingWeights + ((i & 1) * kRingSlots + slot - now.s0) * 4));
+    });
+    if (!more) break;
+    now = next;
+  }
+  __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // (no copy to LDS outlives the workgroup)
+}
+
+// More slots an expert: 256 W rows x 128 slots a workgroup, a wave 64 x 128, two workgroups a CU, a turn each.  W goes straight to
+// the operand registers of the one wave that uses it.  The chip's power bounds it with many slots: 1.6 GHz at half of the MFMA
+// cycles, where the library's plain product of 49152 x 2816 x 2048 runs at 1.06 to 1.27 PFLOP/s and this one (8192 rows, 6 of 64
+// experts) at 0.98, 0.88 before results went by way of LDS; 256 slots a workgroup, both operands through LDS, 0.96.  Slots' chunks
+// trade places by bit 3 of the slot: LDS reads 16 bytes for lanes 0-3, 12-15, 20-27 at a time (by bits 2 and 3, half of its
+// cycles were conflicts).
+constexpr int kStages = 4, kStageBytes = kMoeTile * 64;  // of 32 of K: 16-slot groups of 1 KiB
 
 template <int PRODUCT>
 __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, const int blocks_first, const int blocks_last) {
   constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
   __shared__ __attribute__((aligned(16))) char ring[kStages][kStageBytes];
-  // the tiles of all experts but the last one, then the last one's (the shared expert may be larger): an eighth of each to
-  // every XCD
-  const int tiles_first = p.tiles[4 * p.max_tiles], tiles_all = p.tiles[4 * p.max_tiles + 1];
-  const int xcd = blockIdx.x & 7, turn = blockIdx.x >> 3;
-  const int all_first = tiles_first * blocks_first, all_last = (tiles_all - tiles_first) * blocks_last;
-  const int per_first = (all_first + 7) / 8, per_last = (all_last + 7) / 8;
-  int unit, blocks, tile;
-  if (turn < per_first) {
-    unit = xcd * per_first + turn;
-    if (unit >= all_first) return;
-    blocks = blocks_first;
-    tile = unit / blocks;
-  } else {
-    unit = xcd * per_last + turn - per_first;
-    if (turn - per_first >= per_last || unit >= all_last) return;
-    blocks = blocks_last;
-    tile = tiles_first + unit / blocks;
-    unit += tiles_first * blocks;
-  }
-  constexpr int kSide = 8;
-  const int e = p.tiles[4 * tile], tile0 = p.tiles[4 * tile + 2], count = p.tiles[4 * tile + 3];
-  if (e < 0 || e >= p.experts || count <= 0) return;
-  unit -= tile0 * blocks;  // of this expert's
-  const int group = unit / (kSide * blocks), side = min(kSide, count - group * kSide);
-  unit -= group * kSide * blocks;
-  const int block = unit / side;
-  tile = tile0 + group * kSide + unit - block * side;
-  const int s0 = p.tiles[4 * tile + 1], s1 = min(min(p.offsets[e + 1], s0 + kMoeTile), p.slots);
-  const int ff = p.ff[e], steps = (UP ? p.width : ff) >> 5;
-  const int ntiles = GATED ? ff >> 3 : (UP ? ff : p.width) >> 4;  // of 16 W rows
-  if (block * kTileW >= ntiles || s0 >= s1) return;
+  const TileWork t = tile_work<PRODUCT, kMoeTile>(p, blocks_first, blocks_last, 0);
+  if (!t.any) return;
+  const int e = t.e, s0 = t.s0, s1 = t.s1, block = t.block, steps = t.steps, ntiles = t.ntiles;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
@@ -186,18 +440,18 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, con
   for (int j = 0; j < 2; ++j) {
     const int slot = min(s0 + (wave * 2 + j) * 16 + (lane >> 2), s1 - 1);
     const int64_t row = UP ? min(max(p.token[slot], 0), p.rows - 1) : slot;
-    xsrc[j] = (const uint16_t*)p.x + row * ld + ((lane & 3) ^ (lane >> 4)) * 8;
+    xsrc[j] = (const uint16_t*)p.x + row * ld + ((lane & 3) ^ ((lane >> 4) & 2)) * 8;
   }
   e_u32x4_t a[kStages][4];
   auto issue = [&](int k, int stage) __attribute__((always_inline)) {  // (past the end: the last step once more)
     k = min(k, steps - 1);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) to_lds(xsrc[j] + k * 32, ring[stage] + (wave * 2 + j) * 1024);
+    for (int j = 0; j < 2; ++j) to_lds16((const char*)(xsrc[j] + k * 32), 0, ring[stage] + (wave * 2 + j) * 1024);
 #pragma unroll
     for (int j = 0; j < 4; ++j) a[stage][j] = *reinterpret_cast<const e_u32x4_t*>(wsrc[j] + k * 512);
   };
   constexpr int MT = kMoeTile / 16;
-  const int xoff = c * 64 + ((g ^ (c >> 2)) * 16);
+  const int xoff = c * 64 + ((g ^ ((c >> 2) & 2)) * 16);
   e_f32x4_t acc[4][MT];
 #pragma unroll
   for (int n = 0; n < 4; ++n)
@@ -230,28 +484,9 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, con
   if (k < steps) step(k, 0);
   if (k + 1 < steps) step(k + 1, 1);
   if (k + 2 < steps) step(k + 2, 2);
-  __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // (no copy to LDS outlives the workgroup)
-  [[maybe_unused]] const MoeActivation act(p, GATED ? e : -1);
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int slot = s0 + 16 * m + c;
-    if (slot >= s1) continue;
-    const float f = UP ? slot_weight_of(p, slot) : 1.f;
-#pragma unroll
-    for (int n = 0; n < 4; n += GATED ? 2 : 1) {
-      if (nt0 + n >= ntiles) continue;
-      float v[4];
-      if constexpr (GATED) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = act(acc[n][m][r] * f, acc[n + 1][m][r] * f);
-        store4<BF16>((uint16_t*)p.out + (int64_t)slot * p.ff_max + (nt0 + n) * 8 + 4 * g, v);
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = UP ? relu_squared_of(acc[n][m][r] * f) : acc[n][m][r];
-        store4<BF16>((uint16_t*)p.out + (int64_t)slot * (UP ? p.ff_max : p.width) + (nt0 + n) * 16 + 4 * g, v);
-      }
-    }
-  }
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // (no copy to LDS is under way, and everyone has read the last stage)
+  tile_store<PRODUCT, 4, MT>(p, e, acc, ring[wave], block * kTileW + wave * 4, ntiles, s0, 16, s1,
+                             [&](int slot) { return slot_weight_of(p, min(slot, s1 - 1)); });
 }
 
 // The router's logits on packed weights (experts and the shared gate, up to a multiple of 16 rows): 16 rows of h and a share
@@ -417,9 +652,18 @@ static void go(const MoeParams& p, hipStream_t s) {
   } else {
     auto blocks = [&](int ff) { return ((GATED ? ff / 8 : (UP ? ff : p.width) / 16) + kTileW - 1) / kTileW; };
     const int first = blocks(p.ff_first), last = blocks(p.ff_last);
-    const int64_t last_tiles = (p.rows + kMoeTile - 1) / kMoeTile;  // a token takes an expert once
-    const int64_t wgs = 8 * (((int64_t)p.max_tiles * first + 7) / 8 + (last_tiles * last + 7) / 8);
-    hipLaunchKernelGGL((moe_tile_kernel<PRODUCT>), dim3((unsigned)wgs), dim3(256), 0, s, p, first, last);
+    const int tile = moe_tile(true, p.rows, p.slots, p.experts);
+    const int64_t tiles = std::min<int64_t>(p.max_tiles, p.slots / tile + p.experts);
+    const int64_t last_tiles = (p.rows + tile - 1) / tile;  // a token takes an expert once
+    const int64_t wgs = 8 * ((tiles * first + 7) / 8 + (last_tiles * last + 7) / 8);
+    // of the ring: a workgroup a CU, more only where one would have over 64 turns
+    const unsigned grid = (unsigned)std::min(wgs, std::max<int64_t>(256, (wgs / (kTurns - 2) + 8) / 8 * 8));
+    if (tile == kRingSlots) {
+      (void)hipFuncSetAttribute((const void*)moe_ring_kernel<PRODUCT>, hipFuncAttributeMaxDynamicSharedMemorySize, kRingLds);
+      hipLaunchKernelGGL((moe_ring_kernel<PRODUCT>), dim3(grid), dim3(512), kRingLds, s, p, first, last);
+    } else {
+      hipLaunchKernelGGL((moe_tile_kernel<PRODUCT>), dim3((unsigned)wgs), dim3(256), 0, s, p, first, last);
+    }
   }
 }
 
