@@ -752,6 +752,11 @@ int lvllm_pair_embed(float* x, void* h, const void* table, const void* pairs, co
                      int rows, int vocab, int width, int dtype, void* stream);
 /* out[r, i] = g * sigmoid(1.702 g) * (u + 1), g = min(in[r, i], limit), u = clamp(in[r, d + i], -limit, limit) */
 int lvllm_clamped_unit(void* out, const void* in, int64_t rows, int d, float limit, int dtype, void* stream);
+/* `products` decode projections of one size in one launch, y[p] = x[p] . w[p]^T: x [products, M, K], w_packed and y [products] back
+ * to back, N outputs each, N_last <= N of the last one; bit-identical to lvllm_skinny_gemm of each.  Returns 3 outside the
+ * kernel's envelope: M > 64, K over 4096 (M <= 32) or 2048, fp32 */
+int lvllm_skinny_gemm_products(void* y, const void* x, const void* w_packed, int products, int M, int N, int N_last, int K, int dtype,
+                               void* stream);
 /* ... of a decode projection's result, in its epilogue: w [gate rows | up rows] (N rows, packed or not), y [M, N / 2], gate and up
  * rounded to T first.  The envelope of lvllm_skinny_gemm, N a multiple of 32 */
 int lvllm_skinny_gemm_clamped_unit(void* y, const void* x, const void* w, int M, int N, int K, int64_t ldx, int dtype,

@@ -97,16 +97,24 @@ constexpr unsigned kOutOfRange = 0xfffffff0u;  // >= any descriptor size: load r
 // W8A8 launch used to re-quantise all of X (1 280 vector instructions per wave at K = 4 096: 13 us for a projection
 // whose 25 MB of weights stream in 5), profiles/r03_tuning.md section 5.
 // y8 / y8_scale (SwiGLU epilogue): the activation leaves as fp8 for the down projection (and as T when y != null).
-template <typename T, int MT, int KSTEPS, bool PACKED, int NT, bool W8, bool XQ = false>
+// PRODUCTS: gridDim.z products of rows of their own, the last one with N_last outputs, operands and results back to back.
+template <typename T, int MT, int KSTEPS, bool PACKED, int NT, bool W8, bool XQ = false, bool PRODUCTS = false>
 __global__ __launch_bounds__(kGemmWaves * 64, 2) void skinny_gemm_kernel(
     typename T::store_t* __restrict__ y,   // [M, N]            (ksplit == 1)
     float* __restrict__ partial,           // [ksplit, M, N]    (ksplit > 1)
     const typename T::store_t* __restrict__ x, const typename T::store_t* __restrict__ w,
-    const typename T::store_t* __restrict__ bias, const int M, const int N, const int K,
-    const int64_t ldx, const int steps_per_wave, const int ntiles, const int act, const int stage_tiles,
+    const typename T::store_t* __restrict__ bias, const int M, const int N_each, const int K,
+    const int64_t ldx, const int steps_per_wave, const int ntiles_each, const int act, const int stage_tiles,
     const float* __restrict__ x_scale, const float* __restrict__ w_scale, uint8_t* __restrict__ y8 = nullptr,
-    const float* __restrict__ y8_scale = nullptr, const float limit = 0.f) {
+    const float* __restrict__ y8_scale = nullptr, const float limit = 0.f, const int N_last = 0) {
   using S = typename T::store_t;
+  const bool last = PRODUCTS && blockIdx.z + 1 == gridDim.z;
+  const int N = last ? N_last : N_each, ntiles = last ? N_last >> 4 : ntiles_each;
+  if constexpr (PRODUCTS) {
+    x += (int64_t)blockIdx.z * M * ldx;
+    w += (int64_t)blockIdx.z * N_each * K;
+    y += (int64_t)blockIdx.z * M * N_each;
+  }
   static_assert(!XQ || (W8 && KSTEPS == 8 && MT <= 2), "pre-quantised activations: the W8A8 variants of <= 32 rows");
   LVLLM_TRACE_BEGIN();
   GEMM_TRACE(0);
@@ -827,12 +835,12 @@ __global__ void skinny_gemm_reduce_argmax_kernel(float* __restrict__ cand, const
   }
 }
 
-template <typename T, int MT, int KSTEPS, bool W8 = false, bool XQ = false>
+template <typename T, int MT, int KSTEPS, bool W8 = false, bool XQ = false, bool PRODUCTS = false>
 static void launch_skinny(void* y, float* partial, const void* x, const void* w, const void* bias, int M,
                           int N, int K, int64_t ldx, int steps_per_wave, int ntiles, int groups, int ksplit,
                           bool packed, int act, hipStream_t stream, const float* x_scale = nullptr,
                           const float* w_scale = nullptr, uint8_t* y8 = nullptr, const float* y8_scale = nullptr,
-                          float limit = 0.f) {
+                          float limit = 0.f, int products = 1, int n_last = 0) {
   using S = typename T::store_t;
   constexpr int NT = LVLLM_GEMM_NT / MT > 0 ? LVLLM_GEMM_NT / MT : 1;  // NT * MT slabs per meeting
   const size_t red_bytes = (size_t)2 * kGemmWaves * NT * MT * 64 * sizeof(g_f32x4_t);
@@ -851,11 +859,13 @@ static void launch_skinny(void* y, float* partial, const void* x, const void* w,
   auto go = [&](auto kern) {
     if (smem > 64 * 1024)
       (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    hipLaunchKernelGGL(kern, dim3(groups, ksplit), dim3(kGemmWaves * 64), smem, stream, (S*)y, partial,
+    hipLaunchKernelGGL(kern, dim3(groups, ksplit, products), dim3(kGemmWaves * 64), smem, stream, (S*)y, partial,
                        (const S*)x, (const S*)w, (const S*)bias, M, N, K, ldx, steps_per_wave, ntiles, act,
-                       stage_tiles, x_scale, w_scale, y8, y8_scale, limit);
+                       stage_tiles, x_scale, w_scale, y8, y8_scale, limit, n_last);
   };
-  if constexpr (W8 && XQ) {
+  if constexpr (PRODUCTS) {
+    go(skinny_gemm_kernel<T, MT, KSTEPS, true, NT, false, false, true>);
+  } else if constexpr (W8 && XQ) {
     go(skinny_gemm_kernel<T, MT, KSTEPS, true, NT, true, true>);
   } else if constexpr (W8) {
     go(skinny_gemm_kernel<T, MT, KSTEPS, true, NT, true>);  // fp8 weights are always packed
@@ -1261,6 +1271,41 @@ extern "C" int lvllm_skinny_gemm_ex(void* y, const void* x, const void* w, const
   LV_CHECK(act != 6, "the clamped unit has an entry of its own");
   return skinny_gemm(y, x, w, bias, M, N, K, ldx, dtype, packed, act, 0.f, partial_out, ksplit_out, workspace, workspace_bytes,
                      stream);
+}
+
+// `products` of M rows each: y[p] = x[p] . w[p]^T, x [products, M, K], w and y back to back, N outputs each and N_last of the last
+// one.  One launch where `products` of them were (a launch of a few MB of weights inside a captured step is 7 us, 4.5 of them
+// its start: four of 2048 x 2048 and one of 64 x 2048 for 24 rows 33 us, together 13); bit-identical to them.
+extern "C" int lvllm_skinny_gemm_products(void* y, const void* x, const void* w_packed, int products, int M, int N, int N_last,
+                                          int K, int dtype, void* stream) {
+  if (M <= 0 || products <= 0) return 0;
+  const int steps_per_wave = (K / 32 + kGemmWaves - 1) / kGemmWaves;
+  if (!(dtype == LVLLM_BF16 || dtype == LVLLM_F16) || M > 64 || K % 32 != 0 || N <= 0 || N % 16 != 0 || N_last <= 0 || N_last % 16 != 0 ||
+      N_last > N || products > 64 || steps_per_wave > max_steps_per_wave(M) || (int64_t)N * K * 2 >= ((int64_t)1 << 32) - 16 ||
+      ((((uintptr_t)x | (uintptr_t)w_packed | (uintptr_t)y) & 15) != 0)) {
+    set_error("lvllm_skinny_gemm_products: shape outside the kernel's envelope");
+    return 3;
+  }
+  const int ntiles = N / 16, groups = balanced_groups(ntiles, tuning().gemm_workgroups / products);
+  hipStream_t s = (hipStream_t)stream;
+  const bool k8 = steps_per_wave <= 8;
+#define LV_SP_GO(T_, MT_, KS_)                                                                                              \
+  launch_skinny<T_, MT_, KS_, false, false, true>(y, nullptr, x, w_packed, nullptr, M, N, K, K, steps_per_wave, ntiles, groups, 1, true, 0, s, nullptr, \
+                              nullptr, nullptr, nullptr, 0.f, products, N_last)
+#define LV_SP(T_)                                  \
+  do {                                             \
+    if (M > 32) LV_SP_GO(T_, 4, 8);                \
+    else if (M > 16 && k8) LV_SP_GO(T_, 2, 8);     \
+    else if (M > 16) LV_SP_GO(T_, 2, 16);          \
+    else if (k8) LV_SP_GO(T_, 1, 8);               \
+    else LV_SP_GO(T_, 1, 16);                      \
+  } while (0)
+  if (dtype == LVLLM_BF16) LV_SP(BF16);
+  else LV_SP(F16);
+#undef LV_SP
+#undef LV_SP_GO
+  LV_LAUNCH_CHECK();
+  return 0;
 }
 
 extern "C" int lvllm_skinny_gemm_clamped_unit(void* y, const void* x, const void* w, int M, int N, int K, int64_t ldx, int dtype,

@@ -160,6 +160,23 @@ torch::Tensor skinny_linear_packed(const torch::Tensor& x, const torch::Tensor& 
   return y;
 }
 
+// Projections of rows of their own in one launch: x [P, M, K], the first P - 1 with N outputs (-> [P - 1, M, N]), the last one with
+// n_last (-> [M, n_last]); w_packed: theirs back to back.  Bit-identical to skinny_linear_packed of each.
+std::tuple<torch::Tensor, torch::Tensor> skinny_linear_packed_products(const torch::Tensor& x, const torch::Tensor& w_packed, int64_t N,
+                                                                       int64_t n_last) {
+  const char* op = "skinny_linear_packed_products";
+  TORCH_CHECK(x.dim() == 3 && x.is_contiguous() && x.size(0) > 1 && N > 0 && n_last > 0 &&
+                  w_packed.numel() == ((x.size(0) - 1) * N + n_last) * x.size(2), op, ": bad shapes");
+  TORCH_CHECK(skinny_ok(x[0], w_packed, std::nullopt), op, ": M <= 64 rows of bf16/f16 on the GPU only");
+  const int64_t P = x.size(0), M = x.size(1);
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(x));
+  auto y = torch::empty({M * ((P - 1) * N + n_last)}, x.options());
+  const int64_t first = (P - 1) * M * N;
+  check(lvllm_skinny_gemm_products(y.data_ptr(), x.data_ptr(), w_packed.data_ptr(), (int)P, (int)M, (int)N, (int)n_last, (int)x.size(2),
+                                   dtype_code(x, op), current_stream(x)));
+  return {y.narrow(0, 0, first).view({P - 1, M, N}), y.narrow(0, first, M * n_last).view({M, n_last})};
+}
+
 // lm_head + greedy sampling: int64 [M] = argmax(x . w^T) over the rounded values, no logits tensor (in the
 // projection's epilogue, or inside its split-K reduce pass when K is split over workgroups at this M).
 torch::Tensor skinny_linear_packed_argmax(const torch::Tensor& x, const torch::Tensor& w_packed, int64_t N, int64_t K) {
@@ -660,6 +677,8 @@ TORCH_LIBRARY_FRAGMENT(_C_amd, amd) {
   amd.impl("skinny_linear", torch::kCUDA, &skinny_linear);
   amd.def("skinny_linear_packed(Tensor x, Tensor w_packed, Tensor? bias, int N, int K) -> Tensor");
   amd.impl("skinny_linear_packed", torch::kCUDA, &skinny_linear_packed);
+  amd.def("skinny_linear_packed_products(Tensor x, Tensor w_packed, int N, int n_last) -> (Tensor, Tensor)");
+  amd.impl("skinny_linear_packed_products", torch::kCUDA, &skinny_linear_packed_products);
   amd.def("pack_weight(Tensor w) -> Tensor");
   amd.impl("pack_weight", torch::kCUDA, &pack_weight);
   amd.def("skinny_linear_packed_argmax(Tensor x, Tensor w_packed, int N, int K) -> Tensor");

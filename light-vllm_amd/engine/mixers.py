@@ -16,6 +16,7 @@ from .model import Weight, linear
 amd = torch.ops._C_amd
 DECAY_LOGSIGMOID, DECAY_NEGEXP = 0, 1
 DECODE_ROWS = 64  # steps of up to this many rows take the weight-streaming GEMMs
+DECODE_PRODUCTS_K = 4096  # several products in one launch: K is not split over workgroups (up to 32 rows; 2048 for more)
 
 
 @dataclass
@@ -179,6 +180,15 @@ class TimeMixer:
         w1 = get(name + ".w1")
         self.rank = w1.shape[0]
         self.w1 = make_weight(stack_rows([w1])[0], pack)
+        # steps of single tokens: all five projections in one launch, their packed weights back to back (the five are views)
+        ws, k = [*self.rkvg, self.w1], self.w1.K
+        self.all_packed = None
+        if all(w.packed is not None for w in ws) and self.w1.N <= self.rkvg[0].N and k <= DECODE_PRODUCTS_K:
+            self.all_packed = torch.cat([w.packed.reshape(-1) for w in ws])
+            at = 0
+            for w in ws:
+                w.packed = self.all_packed[at:at + w.numel()].view_as(w.packed)
+                at += w.numel()
         self.decay = LowRankDecay(get(name + ".w2"), get(name + ".w0"), DECAY_NEGEXP)
         self.recurrence = Recurrence(self.decay, get(name + ".u").float().contiguous(), eps)
         self.norm = get(name + ".norm").float()
@@ -187,11 +197,15 @@ class TimeMixer:
     def __call__(self, x, y, norm: DynTanhNorm, cache: LayerCache, step: StepLayout, attn, dtype):
         x, mix = norm.shift_mix(x, y, self.mu, cache.state["shift"], step, dtype)
         rows = x.shape[0]
-        if 0 < rows <= DECODE_ROWS and self.rkvg[0].packed is not None:
-            r, k, v, g = (linear(mix[i], w) for i, w in enumerate(self.rkvg))
+        if self.all_packed is not None and 0 < rows <= (DECODE_ROWS if self.w1.K <= 2048 else 32):
+            (r, k, v, g), u = amd.skinny_linear_packed_products(mix, self.all_packed, self.rkvg[0].N, self.w1.N)
         else:
-            r, k, v, g = torch.bmm(mix[:4], self.rkvg_t)
-        u = linear(mix[4], self.w1)[:, :self.rank]
+            if 0 < rows <= DECODE_ROWS and self.rkvg[0].packed is not None:
+                r, k, v, g = (linear(mix[i], w) for i, w in enumerate(self.rkvg))
+            else:
+                r, k, v, g = torch.bmm(mix[:4], self.rkvg_t)
+            u = linear(mix[4], self.w1)
+        u = u[:, :self.rank]
         cols = self.cfg.heads * self.cfg.dim
         out = (torch.empty if self.out.K == cols else torch.zeros)(rows, self.out.K, dtype=dtype, device=x.device)
         self.recurrence(out[:, :cols], r, k, v, u, g, self.norm, 1.0, 1.0, cache.state["matrix"], step)

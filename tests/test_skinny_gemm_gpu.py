@@ -370,3 +370,20 @@ def test_qkv_splitk_reduce_inside_the_rope_and_cache_launch_is_bit_identical(ops
     torch.cuda.synchronize()
     assert torch.equal(qkv_a.view(torch.int16), qkv_b.view(torch.int16))
     assert torch.equal(kc_a.view(torch.uint8), kc_b.view(torch.uint8)) and torch.equal(vc_a.view(torch.uint8), vc_b.view(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,n_last,K", [(1, 16, 16, 32), (5, 2048, 64, 2048), (16, 48, 32, 4096), (17, 256, 16, 2080), (32, 1040, 64, 4096),
+                                          (33, 64, 16, 2048), (64, 4096, 64, 1024)])
+def test_products_in_one_launch(dtype, M, N, n_last, K):
+    """Several projections of rows of their own, the last one narrower: each as by itself, bit for bit."""
+    amd = torch.ops._C_amd
+    for products in (2, 5):
+        x = torch.randn(products, M, K, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
+        ws = [(torch.randn(n, K, generator=torch.Generator().manual_seed(2 + i)) * K ** -0.5).to(dtype).cuda()
+              for i, n in enumerate([N] * (products - 1) + [n_last])]
+        packed = [amd.pack_weight(w) for w in ws]
+        first, last = amd.skinny_linear_packed_products(x, torch.cat([p.reshape(-1) for p in packed]), N, n_last)
+        for i, (w, p) in enumerate(zip(ws, packed)):
+            got = last if i == products - 1 else first[i]
+            assert torch.equal(got, amd.skinny_linear_packed(x[i], p, None, w.shape[0], K)), (products, i)
