@@ -150,6 +150,19 @@ struct Vec16 {
   typename T::store_t v[N];
 };
 
+// T(a) in the low half, T(b) in the high one.  bf16 as one conversion of both: two of one each, shifted and combined, are four
+// instructions.
+template <typename T>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  if constexpr (T::kDtype == LVLLM_BF16) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+  } else {
+    return (uint32_t)T::from_float(a) | ((uint32_t)T::from_float(b) << 16);
+  }
+}
+
 // 4 consecutive elements <-> floats (the address is a multiple of 4 elements)
 template <typename T>
 __device__ __forceinline__ void load4(const typename T::store_t* p, float (&v)[4]) {
@@ -168,8 +181,8 @@ __device__ __forceinline__ void store4(typename T::store_t* p, const float (&v)[
     *reinterpret_cast<float4*>(p) = float4{v[0], v[1], v[2], v[3]};
   } else {
     uint2 a;
-    a.x = (uint32_t)T::from_float(v[0]) | ((uint32_t)T::from_float(v[1]) << 16);
-    a.y = (uint32_t)T::from_float(v[2]) | ((uint32_t)T::from_float(v[3]) << 16);
+    a.x = pack2<T>(v[0], v[1]);
+    a.y = pack2<T>(v[2], v[3]);
     *reinterpret_cast<uint2*>(p) = a;
   }
 }

@@ -80,7 +80,7 @@ typedef float h_f32x16_t __attribute__((ext_vector_type(16)));
 typedef unsigned int h_u32x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-  return (uint32_t)BF16::from_float(a) | ((uint32_t)BF16::from_float(b) << 16);
+  return pack2<BF16>(a, b);
 }
 
 // bf16, block size 16, sizes of takes_mfma (head_attention.hip)

@@ -1,7 +1,9 @@
 // The chunk body of head_attention.h: causal attention of prompt portions over the paged cache on 32x32x16 bf16 MFMAs.
 //
 // A workgroup is 4 waves = 128 columns, a column being a (query token, head of the GQA group, map) triple; the waves share one
-// stream of 64-key tiles through LDS (two stages, one barrier per tile, the next tile's global loads in flight meanwhile).
+// stream of 64-key tiles, copied straight to LDS: three stages where two workgroups a CU have room for them, else two, one
+// barrier per tile.  A portion's last columns walk all keys one tile after the other, and that walk is how long the launch
+// takes: pages are looked up 16 tiles at a time, and copies are one or two tiles ahead of their use.
 // With two maps, waves 0 and 1 take the first one, waves 2 and 3 the second one of the same 64 (token, head) pairs: each reads
 // its half of the keys, and the two results meet in LDS at the end.
 //   * S^T = K Q^T: a lane holds 32 keys of ONE column, so the column's maximum is in-lane plus one exchange of halves;
@@ -11,7 +13,11 @@
 //   * probabilities never move between lanes: MFMA row i of S^T holds a permuted key (groups of four 1 and 2 of every 16
 //     trade places), which makes a lane's accumulators the consecutive keys that P V wants as its B operand;
 //   * accumulators are rescaled only when a column's maximum grew;
+//   * with two workgroups a CU the vector instructions of the softmax bound a tile (half of them exponentials), so that the scale
+//     goes into the exponential's argument and the maximum takes three scores at a time;
 //   * tiles of kept first keys come ahead of the window's.
+// One prompt of 4096, us, with tiles through registers and an instruction for each of these, and now: 16 heads over 4, 128 + 64,
+// 134, 107; 32 over 8, 128 + 128, 219, 189; two maps 190, 159.  4 prompts of 2048, 16 heads, 192 + 128 (two stages): 155, 147.
 #pragma once
 #include <float.h>
 
@@ -24,12 +30,26 @@ __device__ __forceinline__ h_f32x16_t mfma32(h_u32x4_t a, h_u32x4_t b, h_f32x16_
                                                  0, 0, 0);
 }
 
+__device__ __forceinline__ void to_lds(const uint16_t* src, char* dst) {  // 16 bytes a lane, 1 KiB a wave
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+// The largest of three; fmaxf takes three instructions of what might be a signalling NaN.  The compiler does not look into this
+// one: where b and c are results of MFMAs, `a` has to come from an instruction behind the same ones, which has waited for them.
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float m;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+  return m;
+}
+
+constexpr int prefill_stages(int nk, int nv) { return 3 * 4 * (nk + nv) <= 80 ? 3 : 2; }
+
 template <int NK, int NV, int MAPS>
 __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kernel(const HeadAttnParams p) {
   constexpr int KP = 32 * NK, VP = 32 * NV, KS = 2 * NK / MAPS;  // KS: k-steps of a column
   constexpr int kPrefillCols = 128 / MAPS;                       // (token, head) pairs of a workgroup
   constexpr int kKBlock = KP * 16 * 2, kVBlock = VP * 16 * 2;  // bytes of a block's head slice
-  constexpr int kImageK = 4 * kKBlock, kStage = kImageK + 4 * kVBlock;
+  constexpr int kImageK = 4 * kKBlock, kStage = kImageK + 4 * kVBlock, S = prefill_stages(NK, NV);
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -67,35 +87,29 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
   const int32_t* table = p.block_tables + (int64_t)seq * p.max_blocks;
   const uint16_t* kc = (const uint16_t*)p.k_cache + (int64_t)kvh * KP * 16;
   const uint16_t* vc = (const uint16_t*)p.v_cache + (int64_t)kvh * VP * 16;
-  h_u32x4_t kreg[NK], vreg[NV];
-  auto fetch = [&](int tile) __attribute__((always_inline)) {
-    int64_t blk[4];
+  int pages = 0, run = -1;  // of 16 tiles, a lane each
+  auto copy = [&](int stage, int tile) __attribute__((always_inline)) {
+    if (tile >> 4 != run) {
+      run = tile >> 4;
+      pages = table[min(run * 64 + lane, p.max_blocks - 1)];
+      __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // (here, and not in front of every use)
+    }
+    char* base = smem + stage * kStage;
+    int blk[4];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) blk[b] = min(max(table[min(tile * 4 + b, p.max_blocks - 1)], 0), p.max_block);
+    for (int b = 0; b < 4; ++b) blk[b] = min(max(__builtin_amdgcn_readlane(pages, (tile & 15) * 4 + b), 0), p.max_block);
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
       const int b = (wave + 4 * j) / NK, w = (wave + 4 * j) - b * NK;  // 64-chunk group w of block b
-      const int64_t bk = b == 0 ? blk[0] : b == 1 ? blk[1] : b == 2 ? blk[2] : blk[3];
-      kreg[j] = *reinterpret_cast<const h_u32x4_t*>(kc + bk * p.k_block_stride + (w * 64 + lane) * 8);
+      const int bk = b == 0 ? blk[0] : b == 1 ? blk[1] : b == 2 ? blk[2] : blk[3];
+      to_lds(kc + (int64_t)bk * p.k_block_stride + (w * 64 + lane) * 8, base + b * kKBlock + w * 1024);
     }
 #pragma unroll
-    for (int j = 0; j < NV; ++j) {
+    for (int j = 0; j < NV; ++j) {  // of a 32-row group: the first tokens' chunks of all rows, then the second ones'
       const int b = (wave + 4 * j) / NV, w = (wave + 4 * j) - b * NV;
-      const int64_t bk = b == 0 ? blk[0] : b == 1 ? blk[1] : b == 2 ? blk[2] : blk[3];
-      vreg[j] = *reinterpret_cast<const h_u32x4_t*>(vc + bk * p.v_block_stride + (w * 64 + lane) * 8);
-    }
-  };
-  auto put = [&](int stage) __attribute__((always_inline)) {
-    char* base = smem + stage * kStage;
-#pragma unroll
-    for (int j = 0; j < NK; ++j) {
-      const int b = (wave + 4 * j) / NK, w = (wave + 4 * j) - b * NK;
-      *reinterpret_cast<h_u32x4_t*>(base + b * kKBlock + (w * 64 + lane) * 16) = kreg[j];
-    }
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {  // chunk `lane` of a 32-row group: row lane >> 1, tokens 8 * (lane & 1) ..
-      const int b = (wave + 4 * j) / NV, w = (wave + 4 * j) - b * NV;
-      *reinterpret_cast<h_u32x4_t*>(base + kImageK + b * kVBlock + (w * 64 + (lane & 1) * 32 + (lane >> 1)) * 16) = vreg[j];
+      const int bk = b == 0 ? blk[0] : b == 1 ? blk[1] : b == 2 ? blk[2] : blk[3];
+      to_lds(vc + (int64_t)bk * p.v_block_stride + (w * 64 + (lane & 31) * 2 + (lane >> 5)) * 8,
+             base + kImageK + b * kVBlock + w * 1024);
     }
   };
 
@@ -110,15 +124,21 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
   const int klds = (lc >> 4) * kKBlock + map * (kKBlock / MAPS) + (hi * 16 + key16) * 16;
   const int vlds = kImageK + lane * 16;  // (hi * 32 + lc) * 16
 
-  fetch(tile_of(0));
-  put(0);
-  __syncthreads();
+  constexpr int kCopies = NK + NV;  // of a wave and tile
+  __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // (the queries are here: what is on its way below are copies)
+#pragma unroll
+  for (int t = 0; t < S - 1; ++t)
+    if (t < ntiles) copy(t, tile_of(t));
+  int stage = 0;
   for (int t = 0; t < ntiles; ++t) {
-    const bool more = t + 1 < ntiles;
-    if (more) fetch(tile_of(t + 1));
+    // loads retire in order: with only the youngest tile's copies outstanding (two stages: none), this one's have landed
+    if (S == 3 && t + 1 < ntiles) __builtin_amdgcn_s_waitcnt(kCopies | (7 << 4) | (15 << 8));
+    else __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+    asm volatile("s_barrier" ::: "memory");  // ... for every wave; and everyone is done with the stage that is filled next
+    if (t + S - 1 < ntiles) copy(stage == 0 ? S - 1 : stage - 1, tile_of(t + S - 1));
     const int k0 = tile_of(t) * 64;
     if (wave_ok && k0 <= wave_last && (k0 + 63 >= wave_low || k0 < p.keep_first)) {
-      const char* base = smem + (t & 1) * kStage;
+      const char* base = smem + stage * kStage;
       h_f32x16_t s[2] = {h_f32x16_t{}, h_f32x16_t{}};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
@@ -127,16 +147,14 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
         s[0] = mfma32(a0, qf[ks], s[0]);
         s[1] = mfma32(a1, qf[ks], s[1]);
       }
-      if (score.cap > 0.f) {
+      // scores are mul * s; with a cap, or a scale that does not keep their order, they are made first
+      float mul = score.mul;
+      if (score.cap > 0.f || !(mul > 0.f)) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) s[h][i] = score.capped(s[h][i]);
-      } else {
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) s[h][i] *= score.mul;
+          for (int i = 0; i < 16; ++i) s[h][i] = score.cap > 0.f ? score.capped(s[h][i]) : s[h][i] * mul;
+        mul = 1.f;
       }
       if (k0 + 63 > wave_first || k0 < wave_all) {  // the diagonal or the window's edge passes through it for some column
 #pragma unroll
@@ -144,13 +162,13 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
             const int key = k0 + 32 * h + 16 * (i >> 3) + 8 * hi + (i & 7);
-            s[h][i] = sees(p, key, pos, low) ? s[h][i] : -FLT_MAX;
+            s[h][i] = sees(p, key, pos, low) ? s[h][i] : -INFINITY;
           }
       }
-      float mx = fmaxf(s[0][0], s[1][0]);
+      float mx = fmaxf(s[0][0], s[1][0]);  // (behind this both products' results are there)
 #pragma unroll
-      for (int i = 1; i < 16; ++i) mx = fmaxf(mx, fmaxf(s[0][i], s[1][i]));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      for (int i = 1; i < 16; ++i) mx = max3(mx, s[0][i], s[1][i]);
+      mx = fmaxf(mx, __shfl_xor(mx, 32)) * mul;
       if (__any(mx > m)) {
         const float mn = fmaxf(m, mx), corr = exp2f(m - mn);
         m = mn;
@@ -163,7 +181,7 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          s[h][i] = __builtin_amdgcn_exp2f(s[h][i] - m);
+          s[h][i] = __builtin_amdgcn_exp2f(fmaf(s[h][i], mul, -m));
           sum += s[h][i];
         }
       l += sum;
@@ -179,9 +197,9 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
         }
       }
     }
-    if (more) put((t + 1) & 1);
-    __syncthreads();
+    stage = stage + 1 == S ? 0 : stage + 1;
   }
+  if constexpr (MAPS == 2) __syncthreads();  // (the stages make room for the second map's results)
   l += __shfl_xor(l, 32);
   l += sink_term(p, head, m);
   float f = 1.f / l;
@@ -239,7 +257,7 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
 
 template <int NK, int NV, int MAPS>
 static void go_prefill(const HeadAttnParams& p, hipStream_t s) {
-  constexpr int smem = 2 * 4 * (NK + NV) * 32 * 16 * 2, kCols = 128 / MAPS;
+  constexpr int smem = prefill_stages(NK, NV) * 4 * (NK + NV) * 32 * 16 * 2, kCols = 128 / MAPS;
   static_assert(MAPS == 1 || 64 * (32 * NV + 4) * 4 <= smem, "the second map's results take the place of the stages");
   if (smem > 64 * 1024)
     (void)hipFuncSetAttribute((const void*)head_prefill_kernel<NK, NV, MAPS>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);

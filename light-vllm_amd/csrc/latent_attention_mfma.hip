@@ -148,8 +148,8 @@ __global__ __launch_bounds__(256 * CT, 1) void latent_attention_mfma_kernel(cons
     l += (s[0] + s[1]) + (s[2] + s[3]);
     {
       uint2 w;
-      w.x = (uint32_t)BF16::from_float(s[0]) | ((uint32_t)BF16::from_float(s[1]) << 16);
-      w.y = (uint32_t)BF16::from_float(s[2]) | ((uint32_t)BF16::from_float(s[3]) << 16);
+      w.x = pack2<BF16>(s[0], s[1]);
+      w.y = pack2<BF16>(s[2], s[3]);
       *reinterpret_cast<uint2*>(&sp[ct][c * PP + 16 * kg + 4 * g]) = w;
     }
     lds_barrier();

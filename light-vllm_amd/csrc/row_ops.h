@@ -27,7 +27,7 @@ __device__ __forceinline__ void store_vec(typename T::store_t* p, const float (&
   if constexpr (VEC == 8) {
     uint32_t w[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) w[j] = (uint32_t)T::from_float(v[2 * j]) | ((uint32_t)T::from_float(v[2 * j + 1]) << 16);
+    for (int j = 0; j < 4; ++j) w[j] = pack2<T>(v[2 * j], v[2 * j + 1]);
     *reinterpret_cast<uint4*>(p) = uint4{w[0], w[1], w[2], w[3]};
   } else if constexpr (VEC == 4) {
     store4<T>(p, v);

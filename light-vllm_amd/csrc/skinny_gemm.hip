@@ -220,8 +220,8 @@ __global__ __launch_bounds__(kGemmWaves * 64, 2) void skinny_gemm_kernel(
           for (int r = 0; r < 4; ++r) sum[r] = relu_squared_of(T::to_float(T::from_float(sum[r])));
         }
         uint2 o;
-        o.x = (uint32_t)T::from_float(sum[0]) | ((uint32_t)T::from_float(sum[1]) << 16);
-        o.y = (uint32_t)T::from_float(sum[2]) | ((uint32_t)T::from_float(sum[3]) << 16);
+        o.x = pack2<T>(sum[0], sum[1]);
+        o.y = pack2<T>(sum[2], sum[3]);
         *reinterpret_cast<uint2*>(y + (int64_t)m * N + n0) = o;
       }
     }
@@ -705,8 +705,8 @@ __global__ void skinny_gemm_reduce_kernel(typename T::store_t* __restrict__ y,
     for (int r = 0; r < 4; ++r) sum[r] = relu_squared_of(T::to_float(T::from_float(sum[r])));
   }
   uint2 o;
-  o.x = (uint32_t)T::from_float(sum[0]) | ((uint32_t)T::from_float(sum[1]) << 16);
-  o.y = (uint32_t)T::from_float(sum[2]) | ((uint32_t)T::from_float(sum[3]) << 16);
+  o.x = pack2<T>(sum[0], sum[1]);
+  o.y = pack2<T>(sum[2], sum[3]);
   *reinterpret_cast<uint2*>(y + i) = o;
 }
 
@@ -1031,8 +1031,8 @@ __global__ __launch_bounds__(kGemmWaves * 64, 1) void stream_gemm_kernel(
               for (int r = 0; r < 4; ++r) sum[r] += T::to_float(bias[n0 + r]);
             }
             uint2 o;
-            o.x = (uint32_t)T::from_float(sum[0]) | ((uint32_t)T::from_float(sum[1]) << 16);
-            o.y = (uint32_t)T::from_float(sum[2]) | ((uint32_t)T::from_float(sum[3]) << 16);
+            o.x = pack2<T>(sum[0], sum[1]);
+            o.y = pack2<T>(sum[2], sum[3]);
             *reinterpret_cast<uint2*>(y + (int64_t)m * N + n0) = o;
           }
         }
