@@ -18,10 +18,28 @@ __device__ __forceinline__ float exp_of(float x) {
   return fmaf(r, lo * 0.693147182f, r);
 }
 
+// ln(1 + e), 0 <= e <= 1: 2 artanh(s), s = e / (2 + e) <= 1/3, by its series up to s^17 (what is left out is below 2e-10 of it);
+// log1pf also looks after arguments that do not come here.
+__device__ __forceinline__ float log1p_of(float e) {
+  const float d = 2.f + e, r = __builtin_amdgcn_rcpf(d);
+  float s = e * r;
+  s = fmaf(fmaf(-s, d, e), r, s);
+  const float w = s * s;
+  float p = 1.f / 17.f;
+  p = fmaf(p, w, 1.f / 15.f);
+  p = fmaf(p, w, 1.f / 13.f);
+  p = fmaf(p, w, 1.f / 11.f);
+  p = fmaf(p, w, 1.f / 9.f);
+  p = fmaf(p, w, 1.f / 7.f);
+  p = fmaf(p, w, 1.f / 5.f);
+  p = fmaf(p, w, 1.f / 3.f);
+  return 2.f * fmaf(s * w, p, s);
+}
+
 // `scale`: 1 / tau, or a softplus decay's factor
 __device__ __forceinline__ float log_decay_of(float z, int kind, float scale) {
   if (kind == kDecayNegExp) return -exp_of(fminf(z, 9.f));  // (exp(-exp(9)) is 0: a finite logarithm keeps sums finite)
-  const float small = log1pf(exp_of(-fabsf(z)));
+  const float small = log1p_of(exp_of(-fabsf(z)));
   return kind == kDecaySoftplus ? -scale * (fmaxf(z, 0.f) + small) : (fminf(z, 0.f) - small) * scale;
 }
 
