@@ -199,6 +199,11 @@ __device__ __forceinline__ float relu_squared_of(float x) {
 __device__ __forceinline__ float sigmoid_16bit(float z) {
   return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
 }
+template <typename T>
+__device__ __forceinline__ float sigmoid_for(float z) {  // of a factor of a result in T
+  if constexpr (sizeof(typename T::store_t) == 2) return sigmoid_16bit(z);
+  else return 1.f / (1.f + expf(-z));
+}
 
 // A sigmoid-gated linear unit whose gate is bounded above and whose value on both sides
 __device__ __forceinline__ float clamped_unit_of(float g, float u, float limit) {
@@ -221,30 +226,48 @@ __device__ __forceinline__ int find_seq(const int32_t* __restrict__ query_start_
 
 // Butterflies over 32, 16, 8, 4, 2, 1 lanes in vector registers (a shuffle goes by way of LDS: 448 clocks a sum, 115 here);
 // every lane gets the result, and sums are
-// bit for bit those of shuffles in that order.  Whole waves only (the swaps read lanes that are switched off).
-template <typename V, typename OP>
-__device__ __forceinline__ V over_wave(V v, OP op) {
-  auto dpp = [&](auto ctrl) __attribute__((always_inline)) {
-    const int i = __builtin_bit_cast(int, v);
-    v = op(v, __builtin_bit_cast(V, __builtin_amdgcn_update_dpp(0, i, decltype(ctrl)::value, 0xf, 0xf, true)));
-  };
-  auto swapped = [&](auto r) __attribute__((always_inline)) {
-    const unsigned a = r[0], b = r[1];
-    v = op(__builtin_bit_cast(V, a), __builtin_bit_cast(V, b));
-  };
-  swapped(__builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false));
-  swapped(__builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false));
-  dpp(std::integral_constant<int, 0x128>());  // i + 8 of 16
-  dpp(std::integral_constant<int, 0x124>());  // i + 4 of 16: every eighth lane holds the same now
-  dpp(std::integral_constant<int, 0x4e>());   // i ^ 2
-  dpp(std::integral_constant<int, 0xb1>());   // i ^ 1
-  return v;
+// bit for bit those of shuffles in that order.  Whole groups of lanes
+// only (the swaps read lanes that are switched off).
+template <int CTRL, typename V>
+__device__ __forceinline__ V dpp_of(V v) {
+  return __builtin_bit_cast(V, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kDppXor1 = 0xb1, kDppXor2 = 0x4e, kDppRor4 = 0x124, kDppRor8 = 0x128, kDppMirror8 = 0x141, kDppMirror16 = 0x140;
+// Rows of 16 lanes: (0, 0, 2, 2) and (1, 1, 3, 3); halves: the lower one twice and the upper one twice
+template <typename V>
+struct LanePair { V a, b; };
+template <typename V>
+__device__ __forceinline__ LanePair<V> rows_apart(V v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return {__builtin_bit_cast(V, (unsigned)r[0]), __builtin_bit_cast(V, (unsigned)r[1])};
+}
+template <typename V>
+__device__ __forceinline__ LanePair<V> halves_apart(V v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return {__builtin_bit_cast(V, (unsigned)r[0]), __builtin_bit_cast(V, (unsigned)r[1])};
+}
+template <int L = 64, typename V, typename OP>
+__device__ __forceinline__ V over_lanes(V v, OP op) {  // over L = 16, 32 or 64 neighbouring lanes
+  if constexpr (L == 64) {
+    const auto h = halves_apart(v);
+    v = op(h.a, h.b);
+  }
+  if constexpr (L >= 32) {
+    const auto r = rows_apart(v);
+    v = op(r.a, r.b);
+  }
+  v = op(v, dpp_of<kDppRor8>(v));
+  v = op(v, dpp_of<kDppRor4>(v));  // (every eighth lane holds the same by now: lane i ^ 4)
+  v = op(v, dpp_of<kDppXor2>(v));
+  return op(v, dpp_of<kDppXor1>(v));
 }
 __device__ inline float wave_sum(float v) {
-  return over_wave(v, [](float a, float b) { return a + b; });
+  return over_lanes(v, [](float a, float b) { return a + b; });
 }
 __device__ inline float wave_max(float v) {
-  return over_wave(v, [](float a, float b) { return fmaxf(a, b); });
+  return over_lanes(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Block-wide sum for blocks of up to 16 waves; `red` is 16 floats of LDS.

@@ -375,7 +375,7 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void delta_prepare_kernel(con
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
     const int tile = wave * NT + i, ch = tile * 16 + c;
-    const ChunkSums cs(lv[i], g, c, false);
+    const ChunkSums cs(lv[i], g, false);
     const bool mild = -cs.h1 < kMaxHalfDecay && -cs.h2 < kMaxHalfDecay;
     wild = wild || !mild;
     const uint64_t fast = __ballot(!mild);

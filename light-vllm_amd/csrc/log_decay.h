@@ -57,10 +57,12 @@ struct ChunkSums {
   float h1, h2;              // the chunk's two halves
   float read[4], left[4];    // chunk's start -> what token t reads; token t -> end
   float half_q[4], half_k[4];  // the middle of the chunk -> what token t reads; token t -> the middle
-  __device__ __forceinline__ ChunkSums(const float (&l)[4], int g, int c, bool has_bonus) {
+  __device__ __forceinline__ ChunkSums(const float (&l)[4], int g, bool has_bonus) {
     const float upto[4] = {l[0], l[0] + l[1], (l[0] + l[1]) + l[2], (l[0] + l[1]) + (l[2] + l[3])};
     const float after[4] = {l[1] + (l[2] + l[3]), l[2] + l[3], l[3], 0.f};
-    const float g0 = __shfl(upto[3], c), g1 = __shfl(upto[3], 16 + c), g2 = __shfl(upto[3], 32 + c), g3 = __shfl(upto[3], 48 + c);
+    const auto half = halves_apart(upto[3]);
+    const auto lower = rows_apart(half.a), upper = rows_apart(half.b);
+    const float g0 = lower.a, g1 = lower.b, g2 = upper.a, g3 = upper.b;
     const float before_g = g == 0 ? 0.f : g == 1 ? g0 : g == 2 ? g0 + g1 : g0 + g1 + g2;
     const float after_g = g == 3 ? 0.f : g == 2 ? g3 : g == 1 ? g2 + g3 : g1 + (g2 + g3);
     const float in_half = g == 0 ? g1 : g == 3 ? g2 : 0.f;  // the group of this half between this one and the middle

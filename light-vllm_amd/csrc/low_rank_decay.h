@@ -6,9 +6,6 @@
 // The error against 64 bits is 0.6 to 0.8 of that of fp32 MFMAs and log1pf.  us, 8192 rows, rank 128, 2048 channels, logsigmoid: 107,
 // now 45; exponentials of tanh: 78, 56; 4096 rows, rank 64: 45, 20 and 28, 26.  Writing the results is 14 of the 45, the rest
 // the logarithms' vector instructions.
-// The error against 64 bits is 0.6 to 0.8 of that of fp32 MFMAs and log1pf.  us, 8192 rows, rank 128, 2048 channels, logsigmoid: 107,
-// now 45; exponentials of tanh: 78, 56; 4096 rows, rank 64: 45, 20 and 28, 26.  Writing the results is 14 of the 45, the rest
-// the logarithms' vector instructions.
 #pragma once
 #include "log_decay.h"
 

@@ -112,7 +112,7 @@ __device__ __forceinline__ void choose_experts(float* z, const MoeRouting& r, in
       const int bits = __builtin_bit_cast(int, v + 0.f);  // (one zero)
       int key = lane < experts ? bits ^ (bits >> 31 & 0x7fffffff) : INT32_MIN;
       for (int k = 0; k < top; ++k) {
-        const int best = over_wave(key, [](int a, int b) { return max(a, b); });
+        const int best = over_lanes(key, [](int a, int b) { return max(a, b); });
         const int at = __ffsll((unsigned long long)__ballot(key == best)) - 1;
         if (lane == at) { place = k; key = INT32_MIN; }
       }

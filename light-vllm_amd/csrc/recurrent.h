@@ -121,6 +121,8 @@ struct Packed {
 // channels [w * 16 * NT, (w + 1) * 16 * NT): it scales q and k there, holds those rows of the state as accumulator tiles and
 // forms partial in-chunk products and read-outs, which meet in LDS.  A lane loads channel c, tokens 4g .. 4g + 3 of a tile:
 // scaled k is then the A operand of the state update as it is; q goes through LDS.
+// A chunk is one chain of dependent steps, so that what crosses lanes goes by way of registers.  4096 rows, 16 heads, us with
+// shuffles and now: 81, 68 (64 channels), 74, 66 (128).
 //   STATES: from a zero state, no read-out: a segment's last state and the product of its decays, of all segments but the
 //   last.  Otherwise the segment's first state comes from the slot (sequences that are not cut) or from chunk_combine_kernel.
 template <typename T, typename QT, int NT, int NV, bool STATES, bool FIXED>
@@ -241,7 +243,7 @@ __global__ __launch_bounds__(256, NT == 1 && NV <= 4 ? 3 : 2) void chunk_mix_ker
         else l[r] = ok ? f.l[i][r] : 0.f;
         kv[r] = ok ? QT::to_float(f.k[i][r]) : 0.f;
       }
-      const ChunkSums cs(l, g, c, has_bonus);
+      const ChunkSums cs(l, g, has_bonus);
       end[i] = exp_of(cs.h1 + cs.h2);
       if constexpr (STATES) {
 #pragma unroll
@@ -286,8 +288,10 @@ __global__ __launch_bounds__(256, NT == 1 && NV <= 4 ? 3 : 2) void chunk_mix_ker
       if (has_bonus) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-#pragma unroll
-          for (int m = 1; m < 16; m <<= 1) diag[r] += __shfl_xor(diag[r], m);
+          diag[r] += dpp_of<kDppXor1>(diag[r]);
+          diag[r] += dpp_of<kDppXor2>(diag[r]);
+          diag[r] += dpp_of<kDppMirror8>(diag[r]);   // (four lanes hold the same by now: lane i ^ 4)
+          diag[r] += dpp_of<kDppMirror16>(diag[r]);  // (... and eight: lane i ^ 8)
           if (c == 0) sdiag[wave * 16 + 4 * g + r] = diag[r];
         }
       }
@@ -399,15 +403,14 @@ __global__ __launch_bounds__(256, NT == 1 && NV <= 4 ? 3 : 2) void chunk_mix_ker
             if (d0 + j < p.dv) p.o[(row * p.heads + head) * p.dv + d0 + j] = o[j];
         continue;
       }
-#pragma unroll
-      for (int m = 8; m >= 1; m >>= 1) ss += __shfl_xor(ss, m);
+      ss = over_lanes<16>(ss, [](float a, float b) { return a + b; });
       const float rms = 1.f / sqrtf(ss / p.dv + p.eps);
       if (et < nt) {
         S* out = (S*)p.out + row * p.out_stride + head * p.dv + d0;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
           const float zg = gate.at(j);
-          o[j] = o[j] * rms * nw[j] * (zg / (1.f + expf(-zg)));
+          o[j] = o[j] * rms * nw[j] * (zg * sigmoid_for<T>(zg));
         }
         if constexpr (NV >= 4) {
           if (p.vec_out && d0 + NV <= p.dv) {

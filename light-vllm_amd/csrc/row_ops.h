@@ -37,9 +37,13 @@ __device__ __forceinline__ void store_vec(typename T::store_t* p, const float (&
 }
 template <int L>
 __device__ __forceinline__ float group_sum(float v) {  // over L neighbouring lanes
+  if constexpr (L >= 16) {
+    return over_lanes<L>(v, [](float a, float b) { return a + b; });
+  } else {
 #pragma unroll
-  for (int m = L / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m);
-  return v;
+    for (int m = L / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m);
+    return v;
+  }
 }
 
 // lanes that cover n elements in one pass of VEC each: 8, 16, 32 or 64
