@@ -679,14 +679,20 @@ inline int value_slices(int dk, int dv) { return (dv + 16 * value_tiles(dk, dv) 
 constexpr int mix_wgs_per_cu(int NT, int NV) { return NT == 1 && NV <= 4 ? 3 : 2; }  // (registers; the LDS holds as many)
 
 // Chunks per segment: sequences are cut when (sequence, head, value slice) triples alone leave CUs idle, into as many
-// segments as run at once
-inline int segment_chunks(int rows, int heads, int dk, int dv, int max_query_len) {
+// segments as run at once.  A chunk is a chain of steps that takes 6 to 14 us and a segment walks its own one after the other, so
+// that short portions are cut down to single chunks: 300 rows, us with at least 8 and now: 8 heads of 128 92, 46, with a
+// fixed decay 83, 38; 32 heads of 64 180, 57.  Not below kLeastChunks, where a chunk less does not pay for the two launches more.
+// Every sequence has a workgroup for each segment of the longest: beyond 16384 of them segments are longer, up to kCoarse.
+constexpr int kCoarse = 8, kLeastChunks = 3;
+inline int segment_chunks(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len, bool coarse) {
   const int chunks = (max_query_len + kChunk - 1) / kChunk;
   const int64_t long_seqs = (rows + max_query_len - 1) / max_query_len;
   const int64_t wide = long_seqs * heads * value_slices(dk, dv);
   const int64_t segs = 256 * mix_wgs_per_cu(key_groups(dk), value_tiles(dk, dv)) / wide;
   const int per = segs < 2 ? chunks : (int)((chunks + segs - 1) / segs);
-  return per < 8 ? 8 : per;
+  const int64_t wgs = (int64_t)chunks * num_seqs * heads * value_slices(dk, dv);
+  const int64_t least = coarse || chunks < kLeastChunks ? kCoarse : (wgs + 16383) / 16384;
+  return per < least ? (int)(least < kCoarse ? least : kCoarse) : per;
 }
 inline int64_t segment_slots(int rows, int num_seqs, int per, int max_query_len) {
   return max_query_len <= per * kChunk ? 0 : (int64_t)rows / (kChunk * per) + num_seqs + 1;
@@ -742,26 +748,26 @@ static int launch_single_tokens(const MixParams& p, int dtype, hipStream_t s) {
   return 0;
 }
 
-// The chunked body's segments; `ws`: their workspace.  Returns the floats taken.
-inline int64_t plan_segments(MixParams& p, float* ws, int rows, int max_query_len) {
-  p.seg_chunks = segment_chunks(rows, p.heads, p.dk, p.dv, max_query_len);
+inline int64_t segments_workspace(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len, bool coarse = false) {  // floats
+  const int per = segment_chunks(rows, num_seqs, heads, dk, dv, max_query_len, coarse);
+  const int64_t segs = segment_slots(rows, num_seqs, per, max_query_len) * heads;
+  const int64_t o = value_slices(dk, dv) > 1 ? (int64_t)rows * heads * dv : 0;
+  return segs * ((int64_t)dk * dv + 64 * key_groups(dk)) + o;
+}
+
+// The chunked body's segments; `ws`: their workspace of `room` bytes.  Short portions need more of it than long ones may: what
+// holds segments of kCoarse chunks, but no shorter ones, is enough as well.  Returns whether it is.
+inline bool plan_segments(MixParams& p, float* ws, int64_t room, int rows, int max_query_len) {
+  auto need = [&](bool coarse) { return 4 * segments_workspace(rows, p.num_seqs, p.heads, p.dk, p.dv, max_query_len, coarse); };
+  const bool coarse = room < need(false);
+  if (coarse && room < need(true)) return false;
+  p.seg_chunks = segment_chunks(rows, p.num_seqs, p.heads, p.dk, p.dv, max_query_len, coarse);
   p.max_segs = (max_query_len + kChunk * p.seg_chunks - 1) / (kChunk * p.seg_chunks);
   const int64_t segs = segment_slots(rows, p.num_seqs, p.seg_chunks, max_query_len) * p.heads;
   p.seg_decay = ws;
   p.seg_state = ws + segs * 64 * key_groups(p.dk);
-  int64_t taken = segs * (64 * key_groups(p.dk) + (int64_t)p.dk * p.dv);
-  if (value_slices(p.dk, p.dv) > 1) {
-    p.o = ws + taken;
-    taken += (int64_t)rows * p.heads * p.dv;
-  }
-  return taken;
-}
-
-inline int64_t segments_workspace(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len) {  // floats
-  const int per = segment_chunks(rows, heads, dk, dv, max_query_len);
-  const int64_t segs = segment_slots(rows, num_seqs, per, max_query_len) * heads;
-  const int64_t o = value_slices(dk, dv) > 1 ? (int64_t)rows * heads * dv : 0;
-  return segs * ((int64_t)dk * dv + 64 * key_groups(dk)) + o;
+  if (value_slices(p.dk, p.dv) > 1) p.o = p.seg_state + segs * p.dk * p.dv;
+  return true;
 }
 
 }  // namespace lvllm

@@ -181,13 +181,10 @@ extern "C" int lvllm_recurrent_mix(void* out, int64_t out_stride, const void* q,
   hipStream_t s = (hipStream_t)stream;
   if (max_query_len <= 1) return launch_single_tokens<false>(p, dtype, s);
   LV_CHECK(dtype == LVLLM_BF16 || dtype == LVLLM_F32, "bfloat16 or float32");
-  LV_CHECK(workspace != nullptr &&
-               workspace_bytes >= lvllm_recurrent_mix_workspace_bytes(rows, num_seqs, heads, dk, dv, max_query_len),
+  const int64_t decays = (int64_t)rows * heads * dk;
+  LV_CHECK(workspace != nullptr && plan_segments(p, (float*)workspace + decays, workspace_bytes - decays * 4, rows, max_query_len),
            "workspace too small (see lvllm_recurrent_mix_workspace_bytes)");
-  float* ws = (float*)workspace;
-  p.log_decay = ws;
-  ws += (int64_t)rows * heads * dk;
-  plan_segments(p, ws, rows, max_query_len);
+  p.log_decay = (float*)workspace;
   LV_CHECK((int64_t)num_seqs * p.max_segs <= 65535, "too many sequences or too long portions");
   const int esize = dtype == LVLLM_F32 ? 4 : 2;
   p.vec_in = ((dv | v_stride | gate_stride) & 3) == 0 && (((uintptr_t)v | (uintptr_t)gate) & (4 * esize - 1)) == 0;

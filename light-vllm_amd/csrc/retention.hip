@@ -66,12 +66,10 @@ extern "C" int lvllm_retention(void* out, int64_t out_stride, const void* q, con
   p.norm_weight = norm_weight; p.norm_head_stride = norm_head_stride; p.eps = eps; p.out_scale = out_scale;
   hipStream_t s = (hipStream_t)stream;
   if (max_query_len <= 1) return launch_single_tokens<true>(p, dtype, s);
-  LV_CHECK(workspace != nullptr &&
-               workspace_bytes >= lvllm_retention_workspace_bytes(rows, num_seqs, heads, dk, dv, max_query_len),
+  float *qr = (float*)workspace, *kr = qr + (int64_t)rows * heads * dk;
+  const int64_t rotated = 2 * (int64_t)rows * heads * dk;
+  LV_CHECK(workspace != nullptr && plan_segments(p, qr + rotated, workspace_bytes - rotated * 4, rows, max_query_len),
            "workspace too small (see lvllm_retention_workspace_bytes)");
-  float* ws = (float*)workspace;
-  float *qr = ws, *kr = ws + (int64_t)rows * heads * dk;
-  plan_segments(p, kr + (int64_t)rows * heads * dk, rows, max_query_len);
   LV_CHECK((int64_t)num_seqs * p.max_segs <= 65535, "too many sequences or too long portions");
   LV_DISPATCH_F32_BF16(dtype, {
     using S = typename scalar_t::store_t;

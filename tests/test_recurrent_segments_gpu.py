@@ -1,0 +1,94 @@
+"""Portions cut into segments of single chunks against the token-by-token recurrence: lengths around the chunks' edges (16 tokens; cut from the
+third chunk on), ragged sequences with and without an earlier state, so many sequences that segments get longer, and workspaces that
+hold only the coarse segments of 8 chunks, or not even these."""
+import ctypes
+import os
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def amd():
+    import light_vllm_amd._custom_ops  # noqa: F401
+    return torch.ops._C_amd
+
+
+def operands(lengths, heads, dk, dv, bonus, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    rows, n, rank = sum(lengths), len(lengths), 24
+    r = lambda *s: torch.randn(*s, generator=g)
+    t = {"q": r(rows, heads * dk), "k": r(rows, heads * dk), "v": r(rows, heads * dv), "u": r(rows, rank), "gate": r(rows, heads * dv)}
+    t = {k: v.bfloat16().to(DEV) for k, v in t.items()}
+    t["a_t"], t["bias"] = (0.3 * r(rank, heads * dk)).to(DEV), r(heads * dk).to(DEV)
+    t["bonus"] = r(heads * dk).to(DEV) if bonus else None
+    t["weight"] = r(heads * dv).to(DEV)
+    t["state"] = r(n + 1, heads, dk, dv).to(DEV)
+    t["slots"] = torch.arange(n, 0, -1, dtype=torch.int32, device=DEV)
+    t["start"] = torch.tensor([0] + lengths).cumsum(0).int().to(DEV)
+    t["lens"] = torch.tensor([m + (7 if i % 2 else 0) for i, m in enumerate(lengths)], dtype=torch.int32, device=DEV)  # odd ones go on
+    return t
+
+
+def reference(amd, t, kind, inv_tau, scale):
+    state = t["state"].clone()
+    decay = amd.log_decay(t["u"], t["a_t"], t["bias"], kind, inv_tau)
+    o = amd.recurrent_scan(t["q"], t["k"], t["v"], decay, t["bonus"], scale, state, t["slots"], t["start"], t["lens"])
+    out = torch.empty_like(t["v"])
+    amd.head_norm_gate(out, o, t["gate"], t["weight"], 1e-5, 1.0)
+    return out, state
+
+
+def check(out, state, want, want_state):
+    # both sides: fp32 sums of up to some hundred products, then one rounding to bf16 (2^-8 of the value between neighbours)
+    torch.testing.assert_close(state, want_state, rtol=2e-4, atol=2e-4 * float(want_state.abs().max()))
+    torch.testing.assert_close(out.float(), want.float(), rtol=2 ** -7, atol=2 ** -9 * float(want.float().abs().max()))
+
+
+@pytest.mark.parametrize("heads,dk,dv,kind,bonus", [(8, 128, 128, 0, False), (32, 64, 64, 1, True), (2, 48, 136, 0, False)])
+@pytest.mark.parametrize("lengths", [[32], [33], [47, 1, 48, 49], [65, 16, 17, 2], [300], [128, 129, 127], [40] + [1] * 400],
+                         ids=lambda v: "-".join(map(str, v[:4])))
+def test_segments(amd, lengths, heads, dk, dv, kind, bonus):
+    t = operands(lengths, heads, dk, dv, bonus)
+    inv_tau, scale = (1 / 16, dk ** -0.5) if kind == 0 else (1.0, 1.0)
+    want, want_state = reference(amd, t, kind, inv_tau, scale)
+    out, state = torch.empty_like(t["v"]), t["state"].clone()
+    amd.recurrent_mix(out, t["q"], t["k"], t["v"], t["u"], t["a_t"], t["bias"], kind, inv_tau, t["bonus"], scale, t["gate"], t["weight"],
+                      1e-5, 1.0, state, t["slots"], t["start"], t["lens"], max(lengths))
+    check(out, state, want, want_state)
+
+
+def test_smaller_workspaces(amd):
+    import light_vllm_amd
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(light_vllm_amd.__file__), "lib", "liblvllm_hybrid.so"))
+    lib.lvllm_recurrent_mix_workspace_bytes.restype = ctypes.c_int64
+    heads, dk, dv, lengths, scale = 8, 64, 64, [300, 77], 64 ** -0.5
+    t = operands(lengths, heads, dk, dv, False)
+    rows = sum(lengths)
+    most = lib.lvllm_recurrent_mix_workspace_bytes(rows, 2, heads, dk, dv, max(lengths))
+    # decays, and of segments of 128 rows a state and a decay for each: rows / 128 + sequences + 1
+    coarse = 4 * (rows * heads * dk + (rows // 128 + 3) * heads * (dk * dv + 64))
+    assert most > coarse
+    want, want_state = reference(amd, t, 0, 1 / 16, scale)
+    f, i, i64, p = ctypes.c_float, ctypes.c_int, ctypes.c_int64, lambda x: ctypes.c_void_p(0 if x is None else x.data_ptr())
+    for room, code in ((most, 0), (most - 4, 0), (coarse, 0), (coarse - 4, 1)):
+        out, state = torch.zeros_like(t["v"]), t["state"].clone()
+        ws = torch.empty(most, dtype=torch.uint8, device=DEV)
+        ws[room:] = 77
+        rc = lib.lvllm_recurrent_mix(
+            p(out), i64(out.stride(0)), p(t["q"]), p(t["k"]), p(t["v"]), i64(heads * dk), i64(heads * dk), i64(heads * dv), p(t["u"]),
+            i64(t["u"].stride(0)), p(t["a_t"]), p(t["bias"]), i(t["u"].shape[1]), i(0), f(1 / 16), p(None), f(scale), p(t["gate"]),
+            i64(heads * dv), p(t["weight"]), i(dv), f(1e-5), f(1.0), p(state), i64(state.stride(0)), p(t["slots"]), i(state.shape[0]),
+            p(t["start"]), p(t["lens"]), i(2), i(rows), i(heads), i(dk), i(dv), i(max(lengths)), p(ws), i64(room), i(DTYPE_BF16),
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert (rc != 0) == (code != 0), (room, rc)
+        torch.cuda.synchronize()
+        assert bool((ws[room:] == 77).all())
+        if code == 0:
+            check(out, state, want, want_state)
+
+
+DTYPE_BF16 = 2
