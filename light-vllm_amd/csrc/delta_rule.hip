@@ -283,22 +283,23 @@ __global__ __launch_bounds__(256) void delta_step_kernel(const DeltaStepParams p
 
 // ---- chunks --------------------------------------------------------------------------------------------------------
 __host__ __device__ constexpr int prepare_lds_floats(int NT) {
-  return 5 * kChunk * (64 * NT + 4) + 8 * 256 + kChunk * (kChunk + 4) + 8 * kChunk + kChunk + 4 * NT;
+  return 3 * kChunk * (64 * NT + 4) + 8 * 256 + kChunk * (kChunk + 4) + 8 * kChunk + kChunk + 4 * NT;
 }
 
 // One workgroup per (head, chunk).  Wave w owns key channels [16 NT w, 16 NT (w + 1)); a lane loads channel c, tokens 4g .. 4g + 3
 // of a tile.  Channels that decay too fast for two factors measured from the chunk's middle are added pair by pair.
+// What it moves takes about half of its time, the rest is latency: what the scan reads takes the place of the products' operands
+// in LDS, so that four workgroups share a CU and not three.  8192 rows of 16 heads of 128: 203 us with three, 172 now.
 template <typename T, int NT>
-__global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void delta_prepare_kernel(const DeltaChunkParams p) {
+__global__ __launch_bounds__(256, NT <= 2 ? 4 : 1) void delta_prepare_kernel(const DeltaChunkParams p) {
   using S = typename T::store_t;
   constexpr int DKP = 64 * NT, LD = DKP + 4, LA = kChunk + 4;
   extern __shared__ __attribute__((aligned(16))) float sm[];
   float* sq = sm;                   // [16][LD]: q from the middle of the chunk
   float* sk = sq + kChunk * LD;     // [16][LD]: k to the middle
   float* sr = sk + kChunk * LD;     // [16][LD]: k from the middle (fast decays: ln g)
-  float* sqs = sr + kChunk * LD;    // [16][LD]: q from the chunk's start
-  float* sks = sqs + kChunk * LD;   // [16][LD]: beta k from the chunk's start, then W
-  float* spart = sks + kChunk * LD;  // [2][4 waves][16][16]: products of q and of k with k
+  float *sqs = sq, *sks = sk;       // behind the products: q from the chunk's start; beta k from there, then W
+  float* spart = sr + kChunk * LD;  // [2][4 waves][16][16]: products of q and of k with k
   float* sa = spart + 8 * 256;      // [16][LA]: the system's matrix below its diagonal
   float* sn = sa + kChunk * LA;     // [2][4 waves][16]: squares
   float* sb = sn + 8 * kChunk;      // [16]: beta
@@ -372,6 +373,7 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void delta_prepare_kernel(con
     }
   }
   bool wild = false;
+  float qs[NT][4], ks[NT][4];
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
     const int tile = wave * NT + i, ch = tile * 16 + c;
@@ -390,8 +392,8 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void delta_prepare_kernel(con
       sq[t * LD + ch] = qv[i][r] * from;
       sr[t * LD + ch] = kv[i][r] * from;
       sk[t * LD + ch] = kv[i][r] * to;
-      sqs[t * LD + ch] = qv[i][r] * read;
-      sks[t * LD + ch] = beta[r] * kv[i][r] * read;
+      qs[i][r] = qv[i][r] * read;
+      ks[i][r] = beta[r] * kv[i][r] * read;
       kend[r] = kv[i][r] * (mild ? to * from_mid : exp_of(cs.left[r]));
     }
     *reinterpret_cast<float4*>(ws + p.layout.k() + (tile * 64 + lane) * 4) = float4{kend[0], kend[1], kend[2], kend[3]};
@@ -420,7 +422,8 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void delta_prepare_kernel(con
   }
   const int ti = threadIdx.x >> 4, tj = threadIdx.x & 15;
   float extra_q = 0.f, extra_k = 0.f;
-  if (__syncthreads_or(wild)) {  // the products of the channels left out above
+  const bool any_wild = __syncthreads_or(wild);
+  if (any_wild) {  // the products of the channels left out above
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       const int ch = (wave * NT + i) * 16 + c;
@@ -454,6 +457,15 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void delta_prepare_kernel(con
     ws[p.layout.p() + (tj & 3) * 64 + (tj >> 2) * 16 + ti] = tj <= ti ? pq : 0.f;
     sa[ti * LA + tj] = tj < ti ? sb[ti] * pk : 0.f;
   }
+  if (any_wild) __syncthreads();  // (q and k of those channels are read until here; else the products are behind a barrier already)
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int at = (4 * g + r) * LD + (wave * NT + i) * 16 + c;
+      sqs[at] = qs[i][r];
+      sks[at] = ks[i][r];
+    }
   __syncthreads();
   // substitution: a thread per column of beta G k and of beta v
   for (int col = threadIdx.x; col < DKP + p.layout.dvp; col += 256) {
