@@ -194,17 +194,6 @@ __device__ __forceinline__ float relu_squared_of(float x) {
   return v * v;
 }
 
-// 1 / (1 + e^-z) for what is rounded to 16 bits next: the hardware's 2^x and reciprocal, within 4e-7 of the value for |z| < 8 and
-// 6e-8 |z| beyond, where expf and an IEEE division take 25 instructions.
-__device__ __forceinline__ float sigmoid_16bit(float z) {
-  return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
-}
-template <typename T>
-__device__ __forceinline__ float sigmoid_for(float z) {  // of a factor of a result in T
-  if constexpr (sizeof(typename T::store_t) == 2) return sigmoid_16bit(z);
-  else return 1.f / (1.f + expf(-z));
-}
-
 // A sigmoid-gated linear unit whose gate is bounded above and whose value on both sides
 __device__ __forceinline__ float clamped_unit_of(float g, float u, float limit) {
   g = fminf(g, limit);

@@ -4,6 +4,8 @@
 
 namespace lvllm {
 
+__device__ __forceinline__ float sigmoid_f(float z) { return 1.f / (1.f + expf(-z)); }
+
 // Per head: o / rms(o) * weight * silu(gate) * scale -> T (SILU), or with sigmoid(gate).  o is the fp32 read-out of a recurrent state.
 // weight_head_stride: 0 (one weight of size vdim for all heads) or vdim; weight null: none.  L lanes per (row, head).
 template <typename T, int L, int VEC, bool SILU>
@@ -30,7 +32,7 @@ static __global__ __launch_bounds__(256) void head_norm_gate_kernel(
     load_vec<T, VEC>(gate + row * gate_stride + h * vdim + d, z);
 #pragma unroll
     for (int j = 0; j < VEC; ++j)
-      f[j] = f[j] * r * (weight != nullptr ? weight[h * weight_head_stride + d + j] : 1.f) * (SILU ? z[j] : 1.f) * sigmoid_for<T>(z[j]) * scale;
+      f[j] = f[j] * r * (weight != nullptr ? weight[h * weight_head_stride + d + j] : 1.f) * (SILU ? z[j] * sigmoid_f(z[j]) : sigmoid_f(z[j])) * scale;
     store_vec<T, VEC>(out + row * out_stride + h * vdim + d, f);
   }
 }

@@ -47,13 +47,6 @@ struct MoeActivation {
   __device__ __forceinline__ float operator()(float g, float u) const {
     return silu ? g / (1.f + expf(-g)) * u : clamped_unit_of(g, u, limit);
   }
-  // ... for a result of 16 bits
-  __device__ __forceinline__ float rounded(float g, float u) const {
-    if (silu) return g * sigmoid_16bit(g) * u;
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-    return g * sigmoid_16bit(1.702f * g) * (u + 1.f);
-  }
 };
 __device__ __forceinline__ float slot_weight_of(const MoeParams& p, int slot) {
   return p.slot_weight != nullptr ? p.slot_weight[slot] : 1.f;

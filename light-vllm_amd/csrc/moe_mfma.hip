@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
   if constexpr (GATED) {
     const MoeActivation act(p, e);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = act.rounded(acc[0][r] * f, acc[1][r] * f);
+    for (int r = 0; r < 4; ++r) v[r] = act(acc[0][r] * f, acc[1][r] * f);
     store4<BF16>((uint16_t*)p.out + (int64_t)slot * p.ff_max + 16 * u + 4 * g, v);
   } else {
 #pragma unroll
@@ -207,7 +207,7 @@ __device__ __forceinline__ void tile_store(const MoeParams& p, int e, const e_f3
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          if constexpr (GATED) v[r] = act.rounded(acc[n][m][r] * f, acc[n + 1][m][r] * f);
+          if constexpr (GATED) v[r] = act(acc[n][m][r] * f, acc[n + 1][m][r] * f);
           else v[r] = UP ? relu_squared_of(acc[n][m][r] * f) : acc[n][m][r];
         }
         const int chunk = (GATED ? n - n0 : 2 * (n - n0)) + (g >> 1);

@@ -410,7 +410,7 @@ __global__ __launch_bounds__(256, NT == 1 && NV <= 4 ? 3 : 2) void chunk_mix_ker
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
           const float zg = gate.at(j);
-          o[j] = o[j] * rms * nw[j] * (zg * sigmoid_for<T>(zg));
+          o[j] = o[j] * rms * nw[j] * (zg / (1.f + expf(-zg)));
         }
         if constexpr (NV >= 4) {
           if (p.vec_out && d0 + NV <= p.dv) {
