@@ -13,11 +13,12 @@
 //   * probabilities never move between lanes: MFMA row i of S^T holds a permuted key (groups of four 1 and 2 of every 16
 //     trade places), which makes a lane's accumulators the consecutive keys that P V wants as its B operand;
 //   * accumulators are rescaled only when a column's maximum grew;
-//   * with two workgroups a CU the vector instructions of the softmax bound a tile (half of them exponentials), so that the scale
-//     goes into the exponential's argument and the maximum takes three scores at a time;
+//   * with two workgroups a CU the vector instructions of the softmax bound a tile (half of them exponentials), so that the maximum
+//     takes three scores at a time.  The scale stays a product of its own, rounded ahead of the subtraction (6 to 10 % of such a
+//     launch): fused with it, other roundings moved tokens of a mixture behind the attention to other experts;
 //   * tiles of kept first keys come ahead of the window's.
 // One prompt of 4096, us, with tiles through registers and an instruction for each of these, and now: 16 heads over 4, 128 + 64,
-// 134, 107; 32 over 8, 128 + 128, 219, 189; two maps 190, 159.  4 prompts of 2048, 16 heads, 192 + 128 (two stages): 155, 147.
+// 133, 111; 32 over 8, 128 + 128, 212, 193; two maps 190, 168.  4 prompts of 2048, 16 heads, 192 + 128 (two stages): 145, 133.
 #pragma once
 #include <float.h>
 
@@ -147,14 +148,16 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
         s[0] = mfma32(a0, qf[ks], s[0]);
         s[1] = mfma32(a1, qf[ks], s[1]);
       }
-      // scores are mul * s; with a cap, or a scale that does not keep their order, they are made first
-      float mul = score.mul;
-      if (score.cap > 0.f || !(mul > 0.f)) {
+      if (score.cap > 0.f) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) s[h][i] = score.cap > 0.f ? score.capped(s[h][i]) : s[h][i] * mul;
-        mul = 1.f;
+          for (int i = 0; i < 16; ++i) s[h][i] = score.capped(s[h][i]);
+      } else {  // (rounded here, ahead of the subtraction, as in the other bodies)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[h][i] *= score.mul;
       }
       if (k0 + 63 > wave_first || k0 < wave_all) {  // the diagonal or the window's edge passes through it for some column
 #pragma unroll
@@ -168,7 +171,7 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
       float mx = fmaxf(s[0][0], s[1][0]);  // (behind this both products' results are there)
 #pragma unroll
       for (int i = 1; i < 16; ++i) mx = max3(mx, s[0][i], s[1][i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32)) * mul;
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
       if (__any(mx > m)) {
         const float mn = fmaxf(m, mx), corr = exp2f(m - mn);
         m = mn;
@@ -181,7 +184,7 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          s[h][i] = __builtin_amdgcn_exp2f(fmaf(s[h][i], mul, -m));
+          s[h][i] = __builtin_amdgcn_exp2f(s[h][i] - m);
           sum += s[h][i];
         }
       l += sum;
