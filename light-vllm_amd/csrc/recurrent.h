@@ -680,8 +680,10 @@ constexpr int mix_wgs_per_cu(int NT, int NV) { return NT == 1 && NV <= 4 ? 3 : 2
 
 // Chunks per segment: sequences are cut when (sequence, head, value slice) triples alone leave CUs idle, into as many
 // segments as run at once.  A chunk is a chain of steps that takes 6 to 14 us and a segment walks its own one after the other, so
-// that short portions are cut down to single chunks: 300 rows, us with at least 8 and now: 8 heads of 128 92, 46, with a
-// fixed decay 83, 38; 32 heads of 64 180, 57.  Not below kLeastChunks, where a chunk less does not pay for the two launches more.
+// that short portions are cut down to single chunks: 300 rows, us with at least 8 and now: 8 heads of 128 92, 46; 32 heads of
+// 64 180, 57.  Not below kLeastChunks, where a chunk less does not pay for the two launches more.
+// `coarse`: not below kCoarse chunks.  Fixed decays keep to that (83 us for 300 rows, 38 with single chunks): states and read-outs
+// of other segments are rounded another way, and behind a retention there are mixtures, whose tokens then change experts.
 // Every sequence has a workgroup for each segment of the longest: beyond 16384 of them segments are longer, up to kCoarse.
 constexpr int kCoarse = 8, kLeastChunks = 3;
 inline int segment_chunks(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len, bool coarse) {
@@ -748,7 +750,7 @@ static int launch_single_tokens(const MixParams& p, int dtype, hipStream_t s) {
   return 0;
 }
 
-inline int64_t segments_workspace(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len, bool coarse = false) {  // floats
+inline int64_t segments_workspace(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len, bool coarse) {  // floats
   const int per = segment_chunks(rows, num_seqs, heads, dk, dv, max_query_len, coarse);
   const int64_t segs = segment_slots(rows, num_seqs, per, max_query_len) * heads;
   const int64_t o = value_slices(dk, dv) > 1 ? (int64_t)rows * heads * dv : 0;
@@ -757,9 +759,9 @@ inline int64_t segments_workspace(int rows, int num_seqs, int heads, int dk, int
 
 // The chunked body's segments; `ws`: their workspace of `room` bytes.  Short portions need more of it than long ones may: what
 // holds segments of kCoarse chunks, but no shorter ones, is enough as well.  Returns whether it is.
-inline bool plan_segments(MixParams& p, float* ws, int64_t room, int rows, int max_query_len) {
-  auto need = [&](bool coarse) { return 4 * segments_workspace(rows, p.num_seqs, p.heads, p.dk, p.dv, max_query_len, coarse); };
-  const bool coarse = room < need(false);
+inline bool plan_segments(MixParams& p, float* ws, int64_t room, int rows, int max_query_len, bool coarse = false) {
+  auto need = [&](bool c) { return 4 * segments_workspace(rows, p.num_seqs, p.heads, p.dk, p.dv, max_query_len, c); };
+  coarse = coarse || room < need(false);
   if (coarse && room < need(true)) return false;
   p.seg_chunks = segment_chunks(rows, p.num_seqs, p.heads, p.dk, p.dv, max_query_len, coarse);
   p.max_segs = (max_query_len + kChunk * p.seg_chunks - 1) / (kChunk * p.seg_chunks);

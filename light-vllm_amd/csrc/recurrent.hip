@@ -152,7 +152,7 @@ extern "C" int lvllm_recurrent_scan(float* o, const void* q, const void* k, cons
 
 extern "C" int64_t lvllm_recurrent_mix_workspace_bytes(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len) {
   if (max_query_len <= 1) return 0;
-  return ((int64_t)rows * heads * dk + segments_workspace(rows, num_seqs, heads, dk, dv, max_query_len)) * 4;
+  return ((int64_t)rows * heads * dk + segments_workspace(rows, num_seqs, heads, dk, dv, max_query_len, false)) * 4;
 }
 
 extern "C" int lvllm_recurrent_mix(void* out, int64_t out_stride, const void* q, const void* k, const void* v,

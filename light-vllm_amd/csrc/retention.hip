@@ -40,7 +40,7 @@ using namespace lvllm;
 
 extern "C" int64_t lvllm_retention_workspace_bytes(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len) {
   if (max_query_len <= 1) return 0;
-  return (2 * (int64_t)rows * heads * dk + segments_workspace(rows, num_seqs, heads, dk, dv, max_query_len)) * 4;
+  return (2 * (int64_t)rows * heads * dk + segments_workspace(rows, num_seqs, heads, dk, dv, max_query_len, true)) * 4;
 }
 
 extern "C" int lvllm_retention(void* out, int64_t out_stride, const void* q, const void* k, const void* v, int64_t q_stride,
@@ -68,7 +68,7 @@ extern "C" int lvllm_retention(void* out, int64_t out_stride, const void* q, con
   if (max_query_len <= 1) return launch_single_tokens<true>(p, dtype, s);
   float *qr = (float*)workspace, *kr = qr + (int64_t)rows * heads * dk;
   const int64_t rotated = 2 * (int64_t)rows * heads * dk;
-  LV_CHECK(workspace != nullptr && plan_segments(p, qr + rotated, workspace_bytes - rotated * 4, rows, max_query_len),
+  LV_CHECK(workspace != nullptr && plan_segments(p, qr + rotated, workspace_bytes - rotated * 4, rows, max_query_len, true),
            "workspace too small (see lvllm_retention_workspace_bytes)");
   LV_CHECK((int64_t)num_seqs * p.max_segs <= 65535, "too many sequences or too long portions");
   LV_DISPATCH_F32_BF16(dtype, {

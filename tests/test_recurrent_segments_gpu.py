@@ -1,6 +1,6 @@
 """Portions cut into segments of single chunks against the token-by-token recurrence: lengths around the chunks' edges (16 tokens; cut from the
 third chunk on), ragged sequences with and without an earlier state, so many sequences that segments get longer, and workspaces that
-hold only the coarse segments of 8 chunks, or not even these."""
+hold only the coarse segments of 8 chunks, or not even these; fixed decays, whose segments never get shorter."""
 import ctypes
 import os
 
@@ -89,6 +89,33 @@ def test_smaller_workspaces(amd):
         assert bool((ws[room:] == 77).all())
         if code == 0:
             check(out, state, want, want_state)
+
+
+def test_retention_of_any_workspace(amd):
+    """A retention's bits do not depend on how much scratch there is."""
+    import light_vllm_amd
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(light_vllm_amd.__file__), "lib", "liblvllm_local.so"))
+    heads, dk, dv, lengths = 8, 64, 64, [300, 77, 1]
+    t, rows, n, results = operands(lengths, heads, dk, dv, False), sum(lengths), len(lengths), []
+    decay = torch.linspace(0.9, 0.999, heads, dtype=torch.float64)
+    decay = torch.stack([decay, decay.log()]).float().to(DEV)
+    positions = torch.cat([torch.arange(m) + (7 if i % 2 else 0) for i, m in enumerate(lengths)]).to(DEV)
+    turns = torch.tensor([0.1, 0.01], dtype=torch.float64, device=DEV)
+    # rotated queries and keys, and of segments of 128 rows a state and a decay for each: rows / 128 + sequences + 1
+    least = 4 * (2 * rows * heads * dk + (rows // 128 + n + 1) * heads * (dk * dv + 64))
+    f, i, i64, p = ctypes.c_float, ctypes.c_int, ctypes.c_int64, lambda x: ctypes.c_void_p(0 if x is None else x.data_ptr())
+    for room in (least, 8 * least):
+        out, state, ws = torch.zeros_like(t["v"]), t["state"].clone(), torch.empty(room, dtype=torch.uint8, device=DEV)
+        rc = lib.lvllm_retention(
+            p(out), i64(out.stride(0)), p(t["q"]), p(t["k"]), p(t["v"]), i64(heads * dk), i64(heads * dk), i64(heads * dv), p(positions),
+            p(turns), i(4), p(decay), f(dk ** -0.5), p(t["gate"]), i64(heads * dv), p(t["weight"]), i(dv), f(1e-5), f(1.0), p(state),
+            i64(state.stride(0)), p(t["slots"]), i(state.shape[0]), p(t["start"]), p(t["lens"]), i(n), i(rows), i(heads), i(dk), i(dv),
+            i(max(lengths)), p(ws), i64(room), i(DTYPE_BF16), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0
+        torch.cuda.synchronize()
+        results.append((out, state))
+    (a, sa), (b, sb) = results
+    assert bool(a.any(1).all()) and torch.equal(a, b) and torch.equal(sa, sb)
 
 
 DTYPE_BF16 = 2
