@@ -9,6 +9,7 @@
 #include <algorithm>
 
 #include "moe.h"
+#include "moe_turns.h"
 
 namespace lvllm {
 
@@ -130,9 +131,8 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
 
 constexpr int kTileW = 16;  // W tiles of a workgroup
 
-// A workgroup's turns.  An XCD gets an eighth of the last expert's tiles (the shared expert may be larger: its tiles come first)
-// and of all others', as units: up to 1024 slots of an expert side by side, W block after W block, so that its L2 serves a W
-// block to all of them and their rows to the next blocks.  Its workgroups take units in turn.
+// A workgroup's turn (moe_turns.h).  Units of an expert are up to 1024 of its slots side by side, W block after W block, so that an
+// XCD's L2 serves a W block to all of them and their rows to the next blocks.
 struct TileWork {
   int e, block, s0, s1, steps, ntiles;  // slots s0 .. s1 - 1, k-steps, W tiles of 16 rows of the expert
   bool any;
@@ -142,31 +142,12 @@ __device__ __forceinline__ TileWork tile_work(const MoeParams& p, const int bloc
   constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
   constexpr int kSide = 1024 / TILE;
   TileWork t{};
-  const int xcd = blockIdx.x & 7, cu = blockIdx.x >> 3, cus = gridDim.x >> 3;
-  const int tiles_first = p.tiles[4 * p.max_tiles];
-  const int all_first = tiles_first * blocks_first, all_last = (p.tiles[4 * p.max_tiles + 1] - tiles_first) * blocks_last;
-  const int per_first = (all_first + 7) / 8, per_last = (all_last + 7) / 8;
-  // the first `own` turns are the last expert's, as long as `as_long` of the others (going down, k-steps are its inner size):
-  // workgroups with one turn of them fewer start on the others by so much earlier
-  const int as_long = UP ? 1 : max(1, (p.ff_last + p.ff_first / 2) / p.ff_first);
-  const int full = per_last / cus, rest = per_last % cus;  // (`rest` workgroups have full + 1 of them)
-  const int own = full + (cu < rest);
-  int unit, blocks, tile;
-  if (turn < own) {
-    unit = xcd * per_last + turn * cus + cu;
-    if (unit >= all_last) return t;
-    blocks = blocks_last;
-    tile = tiles_first + unit / blocks;
-    unit += tiles_first * blocks;
-  } else {
-    const int late = cu < rest ? as_long : 0, round = turn - own + late;  // while the others were at their longer turn
-    const int mine = rest == 0 || round >= as_long ? (rest == 0 ? round * cus : as_long * (cus - rest) + (round - as_long) * cus) + cu
-                                                   : round * (cus - rest) + cu - rest;
-    unit = xcd * per_first + mine;
-    if (mine >= per_first || unit >= all_first) return t;
-    blocks = blocks_first;
-    tile = unit / blocks;
-  }
+  const int tiles_first = p.tiles[4 * p.max_tiles], tiles_last = p.tiles[4 * p.max_tiles + 1] - tiles_first;
+  const TurnUnit u = turn_unit(tiles_first * blocks_first, tiles_last * blocks_last, solo_units(UP, p.ff_first, p.ff_last),
+                               blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3, turn);
+  if (!u.any) return t;
+  const int blocks = u.last ? blocks_last : blocks_first;
+  int unit = u.unit + (u.last ? tiles_first * blocks : 0), tile = unit / blocks;
   t.e = p.tiles[4 * tile];
   const int tile0 = p.tiles[4 * tile + 2], count = p.tiles[4 * tile + 3];
   if (t.e < 0 || t.e >= p.experts || count <= 0) return t;
@@ -238,13 +219,13 @@ LV_TO_LDS(to_lds4, 4)
 #undef LV_TO_LDS
 
 // Few slots an expert, behind more than kMoeFewRows rows: bound by the weights' bytes.  256 W rows x 64 slots a workgroup of 8
-// waves, a wave 128 x 16, one workgroup a CU for up to 64 turns.  Both operands come by way of LDS, a ring of six k-steps of
+// waves, a wave 128 x 16, one workgroup a CU for up to kTurns turns.  Both operands come by way of LDS, a ring of six k-steps of
 // 32 of which four are on their way (80 KiB a CU: 2 us of what HBM gives it), and the first steps of a turn are on their way
 // while the turn before stores: no turn waits for memory by itself, as the shared expert's tiles behind all others did.  A
 // step's fragments are read while the step before multiplies.  All turns are looked up at the start, a lane each.
 // 2048 wide, up + down in us, moe_tile_kernel first: 32 experts of 1408, 2 of them and 2816 shared, 80 rows 137, 119, 300 rows
 // 136, 122; 64 experts of 1408, 6 and 2816 shared, 128 rows 238, 227, 512 rows 253, 250; from 45 slots an expert on slower.
-constexpr int kRingSlots = kMoeRingTile, kRingStages = 6, kRingCopies = 3, kTurns = 64;
+constexpr int kRingSlots = kMoeRingTile, kRingStages = 6, kRingCopies = 3;
 struct alignas(16) Turn {
   int64_t w;                // bytes to the block's first W tile
   int s0, s1, steps, left;  // slots s0 .. s1 - 1, k-steps, W tiles from the first one on
@@ -692,14 +673,13 @@ static void go(const MoeParams& p, hipStream_t s) {
     const int tile = moe_tile(true, p.rows, p.slots, p.experts);
     const int64_t tiles = std::min<int64_t>(p.max_tiles, p.slots / tile + p.experts);
     const int64_t last_tiles = (p.rows + tile - 1) / tile;  // a token takes an expert once
-    const int64_t wgs = 8 * ((tiles * first + 7) / 8 + (last_tiles * last + 7) / 8);
-    // of the ring: a workgroup a CU, more only where one would have over 64 turns
-    const unsigned grid = (unsigned)std::min(wgs, std::max<int64_t>(256, (wgs / (kTurns - 2) + 8) / 8 * 8));
     if (tile == kRingSlots) {
+      const unsigned grid = (unsigned)ring_workgroups(tiles * first, last_tiles * last, solo_units(UP, p.ff_first, p.ff_last));
       (void)hipFuncSetAttribute((const void*)moe_ring_kernel<PRODUCT>, hipFuncAttributeMaxDynamicSharedMemorySize, kRingLds);
       hipLaunchKernelGGL((moe_ring_kernel<PRODUCT>), dim3(grid), dim3(512), kRingLds, s, p, first, last);
     } else {
-      hipLaunchKernelGGL((moe_tile_kernel<PRODUCT>), dim3((unsigned)wgs), dim3(256), 0, s, p, first, last);
+      const unsigned grid = (unsigned)unit_workgroups(tiles * first, last_tiles * last);
+      hipLaunchKernelGGL((moe_tile_kernel<PRODUCT>), dim3(grid), dim3(256), 0, s, p, first, last);
     }
   }
 }
