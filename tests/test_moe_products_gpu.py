@@ -63,3 +63,62 @@ def test_products(amd, counts, ff, width, act, weigh):
         assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5).all(), (e, (got - want).abs().max())
         got, want = y[slots[r]], got @ down[e].double().T
         assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5).all(), (e, (got - want).abs().max())
+
+
+@pytest.mark.parametrize("act,weigh", [("clamped", False), ("silu", True), ("relu_squared", True)])
+@pytest.mark.parametrize("width", [4096, 224, 64])
+def test_many_turns_a_workgroup(amd, width, act, weigh):
+    """Few slots an expert, and far more units than workgroups: a turn's first steps come in while the turn before ends, weights of the slots
+    in two buffers by turns, turns of 1 to 12 and of 128 k-steps one after the other, a shared expert of eleven times the others' size
+    (going up its turns come first; going down, workgroups without one take eleven of the others' ahead)."""
+    from light_vllm_amd.engine.moe import ACTIVATIONS, interleave_16
+    g, gated, experts, limit = torch.Generator(device=DEV).manual_seed(width), act != "relu_squared", 40, 1.1
+    counts = [0, 1, 64, 65, 17, 30, 2, 63, 16, 33] * 2 + [7, 20, 11, 9] * 5
+    ff = ([384, 32, 64, 160, 192, 96, 256, 384, 128, 352] * 4)[:experts] + [4096]
+    rows = sum(counts)
+    tiles = sum((n + 63) // 64 for n in counts)
+    assert len(counts) == experts and 64 < rows and 2 * rows < 45 * (experts + 1)  # the ring's range
+    blocks = [-(-n // (128 if gated else 256)) for n in ff]
+    assert sum(b * ((n + 63) // 64) for b, n in zip(blocks, counts + [rows])) > 450 or not gated
+    assert width < 4096 or 16 * tiles > 2 * 256
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
+    of_row = torch.repeat_interleave(torch.arange(experts, device=DEV), torch.tensor(counts, device=DEV))
+    of_row = of_row[torch.randperm(rows, generator=g, device=DEV)]
+    h = 0.5 * rand(rows, width)
+    h[:, :experts] = 0.25 * torch.nn.functional.one_hot(of_row, experts).bfloat16()
+    router = torch.zeros(48, width, dtype=torch.bfloat16, device=DEV)
+    router[:experts, :experts] = 8 * torch.eye(experts)
+    gate, up = ([rand(n, width) * width ** -0.5 for n in ff] for _ in "gu")
+    down = [rand(width, n) * n ** -0.5 for n in ff]
+
+    def packed(parts):
+        parts = [amd.pack_weight(p.contiguous()).reshape(-1) for p in parts]
+        return torch.cat(parts), torch.tensor([0] + [p.numel() for p in parts[:-1]]).cumsum(0).to(DEV)
+    ids, weights, offsets, token, slots, tiles, by_slot = amd.moe_route(h, amd.pack_weight(router), None, 1, True, True, experts, False, 1,
+                                                                        weigh)
+    assert torch.equal(ids[:, 0].long(), of_row) and bool((ids[:, 1] == experts).all())
+    sizes = rows, width, max(ff), max(ff[:-1]), ff[-1]
+    ffs, limits = torch.tensor(ff, dtype=torch.int32, device=DEV), torch.full((experts + 1,), limit, device=DEV)
+    w_up, up_at = packed([interleave_16(a, b) if gated else b for a, b in zip(gate, up)])
+    w_down, down_at = packed(down)
+    a = amd.moe_experts(h, w_up, up_at, ffs, limits, offsets, token, tiles, *sizes, True, True, by_slot if weigh else None, ACTIVATIONS[act])
+    y = amd.moe_experts(a, w_down, down_at, ffs, None, offsets, token, tiles, *sizes, False, True)
+    # fp32 sums of n products in steps of 32, the partial sums below 8 (going up) and 16 (down, of activations up to 6 or so),
+    # then one rounding to 8 bits; the products of two sums have twice the error of one, times the other
+    steps = width // 32
+    atol_up, atol_down = 2.0 ** -23 * 8 * steps * 8, 2.0 ** -23 * 16 * 128
+    for e in range(experts + 1):
+        r = torch.arange(rows, device=DEV) if e == experts else (of_row == e).nonzero()[:, 0]
+        s = slots[r, int(e == experts)].long()
+        x = h[r].double() * (weights[r, int(e == experts)].double()[:, None] if weigh else 1)
+        p, u = x @ gate[e].double().T.contiguous(), x @ up[e].double().T.contiguous()
+        if act == "clamped":
+            p, u = p.clamp(max=limit), u.clamp(-limit, limit)
+            want = p * torch.sigmoid(1.702 * p) * (u + 1)
+        else:
+            want = p * torch.sigmoid(p) * u if gated else u.clamp(min=0).square()
+        got = a[s, :ff[e]].double()
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + atol_up).all(), (e, (got - want).abs().max())
+        want = got @ down[e].double().T.contiguous()
+        got = y[s].double()
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + atol_down).all(), (e, (got - want).abs().max())
