@@ -71,9 +71,11 @@ struct MixParams {
   float* seg_decay;       // [segment slots, heads, dkp]
 };
 
-// Segment k of sequence s has slot query_start_loc[s] / (tokens of a segment) + s + k: unique
+// Segment k of a sequence s of more than one segment has slot base + k.  Sequences of one segment have none: they take at least a
+// row each and no slot, while `base` grows by a segment's worth of rows, and by one more, from one longer sequence to the next.
 __device__ __forceinline__ int seg_slot_base(const MixParams& p, int s) {
-  return p.query_start_loc[s] / (kChunk * p.seg_chunks) + s;
+  const int before = p.query_start_loc[s] / (kChunk * p.seg_chunks);
+  return before + min(s, before);
 }
 
 __host__ __device__ constexpr int mix_smem_floats(int NT, int NV) {
@@ -143,12 +145,14 @@ __global__ __launch_bounds__(256, NT == 1 && NV <= 4 ? 3 : 2) void chunk_mix_ker
   float* sv = so + 4 * kChunk * LO; // [16][LO]: values
   int* swild = reinterpret_cast<int*>(sv + kChunk * LO);  // [4 NT]: channels of a tile that decay too fast for the factors
   const int head = blockIdx.x, v0 = blockIdx.y * 16 * NV;
-  const bool cut = p.max_segs > 1;
-  const int seq = cut ? blockIdx.z / p.max_segs : blockIdx.z, seg = cut ? blockIdx.z - seq * p.max_segs : 0;
+  // First segments side by side, then second ones: segment by segment of a sequence, the workgroups that find nothing would be the
+  // same ones of every few, and with four segments a quarter of the chip would do all of the work.
+  const int seg = p.max_segs > 1 ? blockIdx.z / p.num_seqs : 0, seq = blockIdx.z - seg * p.num_seqs;
   const int qbeg = p.query_start_loc[seq], qlen = p.query_start_loc[seq + 1] - qbeg;
   if (qlen <= 0) return;
   const int all_chunks = (qlen + kChunk - 1) / kChunk;
-  const int first = cut ? seg * p.seg_chunks : 0;
+  const bool cut = p.max_segs > 1 && all_chunks > p.seg_chunks;
+  const int first = seg * p.seg_chunks;
   const int last = cut ? min(first + p.seg_chunks, all_chunks) : all_chunks;
   if (first >= all_chunks || (STATES && last == all_chunks)) return;
   const int lane = threadIdx.x & 63;
@@ -452,7 +456,7 @@ static __global__ __launch_bounds__(256) void chunk_combine_kernel(const MixPara
   const int head = blockIdx.y, seq = blockIdx.z;
   const int qlen = p.query_start_loc[seq + 1] - p.query_start_loc[seq];
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, per_head = (int64_t)p.dk * p.dv;
-  if (qlen <= 0 || i >= per_head) return;
+  if (qlen <= kChunk * p.seg_chunks || i >= per_head) return;
   const int segs = (qlen + kChunk * p.seg_chunks - 1) / (kChunk * p.seg_chunks);
   const int slot = p.state_slots[seq];
   const bool live = slot >= 0 && slot < p.num_slots;
@@ -681,11 +685,14 @@ constexpr int mix_wgs_per_cu(int NT, int NV) { return NT == 1 && NV <= 4 ? 3 : 2
 // Chunks per segment: sequences are cut when (sequence, head, value slice) triples alone leave CUs idle, into as many
 // segments as run at once.  A chunk is a chain of steps that takes 6 to 14 us and a segment walks its own one after the other, so
 // that short portions are cut down to single chunks: 300 rows, us with at least 8 and now: 8 heads of 128 92, 46; 32 heads of
-// 64 180, 57.  Not below kLeastChunks, where a chunk less does not pay for the two launches more.
+// 64 180, 57.  Not into fewer than kLeastSegments, where the chunks saved do not pay for the two launches more.
+// Every sequence has a workgroup for each segment of the longest, and most of them find nothing to do: for segments of n chunks
+// their time falls as 1 / n and that of the walks grows as n, so that n grows with the root of the workgroups of single chunks.
+// One portion beside 255 single tokens, 8 heads of 128, us with at least 8 chunks, with single ones as far as there are workgroups
+// for them, and now: 45 tokens 113, 228, 98; 128 tokens 147, 428, 131; 300 tokens 302, 251, 184.  kSquare = 8192: 136, 152, 171.
 // `coarse`: not below kCoarse chunks.  Fixed decays keep to that (83 us for 300 rows, 38 with single chunks): states and read-outs
 // of other segments are rounded another way, and behind a retention there are mixtures, whose tokens then change experts.
-// Every sequence has a workgroup for each segment of the longest: beyond 16384 of them segments are longer, up to kCoarse.
-constexpr int kCoarse = 8, kLeastChunks = 3;
+constexpr int kCoarse = 8, kLeastSegments = 3, kSquare = 2048;
 inline int segment_chunks(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len, bool coarse) {
   const int chunks = (max_query_len + kChunk - 1) / kChunk;
   const int64_t long_seqs = (rows + max_query_len - 1) / max_query_len;
@@ -693,11 +700,14 @@ inline int segment_chunks(int rows, int num_seqs, int heads, int dk, int dv, int
   const int64_t segs = 256 * mix_wgs_per_cu(key_groups(dk), value_tiles(dk, dv)) / wide;
   const int per = segs < 2 ? chunks : (int)((chunks + segs - 1) / segs);
   const int64_t wgs = (int64_t)chunks * num_seqs * heads * value_slices(dk, dv);
-  const int64_t least = coarse || chunks < kLeastChunks ? kCoarse : (wgs + 16383) / 16384;
-  return per < least ? (int)(least < kCoarse ? least : kCoarse) : per;
+  int least = 1;
+  while (least < kCoarse && (int64_t)least * least * kSquare < wgs) ++least;
+  if (coarse || chunks < kLeastSegments * least) least = kCoarse;
+  return per < least ? least : per;
 }
 inline int64_t segment_slots(int rows, int num_seqs, int per, int max_query_len) {
-  return max_query_len <= per * kChunk ? 0 : (int64_t)rows / (kChunk * per) + num_seqs + 1;
+  const int64_t whole = rows / (kChunk * per);
+  return max_query_len <= per * kChunk ? 0 : whole + (num_seqs < whole ? num_seqs : whole) + 1;
 }
 
 template <typename T, typename QT, int NT, int NV, bool FIXED>

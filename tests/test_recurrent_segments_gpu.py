@@ -61,6 +61,11 @@ def test_segments(amd, lengths, heads, dk, dv, kind, bonus):
     check(out, state, want, want_state)
 
 
+@pytest.mark.parametrize("lengths", [[1] * 20 + [33] + [1] * 3 + [16, 17, 49] + [1] * 9, [3, 64, 1, 1, 65, 2, 15, 48], [1] * 255 + [45], [45] + [1] * 255])
+def test_single_tokens_beside_segments(amd, lengths):
+    test_segments(amd, lengths, 8, 64, 64, 0, False)
+
+
 def test_smaller_workspaces(amd):
     import light_vllm_amd
     lib = ctypes.CDLL(os.path.join(os.path.dirname(light_vllm_amd.__file__), "lib", "liblvllm_hybrid.so"))
