@@ -165,7 +165,9 @@ extern "C" int lvllm_moe_experts(void* out, const void* x, const void* w, const 
                                  int ff_max, int ff_first, int ff_last, int max_tiles, int up, int packed, int dtype,
                                  void* stream) {
   if (slots == 0) return 0;
-  LV_CHECK(experts > 0 && ff_max > 0 && ff_max % 32 == 0 && width > 0 && max_tiles > 0 && max_tiles <= 65535, "sizes of the experts");
+  // tiles are a dimension of the grid but for prompts on matrix cores, whose tiles are counted by 64 slots and made of 128
+  const int most_tiles = packed && rows > kMoeFewRows ? 2 * 65535 : 65535;
+  LV_CHECK(experts > 0 && ff_max > 0 && ff_max % 32 == 0 && width > 0 && max_tiles > 0 && max_tiles <= most_tiles, "sizes of the experts");
   LV_CHECK(!up || act == LVLLM_MOE_SILU || act == LVLLM_MOE_RELU_SQUARED || (act == LVLLM_MOE_CLAMPED && limit != nullptr),
            "unknown activation");
   MoeParams p{};

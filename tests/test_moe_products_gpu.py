@@ -122,3 +122,29 @@ def test_many_turns_a_workgroup(amd, width, act, weigh):
         want = got @ down[e].double().T.contiguous()
         got = y[s].double()
         assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + atol_down).all(), (e, (got - want).abs().max())
+
+
+def test_millions_of_slots(amd):
+    """More tiles of 64 slots than a dimension of a grid: rows of every part of the step against the product in 64 bits."""
+    rows, top, experts, width, ff = 600_000, 8, 16, 32, 32
+    g = torch.Generator(device=DEV).manual_seed(5)
+    h = torch.randn(rows, width, generator=g, device=DEV).bfloat16()
+    router = torch.randn(experts, width, generator=g, device=DEV).bfloat16()
+    up, down = (torch.randn(experts, *s, generator=g, device=DEV).bfloat16() * 32 ** -0.5 for s in ((ff, width), (width, ff)))
+    ids, _, offsets, token, slots, tiles, _ = amd.moe_route(h, amd.pack_weight(router), None, top, False, True, experts, False, 1)
+    assert rows * top > 64 * 65535 and tiles.shape[0] > 65535
+    sizes, at = (rows, width, ff, ff, ff), torch.arange(experts, device=DEV) * ff * width
+    ffs = torch.full((experts,), ff, dtype=torch.int32, device=DEV)
+    pack = lambda w: torch.cat([amd.pack_weight(e.contiguous()).reshape(-1) for e in w])
+    a = amd.moe_experts(h, pack(up), at, ffs, None, offsets, token, tiles, *sizes, True, True, None, 2)
+    y = amd.moe_experts(a, pack(down), at, ffs, None, offsets, token, tiles, *sizes, False, True)
+    r = torch.cat([torch.arange(500, device=DEV), torch.arange(rows - 500, rows, device=DEV), torch.randint(rows, (3000,), generator=g, device=DEV)])
+    e, s = ids[r].long(), slots[r].long()
+    for j in range(experts):
+        row, place = (e == j).nonzero(as_tuple=True)
+        want = (h[r[row]].double() @ up[j].double().T.contiguous()).clamp(min=0).square()
+        got = a[s[row, place]].double()
+        # one k-step: fp32 sums of 32 products, then one rounding to 8 bits
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all(), j
+        want = got @ down[j].double().T.contiguous()
+        assert ((y[s[row, place]].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), j
