@@ -402,7 +402,7 @@ constexpr int kStages = 4, kStageBytes = kMoeTile * 64;  // of 32 of K: 16-slot 
 
 template <int PRODUCT>
 __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, const int blocks_first, const int blocks_last) {
-  constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
+  constexpr bool UP = PRODUCT != kMoeDown;
   __shared__ __attribute__((aligned(16))) char ring[kStages][kStageBytes];
   const TileWork t = tile_work<PRODUCT, kMoeTile>(p, blocks_first, blocks_last, 0);
   if (!t.any) return;
@@ -671,8 +671,11 @@ static void go(const MoeParams& p, hipStream_t s) {
     auto blocks = [&](int ff) { return ((GATED ? ff / 8 : (UP ? ff : p.width) / 16) + kTileW - 1) / kTileW; };
     const int first = blocks(p.ff_first), last = blocks(p.ff_last);
     const int tile = moe_tile(true, p.rows, p.slots, p.experts);
-    const int64_t tiles = std::min<int64_t>(p.max_tiles, p.slots / tile + p.experts);
-    const int64_t last_tiles = (p.rows + tile - 1) / tile;  // a token takes an expert once
+    // more tiles than there are of 64 slots: they may be of 16 (a router that is not packed), which either body takes as well
+    const bool small = p.max_tiles >= p.slots || p.max_tiles > p.slots / kMoeRingTile + p.experts;
+    const int least = small ? kMoeSmallTile : tile;
+    const int64_t tiles = small ? p.max_tiles : std::min<int64_t>(p.max_tiles, p.slots / tile + p.experts);
+    const int64_t last_tiles = (p.rows + least - 1) / least;  // a token takes an expert once
     if (tile == kRingSlots) {
       const unsigned grid = (unsigned)ring_workgroups(tiles * first, last_tiles * last, solo_units(UP, p.ff_first, p.ff_last));
       (void)hipFuncSetAttribute((const void*)moe_ring_kernel<PRODUCT>, hipFuncAttributeMaxDynamicSharedMemorySize, kRingLds);

@@ -148,3 +148,30 @@ def test_millions_of_slots(amd):
         assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all(), j
         want = got @ down[j].double().T.contiguous()
         assert ((y[s[row, place]].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all(), j
+
+
+@pytest.mark.parametrize("rows,experts", [(2000, 4), (300, 8), (100, 200)], ids=["many slots", "few slots", "hardly any"])
+def test_tiles_of_a_plain_router(amd, rows, experts):
+    """Packed products over the tiles of 16 slots that a router that is not packed makes, a shared expert of several times the others' size
+    among them: what they give over the packed router's tiles."""
+    width, ff, shared_ff = 256, 160, 800
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
+    h, marks = rand(rows, width), torch.zeros(experts, width, dtype=torch.bfloat16, device=DEV)
+    marks[torch.arange(experts), torch.arange(experts)] = 4
+    of_row = torch.zeros(rows, width, dtype=torch.bfloat16, device=DEV)  # whole numbers decide: both routers choose alike
+    of_row[torch.arange(rows), torch.arange(rows) % experts] = 1
+    sizes, ffs = (rows, width, shared_ff, ff, shared_ff), torch.tensor([ff] * experts + [shared_ff], dtype=torch.int32, device=DEV)
+    up, down = ([rand(*(s if kind == "up" else s[::-1])) * width ** -0.5 for s in [(ff, width)] * experts + [(shared_ff, width)]]
+                for kind in ("up", "down"))
+    at = torch.arange(experts + 1, device=DEV) * ff * width
+    pack = lambda ws: torch.cat([amd.pack_weight(w.contiguous()).reshape(-1) for w in ws])
+    results = []
+    for packed in (True, False):
+        r = amd.pack_weight(torch.nn.functional.pad(marks, (0, 0, 0, -experts % 16))) if packed else marks
+        ids, _, offsets, token, slots, tiles, _ = amd.moe_route(of_row, r, None, 1, True, packed, experts, False, 1)
+        a = amd.moe_experts(h, pack(up), at, ffs, None, offsets, token, tiles, *sizes, True, True, None, 2)
+        y = amd.moe_experts(a, pack(down), at, ffs, None, offsets, token, tiles, *sizes, False, True)
+        results.append((ids, a[slots.long()][:, 0, :ff], a[slots.long()][:, 1], y[slots.long()]))
+    for one, other in zip(*results):
+        assert torch.equal(one, other)
