@@ -223,8 +223,8 @@ LV_TO_LDS(to_lds4, 4)
 // 32 of which four are on their way (80 KiB a CU: 2 us of what HBM gives it), and the first steps of a turn are on their way
 // while the turn before stores: no turn waits for memory by itself, as the shared expert's tiles behind all others did.  A
 // step's fragments are read while the step before multiplies.  All turns are looked up at the start, a lane each.
-// 2048 wide, up + down in us, moe_tile_kernel first: 32 experts of 1408, 2 of them and 2816 shared, 80 rows 137, 119, 300 rows
-// 136, 122; 64 experts of 1408, 6 and 2816 shared, 128 rows 238, 227, 512 rows 253, 250; from 45 slots an expert on slower.
+// 2048 wide, up + down in us, moe_tile_kernel first: 32 experts of 1408, 2 of them and 2816 shared, 80 rows 137, 125, 300 rows
+// 135, 123; 64 experts of 1408, 6 and 2816 shared, 128 rows 239, 229, 300 rows 245, 240; where it ends: moe_tile (moe.h).
 constexpr int kRingSlots = kMoeRingTile, kRingStages = 6, kRingCopies = 3;
 struct alignas(16) Turn {
   int64_t w;                // bytes to the block's first W tile
@@ -395,7 +395,8 @@ __global__ __launch_bounds__(512, 2) void moe_ring_kernel(const MoeParams p, con
 // More slots an expert: 256 W rows x 128 slots a workgroup, a wave 64 x 128, two workgroups a CU, a turn each.  W goes straight to
 // the operand registers of the one wave that uses it.  The chip's power bounds it with many slots: 1.6 GHz at half of the MFMA
 // cycles, where the library's plain product of 49152 x 2816 x 2048 runs at 1.06 to 1.27 PFLOP/s and this one (8192 rows, 6 of 64
-// experts) at 0.98, 0.88 before results went by way of LDS; 256 slots a workgroup, both operands through LDS, 0.96.  Slots' chunks
+// experts) at 0.95 to 0.99, 0.90 to 0.96 before results went by way of LDS; 256 slots a workgroup, both operands through LDS, were
+// no faster.  Slots' chunks
 // trade places by bit 3 of the slot: LDS reads 16 bytes for lanes 0-3, 12-15, 20-27 at a time (by bits 2 and 3, half of its
 // cycles were conflicts).
 constexpr int kStages = 4, kStageBytes = kMoeTile * 64;  // of 32 of K: 16-slot groups of 1 KiB

@@ -13,8 +13,8 @@
 // Two bodies:
 //   * steps of single tokens (decode): ONE launch per mixer -- decay, state update, read-out, per-head RMS norm and gate --
 //     a workgroup per (sequence, head) that streams the head's state through registers once: HBM-bound;
-//   * everything else: the decays of all heads as one fp32-MFMA product (fixed decays: q and k rotated), then chunks of 16 tokens on fp32 MFMAs
-//     (chunk_mix_kernel): per chunk the decay from its start is folded into q, the decay to its end into k; the masked
+//   * everything else: the decays of all heads as one product (low_rank_decay.h; fixed decays: q and k rotated), then chunks of 16
+//     tokens on fp32 MFMAs (chunk_mix_kernel): per chunk the decay from its start is folded into q, the decay to its end into k; the masked
 //     16 x 16 products inside the chunk, the read-out of the state before it and the state update are matrix products, the
 //     per-head norm and gate its epilogue.  State tiles are MFMA accumulators AND, without a move, the B operands of the
 //     read-out (k-step r of a tile contracts rows {r, 4 + r, 8 + r, 12 + r}: accumulator register r of every lane).
@@ -123,8 +123,8 @@ struct Packed {
 // channels [w * 16 * NT, (w + 1) * 16 * NT): it scales q and k there, holds those rows of the state as accumulator tiles and
 // forms partial in-chunk products and read-outs, which meet in LDS.  A lane loads channel c, tokens 4g .. 4g + 3 of a tile:
 // scaled k is then the A operand of the state update as it is; q goes through LDS.
-// A chunk is one chain of dependent steps, so that what crosses lanes goes by way of registers.  4096 rows, 16 heads, us with
-// shuffles and now: 81, 68 (64 channels), 74, 66 (128).
+// A chunk is one chain of dependent steps, so that what crosses lanes goes by way of registers.  4096 rows, 32 heads of 64
+// channels, us with shuffles and now: 83, 76.
 //   STATES: from a zero state, no read-out: a segment's last state and the product of its decays, of all segments but the
 //   last.  Otherwise the segment's first state comes from the slot (sequences that are not cut) or from chunk_combine_kernel.
 template <typename T, typename QT, int NT, int NV, bool STATES, bool FIXED>

@@ -1275,7 +1275,7 @@ extern "C" int lvllm_skinny_gemm_ex(void* y, const void* x, const void* w, const
 
 // `products` of M rows each: y[p] = x[p] . w[p]^T, x [products, M, K], w and y back to back, N outputs each and N_last of the last
 // one.  One launch where `products` of them were (a launch of a few MB of weights inside a captured step is 7 us, 4.5 of them
-// its start: four of 2048 x 2048 and one of 64 x 2048 for 24 rows 33 us, together 13); bit-identical to them.
+// its start: four of 2048 x 2048 and one of 64 x 2048 for 24 rows 33 us, together 9.6 there); bit-identical to them.
 extern "C" int lvllm_skinny_gemm_products(void* y, const void* x, const void* w_packed, int products, int M, int N, int N_last,
                                           int K, int dtype, void* stream) {
   if (M <= 0 || products <= 0) return 0;

@@ -1,6 +1,6 @@
-"""Sigmoids of gates and activations are those of 32-bit results everywhere: what leaves in bfloat16 is bit for bit the rounded float32 result
-of the same inputs, and the matrix-core mixtures' activation that of the plain body.  Gates far below zero and the largest ones among
-the inputs."""
+"""Sigmoids of gates and activations are those of 32-bit results everywhere: what leaves in bfloat16 is bit for bit the rounded float32
+result of the same inputs, and the matrix-core mixtures' activation that of the plain body.  Gates far below zero and the largest ones
+among the inputs."""
 import pytest
 import torch
 

@@ -1,5 +1,5 @@
-"""Every unit of the grouped products has exactly one turn: csrc/moe_turns.h on the host, over grids of any size, with a last expert of none to
-many times the others' size, up to the most turns that a workgroup can look up."""
+"""Every unit of the grouped products has exactly one turn: csrc/moe_turns.h on the host, over grids of any size, with a last expert of
+none to many times the others' size, up to the most turns that a workgroup can look up."""
 import ctypes
 import os
 import random
@@ -74,7 +74,8 @@ def test_any_ring(lib):
         most_first, most_last, solo = size(), size() - 1, lib.solo(0, 32, 32 * int(2 ** r.uniform(0, 8)))
         grid = lib.ring(most_first, most_last, solo)
         assert grid >= 256 or grid == lib.single(most_first, most_last)
-        for first, last in ((most_first, most_last), (r.randint(0, most_first), r.randint(0, most_last)), (most_first, r.randint(0, most_last))):
+        fewer = r.randint(0, most_last)
+        for first, last in ((most_first, most_last), (r.randint(0, most_first), fewer), (most_first, fewer)):
             assert walk(lib, first, last, solo, grid, lib.turns()) == (0, 0), (first, last, solo, grid)
 
 
