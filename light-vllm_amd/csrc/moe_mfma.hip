@@ -31,9 +31,12 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
   constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
   extern __shared__ __attribute__((aligned(16))) char sx[];  // [k-steps of a chunk][4][16][8]
   __shared__ e_f32x4_t red[KS > 1 ? 4 : 1][2][64];
-  const int e = p.tiles[4 * blockIdx.y];
+  // the last expert's tiles first: it may be larger than the others, and its work is not to be what is left at the end
+  const int tile = p.tiles[4 * p.max_tiles + 1] - 1 - (int)blockIdx.y;
+  if (tile < 0) return;
+  const int e = p.tiles[4 * tile];
   if (e < 0 || e >= p.experts) return;
-  const int s0 = p.tiles[4 * blockIdx.y + 1], s1 = min(min(p.offsets[e + 1], s0 + 16), p.slots);
+  const int s0 = p.tiles[4 * tile + 1], s1 = min(min(p.offsets[e + 1], s0 + 16), p.slots);
   if (s0 >= s1) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -564,52 +567,48 @@ __global__ __launch_bounds__(512) void moe_logits_kernel(float* __restrict__ par
   for (int i = threadIdx.x; i < 16 * ld; i += 512) out[i] = z[i];
 }
 
-// ... and one workgroup adds them, chooses (a wave per row) and groups the assignments.  A wave asks for its next row's shares
-// ahead of a choice; choices and ranks stay in LDS.  One CU does it all, so that the vector instructions of a choice bound it: rounds
-// of maxima take a third of those of counted places.  64 experts, 6 of them, us with counted places and now: 32 rows 17.0, 13.6;
-// 64 rows 29.1, 22.5; 8 rows of 8 groups 8.6, 7.2.
+// ... and one workgroup adds them, chooses (a wave per row) and groups the assignments, `batch` rows at a time.  A thread asks for all
+// shares of its logits at once, up to S of them (further shares stand for the last one: a condition would be a branch, and a wait
+// before the next load); choices and ranks stay in LDS.  One CU does it all, so that round trips to memory and the vector
+// instructions of a choice bound it, and the size of the code, which comes from memory as well.
+template <int S>
 __global__ __launch_bounds__(1024) void moe_choose_group_kernel(int32_t* ids, float* weights, const float* __restrict__ part,
                                                                 const float* __restrict__ bias, const int shares,
                                                                 const int row_tiles, const int ld, const MoeRouting r,
-                                                                const int rows, const int keep, const MoeGroups groups) {
+                                                                const int rows, const int batch, const int keep,
+                                                                const MoeGroups groups) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = r.per_row();
-  float* z = reinterpret_cast<float*>(smem) + wave * ld;
-  int* kept = reinterpret_cast<int*>(smem + 16 * ld * 4);
-  auto bias_of = [&](int e) { return e < r.experts && bias != nullptr ? bias[e] : 0.f; };
-  auto load = [&](int row, int e, float (&t)[kRouteShares]) __attribute__((always_inline)) {
+  const int n = r.per_row();
+  float* z = reinterpret_cast<float*>(smem);  // [batch][ld]
+  int* kept = reinterpret_cast<int*>(smem + batch * ld * 4);
+  const int64_t share = (int64_t)row_tiles * 16 * ld;
+  constexpr int U = 16 / S < 2 ? 2 : 16 / S;  // logits of a thread
+  for (int row0 = 0; row0 < rows; row0 += batch) {
+    const int here = min(batch, rows - row0), count = here * ld;
+    const float* from = part + (int64_t)row0 * ld;
+    if (row0 > 0) __syncthreads();
+    for (int i0 = threadIdx.x; i0 < count; i0 += 1024 * U) {
+      float t[U][S], v[U];
 #pragma unroll
-    for (int s = 0; s < kRouteShares; ++s)
-      if (s < shares) t[s] = part[((int64_t)s * row_tiles * 16 + row) * ld + e];
-  };
-  auto sum = [&](float v, const float (&t)[kRouteShares]) __attribute__((always_inline)) {
+      for (int u = 0; u < U; ++u) {
+        const int i = min(i0 + 1024 * u, count - 1), e = i % ld;
 #pragma unroll
-    for (int s = 0; s < kRouteShares; ++s) v += s < shares ? t[s] : 0.f;
-    return v;
-  };
-  constexpr int A = 2;  // logits of a lane that are asked for ahead
-  float t[A][kRouteShares], b[A] = {0.f, 0.f};
-  auto ahead = [&](int row) __attribute__((always_inline)) {
+        for (int s = 0; s < S; ++s) t[u][s] = from[min(s, shares - 1) * share + i];
+        v[u] = bias != nullptr ? bias[min(e, r.experts - 1)] : 0.f;
+        if (e >= r.experts) v[u] = 0.f;
+      }
 #pragma unroll
-    for (int j = 0; j < A; ++j)
-      if (lane + 64 * j < r.logits()) load(row, lane + 64 * j, t[j]);
-  };
+      for (int u = 0; u < U; ++u) {
 #pragma unroll
-  for (int j = 0; j < A; ++j)
-    if (lane + 64 * j < r.logits()) b[j] = bias_of(lane + 64 * j);
-  if (wave < rows) ahead(wave);
-  for (int row = wave; row < rows; row += 16) {
-#pragma unroll
-    for (int j = 0; j < A; ++j)
-      if (lane + 64 * j < r.logits()) z[lane + 64 * j] = sum(b[j], t[j]);
-    for (int e = lane + 64 * A; e < r.logits(); e += 64) {
-      float v[kRouteShares];
-      load(row, e, v);
-      z[e] = sum(bias_of(e), v);
+        for (int s = 0; s < S; ++s) v[u] += s < shares ? t[u][s] : 0.f;
+        if (i0 + 1024 * u < count) z[i0 + 1024 * u] = v[u];
+      }
     }
-    if (row + 16 < rows) ahead(row + 16);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the wave's own next reads see it)
-    choose_experts(z, r, ids + (int64_t)row * n, weights + (int64_t)row * n, kept + row * n, keep);
+    __syncthreads();
+    for (int i = threadIdx.x >> 6; i < here; i += 16) {
+      const int row = row0 + i;
+      choose_experts(z + i * ld, r, ids + (int64_t)row * n, weights + (int64_t)row * n, kept + row * n, keep);
+    }
   }
   __syncthreads();
   if (keep) group_assignments(kept, kept + rows * n, rows * n, n, r.all(), r.shared, groups);
@@ -632,14 +631,21 @@ int launch_moe_route_mfma(int32_t* ids, float* weights, const void* h, const voi
   if (rows <= kMoeFewRows) {
     const int shares = route_shares(width), per = (width / 32 + shares - 1) / shares, ld = ntiles * 16;
     const int lds = kRouteLds + 16 * ld * 4, numbers = 2 * rows * r.per_row() * 4;
-    const int keep = numbers <= 32 * 1024, lds_choose = 16 * ld * 4 + (keep ? numbers : 0);  // (many experts a row: by way of memory)
+    const int keep = numbers <= 32 * 1024;  // (many experts a row: by way of memory)
+    const int batch = std::min(std::max(1, 64 * 1024 / (ld * 4) / 16), row_tiles) * 16;
+    const int lds_choose = batch * ld * 4 + (keep ? numbers : 0);
     (void)hipFuncSetAttribute((const void*)moe_logits_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    (void)hipFuncSetAttribute((const void*)moe_choose_group_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_choose);
     hipLaunchKernelGGL(moe_logits_kernel, dim3(row_tiles, shares), dim3(512), lds, s, workspace, (const uint16_t*)h,
                        (const uint16_t*)w, ntiles, rows, width, per);
     LV_LAUNCH_CHECK();
-    hipLaunchKernelGGL(moe_choose_group_kernel, dim3(1), dim3(1024), lds_choose, s, ids, weights, workspace, bias, shares,
-                       row_tiles, ld, r, rows, keep, groups);
+    auto choose = [&](auto most) {
+      constexpr int S = decltype(most)::value;
+      (void)hipFuncSetAttribute((const void*)moe_choose_group_kernel<S>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_choose);
+      hipLaunchKernelGGL(moe_choose_group_kernel<S>, dim3(1), dim3(1024), lds_choose, s, ids, weights, workspace, bias, shares,
+                         row_tiles, ld, r, rows, batch, keep, groups);
+    };
+    if (shares <= 4) choose(std::integral_constant<int, 4>{});
+    else choose(std::integral_constant<int, kRouteShares>{});
     LV_LAUNCH_CHECK();
     return 0;
   }
