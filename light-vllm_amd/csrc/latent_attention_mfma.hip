@@ -75,7 +75,9 @@ __global__ __launch_bounds__(256 * CT, 1) void latent_attention_mfma_kernel(cons
     const int i = (j * CT + ct) * 64 + lane, r = i / RC;
     from[j] = r * RE + ((i - r * RC) ^ exchange<NK>(r)) * 8;
   }
-  auto page_of = [&](int t) { return table[min(lo / 16 + 4 * t + kg, p.max_blocks - 1)]; };
+  auto page_of = [&](int t) {  // (a scalar load: it has no place among the copies)
+    return ((const __attribute__((address_space(4))) int32_t*)table)[min(lo / 16 + 4 * t + kg, p.max_blocks - 1)];
+  };
   auto copy = [&](int t, int page) __attribute__((always_inline)) {
     const int64_t blk = min(max(page, 0), p.max_block);
     const uint16_t* src = (const uint16_t*)p.cache + blk * p.block_stride;
@@ -86,15 +88,19 @@ __global__ __launch_bounds__(256 * CT, 1) void latent_attention_mfma_kernel(cons
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + from[j]),
                                          (__attribute__((address_space(3))) void*)(dst + (j * CT + ct) * 1024), 16, 0, 0);
   };
-  if (t0 < t1) copy(t0, page_of(t0));
-  int page = page_of(t0 + 1);  // (looked up a tile ahead)
   m_u32x4_t qf[NK];
   {
     const uint16_t* q = (const uint16_t*)p.q + at * RE + 8 * g;
 #pragma unroll
     for (int j = 0; j < NK; ++j) qf[j] = *reinterpret_cast<const m_u32x4_t*>(q + 32 * j);
   }
-  __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // (q has landed: nothing in the loop waits for it)
+  int page = page_of(t0 + 1);  // (looked up a tile ahead)
+  if (t0 < t1) copy(t0, page_of(t0));
+  if (t0 + 1 < t1) copy(t0 + 1, page);
+  page = page_of(t0 + 2);
+  __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+#pragma unroll
+  for (int j = 0; j < NK; ++j) asm volatile("" : "+v"(qf[j]));  // (q has landed: nothing in the loop waits for it)
   const float sl = p.scale * 1.4426950408889634f;
   float m = -1e30f, l = 0.f;
   m_f32x4_t o[NT];
@@ -106,11 +112,11 @@ __global__ __launch_bounds__(256 * CT, 1) void latent_attention_mfma_kernel(cons
   typedef __attribute__((address_space(3))) m_i16x4_t* lds_tr_t;
 
   for (int t = t0; t < t1; ++t) {
-    // the copies of this tile have landed, for every wave; everyone is done with the tile before
-    __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
-    asm volatile("s_barrier" ::: "memory");
-    if (t + 1 < t1) copy(t + 1, page);
-    page = page_of(t + 2);
+    // Loads return in order: with the next tile's copies outstanding, of which a wave has at least kLeast, this one's have landed ...
+    constexpr int kLeast = NK / CT;
+    if (t + 1 < t1) __builtin_amdgcn_s_waitcnt((kLeast & 15) | (kLeast >> 4) << 14 | (7 << 4) | (15 << 8));
+    else __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+    asm volatile("s_barrier" ::: "memory");  // ... for every wave
     const char* st = tile + ((t - t0) & 1) * kStage;
     m_f32x4_t s{0.f, 0.f, 0.f, 0.f}, s2{0.f, 0.f, 0.f, 0.f};
     constexpr int W = NK < 6 ? NK : 6;  // fragments read ahead
@@ -169,6 +175,11 @@ __global__ __launch_bounds__(256 * CT, 1) void latent_attention_mfma_kernel(cons
         const m_u32x2_t ua = __builtin_bit_cast(m_u32x2_t, a[i]), ub = __builtin_bit_cast(m_u32x2_t, b[i]);
         o[i] = mfma16(m_u32x4_t{ua.x, ua.y, ub.x, ub.y}, pf, o[i]);
       }
+    }
+    if (t + 2 < t1) {
+      lds_barrier();  // everyone is done with this tile: the one after the next takes its place
+      copy(t + 2, page);
+      page = page_of(t + 3);
     }
   }
   l += __shfl_xor(l, 16);
