@@ -451,7 +451,7 @@ __global__ __launch_bounds__(256, NT == 1 && NV <= 4 ? 3 : 2) void chunk_mix_ker
 }
 
 // The first state of every segment, in place of the last state it would have had from zero: a thread per state element,
-// sequential over the segments.
+// sequential over the segments, sixteen of which are asked for at once (behind the store of one, the load of the next waited for it).
 static __global__ __launch_bounds__(256) void chunk_combine_kernel(const MixParams p, const int dkp) {
   const int head = blockIdx.y, seq = blockIdx.z;
   const int qlen = p.query_start_loc[seq + 1] - p.query_start_loc[seq];
@@ -466,11 +466,21 @@ static __global__ __launch_bounds__(256) void chunk_combine_kernel(const MixPara
   float* st = p.seg_state + base * per_head + i;
   const float* de = p.seg_decay + base * dkp + i / p.dv;
   const int64_t st_step = p.heads * per_head, de_step = (int64_t)p.heads * dkp;
-#pragma unroll 4
-  for (int k = 0; k < segs - 1; ++k) {
-    const float own = st[k * st_step], d = de[k * de_step];
-    st[k * st_step] = x;
-    x = fmaf(d, x, own);
+  constexpr int B = 16;
+  for (int k0 = 0; k0 < segs - 1; k0 += B) {
+    float own[B], d[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      const int k = min(k0 + j, segs - 2);
+      own[j] = st[k * st_step];
+      d[j] = de[k * de_step];
+    }
+#pragma unroll
+    for (int j = 0; j < B; ++j)
+      if (k0 + j < segs - 1) {
+        st[(k0 + j) * st_step] = x;
+        x = fmaf(d[j], x, own[j]);
+      }
   }
   st[(segs - 1) * st_step] = x;
 }
