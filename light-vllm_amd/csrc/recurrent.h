@@ -67,6 +67,7 @@ struct MixParams {
   const float* log_decay; // [rows, heads, dk]
   float* o;               // [rows, heads, dv], or null: the epilogue is applied where o is made
   int seg_chunks, max_segs;  // chunks per segment, segments of the longest sequence (1: not cut)
+  int tiles;              // 16-column tiles of a workgroup's value slice
   float* seg_state;       // [segment slots, heads, dk, dv]
   float* seg_decay;       // [segment slots, heads, dkp]
 };
@@ -485,6 +486,49 @@ static __global__ __launch_bounds__(256) void chunk_combine_kernel(const MixPara
   st[(segs - 1) * st_step] = x;
 }
 
+// The epilogue of chunk_mix_kernel for heads whose columns were cut into slices (fine_tiles): the same sums, in the same order.
+// NV: the columns of a thread there, sixteen of which are a row.
+template <typename T, int NV>
+static __global__ __launch_bounds__(256) void chunk_norm_kernel(const MixParams p) {
+  using S = typename T::store_t;
+  const int64_t item = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4), row = item / p.heads;
+  const int head = (int)(item - row * p.heads), d0 = (threadIdx.x & 15) * NV;
+  if (row >= p.query_start_loc[p.num_seqs]) return;  // (the same in a row's sixteen lanes)
+  Packed<T, NV> gate;
+  gate.load((const S*)p.gate + row * p.gate_stride + head * p.dv, d0, p.dv, p.vec_in);
+  float o[NV], nw[NV], ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int d = min(d0 + j, p.dv - 1);
+    o[j] = p.o[item * p.dv + d];
+    nw[j] = p.norm_weight == nullptr ? p.out_scale : p.norm_weight[head * p.norm_head_stride + d] * p.out_scale;
+  }
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    if (d0 + j < p.dv) ss = fmaf(o[j], o[j], ss);
+  ss = over_lanes<16>(ss, [](float a, float b) { return a + b; });
+  const float rms = 1.f / sqrtf(ss / p.dv + p.eps);
+  S* out = (S*)p.out + row * p.out_stride + head * p.dv + d0;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const float zg = gate.at(j);
+    o[j] = o[j] * rms * nw[j] * (zg / (1.f + expf(-zg)));
+  }
+  if constexpr (NV >= 4) {
+    if (p.vec_out && d0 + NV <= p.dv) {
+#pragma unroll
+      for (int j = 0; j < NV; j += 4) {
+        const float w[4] = {o[j], o[j + 1], o[j + 2], o[j + 3]};
+        store4<T>(out + j, w);
+      }
+      return;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+    if (d0 + j < p.dv) out[j] = T::from_float(o[j]);
+}
+
 // ---- single tokens -------------------------------------------------------------------------------------------------
 // state that is not touched again before the next step: past the caches
 __device__ __forceinline__ float4 load_stream(const float* p) {
@@ -720,10 +764,23 @@ inline int64_t segment_slots(int rows, int num_seqs, int per, int max_query_len)
   return max_query_len <= per * kChunk ? 0 : whole + (num_seqs < whole ? num_seqs : whole) + 1;
 }
 
+// Tiles of a value slice that the workgroups of a launch take: fewer than value_tiles() where heads, sequences and segments alone
+// leave CUs idle and a workgroup has a walk of several chunks before it, whose time falls with the columns; the norm over a head is
+// one launch more then.  300 rows, 8 heads of 128 x 128 with fixed decays, all launches in a step, 8 tiles 92 us, 4 72, 2 55, 1 50.
+constexpr int kLeastWalk = 4;
+inline int fine_tiles(int num_seqs, int heads, int dk, int dv, int max_query_len, int per) {
+  const int nv = value_tiles(dk, dv), chunks = (max_query_len + kChunk - 1) / kChunk;
+  if (value_slices(dk, dv) > 1 || (per < chunks ? per : chunks) < kLeastWalk) return nv;
+  const int64_t wgs = (int64_t)heads * num_seqs * ((chunks + per - 1) / per);
+  int n = nv;
+  while (n > 1 && 2 * wgs * (nv / n) <= 256) n /= 2;
+  return n;
+}
+
 template <typename T, typename QT, int NT, int NV, bool FIXED>
 static void launch_mix(const MixParams& p, hipStream_t s) {
   constexpr int smem = mix_smem_floats(NT, NV) * 4;
-  const dim3 grid(p.heads, value_slices(p.dk, p.dv), p.num_seqs * p.max_segs);
+  const dim3 grid(p.heads, (p.dv + 16 * NV - 1) / (16 * NV), p.num_seqs * p.max_segs);
   if (p.max_segs > 1) {
     hipLaunchKernelGGL((chunk_mix_kernel<T, QT, NT, NV, true, FIXED>), grid, dim3(256), 0, s, p);
     hipLaunchKernelGGL(chunk_combine_kernel, dim3((unsigned)(((int64_t)p.dk * p.dv + 255) / 256), p.heads, p.num_seqs),
@@ -736,8 +793,7 @@ static void launch_mix(const MixParams& p, hipStream_t s) {
 
 template <typename T, typename QT, bool FIXED>
 static void launch_mix_sized(const MixParams& p, hipStream_t s) {
-  const int nv = value_tiles(p.dk, p.dv);
-  switch (key_groups(p.dk) * 16 + nv) {
+  switch (key_groups(p.dk) * 16 + p.tiles) {
     case 17: launch_mix<T, QT, 1, 1, FIXED>(p, s); break;
     case 18: launch_mix<T, QT, 1, 2, FIXED>(p, s); break;
     case 20: launch_mix<T, QT, 1, 4, FIXED>(p, s); break;
@@ -750,6 +806,19 @@ static void launch_mix_sized(const MixParams& p, hipStream_t s) {
     case 66: launch_mix<T, QT, 4, 2, FIXED>(p, s); break;
     default: launch_mix<T, QT, 4, 4, FIXED>(p, s); break;
   }
+}
+
+// ... of slices that fine_tiles() made
+template <typename T>
+static int launch_chunk_norm(const MixParams& p, int rows, hipStream_t s) {
+  const dim3 grid((unsigned)(((int64_t)rows * p.heads + 15) / 16));
+  switch (value_tiles(p.dk, p.dv)) {
+    case 2: hipLaunchKernelGGL((chunk_norm_kernel<T, 2>), grid, dim3(256), 0, s, p); break;
+    case 4: hipLaunchKernelGGL((chunk_norm_kernel<T, 4>), grid, dim3(256), 0, s, p); break;
+    default: hipLaunchKernelGGL((chunk_norm_kernel<T, 8>), grid, dim3(256), 0, s, p); break;
+  }
+  LV_LAUNCH_CHECK();
+  return 0;
 }
 
 // every sequence brings one token: sequence s owns row s
@@ -770,17 +839,23 @@ static int launch_single_tokens(const MixParams& p, int dtype, hipStream_t s) {
   return 0;
 }
 
-inline int64_t segments_workspace(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len, bool coarse) {  // floats
+inline int64_t least_segments_workspace(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len, bool coarse) {  // floats
   const int per = segment_chunks(rows, num_seqs, heads, dk, dv, max_query_len, coarse);
   const int64_t segs = segment_slots(rows, num_seqs, per, max_query_len) * heads;
   const int64_t o = value_slices(dk, dv) > 1 ? (int64_t)rows * heads * dv : 0;
   return segs * ((int64_t)dk * dv + 64 * key_groups(dk)) + o;
 }
+inline int64_t segments_workspace(int rows, int num_seqs, int heads, int dk, int dv, int max_query_len, bool coarse) {
+  const int per = segment_chunks(rows, num_seqs, heads, dk, dv, max_query_len, coarse);
+  const bool fine = fine_tiles(num_seqs, heads, dk, dv, max_query_len, per) < value_tiles(dk, dv);
+  return least_segments_workspace(rows, num_seqs, heads, dk, dv, max_query_len, coarse) + (fine ? (int64_t)rows * heads * dv : 0);
+}
 
 // The chunked body's segments; `ws`: their workspace of `room` bytes.  Short portions need more of it than long ones may: what
-// holds segments of kCoarse chunks, but no shorter ones, is enough as well.  Returns whether it is.
+// holds segments of kCoarse chunks, but no shorter ones, is enough as well, and so is what does not hold read-outs of fine slices.
+// Returns whether it is.
 inline bool plan_segments(MixParams& p, float* ws, int64_t room, int rows, int max_query_len, bool coarse = false) {
-  auto need = [&](bool c) { return 4 * segments_workspace(rows, p.num_seqs, p.heads, p.dk, p.dv, max_query_len, c); };
+  auto need = [&](bool c) { return 4 * least_segments_workspace(rows, p.num_seqs, p.heads, p.dk, p.dv, max_query_len, c); };
   coarse = coarse || room < need(false);
   if (coarse && room < need(true)) return false;
   p.seg_chunks = segment_chunks(rows, p.num_seqs, p.heads, p.dk, p.dv, max_query_len, coarse);
@@ -788,7 +863,13 @@ inline bool plan_segments(MixParams& p, float* ws, int64_t room, int rows, int m
   const int64_t segs = segment_slots(rows, p.num_seqs, p.seg_chunks, max_query_len) * p.heads;
   p.seg_decay = ws;
   p.seg_state = ws + segs * 64 * key_groups(p.dk);
-  if (value_slices(p.dk, p.dv) > 1) p.o = p.seg_state + segs * p.dk * p.dv;
+  p.tiles = value_tiles(p.dk, p.dv);
+  if (value_slices(p.dk, p.dv) > 1) {
+    p.o = p.seg_state + segs * p.dk * p.dv;
+  } else if (room >= need(coarse) + 4 * (int64_t)rows * p.heads * p.dv) {
+    p.tiles = fine_tiles(p.num_seqs, p.heads, p.dk, p.dv, max_query_len, p.seg_chunks);
+    if (p.tiles < value_tiles(p.dk, p.dv)) p.o = p.seg_state + segs * p.dk * p.dv;
+  }
   return true;
 }
 

@@ -195,6 +195,7 @@ extern "C" int lvllm_recurrent_mix(void* out, int64_t out_stride, const void* q,
   else launch_mix_sized<F32, F32, false>(p, s);
   LV_LAUNCH_CHECK();
   if (p.o == nullptr) return 0;
+  if (value_slices(dk, dv) == 1) return dtype == LVLLM_BF16 ? launch_chunk_norm<BF16>(p, rows, s) : launch_chunk_norm<F32>(p, rows, s);
   return launch_head_norm_gate<true>(out, out_stride, p.o, gate, gate_stride, norm_weight, norm_head_stride, eps, out_scale, rows,
                                heads, dv, dtype, s);
 }

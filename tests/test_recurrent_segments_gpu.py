@@ -123,4 +123,50 @@ def test_retention_of_any_workspace(amd):
     assert bool(a.any(1).all()) and torch.equal(a, b) and torch.equal(sa, sb)
 
 
+@pytest.mark.parametrize("heads,dk,dv", [(8, 128, 128), (3, 128, 120), (2, 48, 24), (2, 256, 64), (4, 64, 36), (2, 64, 130)])
+@pytest.mark.parametrize("lengths", [[300], [49], [48], [65, 1, 200]], ids=lambda v: "-".join(map(str, v)))
+def test_retention_of_narrow_slices(amd, heads, dk, dv, lengths):
+    """Columns cut finer, with a norm behind, where there is scratch for the read-outs: the same bits as without it."""
+    import light_vllm_amd
+    lib = ctypes.CDLL(os.path.join(os.path.dirname(light_vllm_amd.__file__), "lib", "liblvllm_local.so"))
+    lib.lvllm_retention_workspace_bytes.restype = ctypes.c_int64
+    t, rows, n, results = operands(lengths, heads, dk, dv, False), sum(lengths), len(lengths), []
+    decay = torch.linspace(0.9, 0.999, heads, dtype=torch.float64)
+    decay = torch.stack([decay, decay.log()]).float().to(DEV)
+    positions = torch.cat([torch.arange(m) + (7 if i % 2 else 0) for i, m in enumerate(lengths)]).to(DEV)
+    turns = torch.tensor([0.1, 0.01], dtype=torch.float64, device=DEV)
+    most = lib.lvllm_retention_workspace_bytes(rows, n, heads, dk, dv, max(lengths))
+    f, i, i64, p = ctypes.c_float, ctypes.c_int, ctypes.c_int64, lambda x: ctypes.c_void_p(0 if x is None else x.data_ptr())
+    for room in ((most, most - 4) if dv <= 128 and max(lengths) > 48 else (most,)):
+        out, state, ws = torch.zeros_like(t["v"]), t["state"].clone(), torch.empty(most, dtype=torch.uint8, device=DEV)
+        ws[room:] = 77
+        rc = lib.lvllm_retention(
+            p(out), i64(out.stride(0)), p(t["q"]), p(t["k"]), p(t["v"]), i64(heads * dk), i64(heads * dk), i64(heads * dv), p(positions),
+            p(turns), i(4), p(decay), f(dk ** -0.5), p(t["gate"]), i64(heads * dv), p(t["weight"]), i(dv), f(1e-5), f(1.0), p(state),
+            i64(state.stride(0)), p(t["slots"]), i(state.shape[0]), p(t["start"]), p(t["lens"]), i(n), i(rows), i(heads), i(dk), i(dv),
+            i(max(lengths)), p(ws), i64(room), i(DTYPE_BF16), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0
+        torch.cuda.synchronize()
+        assert bool((ws[room:] == 77).all())
+        results.append((out, state))
+    for a, sa in results:
+        assert bool(a.any(1).all()) and torch.equal(a, results[0][0]) and torch.equal(sa, results[0][1])
+    # against the token-by-token recurrence: fp32 sums of rotated values, one rounding to bf16
+    decays = decay[1].repeat_interleave(dk).expand(rows, -1).contiguous()
+    angles = 2 * torch.pi * positions[:, None].double() * turns
+
+    def rotated(x):
+        x = x.float().view(rows, heads, dk).clone()
+        c, s = angles.cos().float()[:, None], angles.sin().float()[:, None]
+        u, w = x[..., :2].clone(), x[..., 2:4].clone()
+        x[..., :2], x[..., 2:4] = u * c - w * s, w * c + u * s
+        return x.reshape(rows, heads * dk)
+    want_state, g = t["state"].clone(), t["gate"].float()
+    o = amd.recurrent_scan(rotated(t["q"]), rotated(t["k"]), t["v"].float(), decays, None, dk ** -0.5, want_state, t["slots"], t["start"],
+                           t["lens"])
+    want = torch.empty_like(g)
+    amd.head_norm_gate(want, o, g, t["weight"], 1e-5, 1.0)
+    check(results[0][0], results[0][1], want, want_state)
+
+
 DTYPE_BF16 = 2
