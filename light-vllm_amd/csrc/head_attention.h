@@ -31,6 +31,7 @@ struct HeadAttnParams {
   float *part_o, *part_ml;  // decode shares: [rows, heads, maps, nsplit, vpad] and [rows, heads, maps, nsplit, 2]
   int num_seqs, rows, heads, kv_heads, kpad, vpad, vdim, max_blocks, block_size, max_block, nsplit;
   int max_query_len, max_seq_len, window, chunk, keep_first, maps, min_query_len;
+  int fold;  // head_prefill.h
   const float* sink;  // null: none
   float scale, out_scale, softcap, map_weight, map_eps;
   int64_t out_stride, gate_stride, k_block_stride, v_block_stride;
