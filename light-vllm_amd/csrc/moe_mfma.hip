@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
     for (int j = 0; j < kStreamBatch; ++j)
 #pragma unroll
       for (int i = 0; i < 2; ++i)  // (a missing step: the last one again)
-        t[i][j] = *reinterpret_cast<const e_u32x4_t*>(w + ((int64_t)i * steps + min(b + j, steps - 1)) * 512);
+        t[i][j] = __builtin_nontemporal_load(reinterpret_cast<const e_u32x4_t*>(w + ((int64_t)i * steps + min(b + j, steps - 1)) * 512));
   };
   fetch(0, a[0]);
   const int64_t ld = UP ? p.width : p.ff_max;
