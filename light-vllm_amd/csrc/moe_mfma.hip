@@ -212,13 +212,14 @@ __device__ __forceinline__ void tile_store(const MoeParams& p, int e, const e_f3
 }
 
 // 16 (4) bytes a lane to consecutive LDS; base: the same in all lanes
-#define LV_TO_LDS(NAME, BYTES)                                                                                        \
+#define LV_TO_LDS(NAME, BYTES, AUX)                                                                                        \
   __device__ __forceinline__ void NAME(const char* base, uint32_t offset, void* dst) {                               \
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + offset),                 \
-                                     (__attribute__((address_space(3))) void*)dst, BYTES, 0, 0);                     \
+                                     (__attribute__((address_space(3))) void*)dst, BYTES, 0, AUX);                   \
   }
-LV_TO_LDS(to_lds16, 16)
-LV_TO_LDS(to_lds4, 4)
+LV_TO_LDS(to_lds16, 16, 0)
+LV_TO_LDS(to_lds16_past, 16, 2)  // past the caches
+LV_TO_LDS(to_lds4, 4, 0)
 #undef LV_TO_LDS
 
 // Few slots an expert, behind more than kMoeFewRows rows: bound by the weights' bytes.  256 W rows x 64 slots a workgroup of 8
@@ -329,7 +330,7 @@ __global__ __launch_bounds__(512, 2) void moe_ring_kernel(const MoeParams p, con
   auto copy = [&](int k, int stage, int j) __attribute__((always_inline)) {  // behind the last step: of the next turn's
     const bool over = k >= now.steps;
     if (over) k = min(k - now.steps, next.steps - 1);
-    if (j < 2) to_lds16((over ? j ? next.w1 : next.w0 : j ? now.w1 : now.w0) + k * 1024, lane16, ring + stage + (wave * 2 + j) * 1024);
+    if (j < 2) to_lds16_past((over ? j ? next.w1 : next.w0 : j ? now.w1 : now.w0) + k * 1024, lane16, ring + stage + (wave * 2 + j) * 1024);
     else to_lds16((over ? next.x : now.x) + k * 64, 0, ring + stage + (16 + group) * 1024);
   };
   next = now;
