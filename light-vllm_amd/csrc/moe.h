@@ -275,18 +275,10 @@ __device__ __forceinline__ void moe_count_assignments(const int* ids, int row0, 
   }
 }
 
-// slots of a tile: of the matrix-core bodies for prompts, and of those for few rows and for sizes without one
-constexpr int kMoeRingTile = 64, kMoeTile = 128, kMoeSmallTile = 16, kMoeFewRows = 64;
-// Below 45 slots an expert the weights' bytes bound the products and the ring is ahead or level (moe_ring_kernel); from there on
-// tiles of 128 are, but for a strip where the ring is ahead by 2 percent.  Up + down, us, the ring and tiles of 128.  Experts of 1408
-// and a shared one of 2816, 2048 wide: 2 of 32, 300 rows (27 slots an expert) 123, 135; 420 (38) 125, 136; 500 (45) 145, 139; 800 (73)
-// 148, 143; 6 of 64, 300 rows (32) 240, 245; 420 (45) 246, 246; 512 (55) 250, 255; 700 (75) 317, 256.  Both twice as large, 4096 wide:
-// 2 of 32, 300 rows 451, 467; 420 473, 472; 500 513, 484; 6 of 64, 300 rows 854, 856; 420 887, 868; 512 954, 890.
-// `slots` of all `experts`, the shared one's included.
-inline int moe_tile(bool packed, int rows, int64_t slots, int experts) {
-  if (!packed || rows <= kMoeFewRows) return kMoeSmallTile;
-  return slots < (int64_t)45 * experts ? kMoeRingTile : kMoeTile;
-}
+// slots of a tile: of the matrix-core body for prompts, and of those for few rows and for sizes without one
+constexpr int kMoeTile = 128, kMoeSmallTile = 16, kMoeFewRows = 64;
+constexpr int kMoeCountedTile = 64;  // what a prompt's tiles are counted with where room for them is made (lvllm_moe_tile)
+inline int moe_tile(bool packed, int rows) { return packed && rows > kMoeFewRows ? kMoeTile : kMoeSmallTile; }
 
 bool moe_takes_mfma(int width, int dtype);
 int launch_moe_mfma(const MoeParams& p, int product, hipStream_t s);

@@ -114,7 +114,9 @@ __global__ __launch_bounds__(256) void moe_simple_kernel(const MoeParams p) {
 
 using namespace lvllm;
 
-extern "C" int lvllm_moe_tile(int packed, int rows) { return packed && rows > kMoeFewRows ? kMoeRingTile : kMoeSmallTile; }
+extern "C" int lvllm_moe_tile(int packed, int rows) {
+  return packed && rows > kMoeFewRows ? kMoeCountedTile : kMoeSmallTile;
+}
 
 static MoeRouting routing_of(const lvllm_moe_routing& r) {
   return MoeRouting{r.experts, r.top, r.scoring, r.shared != LVLLM_MOE_NO_SHARED, r.shared == LVLLM_MOE_GATED_SHARED,
@@ -140,7 +142,7 @@ extern "C" int lvllm_moe_route(int32_t* ids, float* weights, int32_t* offsets, i
   LV_CHECK(workspace_bytes >= lvllm_moe_route_workspace_bytes(routing, rows, width, packed), "workspace too small");
   hipStream_t s = (hipStream_t)stream;
   const MoeGroups groups{offsets, token, slot, tiles, (int32_t*)workspace,
-                         moe_tile(packed != 0, rows, (int64_t)rows * r.per_row(), r.all()), max_tiles, weights,
+                         moe_tile(packed != 0, rows), max_tiles, weights,
                          slot_weight};
   if (packed) {
     LV_CHECK(moe_takes_mfma(width, dtype), "packed router: bf16, a width that is a multiple of 32");

@@ -4,8 +4,8 @@
 //   * few slots per expert (decode steps): bound by the weights' bytes.  A workgroup takes 16 slots of one expert and a share
 //     of its outputs; the slots' rows sit in LDS in fragment order (2048 of K at a time), every wave streams the two W tiles
 //     of its own (1 KiB a load, eight k-steps in flight behind the eight in use) and needs no other wave;
-//   * prompts: tiles of 64 or 128 slots x 256 W rows, moe_ring_kernel and moe_tile_kernel (moe.h, moe_tile).  A slot's 64 bytes
-//     of a k-step are four chunks, exchanged so that a fragment read is free of bank conflicts.
+//   * prompts: tiles of up to 128 slots x 256 W rows, or 128 where those are few (moe_tile_kernel).  A slot's 64 bytes of a k-step
+//     are four chunks, exchanged so that a fragment read is free of bank conflicts.
 #include <algorithm>
 
 #include "moe.h"
@@ -20,6 +20,15 @@ typedef unsigned int e_u32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ e_f32x4_t moe_mfma(e_u32x4_t a, e_u32x4_t b, e_f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(e_bf16x8_t, a), __builtin_bit_cast(e_bf16x8_t, b), c, 0, 0,
                                                  0);
+}
+
+// Weights that one workgroup reads go past the caches (ONCE); those of an expert with several tiles of slots come by way of the L2
+// that its tiles share.  Up + down, us, without and with: moe_stream_kernel, 32 rows, 6 of 64 experts of 2816, 268, 238; tiles of 128
+// slots, 1000 rows, 6 of 64 experts of 1408 and a shared one 276, 259, 2 of 32 193, 175; all tiles so, 1943 rows 376, 516.
+template <bool ONCE>
+__device__ __forceinline__ e_u32x4_t load_weights(const uint16_t* p) {
+  if constexpr (ONCE) return __builtin_nontemporal_load(reinterpret_cast<const e_u32x4_t*>(p));
+  else return *reinterpret_cast<const e_u32x4_t*>(p);
 }
 
 constexpr int kStreamBatch = 8, kStreamChunk = 64;  // k-steps per batch, per LDS chunk
@@ -58,7 +67,7 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
     for (int j = 0; j < kStreamBatch; ++j)
 #pragma unroll
       for (int i = 0; i < 2; ++i)  // (a missing step: the last one again)
-        t[i][j] = __builtin_nontemporal_load(reinterpret_cast<const e_u32x4_t*>(w + ((int64_t)i * steps + min(b + j, steps - 1)) * 512));
+        t[i][j] = load_weights<true>(w + ((int64_t)i * steps + min(b + j, steps - 1)) * 512);
   };
   fetch(0, a[0]);
   const int64_t ld = UP ? p.width : p.ff_max;
@@ -132,15 +141,13 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
   }
 }
 
-constexpr int kTileW = 16;  // W tiles of a workgroup
-
 // A workgroup's turn (moe_turns.h).  Units of an expert are up to 1024 of its slots side by side, W block after W block, so that an
 // XCD's L2 serves a W block to all of them and their rows to the next blocks.
 struct TileWork {
   int e, block, s0, s1, steps, ntiles;  // slots s0 .. s1 - 1, k-steps, W tiles of 16 rows of the expert
-  bool any;
+  bool any, once;  // once: the expert's only tile
 };
-template <int PRODUCT, int TILE>
+template <int PRODUCT, int TILE, int TILEW>
 __device__ __forceinline__ TileWork tile_work(const MoeParams& p, const int blocks_first, const int blocks_last, const int turn) {
   constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
   constexpr int kSide = 1024 / TILE;
@@ -164,7 +171,8 @@ __device__ __forceinline__ TileWork tile_work(const MoeParams& p, const int bloc
   const int ff = p.ff[t.e];
   t.steps = (UP ? p.width : ff) >> 5;
   t.ntiles = GATED ? ff >> 3 : (UP ? ff : p.width) >> 4;
-  t.any = t.block * kTileW < t.ntiles && t.s0 < t.s1;
+  t.any = t.block * TILEW < t.ntiles && t.s0 < t.s1;
+  t.once = count == 1;
   return t;
 }
 
@@ -176,7 +184,7 @@ __device__ __forceinline__ void tile_store(const MoeParams& p, int e, const e_f3
                                            int slot0, int next, int s1, WEIGHT weight) {
   constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
   [[maybe_unused]] const MoeActivation act(p, GATED ? e : -1);
-  constexpr int kPart = GATED && NT > 4 ? 8 : 4, kOuts = kPart * (GATED ? 8 : 16), kChunks = kOuts / 8;  // of 8 outputs
+  constexpr int kPart = GATED && NT > 4 ? 8 : NT < 4 ? NT : 4, kOuts = kPart * (GATED ? 8 : 16), kChunks = kOuts / 8;  // of 8 outputs
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int64_t out_ld = UP ? p.ff_max : p.width;
 #pragma unroll
@@ -200,8 +208,9 @@ __device__ __forceinline__ void tile_store(const MoeParams& p, int e, const e_f3
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the wave's own next reads see it)
       const int first = (nt0 + n0) * (GATED ? 8 : 16), outs = (ntiles - nt0 - n0) * (GATED ? 8 : 16);
 #pragma unroll
-      for (int j = 0; j < kChunks / 4; ++j) {
+      for (int j = 0; j < (kChunks + 3) / 4; ++j) {
         const int r = j * (64 / kChunks) + lane / kChunks, q = lane % kChunks;
+        if (kChunks < 4 && r >= 16) break;
         const e_u32x4_t v = *reinterpret_cast<const e_u32x4_t*>(lds + r * (kOuts * 2) + ((q ^ r) & (kChunks - 1)) * 16);
         if (slot + r < s1 && q * 8 < outs)
           *reinterpret_cast<e_u32x4_t*>((uint16_t*)p.out + (slot + r) * out_ld + first + q * 8) = v;
@@ -211,243 +220,64 @@ __device__ __forceinline__ void tile_store(const MoeParams& p, int e, const e_f3
   }
 }
 
-// 16 (4) bytes a lane to consecutive LDS; base: the same in all lanes
-#define LV_TO_LDS(NAME, BYTES, AUX)                                                                                        \
-  __device__ __forceinline__ void NAME(const char* base, uint32_t offset, void* dst) {                               \
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + offset),                 \
-                                     (__attribute__((address_space(3))) void*)dst, BYTES, 0, AUX);                   \
-  }
-LV_TO_LDS(to_lds16, 16, 0)
-LV_TO_LDS(to_lds16_past, 16, 2)  // past the caches
-LV_TO_LDS(to_lds4, 4, 0)
-#undef LV_TO_LDS
-
-// Few slots an expert, behind more than kMoeFewRows rows: bound by the weights' bytes.  256 W rows x 64 slots a workgroup of 8
-// waves, a wave 128 x 16, one workgroup a CU for up to kTurns turns.  Both operands come by way of LDS, a ring of six k-steps of
-// 32 of which four are on their way (80 KiB a CU: 2 us of what HBM gives it), and the first steps of a turn are on their way
-// while the turn before stores: no turn waits for memory by itself, as the shared expert's tiles behind all others did.  A
-// step's fragments are read while the step before multiplies.  All turns are looked up at the start, a lane each.
-// 2048 wide, up + down in us, moe_tile_kernel first: 32 experts of 1408, 2 of them and 2816 shared, 80 rows 137, 125, 300 rows
-// 135, 123; 64 experts of 1408, 6 and 2816 shared, 128 rows 239, 229, 300 rows 245, 240; where it ends: moe_tile (moe.h).
-constexpr int kRingSlots = kMoeRingTile, kRingStages = 6, kRingCopies = 3;
-struct alignas(16) Turn {
-  int64_t w;                // bytes to the block's first W tile
-  int s0, s1, steps, left;  // slots s0 .. s1 - 1, k-steps, W tiles from the first one on
-  int block, e;
-};
-constexpr int kRingStep = 16 * 1024 + kRingSlots * 64;       // 1 KiB fragments of W, then of slots
-constexpr int kRingResults = kRingStages * kRingStep;        // 2 KiB a wave
-constexpr int kRingTokens = kRingResults + 8 * 2048;         // its 16 slots' rows, 256 bytes a wave
-constexpr int kRingWeights = kRingTokens + 8 * 256;          // weights of the slots of this turn and of the next one
-constexpr int kRingTable = kRingWeights + 2 * kRingSlots * 4;
-constexpr int kRingLds = kRingTable + kTurns * (int)sizeof(Turn) + 16;
-static_assert(kRingLds <= 160 * 1024, "a CU's LDS");
-
-// Reads of LDS beside copies to it: in one block with their wait (behind an ordinary read the compiler waits for all copies).
-__device__ __forceinline__ uint32_t lds_at(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
-}
-__device__ __forceinline__ uint32_t lds_word(const void* p) {
-  uint32_t v;
-  asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(lds_at(p)) : "memory");
-  return v;
+// 16 bytes a lane to consecutive LDS
+__device__ __forceinline__ void to_lds16(const char* from, void* dst) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
+                                   (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
 
-template <int PRODUCT>
-__global__ __launch_bounds__(512, 2) void moe_ring_kernel(const MoeParams p, const int blocks_first, const int blocks_last) {
+// Prompts: 64 NT W rows x up to 128 slots a workgroup, a wave 16 NT x 128, two workgroups a CU, a unit each.  W goes straight to the
+// operand registers of the one wave that uses it, slots by way of LDS.
+// NT = 4.  With many slots the chip's power bounds it: 1.8 GHz at 55 % of the MFMA cycles, where the library's plain product of
+// 49152 x 2816 x 2048 runs at 1.06 to 1.27 PFLOP/s and this one (8192 rows, 6 of 64 experts) at 0.98 to 1.01; 256 slots a workgroup,
+// both operands through LDS, were no faster.  Between 128 and 400 slots an expert neither memory (4.3 TB/s of weights), the L1, LDS
+// nor MFMA (each near 40 %) is at its limit by itself; one workgroup a CU that goes on from unit to unit, with 8 steps of weights on
+// their way, was slower (1943 rows, 6 of 64 experts of 1408, up: 237 us; 262 with 8 waves, 322 with 4).
+// NT = 2 where units of NT = 4 are fewer than one and a half a CU: a step costs less and eight of them, not four, are under way, so
+// that the memory's latency bounds a walk no more.  Going down 1408 (a shared expert 2816) -> 2048, 2 of 32 experts, us with NT = 4
+// and 2: 300 rows 68, 51; 1000 rows 68, 56; where units are more, going up the same: 300 rows 70, 78; 1000 rows 102, 109.
+// Slots' chunks trade places by bit 3 of the slot: LDS reads 16 bytes for lanes 0-3, 12-15, 20-27 at a time (by bits 2 and 3, half
+// of its cycles were conflicts).
+constexpr int kStageBytes = kMoeTile * 64;  // of 32 of K: 16-slot groups of 1 KiB
+
+constexpr int tile_stages(int NT) { return NT == 4 ? 4 : 8; }
+template <int PRODUCT, bool ONCE, int NT>
+__device__ __forceinline__ void tile_product(const MoeParams& p, const TileWork& t, char (*ring)[kStageBytes]) {
   constexpr bool UP = PRODUCT != kMoeDown;
-  constexpr int S = kRingStages;
-  extern __shared__ __attribute__((aligned(16))) char ring[];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int g = lane >> 4, c = lane & 15;
-  Turn* const table = reinterpret_cast<Turn*>(ring + kRingTable);
-  int* const found = reinterpret_cast<int*>(ring + kRingTable + kTurns * sizeof(Turn));
-  if (wave == 0) {
-    const TileWork t = tile_work<PRODUCT, kRingSlots>(p, blocks_first, blocks_last, lane);
-    const uint64_t any = __ballot(t.any);
-    if (t.any)
-      table[__popcll(any & ((1ull << lane) - 1))] =
-          Turn{(p.w_offset[t.e] + (int64_t)t.block * kTileW * t.steps * 512) * 2, t.s0, t.s1, t.steps,
-               t.ntiles - t.block * kTileW, t.block, t.e};
-    if (lane == 0) *found = __popcll(any);
-  }
-  __syncthreads();
-  const int turns = __builtin_amdgcn_readfirstlane(*found);
-  if (turns == 0) return;
-  const int64_t ld = (int64_t)(UP ? p.width : p.ff_max) * 2;
-  const int wm = wave & 1, wn = wave >> 1, group = wave & 3;  // (two waves copy a group of slots alike)
-
-  struct Work {           // the same in all lanes, but for x
-    const char *w0, *w1;  // this wave's W tiles of a step
-    int s0, s1, steps, left, block, e;
-    const char* x;        // the lane's piece of a step's slots
-  };
-  auto turn_at = [&](int i) __attribute__((always_inline)) {
-    e_u32x4_t u, v;
-    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:16\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(u), "=&v"(v) : "v"(lds_at(table + i)) : "memory");
-    auto one = [](uint32_t z) { return (int)__builtin_amdgcn_readfirstlane((int)z); };
-    Work t;
-    t.s0 = one(u.z), t.s1 = one(u.w), t.steps = one(v.x), t.left = one(v.y), t.block = one(v.z), t.e = one(v.w);
-    const char* w = (const char*)p.w + ((int64_t)one(u.y) << 32 | (uint32_t)one(u.x));
-    t.w0 = w + (int64_t)min(wave * 2, t.left - 1) * t.steps * 1024;
-    t.w1 = w + (int64_t)min(wave * 2 + 1, t.left - 1) * t.steps * 1024;
-    return t;
-  };
-  char* const tokens = ring + kRingTokens + wave * 256;
-  auto ask = [&](const Work& t, int i) __attribute__((always_inline)) {  // older than the copies after it: there once they are
-    if constexpr (UP) {
-      to_lds4((const char*)p.token, (uint32_t)min(t.s0 + group * 16 + c, t.s1 - 1) * 4, tokens);
-      if (p.slot_weight != nullptr && wave == 0)
-        to_lds4((const char*)p.slot_weight, (uint32_t)min(t.s0 + lane, t.s1 - 1) * 4, ring + kRingWeights + (i & 1) * kRingSlots * 4);
-    }
-  };
-  auto take = [&](Work& t) __attribute__((always_inline)) {
-    const int64_t row = UP ? min(max((int)lds_word(tokens + (lane >> 2) * 4), 0), p.rows - 1)
-                           : min(t.s0 + group * 16 + (lane >> 2), t.s1 - 1);
-    t.x = (const char*)p.x + row * ld + ((lane & 3) ^ ((lane >> 4) & 2)) * 16;  // (chunks trade places against bank conflicts)
-  };
-  const uint32_t lane16 = lane * 16;
-  const char* const wread = ring + wm * 8192 + lane * 16;
-  const char* const xread = ring + 16 * 1024 + wn * 1024 + c * 64 + ((g ^ ((c >> 2) & 2)) * 16);
-  auto arrive = [&]() __attribute__((always_inline)) {
-    // loads retire in order: with only the youngest three steps' outstanding, the next one's have landed ...
-    __builtin_amdgcn_s_waitcnt((S - 3) * kRingCopies | (7 << 4) | (15 << 8));
-    asm volatile("s_barrier" ::: "memory");  // ... for every wave; and everyone has read the stage that is filled next
-  };
-  e_f32x4_t acc[8][1];
-  e_u32x4_t a[2][8], x[2];
-  auto read = [&](int stage, int i, int par) __attribute__((always_inline)) {
-    if (i < 8) a[par][i] = *reinterpret_cast<const e_u32x4_t*>(wread + stage + i * 1024);
-    else x[par] = *reinterpret_cast<const e_u32x4_t*>(xread + stage);
-  };
-
-  Work now = turn_at(0), next;
-  ask(now, 0);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  take(now);
-  auto copy = [&](int k, int stage, int j) __attribute__((always_inline)) {  // behind the last step: of the next turn's
-    const bool over = k >= now.steps;
-    if (over) k = min(k - now.steps, next.steps - 1);
-    if (j < 2) to_lds16_past((over ? j ? next.w1 : next.w0 : j ? now.w1 : now.w0) + k * 1024, lane16, ring + stage + (wave * 2 + j) * 1024);
-    else to_lds16((over ? next.x : now.x) + k * 64, 0, ring + stage + (16 + group) * 1024);
-  };
-  next = now;
-  auto after = [&](int stage) __attribute__((always_inline)) { return stage == (S - 1) * kRingStep ? 0 : stage + kRingStep; };
-  auto before = [&](int stage) __attribute__((always_inline)) { return stage == 0 ? (S - 1) * kRingStep : stage - kRingStep; };
-  int stage = 0;      // of the current step
-  bool alone = true;  // no turn before has copied this one's first steps, or not all of them
-  for (int i = 0;; ++i) {
-    if (alone || now.steps < S) {
-      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-      int to = stage;
-#pragma unroll
-      for (int k = 0; k < S - 1; ++k, to = after(to))
-#pragma unroll
-        for (int j = 0; j < kRingCopies; ++j) copy(k, to, j);
-    }
-    alone = now.steps < S;
-    const bool more = i + 1 < turns;
-    auto step = [&](int k, int par) __attribute__((always_inline)) {
-      arrive();
-      const int ahead = after(stage), fill = before(stage);
-#pragma unroll
-      for (int n = 0; n < 8; ++n) {
-        if ((n & 1) == 0 && n / 2 < kRingCopies) copy(k + S - 1, fill, n / 2);
-        read(ahead, n == 0 ? 8 : n, par ^ 1);
-        acc[n][0] = moe_mfma(a[par][n], x[par], acc[n][0]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      read(ahead, 0, par ^ 1);
-      stage = ahead;
-    };
-    int k = 0;
-    auto run_to = [&](int end) __attribute__((always_inline)) {
-      for (; k + 2 <= end; k += 2) {
-        step(k, 0);
-        step(k + 1, 1);
-      }
-    };
-#pragma unroll
-    for (int n = 0; n < 8; ++n) acc[n][0] = e_f32x4_t{0.f, 0.f, 0.f, 0.f};
-    arrive();
-#pragma unroll
-    for (int j = 0; j < 9; ++j) read(stage, j, 0);
-    if (more) {
-      next = turn_at(i + 1);
-      ask(next, i + 1);
-      run_to(min(2 * S, now.steps - S));
-      if (k < S) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      take(next);
-    } else {  // (none: this one's first steps again, and nobody reads them)
-      next = now;
-    }
-    run_to(now.steps);
-    if (k < now.steps) step(k, 0);
-    tile_store<PRODUCT, 8, 1>(p, now.e, acc, ring + kRingResults + wave * 2048, now.block * kTileW + wm * 8,
-                              now.block * kTileW + now.left, now.s0 + wn * 16, 0, now.s1, [&](int slot) {
-      return p.slot_weight == nullptr ? 1.f
-                                      : __builtin_bit_cast(float, lds_word(ring + kRingWeights + ((i & 1) * kRingSlots + slot - now.s0) * 4));
-    });
-    if (!more) break;
-    now = next;
-  }
-  __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // (no copy to LDS outlives the workgroup)
-}
-
-// More slots an expert: 256 W rows x 128 slots a workgroup, a wave 64 x 128, two workgroups a CU, a turn each.  W goes straight to
-// the operand registers of the one wave that uses it.  The chip's power bounds it with many slots: 1.6 GHz at half of the MFMA
-// cycles, where the library's plain product of 49152 x 2816 x 2048 runs at 1.06 to 1.27 PFLOP/s and this one (8192 rows, 6 of 64
-// experts) at 0.95 to 0.99, 0.90 to 0.96 before results went by way of LDS; 256 slots a workgroup, both operands through LDS, were
-// no faster.  Slots' chunks
-// trade places by bit 3 of the slot: LDS reads 16 bytes for lanes 0-3, 12-15, 20-27 at a time (by bits 2 and 3, half of its
-// cycles were conflicts).
-constexpr int kStages = 4, kStageBytes = kMoeTile * 64;  // of 32 of K: 16-slot groups of 1 KiB
-
-template <int PRODUCT>
-__global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, const int blocks_first, const int blocks_last) {
-  constexpr bool UP = PRODUCT != kMoeDown;
-  __shared__ __attribute__((aligned(16))) char ring[kStages][kStageBytes];
-  const TileWork t = tile_work<PRODUCT, kMoeTile>(p, blocks_first, blocks_last, 0);
-  if (!t.any) return;
+  constexpr int S = tile_stages(NT), kOlder = (S - 2) * (NT + 2);
   const int e = t.e, s0 = t.s0, s1 = t.s1, block = t.block, steps = t.steps, ntiles = t.ntiles;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
   const int64_t ld = UP ? p.width : p.ff_max;
-  const int nt0 = block * kTileW + wave * 4;
+  const int nt0 = (block * 4 + wave) * NT;
   // this wave's W tiles, and the two 16-slot groups it copies: lane l moves chunk l % 4, exchanged by slot / 4, of slot l / 4
-  const uint16_t *wsrc[4], *xsrc[2];
+  const uint16_t *wsrc[NT], *xsrc[2];
   const uint16_t* w = (const uint16_t*)p.w + p.w_offset[e] + lane * 8;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) wsrc[j] = w + (int64_t)min(nt0 + j, ntiles - 1) * steps * 512;
+  for (int j = 0; j < NT; ++j) wsrc[j] = w + (int64_t)min(nt0 + j, ntiles - 1) * steps * 512;
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int slot = min(s0 + (wave * 2 + j) * 16 + (lane >> 2), s1 - 1);
     const int64_t row = UP ? min(max(p.token[slot], 0), p.rows - 1) : slot;
     xsrc[j] = (const uint16_t*)p.x + row * ld + ((lane & 3) ^ ((lane >> 4) & 2)) * 8;
   }
-  e_u32x4_t a[kStages][4];
+  e_u32x4_t a[S][NT];
   auto issue = [&](int k, int stage) __attribute__((always_inline)) {  // (past the end: the last step once more)
     k = min(k, steps - 1);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) to_lds16((const char*)(xsrc[j] + k * 32), 0, ring[stage] + (wave * 2 + j) * 1024);
+    for (int j = 0; j < 2; ++j) to_lds16((const char*)(xsrc[j] + k * 32), ring[stage] + (wave * 2 + j) * 1024);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) a[stage][j] = *reinterpret_cast<const e_u32x4_t*>(wsrc[j] + k * 512);
+    for (int j = 0; j < NT; ++j) a[stage][j] = load_weights<ONCE>(wsrc[j] + k * 512);
   };
   constexpr int MT = kMoeTile / 16;
   const int xoff = c * 64 + ((g ^ ((c >> 2) & 2)) * 16);
-  e_f32x4_t acc[4][MT];
+  e_f32x4_t acc[NT][MT];
 #pragma unroll
-  for (int n = 0; n < 4; ++n)
+  for (int n = 0; n < NT; ++n)
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[n][m] = e_f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto step = [&](int k, int stage) __attribute__((always_inline)) {
-    // loads retire in order: with only the two younger steps' six each outstanding, this one's have landed
-    __builtin_amdgcn_s_waitcnt(12 | (7 << 4) | (15 << 8));
-    asm volatile("s_barrier" ::: "memory");  // ... for every wave; and everyone is done with the stage that is filled next
-    issue(k + 3, (stage + 3) % kStages);
+  auto multiply = [&](int stage) __attribute__((always_inline)) {
     e_u32x4_t x[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) x[m] = *reinterpret_cast<const e_u32x4_t*>(ring[stage] + xoff + m * 1024);
@@ -455,24 +285,41 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, con
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-      for (int n = 0; n < 4; ++n) acc[n][m] = moe_mfma(a[stage][n], x[m], acc[n][m]);
+      for (int n = 0; n < NT; ++n) acc[n][m] = moe_mfma(a[stage][n], x[m], acc[n][m]);
   };
-  issue(0, 0);
-  issue(1, 1);
-  issue(2, 2);
-  int k = 0;
-  for (; k + 4 <= steps; k += 4) {
-    step(k, 0);
-    step(k + 1, 1);
-    step(k + 2, 2);
-    step(k + 3, 3);
+#pragma unroll
+  for (int k = 0; k < S - 1; ++k) {
+    issue(k, k);
+    asm volatile("" ::: "memory");  // (in this order: the steps count what is outstanding)
   }
-  if (k < steps) step(k, 0);
-  if (k + 1 < steps) step(k + 1, 1);
-  if (k + 2 < steps) step(k + 2, 2);
-  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // (no copy to LDS is under way, and everyone has read the last stage)
-  tile_store<PRODUCT, 4, MT>(p, e, acc, ring[wave], block * kTileW + wave * 4, ntiles, s0, 16, s1,
+  int k = 0;
+  for (; k + S <= steps; k += S)
+#pragma unroll
+    for (int j = 0; j < S; ++j) {
+      // loads retire in order: with only the younger steps' outstanding, this one's have landed; what was read, too
+      __builtin_amdgcn_s_waitcnt((kOlder & 15) | (kOlder >> 4) << 14 | (7 << 4));
+      asm volatile("s_barrier" ::: "memory");  // ... for every wave; and everyone is done with the stage that is filled next
+      issue(k + j + S - 1, (j + S - 1) % S);
+      multiply(j);
+    }
+  if (k < steps) {  // the rest is on its way (a count would not do: loads that nothing uses any more are not made)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < S - 1; ++j)
+      if (k + j < steps) multiply(j);
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (no copy to LDS is under way, and everyone has read the last stage)
+  tile_store<PRODUCT, NT, MT>(p, e, acc, ring[wave], nt0, ntiles, s0, 16, s1,
                              [&](int slot) { return slot_weight_of(p, min(slot, s1 - 1)); });
+}
+
+template <int PRODUCT, int NT>
+__global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, const int blocks_first, const int blocks_last) {
+  __shared__ __attribute__((aligned(16))) char ring[tile_stages(NT)][kStageBytes];
+  const TileWork t = tile_work<PRODUCT, kMoeTile, 4 * NT>(p, blocks_first, blocks_last, 0);
+  if (!t.any) return;
+  if (t.once) tile_product<PRODUCT, true, NT>(p, t, ring);
+  else tile_product<PRODUCT, false, NT>(p, t, ring);
 }
 
 // The router's logits on packed weights (experts and the shared gate, up to a multiple of 16 rows): 16 rows of h and a share
@@ -676,22 +523,25 @@ static void go(const MoeParams& p, hipStream_t s) {
     else if (wgs <= 512) hipLaunchKernelGGL((moe_stream_kernel<PRODUCT, 2>), dim3((units + 1) / 2, t), dim3(256), smem, s, p);
     else hipLaunchKernelGGL((moe_stream_kernel<PRODUCT, 1>), dim3((units + 3) / 4, t), dim3(256), smem, s, p);
   } else {
-    auto blocks = [&](int ff) { return ((GATED ? ff / 8 : (UP ? ff : p.width) / 16) + kTileW - 1) / kTileW; };
-    const int first = blocks(p.ff_first), last = blocks(p.ff_last);
-    const int tile = moe_tile(true, p.rows, p.slots, p.experts);
-    // more tiles than there are of 64 slots: they may be of 16 (a router that is not packed), which either body takes as well
-    const bool small = p.max_tiles >= p.slots || p.max_tiles > p.slots / kMoeRingTile + p.experts;
+    const int tile = moe_tile(true, p.rows);
+    // more tiles than there are of 64 slots: they may be of 16 (a router that is not packed), which the body takes as well
+    const bool small = p.max_tiles >= p.slots || p.max_tiles > p.slots / kMoeCountedTile + p.experts;
     const int least = small ? kMoeSmallTile : tile;
     const int64_t tiles = small ? p.max_tiles : std::min<int64_t>(p.max_tiles, p.slots / tile + p.experts);
     const int64_t last_tiles = (p.rows + least - 1) / least;  // a token takes an expert once
-    if (tile == kRingSlots) {
-      const unsigned grid = (unsigned)ring_workgroups(tiles * first, last_tiles * last, solo_units(UP, p.ff_first, p.ff_last));
-      (void)hipFuncSetAttribute((const void*)moe_ring_kernel<PRODUCT>, hipFuncAttributeMaxDynamicSharedMemorySize, kRingLds);
-      hipLaunchKernelGGL((moe_ring_kernel<PRODUCT>), dim3(grid), dim3(512), kRingLds, s, p, first, last);
-    } else {
+    auto launch = [&](auto nt) {
+      constexpr int NT = decltype(nt)::value;
+      auto blocks = [&](int ff) { return ((GATED ? ff / 8 : (UP ? ff : p.width) / 16) + 4 * NT - 1) / (4 * NT); };
+      const int first = blocks(p.ff_first), last = blocks(p.ff_last);
+      if (NT == 4) {  // with as many slots for each expert
+        const int64_t each = (p.slots + (int64_t)p.experts * least - 1) / ((int64_t)p.experts * least);
+        if (p.experts * each * first + last_tiles * last <= 384) return false;
+      }
       const unsigned grid = (unsigned)unit_workgroups(tiles * first, last_tiles * last);
-      hipLaunchKernelGGL((moe_tile_kernel<PRODUCT>), dim3(grid), dim3(256), 0, s, p, first, last);
-    }
+      hipLaunchKernelGGL((moe_tile_kernel<PRODUCT, NT>), dim3(grid), dim3(256), 0, s, p, first, last);
+      return true;
+    };
+    if (!launch(std::integral_constant<int, 4>{})) launch(std::integral_constant<int, 2>{});
   }
 }
 

@@ -7,7 +7,7 @@
 
 namespace lvllm {
 
-constexpr int kTurns = 64;  // of a workgroup of the ring, which looks them all up at once, a lane each
+constexpr int kTurns = 64;  // of a workgroup, at most
 
 // Units of the other experts that take as long as one of the last expert's (going down, k-steps are the experts' inner size).  At
 // most kMostSolo, however large the last expert is: a workgroup may have that many turns more than its share.
@@ -45,7 +45,7 @@ __host__ __device__ inline TurnUnit turn_unit(int units_first, int units_last, i
 inline int64_t unit_workgroups(int64_t units_first, int64_t units_last) {
   return 8 * ((units_first + 7) / 8 + (units_last + 7) / 8);
 }
-// The ring's: a workgroup a CU, more only where one might have over kTurns turns.  With `share` units each, every unit has a turn
+// A launch with several units a workgroup: a workgroup a CU, more only where one might have over kTurns turns.  With `share` units each, every unit has a turn
 // below kTurns: a workgroup without a last turn of the last expert's takes at most `solo` units by itself first, and what comes
 // before and after those is floor(last expert's / cus) + ceil(the others' / cus) <= share; one with that turn takes share + 1.
 inline int64_t ring_workgroups(int64_t units_first, int64_t units_last, int solo) {

@@ -65,6 +65,61 @@ def test_products(amd, counts, ff, width, act, weigh):
         assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5).all(), (e, (got - want).abs().max())
 
 
+@pytest.mark.parametrize("act", [0, 2], ids=["clamped", "relu_squared"])
+@pytest.mark.parametrize("copies", [1, 70], ids=["half blocks", "whole blocks"])
+def test_blocks_of_weight_rows(amd, copies, act):
+    """Blocks of 128 and of 256 weight rows a workgroup (few and many units), at their edges: inner sizes around 128 and 256 outputs, walks of
+    1 to 12 k-steps around the steps under way (8 and 4), experts with one tile of slots (weights past the caches) and with several."""
+    g, gated = torch.Generator(device=DEV).manual_seed(copies), act == 0
+    counts, ff, width = [129, 128, 127, 1, 0, 65] * copies, [32, 96, 128, 160, 288, 384] * copies, 288
+    experts, rows, top = len(counts), sum(counts), 1
+    # units of whole blocks, slots spread evenly: where the line lies
+    units = experts * -(-rows // (128 * experts)) * -(-384 // (128 if gated else 256)) + -(-rows // 128) * -(-384 // (128 if gated else 256))
+    assert (units > 384) == (copies > 1)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
+    of_row = torch.repeat_interleave(torch.arange(experts, device=DEV), torch.tensor(counts, device=DEV))
+    of_row = of_row[torch.randperm(rows, generator=g, device=DEV)]
+    # two whole numbers name an expert: 2 a x - a^2 + 2 b y - b^2 is largest at (x, y) = (a, b), and exact
+    marks = torch.zeros(experts, width, device=DEV)
+    e = torch.arange(experts, device=DEV)
+    marks[:, 0], marks[:, 1], marks[:, 2] = 2 * (e // 21), 2 * (e % 21), -((e // 21) ** 2 + (e % 21) ** 2)
+    h = torch.zeros(rows, width, device=DEV)
+    h[:, 0], h[:, 1], h[:, 2] = of_row // 21, of_row % 21, 1
+    assert bool((marks.bfloat16().float() == marks)[:, :2].all())
+    x = 0.5 * rand(rows, width)
+    hi = marks[:, 2].bfloat16().float()
+    marks[:, 3], marks[:, 2], h[:, 3] = marks[:, 2] - hi, hi, 1  # (a square in two parts of 8 bits)
+    router = torch.nn.functional.pad(marks, (0, 0, 0, -experts % 16)).bfloat16()
+    ids, _, offsets, token, slots, tiles, _ = amd.moe_route(h.bfloat16(), amd.pack_weight(router), None, top, False, True, experts, False, 1)
+    assert torch.equal(ids[:, 0].long(), of_row)
+    from light_vllm_amd.engine.moe import interleave_16
+    gate, up = ([rand(n, width) * width ** -0.5 for n in ff] for _ in "gu")
+    down = [rand(width, n) * n ** -0.5 for n in ff]
+
+    def packed(parts):
+        parts = [amd.pack_weight(p.contiguous()).reshape(-1) for p in parts]
+        return torch.cat(parts), torch.tensor([0] + [p.numel() for p in parts[:-1]]).cumsum(0).to(DEV)
+    sizes = rows, width, max(ff), max(ff[:-1]), ff[-1]
+    ffs, limits = torch.tensor(ff, dtype=torch.int32, device=DEV), torch.full((experts,), 1.1, device=DEV)
+    w_up, up_at = packed([interleave_16(a, b) if gated else b for a, b in zip(gate, up)])
+    w_down, down_at = packed(down)
+    a = amd.moe_experts(x, w_up, up_at, ffs, limits, offsets, token, tiles, *sizes, True, True, None, act)
+    y = amd.moe_experts(a, w_down, down_at, ffs, None, offsets, token, tiles, *sizes, False, True)
+    for i in [*range(min(experts, 24)), *range(max(experts - 12, 24), experts)]:
+        r = (of_row == i).nonzero()[:, 0]
+        s, u = slots[r, 0].long(), x[r].double() @ up[i].double().T.contiguous()
+        if gated:
+            p = (x[r].double() @ gate[i].double().T.contiguous()).clamp(max=1.1)
+            want = p * torch.sigmoid(1.702 * p) * (u.clamp(-1.1, 1.1) + 1)
+        else:
+            want = u.clamp(min=0).square()
+        got = a[s, :ff[i]].double()
+        # one rounding to 8 bits behind fp32 sums of at most 384 products of values around 1
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5).all(), (i, (got - want).abs().max())
+        want = got @ down[i].double().T.contiguous()
+        assert ((y[s].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5).all(), (i, (y[s] - want).abs().max())
+
+
 @pytest.mark.parametrize("act,weigh", [("clamped", False), ("silu", True), ("relu_squared", True)])
 @pytest.mark.parametrize("width", [4096, 224, 64])
 def test_many_turns_a_workgroup(amd, width, act, weigh):
