@@ -86,7 +86,7 @@ __global__ __launch_bounds__(256 * CT, 1) void latent_attention_mfma_kernel(cons
     for (int j = 0; j < COPIES; ++j)
       if (j * CT + ct < NK)
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + from[j]),
-                                         (__attribute__((address_space(3))) void*)(dst + (j * CT + ct) * 1024), 16, 0, 0);
+                                         (__attribute__((address_space(3))) void*)(dst + (j * CT + ct) * 1024), 16, 0, 2);  // (past the caches)
   };
   m_u32x4_t qf[NK];
   {
