@@ -238,84 +238,107 @@ __device__ __forceinline__ void to_lds16(const char* from, void* dst) {
 // and 2: 300 rows 68, 51; 1000 rows 68, 56; where units are more, going up the same: 300 rows 70, 78; 1000 rows 102, 109.
 // Slots' chunks trade places by bit 3 of the slot: LDS reads 16 bytes for lanes 0-3, 12-15, 20-27 at a time (by bits 2 and 3, half
 // of its cycles were conflicts).
-constexpr int kStageBytes = kMoeTile * 64;  // of 32 of K: 16-slot groups of 1 KiB
-
-constexpr int tile_stages(int NT) { return NT == 4 ? 4 : 8; }
+constexpr int kStageBytes = kMoeTile * 128;  // two k-steps of 32: a slot's 128 bytes, 8 slots a copy
+constexpr int tile_steps(int NT) { return NT == 4 ? 4 : 8; }  // k-steps of weights in registers; half as many stages of slots
 template <int PRODUCT, bool ONCE, int NT>
 __device__ __forceinline__ void tile_product(const MoeParams& p, const TileWork& t, char (*ring)[kStageBytes]) {
   constexpr bool UP = PRODUCT != kMoeDown;
-  constexpr int S = tile_stages(NT), kOlder = (S - 2) * (NT + 2);
+  constexpr int S = tile_steps(NT), X = S / 2, MT = kMoeTile / 16, kCopies = kMoeTile / 32;
+  constexpr int kYounger = (X - 2) * kCopies + (X - 1) * 2 * NT;  // loads behind a stage's copies when it is needed
+  constexpr int kBehind = (X - 1) * kCopies + (S - 1) * NT;       // ... behind a second k-step's weights
   const int e = t.e, s0 = t.s0, s1 = t.s1, block = t.block, steps = t.steps, ntiles = t.ntiles;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
   const int64_t ld = UP ? p.width : p.ff_max;
   const int nt0 = (block * 4 + wave) * NT;
-  // this wave's W tiles, and the two 16-slot groups it copies: lane l moves chunk l % 4, exchanged by slot / 4, of slot l / 4
-  const uint16_t *wsrc[NT], *xsrc[2];
+  // this wave's W tiles, and the slots it copies: lane l moves chunk l % 8, exchanged by the slot, of slot l / 8 of eight
+  const uint16_t *wsrc[NT], *xsrc[kCopies];
   const uint16_t* w = (const uint16_t*)p.w + p.w_offset[e] + lane * 8;
 #pragma unroll
   for (int j = 0; j < NT; ++j) wsrc[j] = w + (int64_t)min(nt0 + j, ntiles - 1) * steps * 512;
+  const int chunk = (lane & 7) ^ (lane >> 3);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int slot = min(s0 + (wave * 2 + j) * 16 + (lane >> 2), s1 - 1);
+  for (int j = 0; j < kCopies; ++j) {
+    const int slot = min(s0 + (wave * kCopies + j) * 8 + (lane >> 3), s1 - 1);
     const int64_t row = UP ? min(max(p.token[slot], 0), p.rows - 1) : slot;
-    xsrc[j] = (const uint16_t*)p.x + row * ld + ((lane & 3) ^ ((lane >> 4) & 2)) * 8;
+    xsrc[j] = (const uint16_t*)p.x + row * ld;
   }
   e_u32x4_t a[S][NT];
-  auto issue = [&](int k, int stage) __attribute__((always_inline)) {  // (past the end: the last step once more)
+  auto copy = [&](int k, int stage) __attribute__((always_inline)) {  // of k-steps k and k + 1 (a missing one: the one before)
+    k = min(k, (steps - 1) & ~1);
+    const int at = k * 32 + (k + 1 < steps ? chunk : chunk & 3) * 8;
+#pragma unroll
+    for (int j = 0; j < kCopies; ++j) to_lds16((const char*)(xsrc[j] + at), ring[stage] + (wave * kCopies + j) * 1024);
+    asm volatile("" ::: "memory");  // (in this order: what is outstanding is counted)
+  };
+  auto fetch = [&](int k, int at) __attribute__((always_inline)) {  // (past the end: the last step once more)
     k = min(k, steps - 1);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) to_lds16((const char*)(xsrc[j] + k * 32), ring[stage] + (wave * 2 + j) * 1024);
-#pragma unroll
-    for (int j = 0; j < NT; ++j) a[stage][j] = load_weights<ONCE>(wsrc[j] + k * 512);
+    for (int j = 0; j < NT; ++j) a[at][j] = load_weights<ONCE>(wsrc[j] + k * 512);
+    asm volatile("" ::: "memory");
   };
-  constexpr int MT = kMoeTile / 16;
-  const int xoff = c * 64 + ((g ^ ((c >> 2) & 2)) * 16);
   e_f32x4_t acc[NT][MT];
 #pragma unroll
   for (int n = 0; n < NT; ++n)
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[n][m] = e_f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](int stage) __attribute__((always_inline)) {
-    e_u32x4_t x[MT];
+  const int xoff[2] = {c * 128 + ((g ^ (c & 7)) * 16), c * 128 + (((4 + g) ^ (c & 7)) * 16)};
+  auto multiply = [&](int at) __attribute__((always_inline)) {
+    constexpr int W = NT == 4 ? 5 : MT;  // fragments read ahead
+    e_u32x4_t x[W];
+    auto read = [&](int m) { x[m % W] = *reinterpret_cast<const e_u32x4_t*>(ring[at / 2] + xoff[at & 1] + m * 2048); };
 #pragma unroll
-    for (int m = 0; m < MT; ++m) x[m] = *reinterpret_cast<const e_u32x4_t*>(ring[stage] + xoff + m * 1024);
+    for (int m = 0; m < W; ++m) read(m);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < MT; ++m) {
 #pragma unroll
-      for (int n = 0; n < NT; ++n) acc[n][m] = moe_mfma(a[stage][n], x[m], acc[n][m]);
+      for (int n = 0; n < NT; ++n) acc[n][m] = moe_mfma(a[at][n], x[m % W], acc[n][m]);
+      if (m + W < MT) read(m + W);
+      if (W < MT) __builtin_amdgcn_sched_barrier(0);
+    }
   };
 #pragma unroll
-  for (int k = 0; k < S - 1; ++k) {
-    issue(k, k);
-    asm volatile("" ::: "memory");  // (in this order: the steps count what is outstanding)
+  for (int j = 0; j < X - 1; ++j) {
+    copy(2 * j, j);
+    fetch(2 * j, 2 * j);
+    fetch(2 * j + 1, 2 * j + 1);
   }
+  fetch(S - 2, S - 2);
   int k = 0;
   for (; k + S <= steps; k += S)
 #pragma unroll
-    for (int j = 0; j < S; ++j) {
-      // loads retire in order: with only the younger steps' outstanding, this one's have landed; what was read, too
-      __builtin_amdgcn_s_waitcnt((kOlder & 15) | (kOlder >> 4) << 14 | (7 << 4));
+    for (int j = 0; j < X; ++j) {
+      // loads retire in order: with only the younger ones outstanding, this stage's have landed; what was read, too
+      __builtin_amdgcn_s_waitcnt((kYounger & 15) | (kYounger >> 4) << 14 | (7 << 4));
       asm volatile("s_barrier" ::: "memory");  // ... for every wave; and everyone is done with the stage that is filled next
-      issue(k + j + S - 1, (j + S - 1) % S);
-      multiply(j);
+      copy(k + 2 * (j + X - 1), (j + X - 1) % X);
+      fetch(k + 2 * j + S - 1, (2 * j + S - 1) % S);
+      multiply(2 * j);
+      fetch(k + 2 * j + S, 2 * j);
+      __builtin_amdgcn_s_waitcnt((kBehind & 15) | (kBehind >> 4) << 14 | (7 << 4) | (15 << 8));  // (the compiler would wait for all)
+      multiply(2 * j + 1);
     }
-  if (k < steps) {  // the rest is on its way (a count would not do: loads that nothing uses any more are not made)
+  if (k < steps) {  // the rest, but for its last stage, is on its way (a count would not do: loads that nothing uses are not made)
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (steps - k == S - 1) copy(k + S - 2, X - 1);
 #pragma unroll
-    for (int j = 0; j < S - 1; ++j)
+    for (int j = 0; j < S - 2; ++j)
       if (k + j < steps) multiply(j);
+    if (steps - k == S - 1) {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      multiply(S - 2);
+    }
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (no copy to LDS is under way, and everyone has read the last stage)
-  tile_store<PRODUCT, NT, MT>(p, e, acc, ring[wave], nt0, ntiles, s0, 16, s1,
+  tile_store<PRODUCT, NT, MT>(p, e, acc, ring[0] + wave * 2048, nt0, ntiles, s0, 16, s1,
                              [&](int slot) { return slot_weight_of(p, min(slot, s1 - 1)); });
 }
 
 template <int PRODUCT, int NT>
 __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, const int blocks_first, const int blocks_last) {
-  __shared__ __attribute__((aligned(16))) char ring[tile_stages(NT)][kStageBytes];
+  __shared__ __attribute__((aligned(16))) char ring[tile_steps(NT) / 2][kStageBytes];
   const TileWork t = tile_work<PRODUCT, kMoeTile, 4 * NT>(p, blocks_first, blocks_last, 0);
   if (!t.any) return;
   if (t.once) tile_product<PRODUCT, true, NT>(p, t, ring);
