@@ -201,17 +201,23 @@ __device__ __forceinline__ void moe_running_sums(const int* count, int* first, i
   if (threadIdx.x == 0) { first[experts] = base; tile0[experts] = tbase; }
 }
 
+// Slots of each of an expert's n tiles (the last one has what is left): as even as groups of 16 allow, so that no tile multiplies
+// for many slots that are not there (182 slots in tiles of 128: 96 + 86 for 128 + 54).
+__device__ __forceinline__ int moe_tile_slots(int count, int n) { return ((count + n - 1) / n + 15) / 16 * 16; }
+
 // offsets and tiles, by the whole workgroup
 __device__ __forceinline__ void moe_write_tiles(const int* first, const int* tile0, int experts, const MoeGroups& out) {
   int32_t* tiles = out.tiles;
   for (int e = threadIdx.x; e <= experts; e += blockDim.x) out.offsets[e] = first[e];
-  for (int e = threadIdx.x; e < experts; e += blockDim.x)
+  for (int e = threadIdx.x; e < experts; e += blockDim.x) {
+    const int n = tile0[e + 1] - tile0[e], size = n > 0 ? moe_tile_slots(first[e + 1] - first[e], n) : 0;
     for (int t = tile0[e]; t < tile0[e + 1] && t < out.max_tiles; ++t) {
       tiles[4 * t] = e;
-      tiles[4 * t + 1] = first[e] + (t - tile0[e]) * out.tile;
+      tiles[4 * t + 1] = first[e] + (t - tile0[e]) * size;
       tiles[4 * t + 2] = tile0[e];
-      tiles[4 * t + 3] = tile0[e + 1] - tile0[e];
+      tiles[4 * t + 3] = n;
     }
+  }
   for (int t = tile0[experts] + threadIdx.x; t < out.max_tiles; t += blockDim.x) tiles[4 * t] = -1;
   if (threadIdx.x == 0) {
     tiles[4 * out.max_tiles] = min(tile0[experts - 1], out.max_tiles);

@@ -167,7 +167,8 @@ __device__ __forceinline__ TileWork tile_work(const MoeParams& p, const int bloc
   t.block = unit / side;
   tile = tile0 + group * kSide + unit - t.block * side;
   t.s0 = p.tiles[4 * tile + 1];
-  t.s1 = min(min(p.offsets[t.e + 1], t.s0 + TILE), p.slots);
+  const int end = tile + 1 < min(tile0 + count, p.max_tiles) ? p.tiles[4 * tile + 5] : p.offsets[t.e + 1];
+  t.s1 = min(min(end, t.s0 + TILE), p.slots);
   const int ff = p.ff[t.e];
   t.steps = (UP ? p.width : ff) >> 5;
   t.ntiles = GATED ? ff >> 3 : (UP ? ff : p.width) >> 4;
@@ -240,10 +241,10 @@ __device__ __forceinline__ void to_lds16(const char* from, void* dst) {
 // of its cycles were conflicts).
 constexpr int kStageBytes = kMoeTile * 128;  // two k-steps of 32: a slot's 128 bytes, 8 slots a copy
 constexpr int tile_steps(int NT) { return NT == 4 ? 4 : 8; }  // k-steps of weights in registers; half as many stages of slots
-template <int PRODUCT, bool ONCE, int NT>
+template <int PRODUCT, bool ONCE, int NT, int MT>
 __device__ __forceinline__ void tile_product(const MoeParams& p, const TileWork& t, char (*ring)[kStageBytes]) {
   constexpr bool UP = PRODUCT != kMoeDown;
-  constexpr int S = tile_steps(NT), X = S / 2, MT = kMoeTile / 16, kCopies = kMoeTile / 32;
+  constexpr int S = tile_steps(NT), X = S / 2, kCopies = MT / 2;  // (MT groups of 16 slots)
   constexpr int kYounger = (X - 2) * kCopies + (X - 1) * 2 * NT;  // loads behind a stage's copies when it is needed
   constexpr int kBehind = (X - 1) * kCopies + (S - 1) * NT;       // ... behind a second k-step's weights
   const int e = t.e, s0 = t.s0, s1 = t.s1, block = t.block, steps = t.steps, ntiles = t.ntiles;
@@ -285,7 +286,7 @@ __device__ __forceinline__ void tile_product(const MoeParams& p, const TileWork&
     for (int m = 0; m < MT; ++m) acc[n][m] = e_f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int xoff[2] = {c * 128 + ((g ^ (c & 7)) * 16), c * 128 + (((4 + g) ^ (c & 7)) * 16)};
   auto multiply = [&](int at) __attribute__((always_inline)) {
-    constexpr int W = NT == 4 ? 5 : MT;  // fragments read ahead
+    constexpr int W = NT == 4 && MT > 5 ? 5 : MT;  // fragments read ahead
     e_u32x4_t x[W];
     auto read = [&](int m) { x[m % W] = *reinterpret_cast<const e_u32x4_t*>(ring[at / 2] + xoff[at & 1] + m * 2048); };
 #pragma unroll
@@ -341,8 +342,16 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, con
   __shared__ __attribute__((aligned(16))) char ring[tile_steps(NT) / 2][kStageBytes];
   const TileWork t = tile_work<PRODUCT, kMoeTile, 4 * NT>(p, blocks_first, blocks_last, 0);
   if (!t.any) return;
-  if (t.once) tile_product<PRODUCT, true, NT>(p, t, ring);
-  else tile_product<PRODUCT, false, NT>(p, t, ring);
+  const int groups = (t.s1 - t.s0 + 15) >> 4;
+  if (t.once) {
+    if (groups <= 4) tile_product<PRODUCT, true, NT, 4>(p, t, ring);
+    else if (groups <= 6) tile_product<PRODUCT, true, NT, 6>(p, t, ring);
+    else tile_product<PRODUCT, true, NT, 8>(p, t, ring);
+  } else {
+    if (groups <= 4) tile_product<PRODUCT, false, NT, 4>(p, t, ring);
+    else if (groups <= 6) tile_product<PRODUCT, false, NT, 6>(p, t, ring);
+    else tile_product<PRODUCT, false, NT, 8>(p, t, ring);
+  }
 }
 
 // The router's logits on packed weights (experts and the shared gate, up to a multiple of 16 rows): 16 rows of h and a share
