@@ -81,18 +81,16 @@ __global__ __launch_bounds__(256) void qk_norm_cache_kernel(
 // Rows are read VEC values at a time, four loads in flight: 300 rows of 8 heads, us, one value after the other and now: 8.7, 5.4.
 constexpr int kValueTile = 64;
 template <typename S, int VEC>
-__global__ __launch_bounds__(256) void value_cache_tile_kernel(S* __restrict__ value_cache, const S* __restrict__ v,
-                                                               const int64_t row_stride, const int rows, const int vdim,
-                                                               const int vpad, const int64_t* __restrict__ slot_mapping,
-                                                               const int64_t num_slots, const int block_size,
-                                                               const int64_t v_block_stride) {
+__device__ __forceinline__ void write_value_tile(char* smem, const int tile_of_rows, const int head, S* __restrict__ value_cache,
+                                                 const S* __restrict__ v, const int64_t row_stride, const int rows, const int vdim,
+                                                 const int vpad, const int64_t* __restrict__ slot_mapping, const int64_t num_slots,
+                                                 const int block_size, const int64_t v_block_stride) {
   struct alignas(16) Eight { S e[8]; };
   constexpr int LD = kValueTile + 2;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
   S* tile = reinterpret_cast<S*>(smem);  // [vdim][LD]
   __shared__ int64_t slots[kValueTile];
   __shared__ int groups[kValueTile], num_groups;  // first row | length << 8
-  const int row0 = blockIdx.x * kValueTile, head = blockIdx.y, nt = min(kValueTile, rows - row0), tid = threadIdx.x;
+  const int row0 = tile_of_rows * kValueTile, nt = min(kValueTile, rows - row0), tid = threadIdx.x;
   if (tid < kValueTile) {
     int64_t s = tid < nt ? slot_mapping[row0 + tid] : -1;
     if (s >= num_slots) s = -1;
@@ -144,6 +142,17 @@ __global__ __launch_bounds__(256) void value_cache_tile_kernel(S* __restrict__ v
   }
 }
 
+template <typename S, int VEC>
+__global__ __launch_bounds__(256) void value_cache_tile_kernel(S* __restrict__ value_cache, const S* __restrict__ v,
+                                                               const int64_t row_stride, const int rows, const int vdim,
+                                                               const int vpad, const int64_t* __restrict__ slot_mapping,
+                                                               const int64_t num_slots, const int block_size,
+                                                               const int64_t v_block_stride) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  write_value_tile<S, VEC>(smem, blockIdx.x, blockIdx.y, value_cache, v, row_stride, rows, vdim, vpad, slot_mapping, num_slots,
+                           block_size, v_block_stride);
+}
+
 struct RotaryCacheParams {
   void *q_out, *key_cache, *value_cache;
   const void *q, *k, *v;                // rows `row_stride` apart; v may be k
@@ -158,17 +167,27 @@ struct RotaryCacheParams {
   int64_t num_slots;
   int block_size;
   int64_t k_block_stride, v_block_stride;
+  int value_tiles;                      // workgroups ahead of the rows' that write 64 values' rows of a head each
 };
 
 // A workgroup per row.  Entry i of a vector turns with entry i + rot_dims / 2; a thread owns VEC neighbouring entries and reads
-// their partners as well.  The row's angles are shared by its heads through LDS.
+// their partners as well.  The row's angles are shared by its heads through LDS.  Values of many rows go ahead of the rows in the same
+// launch, of which either part alone is mostly the start: 300 rows of 8 heads of 128, us in a prompt step, two launches
+// and one: 11.1, 6.2.
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void rotary_cache_kernel(const RotaryCacheParams p) {
   using S = typename T::store_t;
   constexpr int x = 16 / sizeof(S);
-  extern __shared__ float cs[];  // [rot_dims / 2] cosines, then sines
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  if ((int)blockIdx.x < p.value_tiles) {
+    const int head = blockIdx.x % p.kv_heads;
+    write_value_tile<S, 16 / sizeof(S)>(smem, blockIdx.x / p.kv_heads, head, (S*)p.value_cache, (const S*)p.v, p.row_stride, p.rows,
+                                        p.vdim, p.vpad, p.slot_mapping, p.num_slots, p.block_size, p.v_block_stride);
+    return;
+  }
+  float* cs = reinterpret_cast<float*>(smem);  // [rot_dims / 2] cosines, then sines
   __shared__ float red[32];
-  const int row = blockIdx.x, half = p.rot_dims / 2;
+  const int row = blockIdx.x - p.value_tiles, half = p.rot_dims / 2;
   const S* q = (const S*)p.q + row * p.row_stride;
   const S* k = (const S*)p.k + row * p.row_stride;
   const int64_t pos = p.positions[row], slot = p.slot_mapping[row];
@@ -252,6 +271,10 @@ static bool tiled_values(int rows, int vdim, int esize, int block_size, const vo
   return rows > 64 && vdim * (kValueTile + 2) * esize <= 64 * 1024 && block_size % 8 == 0 && ((uintptr_t)value_cache & 15) == 0 &&
          v_block_stride * esize % 16 == 0;
 }
+// whether the rows of values are read in pieces of 16 bytes
+static bool wide_values(const void* v, int vdim, int64_t row_stride, int esize) {
+  return vdim * esize % 16 == 0 && row_stride * esize % 16 == 0 && ((uintptr_t)v & 15) == 0;
+}
 template <typename S>
 static void write_value_tiles(void* value_cache, const void* v, int64_t row_stride, int rows, int kv_heads, int vdim, int vpad,
                               const int64_t* slot_mapping, int64_t num_slots, int block_size, int64_t v_block_stride, hipStream_t s) {
@@ -261,7 +284,7 @@ static void write_value_tiles(void* value_cache, const void* v, int64_t row_stri
                        (size_t)vdim * (kValueTile + 2) * sizeof(S), s, (S*)value_cache, (const S*)v, row_stride, rows, vdim, vpad,
                        slot_mapping, num_slots, block_size, v_block_stride);
   };
-  if (vdim % N == 0 && row_stride % N == 0 && ((uintptr_t)v & 15) == 0) go(value_cache_tile_kernel<S, N>);
+  if (wide_values(v, vdim, row_stride, sizeof(S))) go(value_cache_tile_kernel<S, N>);
   else go(value_cache_tile_kernel<S, 1>);
 }
 
@@ -337,11 +360,19 @@ extern "C" int lvllm_rotary_cache(void* q_out, void* key_cache, void* value_cach
   LV_DISPATCH_F32_BF16(dtype, {
     using S = typename scalar_t::store_t;
     constexpr int kWide = sizeof(S) == 2 ? 8 : 4;
-    const size_t smem = (size_t)rot_dims * sizeof(float);
-    if (vec8) hipLaunchKernelGGL((rotary_cache_kernel<scalar_t, kWide>), dim3(rows), dim3(256), smem, s, p);
-    else if (vec4) hipLaunchKernelGGL((rotary_cache_kernel<scalar_t, 4>), dim3(rows), dim3(256), smem, s, p);
-    else hipLaunchKernelGGL((rotary_cache_kernel<scalar_t, 1>), dim3(rows), dim3(256), smem, s, p);
-    if (!p.with_values)
+    size_t smem = (size_t)rot_dims * sizeof(float);
+    // (LDS of a tile of values that leaves room for eight workgroups a CU)
+    const size_t tile = (size_t)vdim * (kValueTile + 2) * sizeof(S);
+    const int64_t tiles = (int64_t)((rows + (int64_t)kValueTile - 1) / kValueTile) * kv_heads;
+    if (!p.with_values && tile <= 18 * 1024 && wide_values(v, vdim, row_stride, sizeof(S)) && tiles + rows <= INT32_MAX) {
+      p.value_tiles = (int)tiles;
+      if (smem < tile) smem = tile;
+    }
+    const dim3 grid((unsigned)rows + p.value_tiles);
+    if (vec8) hipLaunchKernelGGL((rotary_cache_kernel<scalar_t, kWide>), grid, dim3(256), smem, s, p);
+    else if (vec4) hipLaunchKernelGGL((rotary_cache_kernel<scalar_t, 4>), grid, dim3(256), smem, s, p);
+    else hipLaunchKernelGGL((rotary_cache_kernel<scalar_t, 1>), grid, dim3(256), smem, s, p);
+    if (!p.with_values && p.value_tiles == 0)
       write_value_tiles<S>(value_cache, v, row_stride, rows, kv_heads, vdim, vpad, slot_mapping, p.num_slots, block_size,
                            v_block_stride, s);
   });

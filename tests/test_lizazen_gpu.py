@@ -229,6 +229,37 @@ def test_rotated_queries_keys_and_cached_values(amd, dtype, heads, kv_heads, dim
         assert (ks[rest] == 7).all() and (vs[rest] == 7).all()
 
 
+@pytest.mark.parametrize("dtype,vdim,own_v", [(BF16, 64, True), (BF16, 128, False), (BF16, 136, True), (BF16, 144, True), (F32, 64, True)])
+@pytest.mark.parametrize("rows", [65, 128, 300])
+def test_values_of_many_rows_in_the_rotary_launch(amd, rows, dtype, vdim, own_v):
+    """Rows that are read in whole pieces and rows that are not, whose values go through a launch of their own: the same bytes."""
+    from light_vllm_amd.attention.head_backend import HeadAttnImpl
+    from light_vllm_amd.engine.hybrid_config import KVSpec
+    from light_vllm_amd.engine.local_config import RotaryConfig
+    from light_vllm_amd.engine.local_layers import turns_of
+    heads, kv_heads, dim = 4, 2, vdim if not own_v else 64
+    turns = turns_of(RotaryConfig(32, 5e4, None), DEV)
+    widths = [heads * dim, kv_heads * dim, kv_heads * vdim]
+    data = rand(rows, sum(widths), seed=3, dtype=dtype).to(DEV)
+    slots = torch.arange(5, 5 + rows, device=DEV)
+    slots[7], slots[rows - 1] = -1, 400
+    spec = KVSpec(kv_heads, dim, vdim)
+    results = []
+    for more in (0, 5):
+        qkv = torch.zeros(rows, sum(widths) + more, dtype=dtype, device=DEV)
+        qkv[:, :sum(widths)] = data
+        q, k, v = qkv[:, :sum(widths)].split(widths, dim=1)
+        cache = torch.full((30, spec.block_elements(16)), 7.0, dtype=dtype, device=DEV)
+        out = amd.rotary_cache(q, k, v if own_v else k, None, None, 1e-3, heads, kv_heads, 1, torch.arange(rows, device=DEV),
+                               turns, *HeadAttnImpl.split_kv_cache(cache, spec, 16), slots)
+        results.append((out, cache))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+    _, vc = HeadAttnImpl.split_kv_cache(results[0][1], spec, 16)
+    stored = vc.permute(0, 3, 1, 2).reshape(480, kv_heads, spec.vpad)[slots[slots >= 0]][..., :vdim]
+    want = data[:, -widths[2]:] if own_v else data[:, widths[0]:widths[0] + widths[1]]
+    assert torch.equal(stored, want.reshape(rows, kv_heads, vdim)[slots >= 0])
+
+
 # ---- attention ----
 def put_keys(kc, vc, table, k, v, spec):
     """k [n, kv_heads * maps, dim], v [n, kv_heads, vdim] of one sequence into its pages."""
