@@ -6,75 +6,12 @@
 //   q_out       [rows, heads, kpad]                                                  (padding zeroed)
 //
 // Norms and angles are fp32; what the attention reads is rounded to T once.
+#include <algorithm>
+
 #include "rotation.h"
 #include "row_ops.h"
 
 namespace lvllm {
-
-// Per-head RMS norm of queries and keys (weights [dim], shared by the heads) and the write of the normed keys and the
-// values into a paged cache whose key and value sizes differ:
-//   key_cache   [num_blocks, kv_heads, kpad / x, block_size, x],  x = 16 / sizeof(T), kpad >= dim (rest zeroed)
-//   value_cache [num_blocks, kv_heads, vpad, block_size],         vpad >= vdim (rest zeroed)
-// q_out [rows, heads, kpad] (padding zeroed).  L lanes per (row, head); the values of few rows ride along as further
-// "heads" (with_values), those of many go through value_cache_tile_kernel.
-template <typename T, int L, int VEC>
-__global__ __launch_bounds__(256) void qk_norm_cache_kernel(
-    typename T::store_t* __restrict__ q_out, typename T::store_t* __restrict__ key_cache,
-    typename T::store_t* __restrict__ value_cache, const typename T::store_t* __restrict__ q,
-    const typename T::store_t* __restrict__ k, const typename T::store_t* __restrict__ v, const int64_t row_stride,
-    const float* __restrict__ q_weight, const float* __restrict__ k_weight, const float eps, const int rows, const int heads,
-    const int kv_heads, const int dim, const int vdim, const int kpad, const int vpad, const bool with_values,
-    const int64_t* __restrict__ slot_mapping, const int64_t num_slots, const int block_size, const int64_t k_block_stride,
-    const int64_t v_block_stride) {
-  using S = typename T::store_t;
-  constexpr int x = 16 / sizeof(S);
-  const int lane = threadIdx.x % L;
-  const int per_row = heads + (with_values ? 2 : 1) * kv_heads;
-  const unsigned item = blockIdx.x * (256 / L) + threadIdx.x / L;
-  const int row = (int)(item / (unsigned)per_row), h = (int)(item - (unsigned)row * per_row);
-  if (row >= rows) return;
-  int64_t block = 0;
-  int off = 0;
-  if (h >= heads) {
-    const int64_t slot = slot_mapping[row];
-    if (slot < 0 || slot >= num_slots) return;
-    block = slot / block_size;
-    off = (int)(slot - block * block_size);
-  }
-  if (h >= heads + kv_heads) {
-    const int g = h - heads - kv_heads;
-    const S* src = v + row * row_stride + (int64_t)g * vdim;
-    S* dst = value_cache + block * v_block_stride + (int64_t)g * vpad * block_size + off;
-    for (int d = lane; d < vpad; d += L) dst[(int64_t)d * block_size] = d < vdim ? src[d] : T::from_float(0.f);
-    return;
-  }
-  const bool is_q = h < heads;
-  const S* src = (is_q ? q + (int64_t)h * dim : k + (int64_t)(h - heads) * dim) + row * row_stride;
-  const float* wt = is_q ? q_weight : k_weight;
-  S* dst = is_q ? q_out + ((int64_t)row * heads + h) * kpad
-                : key_cache + block * k_block_stride + (int64_t)(h - heads) * kpad * block_size + (int64_t)off * x;
-  float f[VEC];
-  float ss = 0.f;
-  for (int d = lane * VEC; d < dim; d += L * VEC) {
-    load_vec<T, VEC>(src + d, f);
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) ss += f[j] * f[j];
-  }
-  const bool one_pass = dim <= L * VEC;  // (the values are still in registers)
-  const float r = 1.f / sqrtf(group_sum<L>(ss) / dim + eps);
-  for (int d = lane * VEC; d < kpad; d += L * VEC) {
-    float o[VEC];
-    if (d < dim) {
-      if (!one_pass) load_vec<T, VEC>(src + d, f);
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) o[j] = f[j] * r * wt[d + j];
-    } else {
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) o[j] = 0.f;
-    }
-    store_vec<T, VEC>(is_q ? dst + d : dst + (int64_t)(d / x) * block_size * x + d % x, o);
-  }
-}
 
 // Values of many rows: a workgroup takes 64 rows of one kv head through LDS.  Its rows are cut into groups of consecutive
 // slots inside one aligned 8-slot window; a thread stores a (d, group) as one piece when the group is full.
@@ -142,6 +79,77 @@ __device__ __forceinline__ void write_value_tile(char* smem, const int tile_of_r
   }
 }
 
+// Per-head RMS norm of queries and keys (weights [dim], shared by the heads) and the write of the normed keys and the
+// values into a paged cache whose key and value sizes differ:
+//   key_cache   [num_blocks, kv_heads, kpad / x, block_size, x],  x = 16 / sizeof(T), kpad >= dim (rest zeroed)
+//   value_cache [num_blocks, kv_heads, vpad, block_size],         vpad >= vdim (rest zeroed)
+// q_out [rows, heads, kpad] (padding zeroed).  L lanes per (row, head); the values of few rows ride along as further
+// "heads" (with_values), those of many go ahead of the rows (value_tiles workgroups) or through value_cache_tile_kernel.
+template <typename T, int L, int VEC>
+__global__ __launch_bounds__(256) void qk_norm_cache_kernel(
+    typename T::store_t* __restrict__ q_out, typename T::store_t* __restrict__ key_cache,
+    typename T::store_t* __restrict__ value_cache, const typename T::store_t* __restrict__ q,
+    const typename T::store_t* __restrict__ k, const typename T::store_t* __restrict__ v, const int64_t row_stride,
+    const float* __restrict__ q_weight, const float* __restrict__ k_weight, const float eps, const int rows, const int heads,
+    const int kv_heads, const int dim, const int vdim, const int kpad, const int vpad, const bool with_values,
+    const int64_t* __restrict__ slot_mapping, const int64_t num_slots, const int block_size, const int64_t k_block_stride,
+    const int64_t v_block_stride, const int value_tiles) {
+  using S = typename T::store_t;
+  constexpr int x = 16 / sizeof(S);
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  if ((int)blockIdx.x < value_tiles) {
+    write_value_tile<S, 16 / sizeof(S)>(smem, blockIdx.x / kv_heads, blockIdx.x % kv_heads, value_cache, v, row_stride, rows, vdim,
+                                        vpad, slot_mapping, num_slots, block_size, v_block_stride);
+    return;
+  }
+  const int lane = threadIdx.x % L;
+  const int per_row = heads + (with_values ? 2 : 1) * kv_heads;
+  const unsigned item = (blockIdx.x - value_tiles) * (256 / L) + threadIdx.x / L;
+  const int row = (int)(item / (unsigned)per_row), h = (int)(item - (unsigned)row * per_row);
+  if (row >= rows) return;
+  int64_t block = 0;
+  int off = 0;
+  if (h >= heads) {
+    const int64_t slot = slot_mapping[row];
+    if (slot < 0 || slot >= num_slots) return;
+    block = slot / block_size;
+    off = (int)(slot - block * block_size);
+  }
+  if (h >= heads + kv_heads) {
+    const int g = h - heads - kv_heads;
+    const S* src = v + row * row_stride + (int64_t)g * vdim;
+    S* dst = value_cache + block * v_block_stride + (int64_t)g * vpad * block_size + off;
+    for (int d = lane; d < vpad; d += L) dst[(int64_t)d * block_size] = d < vdim ? src[d] : T::from_float(0.f);
+    return;
+  }
+  const bool is_q = h < heads;
+  const S* src = (is_q ? q + (int64_t)h * dim : k + (int64_t)(h - heads) * dim) + row * row_stride;
+  const float* wt = is_q ? q_weight : k_weight;
+  S* dst = is_q ? q_out + ((int64_t)row * heads + h) * kpad
+                : key_cache + block * k_block_stride + (int64_t)(h - heads) * kpad * block_size + (int64_t)off * x;
+  float f[VEC];
+  float ss = 0.f;
+  for (int d = lane * VEC; d < dim; d += L * VEC) {
+    load_vec<T, VEC>(src + d, f);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) ss += f[j] * f[j];
+  }
+  const bool one_pass = dim <= L * VEC;  // (the values are still in registers)
+  const float r = 1.f / sqrtf(group_sum<L>(ss) / dim + eps);
+  for (int d = lane * VEC; d < kpad; d += L * VEC) {
+    float o[VEC];
+    if (d < dim) {
+      if (!one_pass) load_vec<T, VEC>(src + d, f);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) o[j] = f[j] * r * wt[d + j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) o[j] = 0.f;
+    }
+    store_vec<T, VEC>(is_q ? dst + d : dst + (int64_t)(d / x) * block_size * x + d % x, o);
+  }
+}
+
 template <typename S, int VEC>
 __global__ __launch_bounds__(256) void value_cache_tile_kernel(S* __restrict__ value_cache, const S* __restrict__ v,
                                                                const int64_t row_stride, const int rows, const int vdim,
@@ -180,9 +188,9 @@ __global__ __launch_bounds__(256) void rotary_cache_kernel(const RotaryCachePara
   constexpr int x = 16 / sizeof(S);
   extern __shared__ __attribute__((aligned(16))) char smem[];
   if ((int)blockIdx.x < p.value_tiles) {
-    const int head = blockIdx.x % p.kv_heads;
-    write_value_tile<S, 16 / sizeof(S)>(smem, blockIdx.x / p.kv_heads, head, (S*)p.value_cache, (const S*)p.v, p.row_stride, p.rows,
-                                        p.vdim, p.vpad, p.slot_mapping, p.num_slots, p.block_size, p.v_block_stride);
+    write_value_tile<S, 16 / sizeof(S)>(smem, blockIdx.x / p.kv_heads, blockIdx.x % p.kv_heads, (S*)p.value_cache, (const S*)p.v,
+                                        p.row_stride, p.rows, p.vdim, p.vpad, p.slot_mapping, p.num_slots, p.block_size,
+                                        p.v_block_stride);
     return;
   }
   float* cs = reinterpret_cast<float*>(smem);  // [rot_dims / 2] cosines, then sines
@@ -275,6 +283,12 @@ static bool tiled_values(int rows, int vdim, int esize, int block_size, const vo
 static bool wide_values(const void* v, int vdim, int64_t row_stride, int esize) {
   return vdim * esize % 16 == 0 && row_stride * esize % 16 == 0 && ((uintptr_t)v & 15) == 0;
 }
+// The workgroups that write tiles of values ahead of `others` in the launch of these; 0: a launch of their own.  (Tiles whose LDS
+// leaves room for eight workgroups a CU.)
+static int tiles_ahead(const void* v, int64_t row_stride, int rows, int kv_heads, int vdim, int esize, int64_t others) {
+  const int64_t tiles = ((int64_t)rows + kValueTile - 1) / kValueTile * kv_heads;
+  return vdim * (kValueTile + 2) * esize <= 18 * 1024 && wide_values(v, vdim, row_stride, esize) && tiles + others <= INT32_MAX ? (int)tiles : 0;
+}
 template <typename S>
 static void write_value_tiles(void* value_cache, const void* v, int64_t row_stride, int rows, int kv_heads, int vdim, int vpad,
                               const int64_t* slot_mapping, int64_t num_slots, int block_size, int64_t v_block_stride, hipStream_t s) {
@@ -306,21 +320,24 @@ extern "C" int lvllm_qk_norm_cache(void* q_out, void* key_cache, void* value_cac
   const int64_t items = (int64_t)rows * (heads + (tiled ? 1 : 2) * kv_heads);
   LV_CHECK(items <= INT32_MAX && kv_heads <= 65535, "too many rows");
 #define LV_QK(VEC_)                                                                                                          \
-  hipLaunchKernelGGL((qk_norm_cache_kernel<scalar_t, kL, VEC_>), grid, dim3(256), 0, (hipStream_t)stream, (S*)q_out,          \
+  hipLaunchKernelGGL((qk_norm_cache_kernel<scalar_t, kL, VEC_>), grid, dim3(256), smem, (hipStream_t)stream, (S*)q_out,       \
                      (S*)key_cache, (S*)value_cache, (const S*)q, (const S*)k, (const S*)v, row_stride, q_weight, k_weight,  \
                      eps, rows, heads, kv_heads, dim, vdim, kpad, vpad, !tiled, slot_mapping, num_blocks * block_size,       \
-                     block_size, k_block_stride, v_block_stride)
+                     block_size, k_block_stride, v_block_stride, ahead)
   LV_DISPATCH_DTYPE(dtype, {
     using S = scalar_t::store_t;
     constexpr int kWide = sizeof(S) == 2 ? 8 : 4;  // elements of a 16-byte piece
     const int lanes = lanes_for(kpad, vec8 ? kWide : vec ? 4 : 1);
-    const dim3 grid((unsigned)((items * lanes + 255) / 256));
+    const int64_t workgroups = (items * lanes + 255) / 256;
+    const int ahead = tiled ? tiles_ahead(v, row_stride, rows, kv_heads, vdim, sizeof(S), workgroups) : 0;
+    const size_t smem = ahead > 0 ? (size_t)vdim * (kValueTile + 2) * sizeof(S) : 0;
+    const dim3 grid((unsigned)(workgroups + ahead));
     LV_LANES(lanes, {
       if (vec8) LV_QK(kWide);
       else if (vec) LV_QK(4);
       else LV_QK(1);
     })
-    if (tiled)
+    if (tiled && ahead == 0)
       write_value_tiles<S>(value_cache, v, row_stride, rows, kv_heads, vdim, vpad, slot_mapping, num_blocks * block_size,
                            block_size, v_block_stride, (hipStream_t)stream);
   });
@@ -361,13 +378,8 @@ extern "C" int lvllm_rotary_cache(void* q_out, void* key_cache, void* value_cach
     using S = typename scalar_t::store_t;
     constexpr int kWide = sizeof(S) == 2 ? 8 : 4;
     size_t smem = (size_t)rot_dims * sizeof(float);
-    // (LDS of a tile of values that leaves room for eight workgroups a CU)
-    const size_t tile = (size_t)vdim * (kValueTile + 2) * sizeof(S);
-    const int64_t tiles = (int64_t)((rows + (int64_t)kValueTile - 1) / kValueTile) * kv_heads;
-    if (!p.with_values && tile <= 18 * 1024 && wide_values(v, vdim, row_stride, sizeof(S)) && tiles + rows <= INT32_MAX) {
-      p.value_tiles = (int)tiles;
-      if (smem < tile) smem = tile;
-    }
+    if (!p.with_values) p.value_tiles = tiles_ahead(v, row_stride, rows, kv_heads, vdim, sizeof(S), rows);
+    if (p.value_tiles > 0) smem = std::max(smem, (size_t)vdim * (kValueTile + 2) * sizeof(S));
     const dim3 grid((unsigned)rows + p.value_tiles);
     if (vec8) hipLaunchKernelGGL((rotary_cache_kernel<scalar_t, kWide>), grid, dim3(256), smem, s, p);
     else if (vec4) hipLaunchKernelGGL((rotary_cache_kernel<scalar_t, 4>), grid, dim3(256), smem, s, p);
