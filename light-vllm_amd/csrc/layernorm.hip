@@ -136,11 +136,21 @@ __global__ void fused_add_rms_norm_splitk_kernel(typename T::store_t* out,  // [
     float acc[N];
 #pragma unroll
     for (int j = 0; j < N; ++j) acc[j] = 0.f;
-    for (int sp = 0; sp < num_partials; ++sp) {
-      const float4* p4 = reinterpret_cast<const float4*>(prow + sp * partial_stride + (int64_t)i * N);
-      const float4 a = p4[0], b = p4[1];
-      acc[0] += a.x; acc[1] += a.y; acc[2] += a.z; acc[3] += a.w;
-      acc[4] += b.x; acc[5] += b.y; acc[6] += b.z; acc[7] += b.w;
+    constexpr int B = 4;  // slabs asked for at once
+    for (int sp0 = 0; sp0 < num_partials; sp0 += B) {
+      float4 a[B], b[B];
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const float4* p4 = reinterpret_cast<const float4*>(prow + min(sp0 + u, num_partials - 1) * partial_stride + (int64_t)i * N);
+        a[u] = p4[0];
+        b[u] = p4[1];
+      }
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        if (sp0 + u >= num_partials) break;
+        acc[0] += a[u].x; acc[1] += a[u].y; acc[2] += a[u].z; acc[3] += a[u].w;
+        acc[4] += b[u].x; acc[5] += b[u].y; acc[6] += b[u].z; acc[7] += b[u].w;
+      }
     }
     const V r = res_v[i];
     V x;

@@ -29,9 +29,17 @@ struct ProjOut {
   __device__ __forceinline__ void at4(int64_t i, float (&v)[4]) const {
     if (partials != nullptr) {
       v[0] = v[1] = v[2] = v[3] = 0.f;
-      for (int p = 0; p < num_partials; ++p) {
-        const float4 a = *reinterpret_cast<const float4*>(partials + p * partial_stride + i);
-        v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
+      constexpr int B = 4;  // slabs asked for at once
+      for (int p0 = 0; p0 < num_partials; p0 += B) {
+        float4 a[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+          a[u] = *reinterpret_cast<const float4*>(partials + min(p0 + u, num_partials - 1) * partial_stride + i);
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+          if (p0 + u >= num_partials) break;
+          v[0] += a[u].x; v[1] += a[u].y; v[2] += a[u].z; v[3] += a[u].w;
+        }
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) v[j] = T::to_float(T::from_float(v[j]));

@@ -387,3 +387,20 @@ def test_products_in_one_launch(dtype, M, N, n_last, K):
         for i, (w, p) in enumerate(zip(ws, packed)):
             got = last if i == products - 1 else first[i]
             assert torch.equal(got, amd.skinny_linear_packed(x[i], p, None, w.shape[0], K)), (products, i)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,K", [(16, 32), (48, 2048), (16, 2080), (4096, 4096), (272, 4128), (2048, 8448), (64, 14336)])
+def test_fine_partials_sum_to_the_projection(dtype, M, N, K):
+    """Parts of K whose waves own at most 8 k-steps: edges of a part, a last part of one k-step, as many parts as there are."""
+    amd = torch.ops._C_amd
+    g = torch.Generator(device=DEV).manual_seed(K + M)
+    x = torch.randn(M, K, generator=g, device=DEV).to(dtype)
+    w = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).to(dtype)
+    parts = amd.skinny_linear_fine_partials(x, amd.pack_weight(w), N, K)
+    assert parts.shape == ((K + 2047) // 2048, M, N) and parts.dtype == torch.float32
+    ref = x.double() @ w.double().t()
+    # K products, exact in fp32, summed in fp32 in any order: K roundings of partial sums, each at most the sum of magnitudes
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert ((parts.double().sum(0) - ref).abs() <= bound).all()
