@@ -38,6 +38,9 @@ __global__ void rms_norm_vec_kernel(typename T::store_t* out,  // == in when FUS
   V* out_v = reinterpret_cast<V*>(out) + row;
   const V* w_v = reinterpret_cast<const V*>(weight);
 
+  // Asked for here, not behind the sum: a step's norm finds its weight in no cache, and a launch of few rows is little but latency.
+  // 9 norms of a decode step of 32 rows, us the step: 16-bit weights 523.1, 521.7 with it, 8-bit ones 352.1, 350.8.
+  const V first_w = w_v[min((int)threadIdx.x, nvec - 1)];
   V cache[kMaxCached];
   float var = 0.f;
   int c = 0;
@@ -75,7 +78,7 @@ __global__ void rms_norm_vec_kernel(typename T::store_t* out,  // == in when FUS
     } else {
       x = FUSED_ADD ? res_v[i] : in_v[i];
     }
-    const V w = w_v[i];
+    const V w = c == 0 ? first_w : w_v[i];
     V o;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
@@ -129,6 +132,7 @@ __global__ void fused_add_rms_norm_splitk_kernel(typename T::store_t* out,  // [
   const bool scaled = scale_a != nullptr;
   const float sc = scaled ? scale_a[0] * scale_b[0] : 1.f;
 
+  const V first_w = w_v[min((int)threadIdx.x, nvec - 1)];  // (as in rms_norm_vec_kernel)
   V cache[kMaxCached];
   float var = 0.f;
   int c = 0;
@@ -136,6 +140,7 @@ __global__ void fused_add_rms_norm_splitk_kernel(typename T::store_t* out,  // [
     float acc[N];
 #pragma unroll
     for (int j = 0; j < N; ++j) acc[j] = 0.f;
+    const V r = res_v[i];
     constexpr int B = 4;  // slabs asked for at once
     for (int sp0 = 0; sp0 < num_partials; sp0 += B) {
       float4 a[B], b[B];
@@ -152,7 +157,6 @@ __global__ void fused_add_rms_norm_splitk_kernel(typename T::store_t* out,  // [
         acc[4] += b[u].x; acc[5] += b[u].y; acc[6] += b[u].z; acc[7] += b[u].w;
       }
     }
-    const V r = res_v[i];
     V x;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
@@ -181,7 +185,7 @@ __global__ void fused_add_rms_norm_splitk_kernel(typename T::store_t* out,  // [
     } else {
       x = res_v[i];
     }
-    const V w = w_v[i];
+    const V w = c == 0 ? first_w : w_v[i];
     V o;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
