@@ -75,7 +75,9 @@ class Worker:
                                       decode_version=decode_version)
         if self.device.type == "cuda":  # free memory before the weights (gpu_worker.py:78-80)
             torch.cuda.empty_cache()
-            self.init_gpu_memory = torch.cuda.mem_get_info(self.device)[0]
+            # what the caching allocator holds unused is free as well: a small model may fit into that alone
+            unused = torch.cuda.memory_reserved(self.device) - torch.cuda.memory_allocated(self.device)
+            self.init_gpu_memory = torch.cuda.mem_get_info(self.device)[0] + unused
         else:
             self.init_gpu_memory = 0
         self.model = model_entry(model_config.architecture).model_cls()(model_config, self.attn_impl, device, seed)

@@ -547,6 +547,16 @@ def test_sizing_without_a_cache(folders):
     assert generate(engine(folders["states"], F32, num_blocks=None), [p], 6) == [greedy(cfg, w, p, 6)]
 
 
+def test_sizing_inside_memory_the_allocator_holds(folders):
+    """A model that fits into what an earlier one left in the caching allocator takes no more of the device."""
+    held = [torch.empty(n, dtype=torch.uint8, device="cuda") for n in [8 << 20] * 16 + [512 << 10] * 32]
+    del held[1:16:2], held[9::2]  # every other one: segments with room in them
+    cfg, w = sc.case("states")
+    p = tokens(cfg, 20, 3)
+    assert generate(engine(folders["states"], F32, num_blocks=None), [p], 6) == [greedy(cfg, w, p, 6)]
+    assert held
+
+
 def test_programs(folders, tmp_path):
     """bin/generate and bin/trace_run as a user starts them."""
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
