@@ -23,7 +23,8 @@ class ModelConfig:
     dtype: torch.dtype = torch.bfloat16
     pack_weights: bool = True       # keep an MFMA-ordered copy of each projection for decode
     fuse_decode_ops: bool = True    # rope+cache write in one launch, split-K sum inside add+norm
-    # the individual fused launches of a decode step (each bit-identical to what it replaces; off = A/B runs)
+    # the individual fused launches of a decode step (each bit-identical to what it replaces, but that the o and down
+    # projections' sums over K are cut in parts of 2048; off = A/B runs)
     rope_in_attention: bool = True  # rotary_embedding + reshape_and_cache inside the attention launch
     rope_in_attention_fp8: bool = True   # the same over an fp8 KV cache (bit-identical too; +2 % on config 5 once the
                                          # new token's cache stores left the prologue, profiles/r03_tuning.md section 10)
