@@ -36,8 +36,9 @@ class ModelConfig:
     stream_gemm_max_rows: int = 256  # 65..this many rows: projections through lvllm_stream_gemm where it wins
     # decode steps of at least this many rows split o_proj's K over workgroups and leave the fp32 partials to the
     # add + norm launch (as the down projection always does); below, K is split inside a workgroup only
-    # (1 row and 32, us a projection and add + norm of 4096: 11.7 and 13.5 below, 10.7 and 12.6 with the partials)
-    o_proj_partials_min_rows: int = 1
+    # (1 row and 32, us a projection and add + norm of 4096: 11.7 and 13.5 below, 10.7 and 12.6 with the partials, but with
+    # two steps in flight they cost 1 % of the tokens a second)
+    o_proj_partials_min_rows: int = 33
     # "fp8": W8A8 projections: per-tensor e4m3 weights, static per-tensor
     # activation scales calibrated once on a random batch (the reference's activation_scheme="static")
     quantization: Optional[str] = None
