@@ -276,11 +276,6 @@ int lvllm_stream_gemm(void* y, const void* x, const void* w_packed, const void* 
 int lvllm_skinny_gemm_ex(void* y, const void* x, const void* w, const void* bias, int M, int N,
                          int K, int64_t ldx, int dtype, int packed, int act, int partial_out,
                          int* ksplit_out, void* workspace, int64_t workspace_bytes, void* stream);
-/* As lvllm_skinny_gemm_ex with partial_out over a packed W, but K is cut so that a wave owns at most 8 k-steps whatever M:
- * partials [lvllm_skinny_gemm_partials_splits(M, N, K)][M][N] fp32, for a launch that sums them.  3 = outside the envelope. */
-int lvllm_skinny_gemm_partials_splits(int M, int N, int K);
-int lvllm_skinny_gemm_partials(float* partials, int64_t partials_bytes, const void* x, const void* w_packed, int M, int N,
-                               int K, int64_t ldx, int dtype, void* stream);
 /* LayerNorm(x + y) of the encoder models (xlm_roberta.py; torch ops in the reference): z = T(x + y),
  * out = T((z - mean) * rsqrt(var + eps) * weight + bias), statistics in fp32.  y may be NULL (plain
  * LayerNorm).  16-bit element types, hidden_size % 8 == 0, contiguous rows, out may alias x. */

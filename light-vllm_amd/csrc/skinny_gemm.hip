@@ -32,8 +32,6 @@
 // KiB (lvllm_pack_weight / `packed` below).
 #include <stdlib.h>
 
-#include <algorithm>
-
 #include "common.h"
 #include "trace.h"
 
@@ -1141,7 +1139,7 @@ extern "C" int lvllm_skinny_gemm(void* y, const void* x, const void* w, const vo
 
 static int skinny_gemm(void* y, const void* x, const void* w, const void* bias, int M, int N, int K, int64_t ldx, int dtype,
                        int packed, int act, float limit, int partial_out, int* ksplit_out, void* workspace,
-                       int64_t workspace_bytes, void* stream, int splits = 0) {
+                       int64_t workspace_bytes, void* stream) {
   if (M <= 0 || N <= 0) return 0;
   if (!(dtype == LVLLM_BF16 || dtype == LVLLM_F16) || M > 64 || (K % 32) != 0 || (N % 16) != 0 ||
       (int64_t)N * K * 2 >= ((int64_t)1 << 32) - 16 || (ldx % 8) != 0 ||
@@ -1160,7 +1158,6 @@ static int skinny_gemm(void* y, const void* x, const void* w, const void* bias, 
   if (partial_out && act == 0 && tuning().gemm_partials_ksplit > ksplit &&
       total_steps >= tuning().gemm_partials_ksplit * kGemmWaves)
     ksplit = tuning().gemm_partials_ksplit;
-  if (splits > ksplit) ksplit = splits;  // (lvllm_skinny_gemm_partials)
   const int steps_per_wg = (total_steps + ksplit - 1) / ksplit;
   const int steps_per_wave = (steps_per_wg + kGemmWaves - 1) / kGemmWaves;  // <= max_steps_per_wave(M)
   const int ntiles = N / 16;
@@ -1266,28 +1263,6 @@ static int skinny_gemm(void* y, const void* x, const void* w, const void* bias, 
     LV_LAUNCH_CHECK();
   }
   return 0;
-}
-
-// Splits of K for a projection whose fp32 partials the next launch sums: waves of at most 8 k-steps, as at more than 32 rows.  A
-// workgroup then reads half of X ahead of its first product, and a wave's loads are all under way at once; more slabs than that cost
-// the next launch more than they save.  us with the launch that sums them, 16 k-steps a wave (4096 -> 4096: a plain product) and 8,
-// 1 / 8 / 24 / 32 rows: 4096 -> 4096 11.7 / 12.1 / 13.2 / 13.5, 10.7 / 11.3 / 12.3 / 12.6; 8448 -> 2048 13.0 / 12.6 / 14.2 / 14.7,
-// 12.0 / 12.4 / 13.1 / 13.4; 14336 -> 4096 24.9 / 24.9 / 26.5 / 26.6, 24.4 / 24.8 / 26.1 / 26.5 (with one slab more than that: 24.2 /
-// 25.6 / 27.1 / 27.3).
-extern "C" int lvllm_skinny_gemm_partials_splits(int M, int N, int K) {
-  // (Where steps share the chip, a launch with fewer workgroups than CUs, the slabs' way through memory costs more: two steps in
-  // flight, 32 rows, 9386 tokens/s with the finer parts in o and down, 9493 without.)
-  const int steps = K / 32, per_wg = kGemmWaves * (tuning().gemm_workgroups >= 256 ? 8 : max_steps_per_wave(M));
-  const int splits = std::max(1, (steps + per_wg - 1) / per_wg);
-  const int forced = tuning().gemm_partials_ksplit;
-  return forced > splits && steps >= forced * kGemmWaves ? forced : splits;
-}
-
-extern "C" int lvllm_skinny_gemm_partials(float* partials, int64_t partials_bytes, const void* x, const void* w_packed, int M, int N,
-                                          int K, int64_t ldx, int dtype, void* stream) {
-  if (M <= 0 || N <= 0) return 0;
-  return skinny_gemm(nullptr, x, w_packed, nullptr, M, N, K, ldx, dtype, 1, 0, 0.f, 1, nullptr, partials, partials_bytes, stream,
-                     lvllm_skinny_gemm_partials_splits(M, N, K));
 }
 
 extern "C" int lvllm_skinny_gemm_ex(void* y, const void* x, const void* w, const void* bias, int M, int N,

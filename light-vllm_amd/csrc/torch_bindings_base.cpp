@@ -318,18 +318,6 @@ torch::Tensor skinny_linear_packed_partials(const torch::Tensor& gate_up, const 
   return ksplit == S ? partials : partials.narrow(0, 0, ksplit);
 }
 
-// The same with K cut finer where few rows would leave a wave more than 8 k-steps (lvllm_skinny_gemm_partials).
-torch::Tensor skinny_linear_fine_partials(const torch::Tensor& x, const torch::Tensor& w_packed, int64_t N, int64_t K) {
-  TORCH_CHECK(x.dim() == 2 && x.size(1) == K && w_packed.numel() == N * K, "bad shapes");
-  TORCH_CHECK(skinny_ok(x, w_packed, std::nullopt), "M <= 64 rows of bf16/f16 on the GPU only");
-  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(x));
-  const int64_t M = x.size(0), S = lvllm_skinny_gemm_partials_splits((int)M, (int)N, (int)K);
-  auto partials = torch::empty({S, M, N}, x.options().dtype(torch::kFloat));
-  check(lvllm_skinny_gemm_partials(partials.data_ptr<float>(), S * M * N * 4, x.data_ptr(), w_packed.data_ptr(), (int)M, (int)N,
-                                   (int)K, x.stride(0), dtype_code(x, "skinny_linear_fine_partials"), current_stream(x)));
-  return partials;
-}
-
 // A W8A8 projection whose K is split over workgroups, leaving the raw fp32 partials [S, M, N] for
 // fused_add_rms_norm_splitk_scaled.  Returns an EMPTY tensor when K is not split at this shape (nothing was done).
 torch::Tensor skinny_linear_w8a8_partials(const torch::Tensor& x, const torch::Tensor& w_packed,
@@ -709,8 +697,6 @@ TORCH_LIBRARY_FRAGMENT(_C_amd, amd) {
   amd.impl("skinny_linear_packed_swiglu", torch::kCUDA, &skinny_linear_packed_swiglu);
   amd.def("skinny_linear_packed_partials(Tensor x, Tensor w_packed, int N, int K, bool swiglu) -> Tensor");
   amd.impl("skinny_linear_packed_partials", torch::kCUDA, &skinny_linear_packed_partials);
-  amd.def("skinny_linear_fine_partials(Tensor x, Tensor w_packed, int N, int K) -> Tensor");
-  amd.impl("skinny_linear_fine_partials", torch::kCUDA, &skinny_linear_fine_partials);
   amd.def("skinny_linear_w8a8(Tensor x, Tensor w_packed, Tensor w_scale, Tensor x_scale, int N, int K, "
           "Tensor? bias) -> Tensor");
   amd.impl("skinny_linear_w8a8", torch::kCUDA, &skinny_linear_w8a8);

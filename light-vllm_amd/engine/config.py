@@ -23,8 +23,7 @@ class ModelConfig:
     dtype: torch.dtype = torch.bfloat16
     pack_weights: bool = True       # keep an MFMA-ordered copy of each projection for decode
     fuse_decode_ops: bool = True    # rope+cache write in one launch, split-K sum inside add+norm
-    # the individual fused launches of a decode step (each bit-identical to what it replaces, but that the o and down
-    # projections' sums over K are cut in parts of 2048; off = A/B runs)
+    # the individual fused launches of a decode step (each bit-identical to what it replaces; off = A/B runs)
     rope_in_attention: bool = True  # rotary_embedding + reshape_and_cache inside the attention launch
     rope_in_attention_fp8: bool = True   # the same over an fp8 KV cache (bit-identical too; +2 % on config 5 once the
                                          # new token's cache stores left the prologue, profiles/r03_tuning.md section 10)
@@ -36,8 +35,6 @@ class ModelConfig:
     stream_gemm_max_rows: int = 256  # 65..this many rows: projections through lvllm_stream_gemm where it wins
     # decode steps of at least this many rows split o_proj's K over workgroups and leave the fp32 partials to the
     # add + norm launch (as the down projection always does); below, K is split inside a workgroup only
-    # (1 row and 32, us a projection and add + norm of 4096: 11.7 and 13.5 below, 10.7 and 12.6 with the partials, but with
-    # two steps in flight they cost 1 % of the tokens a second)
     o_proj_partials_min_rows: int = 33
     # "fp8": W8A8 projections: per-tensor e4m3 weights, static per-tensor
     # activation scales calibrated once on a random batch (the reference's activation_scheme="static")

@@ -70,12 +70,9 @@ def make_weight(w: torch.Tensor, pack: bool) -> Weight:
     return Weight(w.contiguous(), pack and w.dtype != torch.float32)
 
 
-def project_to_residual(x: torch.Tensor, w: Weight, fine: bool = False) -> torch.Tensor:
-    """A projection whose only reader is the next residual add: split-K slabs where that launch sums them.  `fine`: more of them
-    where that is faster; not ahead of routers, whose near-ties a sum in another order decides another way."""
+def project_to_residual(x: torch.Tensor, w: Weight) -> torch.Tensor:
+    """A projection whose only reader is the next residual add: split-K slabs where that launch sums them."""
     if 0 < x.shape[0] <= DECODE_ROWS and w.packed is not None:
-        if fine:
-            return amd.skinny_linear_fine_partials(x, w.packed, w.N, w.K)
         return amd.skinny_linear_packed_partials(x, w.packed, w.N, w.K, False)
     return linear(x, w)
 
@@ -248,4 +245,4 @@ class SquaredReluMlp:
         else:
             a = linear(h, self.up)
             amd.relu_squared(a, a)
-        return project_to_residual(a, self.down, fine=True)
+        return project_to_residual(a, self.down)

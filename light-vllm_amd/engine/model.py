@@ -292,8 +292,9 @@ class DecoderModel:
                 attn_out = self.attn.forward(q, k, v, kv_caches[i] if kv_caches is not None else None,
                                              attn_metadata)
             if decode_only and cfg.o_proj_partials_min_rows <= T <= 64 and lw.o.packed is not None and lw.o.w8_t is None:
-                # the add+norm launch sums the fp32 partials of K's parts (as for the down projection)
-                hidden = torch.ops._C_amd.skinny_linear_fine_partials(attn_out, lw.o.packed, lw.o.N, lw.o.K)
+                # K is split over workgroups at this many rows: the add+norm launch sums the fp32 partials
+                # itself (as for the down projection), one reduce launch less
+                hidden = torch.ops._C_amd.skinny_linear_packed_partials(attn_out, lw.o.packed, lw.o.N, lw.o.K, False)
             elif attn8 is not None:
                 hidden = torch.ops._C_amd.skinny_linear_w8a8_q(attn8, lw.o.w8_packed, lw.o.w_scale, lw.o.x_scale, lw.o.N,
                                                                lw.o.K, None, cfg.dtype)
@@ -328,7 +329,8 @@ class DecoderModel:
             hidden = None
             if decode_only and lw.down.packed is not None and lw.down.w8_t is None:
                 # [S, T, hidden] fp32 split-K partial sums; the next add+norm adds them up
-                hidden = torch.ops._C_amd.skinny_linear_fine_partials(act, lw.down.packed, lw.down.N, lw.down.K)
+                hidden = torch.ops._C_amd.skinny_linear_packed_partials(act, lw.down.packed, lw.down.N,
+                                                                        lw.down.K, False)
             elif decode_only and lw.down.w8_packed is not None and T <= 64:
                 # W8A8: the raw partials and the scales the reduce pass would have applied (empty: K not split here)
                 d = lw.down

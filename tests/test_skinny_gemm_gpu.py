@@ -392,15 +392,50 @@ def test_products_in_one_launch(dtype, M, N, n_last, K):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(16, 32), (48, 2048), (16, 2080), (4096, 4096), (272, 4128), (2048, 8448), (64, 14336)])
-def test_fine_partials_sum_to_the_projection(dtype, M, N, K):
-    """Parts of K whose waves own at most 8 k-steps: edges of a part, a last part of one k-step, as many parts as there are."""
+def test_partials_sum_to_the_projection(dtype, M, N, K):
+    """Parts of K: a workgroup's 8 waves own at most 16 k-steps each, 8 above 32 rows; edges of a part, a last part of one k-step."""
     amd = torch.ops._C_amd
     g = torch.Generator(device=DEV).manual_seed(K + M)
     x = torch.randn(M, K, generator=g, device=DEV).to(dtype)
     w = (torch.randn(N, K, generator=g, device=DEV) * K ** -0.5).to(dtype)
-    parts = amd.skinny_linear_fine_partials(x, amd.pack_weight(w), N, K)
-    assert parts.shape == ((K + 2047) // 2048, M, N) and parts.dtype == torch.float32
+    parts = amd.skinny_linear_packed_partials(x, amd.pack_weight(w), N, K, False)
+    part = 4096 if M <= 32 else 2048
+    assert parts.shape == ((K + part - 1) // part, M, N) and parts.dtype == torch.float32
     ref = x.double() @ w.double().t()
     # K products, exact in fp32, summed in fp32 in any order: K roundings of partial sums, each at most the sum of magnitudes
     bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
     assert ((parts.double().sum(0) - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
+def test_sums_that_the_next_launch_takes_do_not_depend_on_the_workgroups(M):
+    """"gemm_workgroups" says how many workgroups a launch has, not how K is cut: steps of an engine with one in flight and with two,
+    and of one beside an engine of the other kind, have the same bits."""
+    from light_vllm_amd.attention.backend import PagedAttnImpl, PagedAttnMetadata
+    from light_vllm_amd.engine.config import ModelConfig
+    from light_vllm_amd.engine.mixers import SquaredReluMlp
+    from light_vllm_amd.engine.model import DecoderModel
+    g = torch.Generator(device=DEV).manual_seed(M)
+    weights = {"m.up": torch.randn(8448, 256, generator=g, device=DEV) / 16, "m.down": torch.randn(256, 8448, generator=g, device=DEV) / 90}
+    mlp, h = SquaredReluMlp(lambda n: weights[n].bfloat16(), "m", True), torch.randn(M, 256, generator=g, device=DEV).bfloat16()
+    cfg = ModelConfig(hidden_size=4096, intermediate_size=8448, num_hidden_layers=2, vocab_size=512, num_attention_heads=32,
+                      num_key_value_heads=8)
+    impl = PagedAttnImpl(cfg.num_attention_heads, cfg.head_dim, cfg.head_dim ** -0.5, cfg.num_key_value_heads, None, None, "auto")
+    model = DecoderModel(cfg, impl, DEV, seed=0)
+    pages = torch.arange(M, device=DEV, dtype=torch.int32)[:, None]
+    lens = torch.randint(1, 17, (M,), generator=g, device=DEV).to(torch.int32)
+    pos, ids = (lens - 1).long(), torch.randint(0, 512, (M,), generator=g, device=DEV)
+    metadata = PagedAttnMetadata(num_prefills=0, num_prefill_tokens=0, num_decode_tokens=M, slot_mapping=pages[:, 0].long() * 16 + pos,
+                                 seq_lens=None, seq_lens_tensor=lens, max_query_len=1, max_prefill_seq_len=0, max_decode_seq_len=16,
+                                 query_start_loc=None, seq_start_loc=None, context_lens_tensor=None, block_tables=pages)
+    caches = [torch.randn(2, M, 16 * 1024, generator=g, device=DEV).bfloat16() for _ in range(2)]
+    results = []
+    for wgs in (256, 128):
+        torch.ops._C_amd.set_tuning("gemm_workgroups", wgs)
+        try:
+            results.append((mlp(h), model.forward(ids, pos, [c.clone() for c in caches], metadata)))
+        finally:
+            torch.ops._C_amd.set_tuning("gemm_workgroups", 256)
+    (parts, hidden), (parts2, hidden2) = results
+    assert parts.shape == parts2.shape and torch.equal(parts, parts2)
+    assert torch.equal(hidden, hidden2) and bool(torch.isfinite(hidden.float()).all())
