@@ -76,10 +76,10 @@ class Worker:
         if self.device.type == "cuda":  # free memory before the weights (gpu_worker.py:78-80)
             torch.cuda.empty_cache()
             # what the caching allocator holds unused is free as well: a small model may fit into that alone
-            unused = torch.cuda.memory_reserved(self.device) - torch.cuda.memory_allocated(self.device)
-            self.init_gpu_memory = torch.cuda.mem_get_info(self.device)[0] + unused
+            self.held_gpu_memory = torch.cuda.memory_reserved(self.device) - torch.cuda.memory_allocated(self.device)
+            self.init_gpu_memory = self.free_gpu_memory(torch.cuda.memory_allocated(self.device))
         else:
-            self.init_gpu_memory = 0
+            self.init_gpu_memory = self.held_gpu_memory = 0
         self.model = model_entry(model_config.architecture).model_cls()(model_config, self.attn_impl, device, seed)
         self.attn_backend = attn_backend
         self.cache_engine: Optional[CacheEngine] = None
@@ -97,6 +97,12 @@ class Worker:
         # tests: keep the logits of the sampled rows of the last eager step
         self.capture_logits = False
         self.last_logits: Optional[torch.Tensor] = None
+
+    def free_gpu_memory(self, allocated: int) -> int:
+        """The device's free memory and what is unused, with `allocated` bytes in tensors, of what the caching allocator held before
+        the model.  (Its segments since then count as taken, as far as they go beyond that.)"""
+        unused = torch.cuda.memory_reserved(self.device) - allocated
+        return torch.cuda.mem_get_info(self.device)[0] + min(self.held_gpu_memory, max(unused, 0))
 
     # ---- KV-cache sizing (decoding/worker/gpu_worker.py:95-144, runner/model_runner.py:111-145) ----
     @staticmethod
@@ -209,10 +215,13 @@ class Worker:
         streams; the rest of `gpu_memory_utilization` x total memory, less the graph reserve, is KV cache."""
         scheduler_config = scheduler_config or SchedulerConfig()
         torch.cuda.empty_cache()
-        free_after_load = torch.cuda.mem_get_info(self.device)[0]
+        free_after_load = self.free_gpu_memory(torch.cuda.memory_allocated(self.device))
+        if self.held_gpu_memory > 0:  # (else nothing asks for the peak)
+            torch.cuda.reset_peak_memory_stats(self.device)
         self.profile_run(scheduler_config)
         torch.cuda.synchronize(self.device)
-        free_after_profile, total = torch.cuda.mem_get_info(self.device)
+        free_after_profile = self.free_gpu_memory(torch.cuda.max_memory_allocated(self.device))
+        total = torch.cuda.mem_get_info(self.device)[1]
         block_bytes = CacheEngine.get_cache_block_footprint(self.cache_config, self.model_config)
         out = self.kv_blocks_from_profile(total, self.init_gpu_memory, free_after_load, free_after_profile,
                                           self.cache_config.gpu_memory_utilization, scheduler_config.scheduling,

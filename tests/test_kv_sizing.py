@@ -91,6 +91,35 @@ def test_profile_run_sizes_the_cache_on_the_gpu():
 
 
 @pytest.mark.gpu
+def test_memory_that_the_allocator_holds_is_free_in_every_reading():
+    """What earlier work left in partly used segments is neither the model's nor its activations': as many blocks as without it, and
+    the activations count where they fit into it."""
+    import gc
+    from light_vllm_amd.attention.backend import PagedAttnBackend
+    sc = SchedulerConfig(max_num_batched_tokens=2048, max_num_seqs=16, max_model_len=2048)
+
+    def sized():
+        gc.collect()
+        w = Worker(ModelConfig.tiny(), CacheConfig(block_size=16, gpu_memory_utilization=0.05, swap_space_bytes=1 << 20), PagedAttnBackend(),
+                   "cuda:0", use_hip_graph=False)
+        blocks = w.determine_num_available_blocks(sc)[0]
+        p = w.profile
+        return blocks, p["block_bytes"], p["init_free"] - p["free_after_load"], p["free_after_load"] - p["free_after_profile"]
+    sized()  # (what a first run loads stays)
+    blocks, block_bytes, weights, activations = sized()
+    assert activations > 2 << 20
+    held = [torch.empty(n, dtype=torch.uint8, device="cuda:0") for n in [8 << 20] * 128 + [512 << 10] * 128]
+    del held[1:128:2], held[65::2]  # every other one: segments with room in them, 500 MB and more
+    again, _, held_weights, held_activations = sized()
+    # a segment of tensors of 1 to 10 MB is 20 MB; weights and activations leave parts of a few of them
+    slack = 6 * (20 << 20)
+    assert abs(held_weights - weights) <= slack and abs(held_activations - activations) <= slack
+    assert held_activations > 2 << 20
+    assert abs(again - blocks) * block_bytes <= slack, (again, blocks, block_bytes)
+    assert held
+
+
+@pytest.mark.gpu
 def test_rocm_platform_answers_on_the_gpu():
     """the capability the reference indexes (`[0] >= 8` for bf16, gpu_worker.py:227-238) exists."""
     from light_vllm_amd.platforms import RocmPlatform
