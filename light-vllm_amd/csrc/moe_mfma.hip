@@ -22,9 +22,10 @@ __device__ __forceinline__ e_f32x4_t moe_mfma(e_u32x4_t a, e_u32x4_t b, e_f32x4_
                                                  0);
 }
 
-// Weights that one workgroup reads go past the caches (ONCE); those of an expert with several tiles of slots come by way of the L2
-// that its tiles share.  Up + down, us, without and with: moe_stream_kernel, 32 rows, 6 of 64 experts of 2816, 268, 238; tiles of 128
-// slots, 1000 rows, 6 of 64 experts of 1408 and a shared one 276, 259, 2 of 32 193, 175; all tiles so, 1943 rows 376, 516.
+// Weights past the caches (ONCE) or by way of the L2.  Those that one workgroup reads go past them.  Up + down, us, without and with:
+// moe_stream_kernel, 32 rows, 6 of 64 experts of 2816, 268, 238; tiles of 128 slots, 1000 rows, 6 of 64 experts of 1408 and a shared
+// one 276, 259, 2 of 32 193, 175.  What several tiles of 128 slots share does not: all tiles so, 1943 rows 376, 516; for several of 16
+// see moe_stream_kernel.
 template <bool ONCE>
 __device__ __forceinline__ e_u32x4_t load_weights(const uint16_t* p) {
   if constexpr (ONCE) return __builtin_nontemporal_load(reinterpret_cast<const e_u32x4_t*>(p));
@@ -35,18 +36,10 @@ constexpr int kStreamBatch = 8, kStreamChunk = 64;  // k-steps per batch, per LD
 
 // grid (shares of the outputs, tiles of 16 slots); a wave computes W tiles 2 u and 2 u + 1, or (KS > 1, when few
 // experts have work) a KS-th of their k-steps, 64 / KS of every LDS chunk
-template <int PRODUCT, int KS>
-__global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
+template <int PRODUCT, int KS, bool ONCE>
+__device__ __forceinline__ void stream_product(const MoeParams& p, const int e, const int s0, const int s1, char* sx,
+                                               e_f32x4_t (*red)[2][64]) {
   constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
-  extern __shared__ __attribute__((aligned(16))) char sx[];  // [k-steps of a chunk][4][16][8]
-  __shared__ e_f32x4_t red[KS > 1 ? 4 : 1][2][64];
-  // the last expert's tiles first: it may be larger than the others, and its work is not to be what is left at the end
-  const int tile = p.tiles[4 * p.max_tiles + 1] - 1 - (int)blockIdx.y;
-  if (tile < 0) return;
-  const int e = p.tiles[4 * tile];
-  if (e < 0 || e >= p.experts) return;
-  const int s0 = p.tiles[4 * tile + 1], s1 = min(min(p.offsets[e + 1], s0 + 16), p.slots);
-  if (s0 >= s1) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
@@ -67,7 +60,7 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
     for (int j = 0; j < kStreamBatch; ++j)
 #pragma unroll
       for (int i = 0; i < 2; ++i)  // (a missing step: the last one again)
-        t[i][j] = load_weights<true>(w + ((int64_t)i * steps + min(b + j, steps - 1)) * 512);
+        t[i][j] = load_weights<ONCE>(w + ((int64_t)i * steps + min(b + j, steps - 1)) * 512);
   };
   fetch(0, a[0]);
   const int64_t ld = UP ? p.width : p.ff_max;
@@ -139,6 +132,28 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
       store4<BF16>((uint16_t*)p.out + (int64_t)slot * (UP ? p.ff_max : p.width) + 32 * u + 16 * i + 4 * g, v);
     }
   }
+}
+
+// Of an expert's two to four tiles of 16 slots those that run at the same time share little by way of the L2 (they are on several
+// XCDs), and past the caches is faster as long as other experts' weights are most of what is read: 2 of 8 experts of 1408 and a shared
+// one of 2816, 2048 wide, up, us by way of the L2 and past it: 32 rows 38.2, 32.0, 64 rows 39.5, 37.8; 6 of 64, down, 64 rows 76.4,
+// 70.2.  Not going up where the launch is experts that most rows take and as large as needs no KS: 64 rows that all take the same 2 of
+// 16 experts of 2816, 4096 wide, 50, 68, the same 8 163, 207; down 27.7, 24.2 and 73, 84, with a shared expert 54, 51.  There the
+// tiles are full: 14 slots of 16 and more (12.8 in the second case above, 16 in these).
+template <int PRODUCT, int KS>
+__global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
+  extern __shared__ __attribute__((aligned(16))) char sx[];  // [k-steps of a chunk][4][16][8]
+  __shared__ e_f32x4_t red[KS > 1 ? 4 : 1][2][64];
+  // the last expert's tiles first: it may be larger than the others, and its work is not to be what is left at the end
+  const int all = p.tiles[4 * p.max_tiles + 1], tile = all - 1 - (int)blockIdx.y;
+  if (tile < 0) return;
+  const int e = p.tiles[4 * tile];
+  if (e < 0 || e >= p.experts) return;
+  const int s0 = p.tiles[4 * tile + 1], s1 = min(min(p.offsets[e + 1], s0 + 16), p.slots);
+  if (s0 >= s1) return;
+  if constexpr (PRODUCT != kMoeDown && KS == 1)
+    if (p.tiles[4 * tile + 3] >= 3 && p.slots >= 14 * all) return stream_product<PRODUCT, KS, false>(p, e, s0, s1, sx, red);
+  stream_product<PRODUCT, KS, true>(p, e, s0, s1, sx, red);
 }
 
 // A workgroup's turn (moe_turns.h).  Units of an expert are up to 1024 of its slots side by side, W block after W block, so that an

@@ -65,6 +65,19 @@ def test_products(amd, counts, ff, width, act, weigh):
         assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5).all(), (e, (got - want).abs().max())
 
 
+@pytest.mark.parametrize("act", ["clamped", "relu_squared"])
+@pytest.mark.parametrize("width", [64, 2400])
+@pytest.mark.parametrize("counts,full", [([64, 0, 0, 0], True), ([0, 48, 16, 0], True), ([0, 0, 15, 48], True), ([33, 1, 30, 0], False),
+                                         ([49, 1, 1, 1], False), ([0, 32, 0, 31], True)], ids=lambda v: "-".join(map(str, v)) if isinstance(v, list) else "")
+def test_products_of_few_rows(amd, counts, full, width, act):
+    """Up to 64 rows, tiles of 16: experts of one to four tiles.  Going up, those of three and more among full tiles read their weights
+    by way of the L2 where there are workgroups for whole units, all others past it."""
+    tiles = sum(-(-n // 16) for n in counts)
+    assert (sum(counts) >= 14 * tiles) == full
+    ff = 4480 if act == "clamped" else 8320  # a fourth of its units, for each of 8 tiles that there may be, is more than 512
+    test_products(amd, counts, [ff, 96, 1408, 352], width, act, True)
+
+
 @pytest.mark.parametrize("act", [0, 2], ids=["clamped", "relu_squared"])
 @pytest.mark.parametrize("copies", [1, 70], ids=["half blocks", "whole blocks"])
 def test_blocks_of_weight_rows(amd, copies, act):
