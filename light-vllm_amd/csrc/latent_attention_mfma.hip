@@ -32,28 +32,26 @@ __device__ __forceinline__ int exchange(int r) {
   return NK % 4 == 0 ? r & 15 : NK % 2 == 0 ? (r >> 1) & 7 : (r >> 2) & 3;
 }
 
+constexpr int kColumnPitch = 72;  // elements between columns of P
+
 // everything written to LDS so far is seen by the workgroup; copies in flight stay in flight
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// NC, NR: latent and rotated part in units of 32 entries
-template <int NC, int NR, int CT>
-__global__ __launch_bounds__(256 * CT, 1) void latent_attention_mfma_kernel(const LatentAttnParams p) {
+// NC, NR: latent and rotated part in units of 32 entries; ONCE: one workgroup has all columns of the sequence
+template <int NC, int NR, int CT, bool ONCE>
+__device__ __forceinline__ void latent_columns(const LatentAttnParams& p, const int qbeg, const int qlen, char* tile,
+                                               uint16_t (*sp)[16 * kColumnPitch], float (*sm)[4][16]) {
   constexpr int NK = NC + NR, RE = 32 * NK, CP = 32 * NC;
   constexpr int RC = 4 * NK, RB = 64 * NK;  // 16-byte chunks and bytes of a row
   constexpr int kStage = 64 * RB;
   constexpr int COPIES = (NK + CT - 1) / CT;  // of 1 KiB, per wave and tile: a page is NK KiB
   constexpr int NT = NC / 2;               // 16-entry tiles of O a wave owns
-  constexpr int PP = 72;                   // elements between columns of P
-  extern __shared__ __attribute__((aligned(16))) char tile[];  // [2][64][RB]
-  __shared__ __attribute__((aligned(16))) uint16_t sp[CT][16 * PP];
-  __shared__ float sm[CT][4][16];
+  constexpr int PP = kColumnPitch;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kg = CT == 1 ? wave : wave & 3, ct = CT == 1 ? 0 : wave >> 2;
   const int g = lane >> 4, c = lane & 15;
   const int seq = blockIdx.y, share = blockIdx.z;
-  const int qbeg = p.query_start_loc[seq], qlen = p.query_start_loc[seq + 1] - qbeg;
-  if (qlen <= 0 || qlen > p.absorbed_max) return;
   const int ncols = qlen * p.heads, col_wg = blockIdx.x * 16 * CT;
   if (col_wg >= ncols) return;
   const int ctx = p.seq_lens[seq] - qlen;
@@ -86,7 +84,7 @@ __global__ __launch_bounds__(256 * CT, 1) void latent_attention_mfma_kernel(cons
     for (int j = 0; j < COPIES; ++j)
       if (j * CT + ct < NK)
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + from[j]),
-                                         (__attribute__((address_space(3))) void*)(dst + (j * CT + ct) * 1024), 16, 0, 2);  // (past the caches)
+                                         (__attribute__((address_space(3))) void*)(dst + (j * CT + ct) * 1024), 16, 0, ONCE ? 2 : 0);  // (past the caches)
   };
   m_u32x4_t qf[NK];
   {
@@ -196,6 +194,20 @@ __global__ __launch_bounds__(256 * CT, 1) void latent_attention_mfma_kernel(cons
     p.part_ml[2 * part] = m;
     p.part_ml[2 * part + 1] = (sm[ct][0][c] + sm[ct][1][c]) + (sm[ct][2][c] + sm[ct][3][c]);
   }
+}
+
+// Cached rows that one workgroup of a share reads go past the caches, those that several read by way of them.  Both launches, us, by
+// way of them and past: 16 tokens after 4000 of 16 heads 35.6, 31.9, of 64 heads 47.9, 50.5; 4 portions of 16 tokens after 4000, 16
+// heads 46.6, 53.4; 64 tokens after 4000 of 128 heads 213, 243.
+template <int NC, int NR, int CT>
+__global__ __launch_bounds__(256 * CT, 1) void latent_attention_mfma_kernel(const LatentAttnParams p) {
+  extern __shared__ __attribute__((aligned(16))) char tile[];  // [2][64] rows
+  __shared__ __attribute__((aligned(16))) uint16_t sp[CT][16 * kColumnPitch];
+  __shared__ float sm[CT][4][16];
+  const int qbeg = p.query_start_loc[blockIdx.y], qlen = p.query_start_loc[blockIdx.y + 1] - qbeg;
+  if (qlen <= 0 || qlen > p.absorbed_max) return;
+  if (CT == 1 || qlen * p.heads <= 16 * CT) latent_columns<NC, NR, CT, true>(p, qbeg, qlen, tile, sp, sm);
+  else latent_columns<NC, NR, CT, false>(p, qbeg, qlen, tile, sp, sm);
 }
 
 // The shares of R rows of one head -> their weighted sum o in latent space (bf16, as W's product reads it) -> out = V_h o * gate.
