@@ -249,9 +249,8 @@ __device__ __forceinline__ void to_lds16(const char* from, void* dst) {
 // both operands through LDS, were no faster.  Between 128 and 400 slots an expert neither memory (4.3 TB/s of weights), the L1, LDS
 // nor MFMA (each near 40 %) is at its limit by itself; one workgroup a CU that goes on from unit to unit, with 8 steps of weights on
 // their way, was slower (1943 rows, 6 of 64 experts of 1408, up: 237 us; 262 with 8 waves, 322 with 4).
-// NT = 2 where units of NT = 4 are fewer than one and a half a CU: a step costs less and eight of them, not four, are under way, so
-// that the memory's latency bounds a walk no more.  Going down 1408 (a shared expert 2816) -> 2048, 2 of 32 experts, us with NT = 4
-// and 2: 300 rows 68, 51; 1000 rows 68, 56; where units are more, going up the same: 300 rows 70, 78; 1000 rows 102, 109.
+// NT = 2 (takes_half_blocks, moe_turns.h): a step costs less and eight of them, not four, are under way, so that the memory's latency
+// bounds a walk no more.
 // Slots' chunks trade places by bit 3 of the slot: LDS reads 16 bytes for lanes 0-3, 12-15, 20-27 at a time (by bits 2 and 3, half
 // of its cycles were conflicts).
 constexpr int kStageBytes = kMoeTile * 128;  // two k-steps of 32: a slot's 128 bytes, 8 slots a copy
@@ -576,19 +575,16 @@ static void go(const MoeParams& p, hipStream_t s) {
     const int least = small ? kMoeSmallTile : tile;
     const int64_t tiles = small ? p.max_tiles : std::min<int64_t>(p.max_tiles, p.slots / tile + p.experts);
     const int64_t last_tiles = (p.rows + least - 1) / least;  // a token takes an expert once
-    auto launch = [&](auto nt) {
-      constexpr int NT = decltype(nt)::value;
-      auto blocks = [&](int ff) { return ((GATED ? ff / 8 : (UP ? ff : p.width) / 16) + 4 * NT - 1) / (4 * NT); };
-      const int first = blocks(p.ff_first), last = blocks(p.ff_last);
-      if (NT == 4) {  // with as many slots for each expert
-        const int64_t each = (p.slots + (int64_t)p.experts * least - 1) / ((int64_t)p.experts * least);
-        if (p.experts * each * first + last_tiles * last <= 384) return false;
-      }
-      const unsigned grid = (unsigned)unit_workgroups(tiles * first, last_tiles * last);
-      hipLaunchKernelGGL((moe_tile_kernel<PRODUCT, NT>), dim3(grid), dim3(256), 0, s, p, first, last);
-      return true;
+    auto blocks = [&](int nt, int ff) { return ((GATED ? ff / 8 : (UP ? ff : p.width) / 16) + 4 * nt - 1) / (4 * nt); };
+    const BlockCounts whole{blocks(4, p.ff_first), blocks(4, p.ff_last)}, half{blocks(2, p.ff_first), blocks(2, p.ff_last)};
+    auto launch = [&](auto nt, const BlockCounts& b) {
+      const unsigned grid = (unsigned)unit_workgroups(tiles * b.first, last_tiles * b.last);
+      hipLaunchKernelGGL((moe_tile_kernel<PRODUCT, decltype(nt)::value>), dim3(grid), dim3(256), 0, s, p, b.first, b.last);
     };
-    if (!launch(std::integral_constant<int, 4>{})) launch(std::integral_constant<int, 2>{});
+    if (takes_half_blocks(p.rows, p.slots, p.experts, least, whole, half, UP, p.ff_last > p.ff_first))
+      launch(std::integral_constant<int, 2>{}, half);
+    else
+      launch(std::integral_constant<int, 4>{}, whole);
   }
 }
 

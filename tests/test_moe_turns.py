@@ -29,6 +29,9 @@ extern "C" int solo(int up, int ff_first, int ff_last) { return solo_units(up, f
 extern "C" long ring(long units_first, long units_last, int solo) { return ring_workgroups(units_first, units_last, solo); }
 extern "C" long single(long units_first, long units_last) { return unit_workgroups(units_first, units_last); }
 extern "C" int turns() { return kTurns; }
+extern "C" int half(int rows, long slots, int experts, int first4, int last4, int first2, int last2, int up, int larger) {
+  return takes_half_blocks(rows, slots, experts, 128, {first4, last4}, {first2, last2}, up, larger);
+}
 """
 
 
@@ -40,6 +43,7 @@ def lib(tmp_path_factory):
                     str(d / "t.so")], check=True)
     t = ctypes.CDLL(str(d / "t.so"))
     t.ring.restype = t.single.restype = ctypes.c_long
+    t.half.argtypes = [ctypes.c_int, ctypes.c_long] + [ctypes.c_int] * 7
     t.ring.argtypes, t.single.argtypes = [ctypes.c_long, ctypes.c_long, ctypes.c_int], [ctypes.c_long] * 2
     return t
 
@@ -85,3 +89,24 @@ def test_a_unit_a_workgroup(lib):
         most_first, most_last = r.randint(1, 3000), r.randint(0, 1000)
         first, last = r.randint(0, most_first), r.randint(0, most_last)
         assert walk(lib, first, last, r.randint(1, 16), lib.single(most_first, most_last), 1) == (0, 0), (first, last)
+
+
+# rows, experts taken by a row, experts, their inner size, the shared one's (0: none), width; whether half blocks were ahead, going up (None:
+# level) and down
+HALF = [(300, 2, 32, 1408, 2816, 2048, None, True), (1000, 2, 32, 1408, 2816, 2048, None, True), (1943, 6, 64, 1408, 2816, 2048, False, False),
+        (65, 2, 8, 1408, 2816, 2048, True, True), (420, 2, 8, 1408, 2816, 2048, False, True), (8192, 6, 64, 2816, 2816, 2048, False, False),
+        (500, 2, 16, 1408, 0, 2048, False, True), (1000, 2, 16, 1408, 0, 2048, True, False), (1500, 4, 32, 512, 0, 1024, None, False),
+        (1500, 2, 16, 512, 0, 1024, True, True), (2000, 2, 16, 512, 0, 1024, None, False), (300, 2, 16, 2816, 2816, 2048, None, False),
+        (100, 4, 16, 768, 768, 2048, True, False), (700, 2, 16, 512, 512, 1024, True, True), (1000, 2, 16, 512, 512, 1024, True, True),
+        (1000, 2, 8, 512, 0, 2048, True, False), (300, 2, 64, 512, 0, 1024, True, True), (65, 2, 8, 7168, 0, 4096, None, True)]
+
+
+@pytest.mark.parametrize("rows,top,experts,ff,shared,width,up,down", HALF)
+def test_half_blocks(lib, rows, top, experts, ff, shared, width, up, down):
+    """Where measurements put the line between half and whole blocks of weight rows (gated experts)."""
+    all_experts, slots, last = experts + (shared > 0), rows * (top + (shared > 0)), shared or ff
+    blocks = lambda n, nt: -(-n // (4 * nt))
+    for is_up, want, tiles in ((1, up, lambda f: f // 8), (0, down, lambda f: width // 16)):
+        got = lib.half(rows, slots, all_experts, blocks(tiles(ff), 4), blocks(tiles(last), 4), blocks(tiles(ff), 2), blocks(tiles(last), 2),
+                       is_up, last > ff)
+        assert want is None or bool(got) == want
