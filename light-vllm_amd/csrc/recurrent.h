@@ -27,6 +27,8 @@
 // the read-out.  Rows are the new tokens of `num_seqs` sequences back to back (query_start_loc); a sequence whose tokens
 // are all in this step (seq_lens == its rows) starts from a zero state, every other one from its slot.
 #pragma once
+#include <type_traits>
+
 #include "head_norm_gate.h"
 #include "log_decay.h"
 #include "rotation.h"
@@ -451,10 +453,11 @@ __global__ __launch_bounds__(256, NT == 1 && NV <= 4 ? 3 : 2) void chunk_mix_ker
   }
 }
 
-// The first state of every segment, in place of the last state it would have had from zero: a thread per state element
-// or four, sequential over the segments, sixteen of which are asked for at once (behind the store of one, the load of the next waited
-// for it).  64 segments of 8
-// heads of 128 x 128 and 24 of 32 heads of 64 x 64 took 33 us together an element a thread, 25 with four.
+// The first state of every segment, in place of the last state it would have had from zero: a thread per state element or four,
+// sequential over the segments, B of which are asked for at once (behind the store of one, the load of the next waited for it).  64
+// segments of 8 heads of 128 x 128 and 24 of 32 heads of 64 x 64 took 33 us together an element a thread, 25 with four.  Few segments
+// take B = 4: a missing one is asked for like the others (the last one again), which with sixteen cost 0.9 of 26 us at 4 segments of 16
+// heads of 64 x 64.
 template <int VEC>
 static __global__ __launch_bounds__(256) void chunk_combine_kernel(const MixParams p, const int dkp) {
   const int head = blockIdx.y, seq = blockIdx.z;
@@ -472,23 +475,27 @@ static __global__ __launch_bounds__(256) void chunk_combine_kernel(const MixPara
   float* st = p.seg_state + base * per_head + i;
   const float* de = p.seg_decay + base * dkp + i / p.dv;
   const int64_t st_step = p.heads * per_head, de_step = (int64_t)p.heads * dkp;
-  constexpr int B = 16;
-  for (int k0 = 0; k0 < segs - 1; k0 += B) {
-    float own[B][VEC], d[B];
+  auto walk = [&](auto at_once) __attribute__((always_inline)) {
+    constexpr int B = decltype(at_once)::value;
+    for (int k0 = 0; k0 < segs - 1; k0 += B) {
+      float own[B][VEC], d[B];
 #pragma unroll
-    for (int j = 0; j < B; ++j) {
-      const int k = min(k0 + j, segs - 2);
-      load_vec<F32, VEC>(st + k * st_step, own[j]);
-      d[j] = de[k * de_step];
-    }
-#pragma unroll
-    for (int j = 0; j < B; ++j)
-      if (k0 + j < segs - 1) {
-        store_vec<F32, VEC>(st + (k0 + j) * st_step, x);
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) x[v] = fmaf(d[j], x[v], own[j][v]);
+      for (int j = 0; j < B; ++j) {
+        const int k = min(k0 + j, segs - 2);
+        load_vec<F32, VEC>(st + k * st_step, own[j]);
+        d[j] = de[k * de_step];
       }
-  }
+#pragma unroll
+      for (int j = 0; j < B; ++j)
+        if (k0 + j < segs - 1) {
+          store_vec<F32, VEC>(st + (k0 + j) * st_step, x);
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) x[v] = fmaf(d[j], x[v], own[j][v]);
+        }
+    }
+  };
+  if (segs <= 5) walk(std::integral_constant<int, 4>{});
+  else walk(std::integral_constant<int, 16>{});
   store_vec<F32, VEC>(st + (segs - 1) * st_step, x);
 }
 

@@ -61,6 +61,13 @@ def test_segments(amd, lengths, heads, dk, dv, kind, bonus):
     check(out, state, want, want_state)
 
 
+@pytest.mark.parametrize("heads,dk,dv", [(3, 64, 64), (2, 128, 30)])
+@pytest.mark.parametrize("lengths", [[80], [81], [64, 65, 80, 81, 96, 97]], ids=lambda v: "-".join(map(str, v)))
+def test_few_segments_and_more(amd, lengths, heads, dk, dv):
+    """Up to five segments of a sequence are asked for four at a time, more of them sixteen at a time; columns in fours and one by one."""
+    test_segments(amd, lengths, heads, dk, dv, 0, False)
+
+
 @pytest.mark.parametrize("lengths", [[1] * 20 + [33] + [1] * 3 + [16, 17, 49] + [1] * 9, [3, 64, 1, 1, 65, 2, 15, 48], [1] * 255 + [45], [45] + [1] * 255])
 def test_single_tokens_beside_segments(amd, lengths):
     test_segments(amd, lengths, 8, 64, 64, 0, False)
