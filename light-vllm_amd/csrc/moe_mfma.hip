@@ -4,8 +4,8 @@
 //   * few slots per expert (decode steps): bound by the weights' bytes.  A workgroup takes 16 slots of one expert and a share
 //     of its outputs; the slots' rows sit in LDS in fragment order (2048 of K at a time), every wave streams the two W tiles
 //     of its own (1 KiB a load, eight k-steps in flight behind the eight in use) and needs no other wave;
-//   * prompts: tiles of up to 128 slots x 256 W rows, or 128 where those are few (moe_tile_kernel).  A slot's 64 bytes of a k-step
-//     are four chunks, exchanged so that a fragment read is free of bank conflicts.
+//   * prompts: tiles of up to 128 slots x 256 W rows, or 128 where those are few (moe_tile_kernel).  A slot's 128 bytes of two k-steps
+//     are eight chunks, exchanged so that a fragment read is free of bank conflicts.
 #include <algorithm>
 
 #include "moe.h"
@@ -156,20 +156,19 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const MoeParams p) {
   stream_product<PRODUCT, KS, true>(p, e, s0, s1, sx, red);
 }
 
-// A workgroup's turn (moe_turns.h).  Units of an expert are up to 1024 of its slots side by side, W block after W block, so that an
+// A workgroup's unit (moe_turns.h).  Units of an expert are up to 1024 of its slots side by side, W block after W block, so that an
 // XCD's L2 serves a W block to all of them and their rows to the next blocks.
 struct TileWork {
   int e, block, s0, s1, steps, ntiles;  // slots s0 .. s1 - 1, k-steps, W tiles of 16 rows of the expert
   bool any, once;  // once: the expert's only tile
 };
 template <int PRODUCT, int TILE, int TILEW>
-__device__ __forceinline__ TileWork tile_work(const MoeParams& p, const int blocks_first, const int blocks_last, const int turn) {
+__device__ __forceinline__ TileWork tile_work(const MoeParams& p, const int blocks_first, const int blocks_last) {
   constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
   constexpr int kSide = 1024 / TILE;
   TileWork t{};
   const int tiles_first = p.tiles[4 * p.max_tiles], tiles_last = p.tiles[4 * p.max_tiles + 1] - tiles_first;
-  const TurnUnit u = turn_unit(tiles_first * blocks_first, tiles_last * blocks_last, solo_units(UP, p.ff_first, p.ff_last),
-                               blockIdx.x & 7, blockIdx.x >> 3, gridDim.x >> 3, turn);
+  const TurnUnit u = turn_unit(tiles_first * blocks_first, tiles_last * blocks_last, blockIdx.x & 7, blockIdx.x >> 3);
   if (!u.any) return t;
   const int blocks = u.last ? blocks_last : blocks_first;
   int unit = u.unit + (u.last ? tiles_first * blocks : 0), tile = unit / blocks;
@@ -192,47 +191,43 @@ __device__ __forceinline__ TileWork tile_work(const MoeParams& p, const int bloc
   return t;
 }
 
-// A wave's results by way of 2 KiB of LDS of its own: W tiles nt0 .. of groups of 16 slots, slot0 + m * next ..; 64 outputs of a
-// group at a time, so that a store is a line of a slot's row (8 bytes a lane as the products leave them took 17 000 clocks of a
-// turn's 110 000).
-template <int PRODUCT, int NT, int MT, typename WEIGHT>
+// A wave's results by way of 2 KiB of LDS of its own: W tiles nt0 .. of groups of 16 slots from slot0 on, a group at a time, so that a
+// store is a line of a slot's row and not the 8 bytes a lane that the products leave.
+template <int PRODUCT, int NT, int MT>
 __device__ __forceinline__ void tile_store(const MoeParams& p, int e, const e_f32x4_t (&acc)[NT][MT], char* lds, int nt0, int ntiles,
-                                           int slot0, int next, int s1, WEIGHT weight) {
+                                           int slot0, int s1) {
   constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
   [[maybe_unused]] const MoeActivation act(p, GATED ? e : -1);
-  constexpr int kPart = GATED && NT > 4 ? 8 : NT < 4 ? NT : 4, kOuts = kPart * (GATED ? 8 : 16), kChunks = kOuts / 8;  // of 8 outputs
+  constexpr int kOuts = NT * (GATED ? 8 : 16), kChunks = kOuts / 8;  // of 8 outputs
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int64_t out_ld = UP ? p.ff_max : p.width;
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    const int slot = slot0 + m * next;
+    const int slot = slot0 + m * 16;
     if (slot >= s1) break;
-    const float f = UP ? weight(slot + c) : 1.f;
+    const float f = UP ? slot_weight_of(p, min(slot + c, s1 - 1)) : 1.f;
 #pragma unroll
-    for (int n0 = 0; n0 < NT; n0 += kPart) {
+    for (int n = 0; n < NT; n += GATED ? 2 : 1) {
+      float v[4];
 #pragma unroll
-      for (int n = n0; n < n0 + kPart; n += GATED ? 2 : 1) {
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if constexpr (GATED) v[r] = act(acc[n][m][r] * f, acc[n + 1][m][r] * f);
-          else v[r] = UP ? relu_squared_of(acc[n][m][r] * f) : acc[n][m][r];
-        }
-        const int chunk = (GATED ? n - n0 : 2 * (n - n0)) + (g >> 1);
-        store4<BF16>(reinterpret_cast<uint16_t*>(lds + c * (kOuts * 2) + ((chunk ^ c) & (kChunks - 1)) * 16 + (g & 1) * 8), v);
+      for (int r = 0; r < 4; ++r) {
+        if constexpr (GATED) v[r] = act(acc[n][m][r] * f, acc[n + 1][m][r] * f);
+        else v[r] = UP ? relu_squared_of(acc[n][m][r] * f) : acc[n][m][r];
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the wave's own next reads see it)
-      const int first = (nt0 + n0) * (GATED ? 8 : 16), outs = (ntiles - nt0 - n0) * (GATED ? 8 : 16);
-#pragma unroll
-      for (int j = 0; j < (kChunks + 3) / 4; ++j) {
-        const int r = j * (64 / kChunks) + lane / kChunks, q = lane % kChunks;
-        if (kChunks < 4 && r >= 16) break;
-        const e_u32x4_t v = *reinterpret_cast<const e_u32x4_t*>(lds + r * (kOuts * 2) + ((q ^ r) & (kChunks - 1)) * 16);
-        if (slot + r < s1 && q * 8 < outs)
-          *reinterpret_cast<e_u32x4_t*>((uint16_t*)p.out + (slot + r) * out_ld + first + q * 8) = v;
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read before it is written again)
+      const int chunk = (GATED ? n : 2 * n) + (g >> 1);
+      store4<BF16>(reinterpret_cast<uint16_t*>(lds + c * (kOuts * 2) + ((chunk ^ c) & (kChunks - 1)) * 16 + (g & 1) * 8), v);
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the wave's own next reads see it)
+    const int first = nt0 * (GATED ? 8 : 16), outs = (ntiles - nt0) * (GATED ? 8 : 16);
+#pragma unroll
+    for (int j = 0; j < (kChunks + 3) / 4; ++j) {
+      const int r = j * (64 / kChunks) + lane / kChunks, q = lane % kChunks;
+      if (kChunks < 4 && r >= 16) break;
+      const e_u32x4_t v = *reinterpret_cast<const e_u32x4_t*>(lds + r * (kOuts * 2) + ((q ^ r) & (kChunks - 1)) * 16);
+      if (slot + r < s1 && q * 8 < outs)
+        *reinterpret_cast<e_u32x4_t*>((uint16_t*)p.out + (slot + r) * out_ld + first + q * 8) = v;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (read before it is written again)
   }
 }
 
@@ -244,15 +239,15 @@ __device__ __forceinline__ void to_lds16(const char* from, void* dst) {
 
 // Prompts: 64 NT W rows x up to 128 slots a workgroup, a wave 16 NT x 128, two workgroups a CU, a unit each.  W goes straight to the
 // operand registers of the one wave that uses it, slots by way of LDS.
-// NT = 4.  With many slots the chip's power bounds it: 1.8 GHz at 55 % of the MFMA cycles, where the library's plain product of
-// 49152 x 2816 x 2048 runs at 1.06 to 1.27 PFLOP/s and this one (8192 rows, 6 of 64 experts) at 0.98 to 1.01; 256 slots a workgroup,
-// both operands through LDS, were no faster.  Between 128 and 400 slots an expert neither memory (4.3 TB/s of weights), the L1, LDS
+// NT = 4.  With many slots the chip's power bounds it: 1.8 GHz at 55 % of the MFMA cycles.  8192 rows, 6 of 64 experts of 2816, 2048
+// wide: 1.08 PFLOP/s going up and 1.10 down, where the library's plain products of these sizes run at 1.33 and 1.45; 256 slots a
+// workgroup, both operands through LDS, were no faster.  Between 128 and 400 slots an expert neither memory (4.3 TB/s of weights), the L1, LDS
 // nor MFMA (each near 40 %) is at its limit by itself; one workgroup a CU that goes on from unit to unit, with 8 steps of weights on
 // their way, was slower (1943 rows, 6 of 64 experts of 1408, up: 237 us; 262 with 8 waves, 322 with 4).
 // NT = 2 (takes_half_blocks, moe_turns.h): a step costs less and eight of them, not four, are under way, so that the memory's latency
 // bounds a walk no more.
-// Slots' chunks trade places by bit 3 of the slot: LDS reads 16 bytes for lanes 0-3, 12-15, 20-27 at a time (by bits 2 and 3, half
-// of its cycles were conflicts).
+// A slot's eight chunks trade places by the slot's three low bits: a fragment read takes one chunk of each of 16 slots, 128 bytes
+// apart.  4 to 8 % of the cycles in which LDS is active are conflicts, those of the results' way out included.
 constexpr int kStageBytes = kMoeTile * 128;  // two k-steps of 32: a slot's 128 bytes, 8 slots a copy
 constexpr int tile_steps(int NT) { return NT == 4 ? 4 : 8; }  // k-steps of weights in registers; half as many stages of slots
 template <int PRODUCT, bool ONCE, int NT, int MT>
@@ -347,14 +342,13 @@ __device__ __forceinline__ void tile_product(const MoeParams& p, const TileWork&
     }
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (no copy to LDS is under way, and everyone has read the last stage)
-  tile_store<PRODUCT, NT, MT>(p, e, acc, ring[0] + wave * 2048, nt0, ntiles, s0, 16, s1,
-                             [&](int slot) { return slot_weight_of(p, min(slot, s1 - 1)); });
+  tile_store<PRODUCT, NT, MT>(p, e, acc, ring[0] + wave * 2048, nt0, ntiles, s0, s1);
 }
 
 template <int PRODUCT, int NT>
 __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, const int blocks_first, const int blocks_last) {
   __shared__ __attribute__((aligned(16))) char ring[tile_steps(NT) / 2][kStageBytes];
-  const TileWork t = tile_work<PRODUCT, kMoeTile, 4 * NT>(p, blocks_first, blocks_last, 0);
+  const TileWork t = tile_work<PRODUCT, kMoeTile, 4 * NT>(p, blocks_first, blocks_last);
   if (!t.any) return;
   const int groups = (t.s1 - t.s0 + 15) >> 4;
   if (t.once) {

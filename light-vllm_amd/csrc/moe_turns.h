@@ -1,57 +1,32 @@
 // Which workgroup of the grouped products' launches takes which piece of work, in whole numbers that the host counts as well.
 //
-// A unit is a block of W rows of one tile of slots.  An XCD gets an eighth of the last expert's units (the shared expert may be
-// larger: its units come first) and an eighth of all others'; its workgroups take them in turn.
+// A unit is a block of W rows of one tile of slots; a workgroup takes one.  An XCD gets an eighth of the last expert's units, which come
+// first (the shared expert may be larger), and an eighth of all others'.
 #pragma once
 #include <math.h>
 #include <stdint.h>
 
 namespace lvllm {
 
-constexpr int kTurns = 64;  // of a workgroup, at most
-
-// Units of the other experts that take as long as one of the last expert's (going down, k-steps are the experts' inner size).  At
-// most kMostSolo, however large the last expert is: a workgroup may have that many turns more than its share.
-constexpr int kMostSolo = 16;
-__host__ __device__ constexpr int solo_units(bool up, int ff_first, int ff_last) {
-  if (up) return 1;
-  const int64_t n = ((int64_t)ff_last + ff_first / 2) / ff_first;
-  return n < 1 ? 1 : n > kMostSolo ? kMostSolo : (int)n;
-}
-
 struct TurnUnit {
   int unit;   // among the last expert's, or among all others'
   bool last;  // the last expert's
   bool any;
 };
-// Turn `turn` of workgroup `cu` of `cus` of an XCD; units_first, units_last: of all XCDs.  The first `own` turns are the last
-// expert's; workgroups with one of them fewer start on the others by so much earlier.
-__host__ __device__ inline TurnUnit turn_unit(int units_first, int units_last, int solo, int xcd, int cu, int cus, int turn) {
+// Workgroup `cu` of an XCD; units_first, units_last: of all XCDs.
+__host__ __device__ inline TurnUnit turn_unit(int units_first, int units_last, int xcd, int cu) {
   const int per_first = (units_first + 7) / 8, per_last = (units_last + 7) / 8;
-  const int full = per_last / cus, rest = per_last % cus;  // (`rest` workgroups have full + 1 of them)
-  const int own = full + (cu < rest);
-  if (turn < own) {
-    const int unit = xcd * per_last + turn * cus + cu;
+  if (cu < per_last) {
+    const int unit = xcd * per_last + cu;
     return {unit, true, unit < units_last};
   }
-  const int late = cu < rest ? solo : 0, round = turn - own + late;  // while the others were at their longer turn
-  const int mine = rest == 0     ? round * cus + cu
-                   : round >= solo ? solo * (cus - rest) + (round - solo) * cus + cu
-                                   : round * (cus - rest) + cu - rest;
-  const int unit = xcd * per_first + mine;
+  const int mine = cu - per_last, unit = xcd * per_first + mine;
   return {unit, false, mine < per_first && unit < units_first};
 }
 
-// A launch with a unit a workgroup: an eighth of both kinds, rounded up, eight times.
+// Their workgroups: an eighth of both kinds, rounded up, eight times.
 inline int64_t unit_workgroups(int64_t units_first, int64_t units_last) {
   return 8 * ((units_first + 7) / 8 + (units_last + 7) / 8);
-}
-// A launch with several units a workgroup: a workgroup a CU, more only where one might have over kTurns turns.  With `share` units each, every unit has a turn
-// below kTurns: a workgroup without a last turn of the last expert's takes at most `solo` units by itself first, and what comes
-// before and after those is floor(last expert's / cus) + ceil(the others' / cus) <= share; one with that turn takes share + 1.
-inline int64_t ring_workgroups(int64_t units_first, int64_t units_last, int solo) {
-  const int64_t all = unit_workgroups(units_first, units_last), share = kTurns - solo, cus = (all / 8 + share - 1) / share;
-  return cus > 32 ? 8 * cus : all < 256 ? all : 256;
 }
 
 // Blocks of W rows of the other experts and of the last one.

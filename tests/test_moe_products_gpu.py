@@ -1,11 +1,11 @@
-"""Grouped products of prompts at the edges of their tiles: experts with 0, 1, 63 .. 65 and 127 .. 129 rows, inner sizes from one k-step on
-and of unequal length, weights on what an expert reads; both bodies (few and many rows an expert)."""
+"""Grouped products at the edges of their tiles: experts with 0, 1, 63 .. 65 and 127 .. 129 rows, inner sizes from one k-step on
+and of unequal length, weights on what an expert reads; few and many rows an expert, tiles of 16 slots and of up to 128."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-# rows of every expert, inner sizes (multiples of 32), width; below and above 45 rows an expert
+# rows of every expert, inner sizes (multiples of 32), width; few and many rows an expert
 FEW = ([0, 1, 63, 64, 65, 0, 17, 30], [32, 64, 96, 128, 160, 192, 224, 704], 352)
 MANY = ([129, 128, 127, 1, 0, 65, 300], [32, 96, 160, 224, 288, 352, 736], 288)
 
@@ -86,7 +86,7 @@ def test_blocks_of_weight_rows(amd, copies, act):
     g, gated = torch.Generator(device=DEV).manual_seed(copies), act == 0
     counts, ff, width = [129, 128, 127, 1, 0, 65] * copies, [32, 96, 128, 160, 288, 384] * copies, 288
     experts, rows, top = len(counts), sum(counts), 1
-    # units of whole blocks, slots spread evenly: where the line lies
+    # units of whole blocks, slots spread evenly: far from the lines between half and whole ones
     units = experts * -(-rows // (128 * experts)) * -(-384 // (128 if gated else 256)) + -(-rows // 128) * -(-384 // (128 if gated else 256))
     assert (units > 384) == (copies > 1)
     rand = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
@@ -135,20 +135,15 @@ def test_blocks_of_weight_rows(amd, copies, act):
 
 @pytest.mark.parametrize("act,weigh", [("clamped", False), ("silu", True), ("relu_squared", True)])
 @pytest.mark.parametrize("width", [4096, 224, 64])
-def test_many_turns_a_workgroup(amd, width, act, weigh):
-    """Few slots an expert, and far more units than workgroups: a turn's first steps come in while the turn before ends, weights of the slots
-    in two buffers by turns, turns of 1 to 12 and of 128 k-steps one after the other, a shared expert of eleven times the others' size
-    (going up its turns come first; going down, workgroups without one take eleven of the others' ahead)."""
+def test_few_slots_an_expert_and_a_large_shared_one(amd, width, act, weigh):
+    """Single tiles of few slots, walks of 1 to 12 k-steps going down, and a shared expert of eleven times the others' size, whose
+    units come first: its walks have 128 k-steps and its tiles are several."""
     from light_vllm_amd.engine.moe import ACTIVATIONS, interleave_16
     g, gated, experts, limit = torch.Generator(device=DEV).manual_seed(width), act != "relu_squared", 40, 1.1
     counts = [0, 1, 64, 65, 17, 30, 2, 63, 16, 33] * 2 + [7, 20, 11, 9] * 5
     ff = ([384, 32, 64, 160, 192, 96, 256, 384, 128, 352] * 4)[:experts] + [4096]
     rows = sum(counts)
-    tiles = sum((n + 63) // 64 for n in counts)
-    assert len(counts) == experts and 64 < rows and 2 * rows < 45 * (experts + 1)  # the ring's range
-    blocks = [-(-n // (128 if gated else 256)) for n in ff]
-    assert sum(b * ((n + 63) // 64) for b, n in zip(blocks, counts + [rows])) > 450 or not gated
-    assert width < 4096 or 16 * tiles > 2 * 256
+    assert len(counts) == experts and max(counts) < 128 and 64 < rows
     rand = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
     of_row = torch.repeat_interleave(torch.arange(experts, device=DEV), torch.tensor(counts, device=DEV))
     of_row = of_row[torch.randperm(rows, generator=g, device=DEV)]

@@ -1,5 +1,5 @@
-"""Every unit of the grouped products has exactly one turn: csrc/moe_turns.h on the host, over grids of any size, with a last expert of
-none to many times the others' size, up to the most turns that a workgroup can look up."""
+"""Every unit of the grouped products has exactly one workgroup, and which products take half blocks of weight rows: csrc/moe_turns.h
+on the host, over grids of any size, with a last expert of none to many times the others' size."""
 import ctypes
 import os
 import random
@@ -12,23 +12,19 @@ SOURCE = r"""
 #include <vector>
 #include "moe_turns.h"
 using namespace lvllm;
-// units without a turn of `lookups`, and with several; cus: workgroups of an XCD
-extern "C" void walk(int units_first, int units_last, int solo, int cus, int lookups, int* missing, int* twice) {
+// units without a workgroup, and with several; cus: workgroups of an XCD
+extern "C" void walk(int units_first, int units_last, int cus, int* missing, int* twice) {
   std::vector<int> first(units_first), last(units_last);
   for (int xcd = 0; xcd < 8; ++xcd)
-    for (int cu = 0; cu < cus; ++cu)
-      for (int turn = 0; turn < lookups; ++turn) {
-        const TurnUnit u = turn_unit(units_first, units_last, solo, xcd, cu, cus, turn);
-        if (u.any) ++(u.last ? last : first).at(u.unit);
-      }
+    for (int cu = 0; cu < cus; ++cu) {
+      const TurnUnit u = turn_unit(units_first, units_last, xcd, cu);
+      if (u.any) ++(u.last ? last : first).at(u.unit);
+    }
   *missing = *twice = 0;
   for (auto* v : {&first, &last})
     for (int n : *v) { *missing += n == 0; *twice += n > 1; }
 }
-extern "C" int solo(int up, int ff_first, int ff_last) { return solo_units(up, ff_first, ff_last); }
-extern "C" long ring(long units_first, long units_last, int solo) { return ring_workgroups(units_first, units_last, solo); }
 extern "C" long single(long units_first, long units_last) { return unit_workgroups(units_first, units_last); }
-extern "C" int turns() { return kTurns; }
 extern "C" int half(int rows, long slots, int experts, int first4, int last4, int first2, int last2, int up, int larger) {
   return takes_half_blocks(rows, slots, experts, 128, {first4, last4}, {first2, last2}, up, larger);
 }
@@ -42,53 +38,27 @@ def lib(tmp_path_factory):
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-D__host__=", "-D__device__=", "-I", CSRC, str(d / "t.cpp"), "-o",
                     str(d / "t.so")], check=True)
     t = ctypes.CDLL(str(d / "t.so"))
-    t.ring.restype = t.single.restype = ctypes.c_long
+    t.single.restype = ctypes.c_long
     t.half.argtypes = [ctypes.c_int, ctypes.c_long] + [ctypes.c_int] * 7
-    t.ring.argtypes, t.single.argtypes = [ctypes.c_long, ctypes.c_long, ctypes.c_int], [ctypes.c_long] * 2
+    t.single.argtypes = [ctypes.c_long] * 2
     return t
 
 
-def walk(lib, first, last, solo, workgroups, lookups):
+def walk(lib, first, last, workgroups):
     missing, twice = ctypes.c_int(), ctypes.c_int()
     assert workgroups % 8 == 0 and workgroups > 0
-    lib.walk(first, last, solo, workgroups // 8, lookups, ctypes.byref(missing), ctypes.byref(twice))
+    lib.walk(first, last, workgroups // 8, ctypes.byref(missing), ctypes.byref(twice))
     return missing.value, twice.value
 
 
-# width, experts but the last, their inner size, the last one's, taken by a row, rows: going down, a tile of 64 slots for each expert
-# of the first kind at least
-DOWN = [(2048, 384, 256, 14336, 8, 1921), (7168, 512, 512, 8192, 8, 321), (7168, 512, 1024, 14336, 8, 321), (4096, 1000, 64, 512, 1, 1000),
-        (7168, 384, 128, 3456, 8, 500), (7168, 256, 64, 2752, 8, 500), (2048, 32, 1408, 2816, 2, 300), (2048, 64, 32, 1 << 20, 6, 700)]
-
-
-@pytest.mark.parametrize("width,experts,ff,last_ff,top,rows", DOWN)
-def test_ring_going_down(lib, width, experts, ff, last_ff, top, rows):
-    blocks = (width // 16 + 15) // 16
-    solo, tiles, last = lib.solo(0, ff, last_ff), rows * (top + 1) // 64 + experts + 1, (rows + 63) // 64
-    grid = lib.ring(tiles * blocks, last * blocks, solo)
-    for n in {experts, tiles - last, min(tiles, experts + rows * top // 64)}:
-        assert walk(lib, n * blocks, last * blocks, solo, grid, lib.turns()) == (0, 0), n
-
-
-def test_any_ring(lib):
+def test_a_unit_a_workgroup(lib):
     """Units up to what the launch was sized for."""
-    r = random.Random(1)
-    size = lambda: int(2 ** r.uniform(0, 14))
-    for _ in range(400):
-        most_first, most_last, solo = size(), size() - 1, lib.solo(0, 32, 32 * int(2 ** r.uniform(0, 8)))
-        grid = lib.ring(most_first, most_last, solo)
-        assert grid >= 256 or grid == lib.single(most_first, most_last)
+    r = random.Random(2)
+    for _ in range(600):
+        most_first, most_last = int(2 ** r.uniform(0, 14)), int(2 ** r.uniform(0, 12)) - 1
         fewer = r.randint(0, most_last)
         for first, last in ((most_first, most_last), (r.randint(0, most_first), fewer), (most_first, fewer)):
-            assert walk(lib, first, last, solo, grid, lib.turns()) == (0, 0), (first, last, solo, grid)
-
-
-def test_a_unit_a_workgroup(lib):
-    r = random.Random(2)
-    for _ in range(200):
-        most_first, most_last = r.randint(1, 3000), r.randint(0, 1000)
-        first, last = r.randint(0, most_first), r.randint(0, most_last)
-        assert walk(lib, first, last, r.randint(1, 16), lib.single(most_first, most_last), 1) == (0, 0), (first, last)
+            assert walk(lib, first, last, lib.single(most_first, most_last)) == (0, 0), (first, last)
 
 
 # rows, experts taken by a row, experts, their inner size, the shared one's (0: none), width; whether half blocks were ahead, going up (None:
