@@ -32,7 +32,8 @@ OBJDIR = os.path.join(ROOT, "build", "obj")
 ARCH = "gfx950"
 
 SOURCES = {
-    "base": ["capi.hip", "cache.hip", "skinny_gemm.hip", "prepare_inputs.hip", "sampler.hip", "activation.hip"],
+    "base": ["capi.hip", "cache.hip", "skinny_gemm.hip", "prepare_inputs.hip", "sampler.hip", "activation.hip",
+             "wide_linear.hip", "tile_linear.hip"],
     "heads": ["head_attention.hip", "head_attention_prefill.hip", "head_attention_decode.hip", "head_attention_maps.hip",
               "head_cache.hip"],
     "moe": ["moe.hip", "moe_mfma.hip"],

@@ -251,6 +251,34 @@ torch::Tensor skinny_linear_packed_relu_squared(const torch::Tensor& x, const to
   return y;
 }
 
+// act(x w^T + bias) of a prompt in one launch; nothing where the library's product and a launch of the activation are faster, or the
+// operands are none that the kernels take
+std::optional<torch::Tensor> prompt_linear(const torch::Tensor& x, const std::optional<torch::Tensor>& w,
+                                           const std::optional<torch::Tensor>& w_packed, const std::optional<torch::Tensor>& bias,
+                                           int64_t outputs, int64_t act) {
+  const char* op = "prompt_linear";
+  LV_CHECK_DEVICE(x);
+  TORCH_CHECK(x.dim() == 2, op, ": x must be [rows, k]");
+  const int64_t rows = x.size(0), k = x.size(1), n = outputs * (act == LVLLM_ACT_SILU_AND_MUL ? 2 : 1);
+  auto aligned = [](const torch::Tensor& t) { return ((uintptr_t)t.data_ptr() & 15) == 0; };
+  auto takes = [&](const std::optional<torch::Tensor>& t, int64_t numel) {
+    if (!t) return false;
+    TORCH_CHECK(t->numel() == numel && t->device() == x.device(), op, ": weights [n, k] and a bias [n] on x's device");
+    return t->is_contiguous() && t->scalar_type() == x.scalar_type() && aligned(*t);
+  };
+  const bool row_major = takes(w, n * k), packed = takes(w_packed, n * k), biased = takes(bias, n);
+  if (x.scalar_type() != at::kBFloat16 || !x.is_contiguous() || !aligned(x) || bias.has_value() != (act == LVLLM_ACT_GELU) ||
+      bias.has_value() != biased || rows >= (1 << 24) || outputs >= (1 << 24) || k >= (1 << 24) ||
+      lvllm_prompt_linear_body((int)rows, (int)outputs, (int)k, (int)act, row_major, packed) == LVLLM_PROMPT_NONE)
+    return std::nullopt;
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(x));
+  auto out = torch::empty({rows, outputs}, x.options());
+  check(lvllm_prompt_linear(out.data_ptr(), x.data_ptr(), row_major ? w->data_ptr() : nullptr, packed ? w_packed->data_ptr() : nullptr,
+                            biased ? bias->data_ptr() : nullptr, (int)rows, (int)outputs, (int)k, (int)act, dtype_code(x, op),
+                            current_stream(x)));
+  return out;
+}
+
 // The clamped unit of a feed-forward's gate and up projection, [gate rows | up rows], in one launch: clamped_unit of the plain
 // projection
 torch::Tensor skinny_linear_packed_clamped_unit(const torch::Tensor& x, const torch::Tensor& w_packed, int64_t N, int64_t K,
@@ -687,6 +715,8 @@ TORCH_LIBRARY_FRAGMENT(_C_amd, amd) {
   amd.impl("skinny_linear_packed_clamped_unit", torch::kCUDA, &skinny_linear_packed_clamped_unit);
   amd.def("clamped_unit(Tensor x, float limit) -> Tensor");
   amd.impl("clamped_unit", torch::kCUDA, &clamped_unit);
+  amd.def("prompt_linear(Tensor x, Tensor? w, Tensor? w_packed, Tensor? bias, int outputs, int act) -> Tensor?");
+  amd.impl("prompt_linear", torch::kCUDA, &prompt_linear);
   amd.def("silu_unit(Tensor x) -> Tensor");
   amd.impl("silu_unit", torch::kCUDA, &silu_unit);
   amd.def("skinny_linear_packed_relu_squared(Tensor x, Tensor w_packed, int N, int K) -> Tensor");

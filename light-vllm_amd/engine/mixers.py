@@ -11,7 +11,7 @@ import torch
 import torch.nn.functional as F
 
 from .hybrid_config import KVSpec, LinearHeadsConfig, ParallelMixerConfig, SoftmaxHeadsConfig, TimeMixerConfig
-from .model import Weight, linear
+from .model import Weight, linear, linear_act
 
 amd = torch.ops._C_amd
 DECAY_LOGSIGMOID, DECAY_NEGEXP = 0, 1
@@ -227,7 +227,8 @@ class SiluMlp:
         if 0 < h.shape[0] <= DECODE_ROWS and self.up.packed is not None:
             a = amd.skinny_linear_packed_swiglu(h, self.up.packed, None, self.up.N, self.up.K)
         else:
-            a = amd.silu_unit(linear(h, self.up))
+            a = linear_act(h, self.up, "silu_and_mul", self.up.N // 2)
+            a = amd.silu_unit(linear(h, self.up)) if a is None else a
         return project_to_residual(a, self.down)
 
 
@@ -243,6 +244,8 @@ class SquaredReluMlp:
         if 0 < h.shape[0] <= DECODE_ROWS and self.up.packed is not None:
             a = amd.skinny_linear_packed_relu_squared(h, self.up.packed, self.up.N, self.up.K)
         else:
-            a = linear(h, self.up)
-            amd.relu_squared(a, a)
+            a = linear_act(h, self.up, "relu_squared", self.up.N)
+            if a is None:
+                a = linear(h, self.up)
+                amd.relu_squared(a, a)
         return project_to_residual(a, self.down)

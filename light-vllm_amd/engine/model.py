@@ -72,6 +72,16 @@ def linear(x: torch.Tensor, w: "Weight", bias: Optional[torch.Tensor] = None) ->
     return F.linear(x, w.w, bias)
 
 
+PROMPT_ACTS = {"gelu": 1, "silu_and_mul": 2, "relu_squared": 3}  # include/lvllm_hip.h LVLLM_ACT_*
+
+
+def linear_act(x: torch.Tensor, w: "Weight", act: str, outputs: int) -> Optional[torch.Tensor]:
+    """A prompt's projection with its activation in one launch; None where two are faster (csrc/prompt_linear.h)."""
+    if not x.is_cuda or _CALIBRATING or w.w is None:
+        return None
+    return torch.ops._C_amd.prompt_linear(x, w.w, w.packed, None, outputs, PROMPT_ACTS[act])
+
+
 _CALIBRATING = False
 _STREAM_GEMM_MAX_ROWS = 256  # set from ModelConfig.stream_gemm_max_rows by DecoderModel
 
@@ -323,6 +333,8 @@ class DecoderModel:
                 act = torch.ops._C_amd.skinny_linear_packed_swiglu(hidden, lw.gate_up.packed, None,
                                                                    lw.gate_up.N, lw.gate_up.K)
             else:
+                act = linear_act(hidden, lw.gate_up, "silu_and_mul", cfg.intermediate_size)
+            if act is None:
                 gate_up = linear(hidden, lw.gate_up)
                 act = torch.empty(T, cfg.intermediate_size, dtype=gate_up.dtype, device=gate_up.device)
                 ops.silu_and_mul(act, gate_up)

@@ -5,7 +5,8 @@ attention -> output projection -> add & LayerNorm -> GELU MLP -> add & LayerNorm
 
 Attention is this package's HIP varlen kernel (AttentionType.ENCODER); the residual add and the LayerNorm
 behind it are one launch (`_C_amd.add_layer_norm`; the reference leaves both to torch),
-exact GELU is an in-place kernel of this package too; the projections are library GEMMs (prompt batches are hundreds to thousands of rows).
+exact GELU leaves the projection in front of it (csrc/tile_linear.hip) or is an in-place kernel of this package; the other projections
+are library GEMMs (prompt batches are hundreds to thousands of rows).
 Weights are random-initialised: no checkpoint is available offline."""
 from dataclasses import dataclass
 from typing import List
@@ -14,7 +15,7 @@ import torch
 import torch.nn.functional as F
 
 from ..attention.prefill_only import AttentionType, PrefillOnlyHIPVarlenBackend
-
+from ..engine.model import PROMPT_ACTS
 
 
 @dataclass
@@ -63,6 +64,9 @@ class EncoderLayerWeights:
         self.out_w, self.out_b = w(hid, hid), w(hid)
         self.attn_ln = ln()
         self.fc1_w, self.fc1_b = w(inter, hid), w(inter)
+        # once more in fragment order, for the kernel with GELU behind the product
+        pack = self.fc1_w.is_cuda and cfg.dtype == torch.bfloat16 and inter % 16 == 0 and hid % 32 == 0
+        self.fc1_packed = torch.ops._C_amd.pack_weight(self.fc1_w) if pack else None
         self.fc2_w, self.fc2_b = w(hid, inter), w(hid)
         self.out_ln = ln()
 
@@ -103,6 +107,17 @@ class EncoderModel:
                 return out
             return F.layer_norm(a if b is None else a + b, (hid,), ln[0], ln[1], eps)
 
+        def fc1_gelu(a, lw):
+            if fused and lw.fc1_packed is not None:
+                h = torch.ops._C_amd.prompt_linear(a, None, lw.fc1_packed, lw.fc1_b, cfg.intermediate_size, PROMPT_ACTS["gelu"])
+                if h is not None:
+                    return h
+            h = F.linear(a, lw.fc1_w, lw.fc1_b)
+            if fused and h.numel() % 8 == 0:
+                torch.ops._C_amd.gelu(h, h)  # exact GELU in place
+                return h
+            return F.gelu(h)
+
         x = add_ln(x, None, self.emb_ln)
         for lw in self.layers:
             qkv = F.linear(x, lw.qkv_w, lw.qkv_b)
@@ -113,18 +128,9 @@ class EncoderModel:
             if blk > 0 and x.shape[0] > blk:
                 y = torch.empty_like(x)
                 for r0 in range(0, x.shape[0], blk):
-                    hb = F.linear(x[r0:r0 + blk], lw.fc1_w, lw.fc1_b)
-                    if fused and hb.numel() % 8 == 0:
-                        torch.ops._C_amd.gelu(hb, hb)
-                    else:
-                        hb = F.gelu(hb)
+                    hb = fc1_gelu(x[r0:r0 + blk], lw)
                     torch.addmm(lw.fc2_b, hb, lw.fc2_w.t(), out=y[r0:r0 + blk])
             else:
-                h = F.linear(x, lw.fc1_w, lw.fc1_b)
-                if fused and h.numel() % 8 == 0:
-                    torch.ops._C_amd.gelu(h, h)  # exact GELU in place
-                else:
-                    h = F.gelu(h)
-                y = F.linear(h, lw.fc2_w, lw.fc2_b)
+                y = F.linear(fc1_gelu(x, lw), lw.fc2_w, lw.fc2_b)
             x = add_ln(x, y, lw.out_ln)
         return x

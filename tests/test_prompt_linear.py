@@ -1,0 +1,62 @@
+"""Which kernel takes a prompt's projection with an activation behind it (csrc/prompt_linear.h), on the host: at sizes that were measured,
+and what no size may lead to."""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "light-vllm_amd", "csrc")
+SOURCE = r"""
+#include "prompt_linear.h"
+extern "C" int plan(int rows, int outputs, int k, int act, int row_major, int packed, int* groups, int* nt) {
+  const lvllm::PromptLinearPlan p = lvllm::prompt_linear_plan(rows, outputs, k, act, row_major, packed);
+  *groups = p.groups;
+  *nt = p.nt;
+  return p.body;
+}
+"""
+GELU, SILU, RELU2 = 1, 2, 3
+NONE, WIDE, TILE = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    (d / "t.cpp").write_text(SOURCE)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, str(d / "t.cpp"), "-o", str(d / "t.so")], check=True)
+    lib = ctypes.CDLL(str(d / "t.so"))
+
+    def f(rows, outputs, k, act, row_major=True, packed=True):
+        g, n = ctypes.c_int(), ctypes.c_int()
+        body = lib.plan(rows, outputs, k, act, row_major, packed, ctypes.byref(g), ctypes.byref(n))
+        return body, g.value if body == WIDE else n.value
+    return f
+
+
+MEASURED = [  # rows, outputs, k, activation -> body, groups or blocks
+    (4875, 14336, 4096, SILU, WIDE, 4), (3000, 14336, 4096, SILU, WIDE, 3), (1000, 14336, 4096, SILU, NONE, 0), (700, 14336, 4096, SILU, WIDE, 3),
+    (300, 14336, 4096, SILU, WIDE, 3), (100, 14336, 4096, SILU, NONE, 0), (8192, 11264, 2048, SILU, WIDE, 4), (300, 5632, 2048, SILU, NONE, 0),
+    (4096, 8448, 2048, RELU2, WIDE, 3), (1000, 8448, 2048, RELU2, WIDE, 3), (700, 8448, 2048, RELU2, TILE, 4), (300, 8448, 2048, RELU2, TILE, 2),
+    (100, 8448, 2048, RELU2, NONE, 0), (16384, 4096, 1024, GELU, TILE, 4), (2000, 4096, 1024, GELU, TILE, 2), (100, 4096, 1024, GELU, NONE, 0)]
+
+
+@pytest.mark.parametrize("rows,outputs,k,act,body,size", MEASURED)
+def test_measured_sizes(plan, rows, outputs, k, act, body, size):
+    got = plan(rows, outputs, k, act)
+    assert got[0] == body and (body == NONE or got[1] == size)
+
+
+def test_any_size(plan):
+    rng = random.Random(0)
+    for _ in range(20000):
+        rows, outputs, k = rng.randint(1, 40000), rng.choice([8, 16]) * rng.randint(1, 2000), rng.choice([8, 32, 64]) * rng.randint(1, 128)
+        act, row_major, packed = rng.choice([GELU, SILU, RELU2]), rng.random() < 0.5, rng.random() < 0.5
+        body, size = plan(rows, outputs, k, act, row_major, packed)
+        if body == WIDE:
+            assert row_major and act != GELU and k % 64 == 0 and outputs % 16 == 0 and 2 <= size <= 4
+        elif body == TILE:
+            assert packed and act != SILU and k % 32 == 0 and outputs % 16 == 0 and size in (2, 4)
+        if body != NONE:
+            assert rows > 64 and outputs * k * (2 if act == SILU else 1) * 2 < 2 ** 31

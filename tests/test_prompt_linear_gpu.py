@@ -1,0 +1,99 @@
+"""Projections of prompts with an activation in the same launch: tiles with remainders of rows and outputs, every number of 64-row groups,
+the smallest k, and which sizes the kernels take."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+GELU, SILU, RELU2 = 1, 2, 3
+
+
+@pytest.fixture(scope="module")
+def amd():
+    import light_vllm_amd._custom_ops  # noqa: F401
+    return torch.ops._C_amd
+
+
+# rows, outputs, k: whole tiles and one row more, remainders of 1 to 4 groups of 64 rows, outputs that end inside a block and inside a
+# wave's part of one, odd numbers of stages, one tile a workgroup and several
+WIDE = [(769, 8464, 512), (1100, 5904, 576), (1500, 4096, 512), (3000, 2832, 640), (2113, 8192, 1088), (600, 16400, 512)]
+TILE = [(300, 4096, 64), (1000, 4112, 96), (129, 6160, 1024), (2500, 4096, 160), (4097, 784, 32), (513, 4224, 2048)]
+
+
+def check(amd, rows, outputs, k, act, row_major, pack):
+    gen = torch.Generator().manual_seed(rows + outputs + k)
+    n = outputs * (2 if act == SILU else 1)
+    x = torch.randn(rows, k, generator=gen).bfloat16().to(DEV)
+    w = (torch.randn(n, k, generator=gen) * 2 * k ** -0.5).bfloat16().to(DEV)
+    bias = (0.2 * torch.randn(n, generator=gen)).bfloat16().to(DEV) if act == GELU else None
+    got = amd.prompt_linear(x, w if row_major else None, amd.pack_weight(w) if pack else None, bias, outputs, act)
+    assert got is not None and got.shape == (rows, outputs)
+    z = x.double() @ w.double().T
+    # sums of up to 2048 products of values around 1 in fp32, rounded to 8 bits behind the product (not GELU) and behind the activation,
+    # SwiGLU once more between
+    sums, eps = 1e-5, 2.0 ** -8
+    if act == GELU:
+        z = z + bias.double()
+        want, slack = F.gelu(z), eps * F.gelu(z).abs() + 1.13 * sums
+    elif act == SILU:
+        g, u = z[:, :outputs], z[:, outputs:]
+        want = F.silu(g) * u
+        slack = eps * (2 * want.abs() + 1.1 * g.abs() * u.abs() + F.silu(g).abs() * u.abs()) + 4 * sums * (1 + g.abs() + u.abs())
+    else:
+        want = z.clamp(min=0).square()
+        slack = eps * 3.1 * want + 2 * sums * (z.abs() + 1)
+    assert ((got.double() - want).abs() <= slack).all(), ((got.double() - want).abs() - slack).max()
+
+
+@pytest.mark.parametrize("act", [SILU, RELU2])
+@pytest.mark.parametrize("rows,outputs,k", WIDE)
+def test_wide_tiles(amd, rows, outputs, k, act):
+    check(amd, rows, outputs, k, act, True, False)
+
+
+@pytest.mark.parametrize("rows,outputs,k", TILE)
+def test_tiles(amd, rows, outputs, k):
+    check(amd, rows, outputs, k, GELU, False, True)
+
+
+@pytest.mark.parametrize("rows,outputs,k", [(200, 8448, 96), (129, 12304, 1024), (640, 8464, 160)])
+def test_tiles_of_squared_relu(amd, rows, outputs, k):
+    check(amd, rows, outputs, k, RELU2, False, True)
+
+
+def test_activations_of_the_largest_and_smallest_values(amd):
+    """GELU and SwiGLU of products from far below to far above their bends, infinities and NaN included."""
+    rows, outputs, k = 2048, 4096, 512
+    v = torch.cat([torch.linspace(-120, 120, rows - 8), torch.tensor([3e38, -3e38, float("inf"), float("nan"), 1e-30, -1e-30, 0., 88.])])
+    x = torch.zeros(rows, k, dtype=torch.bfloat16)
+    x[:, 0] = v.bfloat16()
+    w = torch.zeros(2 * outputs, k, dtype=torch.bfloat16)
+    w[:, 0] = 1
+    x, w = x.to(DEV), w.to(DEV)
+    z = x[:, :1].double()
+    gelu = amd.prompt_linear(x, None, amd.pack_weight(w[:outputs].contiguous()), torch.zeros(outputs, dtype=torch.bfloat16, device=DEV), outputs,
+                             GELU)
+    silu = amd.prompt_linear(x, w, None, None, outputs, SILU)
+    for got, want, floor in (gelu, F.gelu(z), 1e-6), (silu, F.silu(z) * z, 1e-30):
+        got, want = got.double(), want.expand(rows, outputs)
+        nan, big = want.isnan(), want.abs() > 3.3e38
+        assert (got.isnan() == nan).all() and (got[big] == got[big].sign() * float("inf")).all()
+        keep = ~nan & ~big
+        # (SwiGLU: two roundings; GELU's polynomial: 6.7e-8)
+        assert ((got - want)[keep].abs() <= 2.1 * 2.0 ** -8 * want[keep].abs() + floor).all()
+
+
+def test_what_is_refused(amd):
+    x = torch.randn(2048, 512, device=DEV).bfloat16()
+    w = torch.randn(8192, 512, device=DEV).bfloat16()
+    assert amd.prompt_linear(x, w, None, None, 4096, SILU) is not None
+    assert amd.prompt_linear(x[:64].contiguous(), w, None, None, 4096, SILU) is None
+    assert amd.prompt_linear(x[:, ::2], w[:, ::2].contiguous(), None, None, 4096, SILU) is None   # rows that are not back to back
+    assert amd.prompt_linear(x.half(), w.half(), None, None, 4096, SILU) is None
+    assert amd.prompt_linear(x, None, None, None, 4096, SILU) is None
+    assert amd.prompt_linear(x, None, amd.pack_weight(w), None, 8192, GELU) is None   # no bias
+    flat = torch.randn(2048 * 512 + 1, device=DEV).bfloat16()
+    assert amd.prompt_linear(flat[1:].view(2048, 512), w, None, None, 4096, SILU) is None   # not aligned
+    with pytest.raises(RuntimeError):
+        amd.prompt_linear(x, w, None, None, 8192, SILU)
