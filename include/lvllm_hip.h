@@ -281,6 +281,11 @@ int lvllm_skinny_gemm_ex(void* y, const void* x, const void* w, const void* bias
  * LayerNorm).  16-bit element types, hidden_size % 8 == 0, contiguous rows, out may alias x. */
 int lvllm_add_layer_norm(void* out, const void* x, const void* y, const void* weight, const void* bias,
                          float epsilon, int num_tokens, int hidden_size, int dtype, void* stream);
+/* LayerNorm(T(T(word[ids] + pos[positions + shift]) + type)) of an encoder's embeddings: word [words, hidden], pos [places, hidden], type
+ * [hidden].  16-bit element types, hidden_size a multiple of 8 up to 2048; rows of an id or position outside its table become NaN. */
+int lvllm_embed_layer_norm(void* out, const int64_t* ids, const int64_t* positions, int64_t shift, const void* word, const void* pos,
+                           const void* type, const void* weight, const void* bias, float epsilon, int num_tokens, int hidden_size,
+                           int64_t words, int64_t places, int dtype, void* stream);
 /* fused_add_rms_norm whose input is the fp32 split-K partials of the preceding projection:
  * x = T(sum_s partials[s]); residual = T(x + residual); out = norm(residual) * weight. */
 int lvllm_fused_add_rms_norm_splitk(void* out, void* residual, const float* partials,

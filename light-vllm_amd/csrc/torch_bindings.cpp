@@ -144,6 +144,28 @@ void add_layer_norm(torch::Tensor& out, const torch::Tensor& x, const std::optio
                              dtype_code(x, "add_layer_norm"), current_stream(x)));
 }
 
+torch::Tensor embed_layer_norm(const torch::Tensor& ids, const torch::Tensor& positions, int64_t shift, const torch::Tensor& word,
+                               const torch::Tensor& pos, const torch::Tensor& type, const torch::Tensor& weight, const torch::Tensor& bias,
+                               double epsilon) {
+  const char* op = "embed_layer_norm";
+  LV_CHECK_DEVICE(ids);
+  TORCH_CHECK(ids.dim() == 1 && positions.sizes() == ids.sizes() && ids.is_contiguous() && positions.is_contiguous() &&
+                  ids.scalar_type() == at::kLong && positions.scalar_type() == at::kLong && positions.device() == ids.device(),
+              op, ": int64 ids and positions of the same rows");
+  TORCH_CHECK(word.dim() == 2 && pos.dim() == 2 && word.size(1) == pos.size(1), op, ": tables of one width");
+  const int64_t hidden = word.size(1);
+  for (const auto* t : {&word, &pos, &type, &weight, &bias})
+    TORCH_CHECK(t->device() == ids.device() && t->is_contiguous() && t->scalar_type() == word.scalar_type(), op,
+                ": contiguous tables, weight and bias of one type");
+  TORCH_CHECK(type.numel() == hidden && weight.numel() == hidden && bias.numel() == hidden, op, ": type, weight and bias of [hidden]");
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(ids));
+  auto out = torch::empty({ids.size(0), hidden}, word.options());
+  check(lvllm_embed_layer_norm(out.data_ptr(), ids.data_ptr<int64_t>(), positions.data_ptr<int64_t>(), shift, word.data_ptr(),
+                               pos.data_ptr(), type.data_ptr(), weight.data_ptr(), bias.data_ptr(), (float)epsilon, (int)ids.size(0),
+                               (int)hidden, word.size(0), pos.size(0), dtype_code(word, op), current_stream(ids)));
+  return out;
+}
+
 void fused_add_rms_norm_splitk_scaled(torch::Tensor& out, torch::Tensor& residual, const torch::Tensor& partials,
                                       const torch::Tensor& weight, double epsilon,
                                       const c10::optional<torch::Tensor>& x_scale,
@@ -557,6 +579,9 @@ TORCH_LIBRARY_FRAGMENT(_C_amd, amd) {
   amd.impl("gelu", torch::kCUDA, &gelu);
   amd.def("add_layer_norm(Tensor! out, Tensor x, Tensor? y, Tensor weight, Tensor bias, float epsilon) -> ()");
   amd.impl("add_layer_norm", torch::kCUDA, &add_layer_norm);
+  amd.def("embed_layer_norm(Tensor ids, Tensor positions, int shift, Tensor word, Tensor pos, Tensor type, Tensor weight, Tensor bias, "
+          "float epsilon) -> Tensor");
+  amd.impl("embed_layer_norm", torch::kCUDA, &embed_layer_norm);
   amd.def("fused_add_rms_norm_splitk(Tensor! out, Tensor! residual, Tensor partials, Tensor weight, "
           "float epsilon) -> ()");
   amd.impl("fused_add_rms_norm_splitk", torch::kCUDA, &fused_add_rms_norm_splitk);

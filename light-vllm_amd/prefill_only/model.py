@@ -95,10 +95,8 @@ class EncoderModel:
         cfg = self.cfg
         eps = cfg.layer_norm_eps
         hid = cfg.hidden_size
-        # xlm_roberta.py: position ids start after the padding index
-        x = (F.embedding(input_ids, self.word_emb) + F.embedding(positions + cfg.pad_token_id + 1, self.pos_emb)
-             + self.type_emb[0])
-        fused = x.is_cuda and hid % 8 == 0 and x.dtype in (torch.bfloat16, torch.float16) and self.cfg.fused_layer_norm
+        emb, shift = self.word_emb, cfg.pad_token_id + 1  # xlm_roberta.py: position ids start after the padding index
+        fused = emb.is_cuda and hid % 8 == 0 and emb.dtype in (torch.bfloat16, torch.float16) and self.cfg.fused_layer_norm
 
         def add_ln(a, b, ln):  # LayerNorm(a + b), b optional
             if fused:
@@ -118,7 +116,12 @@ class EncoderModel:
                 return h
             return F.gelu(h)
 
-        x = add_ln(x, None, self.emb_ln)
+        if fused and hid <= 2048 and input_ids.dtype == positions.dtype == torch.int64:  # (one launch: csrc/layernorm.hip)
+            x = torch.ops._C_amd.embed_layer_norm(input_ids.contiguous(), positions.contiguous(), shift, self.word_emb, self.pos_emb,
+                                                  self.type_emb, *self.emb_ln, eps)
+        else:
+            x = F.embedding(input_ids, self.word_emb) + F.embedding(positions + shift, self.pos_emb) + self.type_emb[0]
+            x = add_ln(x, None, self.emb_ln)
         for lw in self.layers:
             qkv = F.linear(x, lw.qkv_w, lw.qkv_b)
             q, k, v = qkv.split([hid, hid, hid], dim=-1)  # strided views of the fused projection

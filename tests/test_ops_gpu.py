@@ -599,6 +599,25 @@ def test_add_layer_norm_matches_torch(ops, dtype, T, hidden, with_y):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,hidden", [(1, 8), (5, 128), (33, 1000), (4, 1024), (3, 2048)])
+def test_embed_layer_norm(ops, dtype, T, hidden):
+    """The norm of an encoder's summed embeddings: the bits of the sums, then of the norm by itself; a row outside the tables is NaN."""
+    g = torch.Generator(device=DEV).manual_seed(T + hidden)
+    word, pos, typ = ((torch.randn(n, hidden, generator=g, device=DEV)).to(dtype) for n in (50, 40, 1))
+    w, b = (1 + 0.1 * torch.randn(hidden, generator=g, device=DEV)).to(dtype), (0.1 * torch.randn(hidden, generator=g, device=DEV)).to(dtype)
+    ids, at = torch.randint(0, 50, (T,), generator=g, device=DEV), torch.randint(0, 38, (T,), generator=g, device=DEV)
+    ids[0], at[0] = 49, 37
+    got = torch.ops._C_amd.embed_layer_norm(ids, at, 2, word, pos, typ, w, b, 1e-5)
+    z, want = word[ids] + pos[at + 2] + typ[0], torch.empty_like(got)
+    torch.ops._C_amd.add_layer_norm(want, z, None, w, b, 1e-5)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    for bad_id, bad_at in ((50, 0), (-1, 0), (0, 38), (0, -3)):
+        ids[0], at[0] = bad_id, bad_at
+        got2 = torch.ops._C_amd.embed_layer_norm(ids, at, 2, word, pos, typ, w, b, 1e-5)
+        assert got2[0].isnan().all() and torch.equal(got2[1:].view(torch.int16), got[1:].view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gelu_matches_torch(ops, dtype):
     g = torch.Generator(device=DEV).manual_seed(1)
     x = (torch.randn(37, 4096, generator=g, device=DEV) * 3).to(dtype)
