@@ -692,15 +692,15 @@ int lvllm_latent_rotate_query(void* out, const void* q, int64_t q_stride, int he
                               const int64_t* positions, const double* turns, int rot_dims, float grow, int rows, int dtype,
                               void* stream);
 /* ---- projections of prompts with an activation behind them (csrc/wide_linear.hip, tile_linear.hip) ---- */
-enum { LVLLM_ACT_GELU = 1, LVLLM_ACT_SILU_AND_MUL = 2, LVLLM_ACT_RELU_SQUARED = 3 };
+enum { LVLLM_ACT_GELU = 1, LVLLM_ACT_SILU_AND_MUL = 2, LVLLM_ACT_RELU_SQUARED = 3, LVLLM_ACT_CLAMPED_UNIT = 4 };
 enum { LVLLM_PROMPT_NONE = 0, LVLLM_PROMPT_WIDE = 1, LVLLM_PROMPT_TILE = 2 };
 /* what takes out [rows, outputs] = act(x w^T + bias), with the weights row-major, packed (lvllm_pack_weight) or both: NONE where the
  * library's product and a launch of the activation are faster */
 int lvllm_prompt_linear_body(int rows, int outputs, int k, int act, int row_major, int packed);
-/* x [rows, k]; w [outputs, k] (SILU_AND_MUL: [2 outputs, k], gate rows first) row-major and packed, either may be null; bias [outputs]:
- * GELU only.  bf16.  SILU_AND_MUL and RELU_SQUARED round the product as the library's result is before they act. */
+/* x [rows, k]; w [outputs, k] (SILU_AND_MUL, CLAMPED_UNIT: [2 outputs, k], gate rows first) row-major and packed, either may be null;
+ * bias [outputs]: GELU only; limit: CLAMPED_UNIT only.  bf16.  All but GELU round the product as the library's result is before they act. */
 int lvllm_prompt_linear(void* out, const void* x, const void* w, const void* w_packed, const void* bias, int rows, int outputs, int k,
-                        int act, int dtype, void* stream);
+                        int act, float limit, int dtype, void* stream);
 /* ---- mixtures of experts (csrc/moe*.hip, moe.h) ---- */
 enum { LVLLM_MOE_SOFTMAX = 0, LVLLM_MOE_SIGMOID = 1 };  /* weights: softmax over the chosen logits, or each logit's sigmoid */
 enum { LVLLM_MOE_NO_SHARED = 0, LVLLM_MOE_GATED_SHARED = 1, LVLLM_MOE_PLAIN_SHARED = 2 };

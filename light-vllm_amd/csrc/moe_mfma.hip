@@ -173,7 +173,7 @@ __device__ __forceinline__ void tile_product(const MoeParams& p, const TileWork&
   constexpr bool UP = PRODUCT != kMoeDown, GATED = PRODUCT == kMoeGated;
   e_f32x4_t acc[NT][MT];
   tile_sums<ONCE>(acc, (const uint16_t*)p.x, UP ? p.width : p.ff_max, (const uint16_t*)p.w + p.w_offset[t.e], t, ring,
-                  [&](int slot) { return UP ? min(max(p.token[slot], 0), p.rows - 1) : slot; });
+                  [&](int slot) { return UP ? min(max(p.token[slot], 0), p.rows - 1) : slot; }, [](int tile) { return tile; });
   [[maybe_unused]] const MoeActivation act(p, GATED ? t.e : -1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   tile_store<GATED>((uint16_t*)p.out, UP ? p.ff_max : p.width, acc, ring[0] + wave * 2048, (t.block * 4 + wave) * NT, t.ntiles, t.s0,

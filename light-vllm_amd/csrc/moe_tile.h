@@ -1,5 +1,5 @@
 // Tiles of up to 128 rows x 64 NT W rows on 16x16x32 bf16 MFMAs over packed weights, two workgroups a CU: the grouped products of prompts
-// (moe_mfma.hip) and plain projections with GELU behind them (prompt_linear.hip).
+// (moe_mfma.hip) and projections with an activation behind them (tile_linear.hip).
 #pragma once
 #include "moe.h"
 
@@ -81,10 +81,10 @@ __device__ __forceinline__ void to_lds16(const char* from, void* dst) {
 // apart.  4 to 8 % of the cycles in which LDS is active are conflicts, those of the results' way out included.
 constexpr int kStageBytes = kMoeTile * 128;  // two k-steps of 32: a slot's 128 bytes, 8 slots a copy
 constexpr int tile_steps(int NT) { return NT == 4 ? 4 : 8; }  // k-steps of weights in registers; half as many stages of slots
-// row_of: where in x (of row length ld) a slot's row lies.  Ends with LDS free, for every wave.
-template <bool ONCE, int NT, int MT, class ROW>
+// row_of: where in x (of row length ld) a slot's row lies; tile_of: where in w a W tile lies.  Ends with LDS free, for every wave.
+template <bool ONCE, int NT, int MT, class ROW, class TILE>
 __device__ __forceinline__ void tile_sums(e_f32x4_t (&acc)[NT][MT], const uint16_t* x_rows, const int64_t ld, const uint16_t* w_tiles,
-                                          const TileWork& t, char (*ring)[kStageBytes], ROW row_of) {
+                                          const TileWork& t, char (*ring)[kStageBytes], ROW row_of, TILE tile_of) {
   constexpr int S = tile_steps(NT), X = S / 2, kCopies = MT / 2;  // (MT groups of 16 slots)
   constexpr int kYounger = (X - 2) * kCopies + (X - 1) * 2 * NT;  // loads behind a stage's copies when it is needed
   constexpr int kBehind = (X - 1) * kCopies + (S - 1) * NT;       // ... behind a second k-step's weights
@@ -97,7 +97,7 @@ __device__ __forceinline__ void tile_sums(e_f32x4_t (&acc)[NT][MT], const uint16
   const uint16_t *wsrc[NT], *xsrc[kCopies];
   const uint16_t* w = w_tiles + lane * 8;
 #pragma unroll
-  for (int j = 0; j < NT; ++j) wsrc[j] = w + (int64_t)min(nt0 + j, ntiles - 1) * steps * 512;
+  for (int j = 0; j < NT; ++j) wsrc[j] = w + (int64_t)tile_of(min(nt0 + j, ntiles - 1)) * steps * 512;
   const int chunk = (lane & 7) ^ (lane >> 3);
 #pragma unroll
   for (int j = 0; j < kCopies; ++j) {

@@ -6,66 +6,68 @@
 
 namespace lvllm {
 
+// Gated units: an output is made of a gate row and a value row.
+constexpr bool prompt_pairs(int act) { return act == LVLLM_ACT_SILU_AND_MUL || act == LVLLM_ACT_CLAMPED_UNIT; }
+
 // What takes a projection: the library and a launch of the activation (none of these), tiles of up to 64 groups rows x 256 W rows one a CU
-// over row-major weights (wide_linear.hip), or tiles of 128 rows x 64 nt outputs two a CU over packed weights (tile_linear.hip).
+// over row-major weights (wide_linear.hip), or tiles of 128 rows x 64 nt W rows two a CU over packed weights (tile_linear.hip).
 struct PromptLinearPlan {
   int body;    // LVLLM_PROMPT_*
   int groups;  // wide
   int nt;      // tile
 };
 
-// Wide tiles take turns of one a CU, 256 at a time; a turn of 64, 128, 192, 256 rows takes 40, 59, 78, 100 %.  `fill`: the share of the
-// turns' time that is work on rows and outputs that are there.  us, library and activation, then this:
-//   * SwiGLU of 14336, 4096 wide: 3000 rows (fill 94 %) 575, 524; 4875 964, 842; 8192 (100 %) 1397, 1323; 2000 (88 %) 380, 373; but 1000
-//     (85 %) 201, 207; 1500 (85 %) 285, 292.  Of 11264, 2048 wide, where the activation is twice as large a part: 1000 (76 %) 104, 95;
-//     4096 408, 308; 8192 632, 576; of 5632: 2000 (86 %) 95, 80; 8192 407, 301;
-//   * at a few hundred rows the library fills the chip no better: 14336, 4096 wide, 300 rows (66 %) 88, 78; 700 (77 %) 164, 135; 512 (88 %)
-//     109, 106; of 5632, 2048 wide, 512 (58 %) 38, 35; 300 (34 %) 33, 34;
-//   * squared ReLU of 8448, 2048 wide: 1000 (65 %) 43.6, 40.3; 2000 80, 73; 4096 138, 114; 8192 311, 223.
-inline PromptLinearPlan wide_plan(int rows, int outputs, int k, int act) {
-  static const int kTurn[5] = {0, 40, 59, 78, 100};
-  const int pairs = act == LVLLM_ACT_SILU_AND_MUL ? 2 : 1;
-  const int64_t blocks = ((int64_t)pairs * outputs + 255) / 256;
-  int64_t best = 0;
-  int groups = 0;
-  for (int g = 4; g >= 2; --g) {
-    const int64_t turns = (((rows + 64 * g - 1) / (64 * g)) * blocks + 255) / 256, time = turns * kTurn[g];
-    if (groups == 0 || time < best) best = time, groups = g;
-  }
-  const int64_t fill = (int64_t)rows * pairs * outputs * 100 / 256 / 256 * 100 / 256 / best;  // in per cent
-  const int64_t least = rows <= 768 ? 50 : k <= 2048 ? 60 : 87;
-  return {fill >= least ? LVLLM_PROMPT_WIDE : LVLLM_PROMPT_NONE, groups, 0};
+// Times in hundredths of a launch of at most one whole tile (nt = 4) a CU, 32 us at k = 2048, as measured (gated units of 5632 and
+// 11264, 2048 wide, 65 to 8192 rows):
+//   * whole tiles: a CU's second one beside the first 0.50 to 0.81 (0.65 to 0.81 from k = 3072 on); from the third on a round of both at 1.58
+//     (1.64), and 0.70 of ends;
+//   * half tiles (nt = 2): 0.71 alone, 0.85 to 1.19 two, then 1.05 a round and 0.45;
+//   * wide ones take turns, 256 tiles at a time, of 0.97, 1.28 and 1.64 with 2, 3 and 4 groups; of 0.88, 1.17, 1.50 from k = 3072 on, where
+//     their way in and out counts less.  Nothing covers their activations: 4 % more with SwiGLU, 10 % with the clamped unit, whose
+//     exponential and division are the mathematical library's.
+inline int64_t tile_time(int64_t units, int nt, int k) {
+  const int second = k < 3072 ? 150 : 165;
+  if (nt == 4) return units <= 256 ? 100 : units <= 512 ? second + (181 - second) * (units - 256) / 256 : (k < 3072 ? 158 : 164) * units / 512 + 70;
+  return units <= 256 ? 71 : units <= 512 ? 85 + 34 * (units - 256) / 256 : 105 * units / 512 + 45;
+}
+inline int64_t wide_time(int64_t units, int groups, int k, int act) {
+  static const int kTurn[2][5] = {{0, 0, 97, 128, 164}, {0, 0, 88, 117, 150}};
+  const int more = act == LVLLM_ACT_CLAMPED_UNIT ? 110 : act == LVLLM_ACT_SILU_AND_MUL ? 104 : 100;
+  return (units + 255) / 256 * kTurn[k >= 3072][groups] * more / 100;
 }
 
-// Tiles of 64 nt outputs: GELU, whose instructions then run beside another tile's MFMAs (a wide tile has nobody beside it), and squared ReLU
-// of few rows.  Half blocks (nt = 2) up to 512 of them, from 96 on; whole ones of squared ReLU while they fit a CU each.  us, library and
-// activation, then half and whole blocks: GELU of 4096, 1024 wide, 100 rows (32 half blocks) 11.7, 12.3, 18.6; 300 rows (96) 13.9,
-// 12.6, 18.9; 1000 (256) 20.8, 14.2, 20.3; 2000 (512) 29.8, 22.8, 23.0; 3000 37.3, 33.7, 31.8; 16384 154, 125 whole, 149 wide; squared ReLU
-// of 8448, 2048 wide, 100 rows (66) 19.4, 20.8, 29.8; 300 (198) 27.9, 21.4, 29.6; 700 (396; 198 whole) 37.7, 33.4, 31.1; 1000 (528; 264) 43.7, 50.4,
-// 47.4.
-inline PromptLinearPlan tile_plan(int rows, int outputs, int act) {
-  const int64_t tiles = (rows + 127) / 128, half = tiles * ((outputs + 127) / 128), whole = tiles * ((outputs + 255) / 256);
-  if (half < 96) return {LVLLM_PROMPT_NONE, 0, 0};
-  if (act == LVLLM_ACT_GELU) return {LVLLM_PROMPT_TILE, 0, half <= 512 ? 2 : 4};
-  if (half <= 264) return {LVLLM_PROMPT_TILE, 0, 2};
-  return {whole <= 256 ? LVLLM_PROMPT_TILE : LVLLM_PROMPT_NONE, 0, 4};
-}
-
-// `row_major`, `packed`: the orders of the weights that are there.
+// The shortest of these; `row_major`, `packed`: the orders of the weights that are there.  Nothing where the half tiles are too few to fill
+// half of the chip: the library cuts K then.  us, library and activation, then this:
+//   * SwiGLU of 14336, 4096 wide: 65 rows 58, 45; 300 88, 84; 700 163, 144; 1000 206, 195; 2000 382, 376; 3000 575, 515; 4875 990, 855; 8192 1398,
+//     1346; of 11264, 2048 wide: 128 rows 32, 27; 700 99, 77; 1000 106, 85; 2000 193, 164; 4096 402, 320; 8192 634, 577;
+//   * the clamped unit of 5632, 2048 wide: 100 rows (88 half tiles) 21.1, 23.0; 200 30.6, 22.7; 300 32.6, 27.2; 512 39, 34; 1000 58, 55; 2000 99, 88;
+//     4096 191, 161; of 11008, 4096 wide: 300 75, 76; 2000 425, 300;
+//   * squared ReLU of 8448, 2048 wide: 100 rows (66) 19.4, 20.8; 300 27.9, 21.4; 700 37.7, 31.1; 1000 43.6, 40.4; 4096 141, 120; 8192 311, 223;
+//   * GELU of 4096, 1024 wide: 100 rows (32) 11.7, 12.3; 300 (96) 13.9, 12.6; 1000 20.8, 14.2; 3000 37.3, 31.8; 16384 164, 131.  Its
+//     instructions run beside another tile's MFMAs, where a wide tile (149) has nobody beside it.
 inline PromptLinearPlan prompt_linear_plan(int rows, int outputs, int k, int act, bool row_major, bool packed) {
-  const PromptLinearPlan none{LVLLM_PROMPT_NONE, 0, 0};
-  const int64_t weights = (int64_t)outputs * (act == LVLLM_ACT_SILU_AND_MUL ? 2 : 1) * k;
-  if (rows <= 64 || outputs < 128 || weights >= (int64_t)1 << 30) return none;
-  if (packed && act != LVLLM_ACT_SILU_AND_MUL && outputs % 16 == 0 && k % 32 == 0 && k <= 2048) {
-    const PromptLinearPlan t = tile_plan(rows, outputs, act);
-    if (t.body != LVLLM_PROMPT_NONE) return t;
+  PromptLinearPlan plan{LVLLM_PROMPT_NONE, 0, 0};
+  const int64_t wrows = (int64_t)outputs * (prompt_pairs(act) ? 2 : 1);
+  const bool gelu = act == LVLLM_ACT_GELU;
+  if (rows <= 64 || outputs < 128 || outputs % 16 != 0 || wrows * k >= (int64_t)1 << 30) return plan;
+  const int64_t tiles = (rows + 127) / 128, half = tiles * ((wrows + 127) / 128);
+  if (half < (gelu ? 96 : 128)) return plan;
+  int64_t best = 0;
+  auto take = [&](int body, int groups, int nt, int64_t time) {
+    if (plan.body == LVLLM_PROMPT_NONE || time < best) plan = {body, groups, nt}, best = time;
+  };
+  if (row_major && !gelu && k % 64 == 0 && k >= 512)
+    for (int g = 4; g >= 2; --g) take(LVLLM_PROMPT_WIDE, g, 0, wide_time((rows + 64 * g - 1) / (64 * g) * ((wrows + 255) / 256), g, k, act));
+  if (packed && k % 32 == 0 && (!gelu || k <= 2048)) {
+    take(LVLLM_PROMPT_TILE, 0, 4, tile_time(tiles * ((wrows + 255) / 256), 4, k));
+    take(LVLLM_PROMPT_TILE, 0, 2, tile_time(half, 2, k));
   }
-  if (row_major && act != LVLLM_ACT_GELU && outputs % 16 == 0 && k % 64 == 0 && k >= 512) return wide_plan(rows, outputs, k, act);
-  return none;
+  return plan;
 }
 
-int launch_wide_linear(void* out, const void* x, const void* w, int rows, int outputs, int k, int act, int groups, void* stream);
-int launch_tile_linear(void* out, const void* x, const void* w, const void* bias, int rows, int outputs, int k, int act, int nt,
+int launch_wide_linear(void* out, const void* x, const void* w, int rows, int outputs, int k, int act, float limit, int groups,
                        void* stream);
+int launch_tile_linear(void* out, const void* x, const void* w, const void* bias, int rows, int outputs, int k, int act, float limit,
+                       int nt, void* stream);
 
 }  // namespace lvllm

@@ -5,32 +5,36 @@
 
 #include "gelu.h"
 #include "moe_tile.h"
+#include "prompt_act.h"
 #include "prompt_linear.h"
 
 namespace lvllm {
 
 struct TileLinear {
-  uint16_t* out;                  // [rows, n]
-  const uint16_t *x, *w, *bias;   // x [rows, k], w packed [n, k], bias [n] (GELU)
-  int rows, n, k, tiles, blocks;  // tiles of 128 rows, blocks of outputs
+  uint16_t* out;                  // [rows, outputs]
+  const uint16_t *x, *w, *bias;   // x [rows, k], w packed [n, k] (pairs: [gate rows | value rows]), bias [n] (GELU)
+  int rows, outputs, k, tiles, blocks;  // tiles of 128 rows, blocks of W rows
+  float limit;                    // CLAMPED_UNIT
 };
 
 template <int ACT, int NT, int MT>
 __device__ __forceinline__ void tile_linear(const TileLinear& p, const TileWork& t, char (*ring)[kStageBytes]) {
-  constexpr bool GELU = ACT == LVLLM_ACT_GELU;
+  constexpr bool GELU = ACT == LVLLM_ACT_GELU, PAIRS = prompt_pairs(ACT);
   e_f32x4_t acc[NT][MT];
-  tile_sums<false>(acc, p.x, p.k, p.w, t, ring, [](int slot) { return slot; });
+  // PAIRS: 16 gate rows, the 16 value rows that belong to them, ...
+  tile_sums<false>(acc, p.x, p.k, p.w, t, ring, [](int slot) { return slot; },
+                   [&](int tile) { return PAIRS ? (tile & 1) * (p.outputs >> 4) + (tile >> 1) : tile; });
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nt0 = (t.block * 4 + wave) * NT, g = (threadIdx.x & 63) >> 4;
   float z[NT][4];
   if constexpr (GELU)
 #pragma unroll
     for (int n = 0; n < NT; ++n) load4<BF16>(p.bias + min(nt0 + n, t.ntiles - 1) * 16 + 4 * g, z[n]);
-  tile_store<false>(p.out, p.n, acc, ring[0] + wave * 2048, nt0, t.ntiles, t.s0, t.s1, [](int) { return 1.f; },
-                    [&](float, int n, const e_f32x4_t& a, const e_f32x4_t&, float (&v)[4]) {
+  tile_store<PAIRS>(p.out, p.outputs, acc, ring[0] + wave * 2048, nt0, t.ntiles, t.s0, t.s1, [](int) { return 1.f; },
+                    [&](float, int n, const e_f32x4_t& a, const e_f32x4_t& b, float (&v)[4]) {
 #pragma unroll
                       for (int r = 0; r < 4; ++r) {
                         if constexpr (GELU) v[r] = gelu_of(a[r] + z[n][r]);
-                        else v[r] = relu_squared_of(BF16::to_float(BF16::from_float(a[r])));  // (of the projection's result)
+                        else v[r] = prompt_act<ACT>(a[r], b[r], p.limit);
                       }
                     });
 }
@@ -50,22 +54,22 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(const TileLinear p)
   t.s1 = min(t.s0 + size, p.rows);
   if (t.s0 >= t.s1) return;
   t.steps = p.k >> 5;
-  t.ntiles = p.n >> 4;
+  t.ntiles = (prompt_pairs(ACT) ? 2 : 1) * (p.outputs >> 4);
   const int groups = (t.s1 - t.s0 + 15) >> 4;
   if (groups <= 4) tile_linear<ACT, NT, 4>(p, t, ring);
   else if (groups <= 6) tile_linear<ACT, NT, 6>(p, t, ring);
   else tile_linear<ACT, NT, 8>(p, t, ring);
 }
 
-int launch_tile_linear(void* out, const void* x, const void* w, const void* bias, int rows, int outputs, int k, int act, int nt,
-                       void* stream) {
+int launch_tile_linear(void* out, const void* x, const void* w, const void* bias, int rows, int outputs, int k, int act, float limit,
+                       int nt, void* stream) {
   TileLinear p{};
   p.out = (uint16_t*)out; p.x = (const uint16_t*)x; p.w = (const uint16_t*)w; p.bias = (const uint16_t*)bias;
-  p.rows = rows; p.n = outputs; p.k = k;
+  p.rows = rows; p.outputs = outputs; p.k = k; p.limit = limit;
   p.tiles = (rows + kMoeTile - 1) / kMoeTile;
   auto launch = [&](auto act, auto nt) {
     constexpr int ACT = decltype(act)::value, NT = decltype(nt)::value;
-    p.blocks = (outputs + 64 * NT - 1) / (64 * NT);
+    p.blocks = ((prompt_pairs(ACT) ? 2 : 1) * outputs + 64 * NT - 1) / (64 * NT);
     hipLaunchKernelGGL((tile_linear_kernel<ACT, NT>), dim3((p.tiles * p.blocks + 7) / 8 * 8), dim3(256), 0, (hipStream_t)stream, p);
   };
   auto with = [&](auto act) {
@@ -73,7 +77,9 @@ int launch_tile_linear(void* out, const void* x, const void* w, const void* bias
     else launch(act, std::integral_constant<int, 2>{});
   };
   if (act == LVLLM_ACT_GELU) with(std::integral_constant<int, LVLLM_ACT_GELU>{});
-  else with(std::integral_constant<int, LVLLM_ACT_RELU_SQUARED>{});
+  else if (act == LVLLM_ACT_RELU_SQUARED) with(std::integral_constant<int, LVLLM_ACT_RELU_SQUARED>{});
+  else if (act == LVLLM_ACT_SILU_AND_MUL) with(std::integral_constant<int, LVLLM_ACT_SILU_AND_MUL>{});
+  else with(std::integral_constant<int, LVLLM_ACT_CLAMPED_UNIT>{});
   LV_LAUNCH_CHECK();
   return 0;
 }

@@ -255,11 +255,11 @@ torch::Tensor skinny_linear_packed_relu_squared(const torch::Tensor& x, const to
 // operands are none that the kernels take
 std::optional<torch::Tensor> prompt_linear(const torch::Tensor& x, const std::optional<torch::Tensor>& w,
                                            const std::optional<torch::Tensor>& w_packed, const std::optional<torch::Tensor>& bias,
-                                           int64_t outputs, int64_t act) {
+                                           int64_t outputs, int64_t act, double limit) {
   const char* op = "prompt_linear";
   LV_CHECK_DEVICE(x);
   TORCH_CHECK(x.dim() == 2, op, ": x must be [rows, k]");
-  const int64_t rows = x.size(0), k = x.size(1), n = outputs * (act == LVLLM_ACT_SILU_AND_MUL ? 2 : 1);
+  const int64_t rows = x.size(0), k = x.size(1), n = outputs * (act == LVLLM_ACT_SILU_AND_MUL || act == LVLLM_ACT_CLAMPED_UNIT ? 2 : 1);
   auto aligned = [](const torch::Tensor& t) { return ((uintptr_t)t.data_ptr() & 15) == 0; };
   auto takes = [&](const std::optional<torch::Tensor>& t, int64_t numel) {
     if (!t) return false;
@@ -274,7 +274,7 @@ std::optional<torch::Tensor> prompt_linear(const torch::Tensor& x, const std::op
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(x));
   auto out = torch::empty({rows, outputs}, x.options());
   check(lvllm_prompt_linear(out.data_ptr(), x.data_ptr(), row_major ? w->data_ptr() : nullptr, packed ? w_packed->data_ptr() : nullptr,
-                            biased ? bias->data_ptr() : nullptr, (int)rows, (int)outputs, (int)k, (int)act, dtype_code(x, op),
+                            biased ? bias->data_ptr() : nullptr, (int)rows, (int)outputs, (int)k, (int)act, (float)limit, dtype_code(x, op),
                             current_stream(x)));
   return out;
 }
@@ -715,7 +715,7 @@ TORCH_LIBRARY_FRAGMENT(_C_amd, amd) {
   amd.impl("skinny_linear_packed_clamped_unit", torch::kCUDA, &skinny_linear_packed_clamped_unit);
   amd.def("clamped_unit(Tensor x, float limit) -> Tensor");
   amd.impl("clamped_unit", torch::kCUDA, &clamped_unit);
-  amd.def("prompt_linear(Tensor x, Tensor? w, Tensor? w_packed, Tensor? bias, int outputs, int act) -> Tensor?");
+  amd.def("prompt_linear(Tensor x, Tensor? w, Tensor? w_packed, Tensor? bias, int outputs, int act, float limit=0.) -> Tensor?");
   amd.impl("prompt_linear", torch::kCUDA, &prompt_linear);
   amd.def("silu_unit(Tensor x) -> Tensor");
   amd.impl("silu_unit", torch::kCUDA, &silu_unit);

@@ -1,9 +1,10 @@
-// Projections of prompts with SwiGLU or squared ReLU behind them, in the tiles of wide_tile.h over the library's row-major weights: what
+// Projections of prompts with a gated unit or squared ReLU behind them, in the tiles of wide_tile.h over the library's row-major weights: what
 // they leave is the activation of what the projection would, in one launch and without its way through memory.  4875 rows of 4096, SwiGLU of
 // 14336: 842 us (1.36 PFLOP/s) for 891 and 73 in two launches; prompt_linear.h has more.
 #include <algorithm>
 #include <type_traits>
 
+#include "prompt_act.h"
 #include "prompt_linear.h"
 #include "wide_tile.h"
 
@@ -11,23 +12,11 @@ namespace lvllm {
 
 struct WideLinear {
   uint16_t* out;                      // [rows, outputs]
-  const uint16_t *x, *w;              // x [rows, k], w [n, k]; SwiGLU: [gate rows | value rows]
+  const uint16_t *x, *w;              // x [rows, k], w [n, k]; gated units: [gate rows | value rows]
   int rows, outputs, k, tile, tiles;  // tiles of `tile` rows
   int blocks;                         // of 256 W rows
+  float limit;                        // CLAMPED_UNIT
 };
-
-// x / (1 + e^-x) to the last bit or so: what the product with log2(e) loses goes into the power behind it, and a Newton step takes the
-// reciprocal's error.  The power is taken between +-87; below, the sigmoid is 0 to any bit that x could bring back.
-__device__ __forceinline__ float wide_silu(float x) {
-  const float y = -__builtin_amdgcn_fmed3f(x, -87.f, 87.f), t = y * 1.44269504f;
-  const float lost = fmaf(y, 1.92596303e-08f, fmaf(y, 1.44269504f, -t));
-  float e = __builtin_amdgcn_exp2f(t);
-  e = fmaf(e, lost * 0.693147181f, e);
-  const float d = 1.f + e;
-  float r = __builtin_amdgcn_rcpf(d);
-  r = fmaf(fmaf(-d, r, 1.f), r, r);
-  return x * (x < -87.f ? 0.f : r);
-}
 
 // W block `block` of rows row0 .. row1 - 1
 struct WideLinearUnit {
@@ -35,7 +24,7 @@ struct WideLinearUnit {
 };
 template <int ACT>
 __device__ __forceinline__ void wide_linear_tile(const WideLinear& p, const WideLinearUnit& u, WideTile& t) {
-  constexpr bool PAIRS = ACT == LVLLM_ACT_SILU_AND_MUL;
+  constexpr bool PAIRS = prompt_pairs(ACT);
   const int lane = wide_lane(), wave = wide_wave(), ld = p.k * 2;
   t.iters = p.k >> 6;
   t.groups = (u.row1 - u.row0 + 63) >> 6;
@@ -56,15 +45,13 @@ __device__ __forceinline__ void wide_linear_tile(const WideLinear& p, const Wide
 
 template <int ACT, int MT>
 __device__ __forceinline__ void wide_linear_store(const WideLinear& p, const WideLinearUnit& u, const WideSums<MT>& sums, char* lds) {
-  constexpr bool PAIRS = ACT == LVLLM_ACT_SILU_AND_MUL;
+  constexpr bool PAIRS = prompt_pairs(ACT);
   constexpr int kOuts = PAIRS ? 64 : 128;  // of a wave
   const int wave = wide_wave(), first = (u.block * 2 + (wave >> 1)) * kOuts, r0 = u.row0 + (wave & 1) * 32 * MT;
   wide_store<PAIRS>(sums, lds, p.out + (int64_t)r0 * p.outputs + first, p.outputs, u.row1 - r0, p.outputs - first,
                     [&](int, const w_f32x4_t& a, const w_f32x4_t& b, float (&v)[4]) {
-                      auto rounded = [](float f) { return BF16::to_float(BF16::from_float(f)); };
 #pragma unroll
-                      for (int r = 0; r < 4; ++r)
-                        v[r] = PAIRS ? rounded(wide_silu(rounded(a[r]))) * rounded(b[r]) : relu_squared_of(rounded(a[r]));
+                      for (int r = 0; r < 4; ++r) v[r] = prompt_act<ACT>(a[r], b[r], p.limit);
                     });
 }
 
@@ -119,16 +106,19 @@ static int launch(const WideLinear& p, hipStream_t s) {
   return 0;
 }
 
-int launch_wide_linear(void* out, const void* x, const void* w, int rows, int outputs, int k, int act, int groups, void* stream) {
+int launch_wide_linear(void* out, const void* x, const void* w, int rows, int outputs, int k, int act, float limit, int groups,
+                       void* stream) {
   WideLinear p{};
   p.out = (uint16_t*)out; p.x = (const uint16_t*)x; p.w = (const uint16_t*)w;
-  p.rows = rows; p.outputs = outputs; p.k = k;
+  p.rows = rows; p.outputs = outputs; p.k = k; p.limit = limit;
   p.tile = 64 * groups;
   p.tiles = (rows + p.tile - 1) / p.tile;
-  const int per = act == LVLLM_ACT_SILU_AND_MUL ? 128 : 256;
+  const int per = prompt_pairs(act) ? 128 : 256;
   p.blocks = (outputs + per - 1) / per;
-  return act == LVLLM_ACT_SILU_AND_MUL ? launch<LVLLM_ACT_SILU_AND_MUL>(p, (hipStream_t)stream)
-                                       : launch<LVLLM_ACT_RELU_SQUARED>(p, (hipStream_t)stream);
+  hipStream_t s = (hipStream_t)stream;
+  if (act == LVLLM_ACT_SILU_AND_MUL) return launch<LVLLM_ACT_SILU_AND_MUL>(p, s);
+  if (act == LVLLM_ACT_CLAMPED_UNIT) return launch<LVLLM_ACT_CLAMPED_UNIT>(p, s);
+  return launch<LVLLM_ACT_RELU_SQUARED>(p, s);
 }
 
 }  // namespace lvllm
@@ -140,14 +130,14 @@ extern "C" int lvllm_prompt_linear_body(int rows, int outputs, int k, int act, i
 }
 
 extern "C" int lvllm_prompt_linear(void* out, const void* x, const void* w, const void* w_packed, const void* bias, int rows, int outputs,
-                                   int k, int act, int dtype, void* stream) {
+                                   int k, int act, float limit, int dtype, void* stream) {
   if (rows == 0) return 0;
-  LV_CHECK(act == LVLLM_ACT_GELU || act == LVLLM_ACT_SILU_AND_MUL || act == LVLLM_ACT_RELU_SQUARED, "unknown activation");
+  LV_CHECK(act >= LVLLM_ACT_GELU && act <= LVLLM_ACT_CLAMPED_UNIT, "unknown activation");
   LV_CHECK(dtype == LVLLM_BF16, "bf16 only");
   LV_CHECK((bias != nullptr) == (act == LVLLM_ACT_GELU), "GELU takes a bias, the others none");
   LV_CHECK((((uintptr_t)out | (uintptr_t)x | (uintptr_t)w | (uintptr_t)w_packed | (uintptr_t)bias) & 15) == 0, "16-byte aligned pointers");
   const PromptLinearPlan plan = prompt_linear_plan(rows, outputs, k, act, w != nullptr, w_packed != nullptr);
   LV_CHECK(plan.body != LVLLM_PROMPT_NONE, "sizes that lvllm_prompt_linear_body does not take");
-  if (plan.body == LVLLM_PROMPT_TILE) return launch_tile_linear(out, x, w_packed, bias, rows, outputs, k, act, plan.nt, stream);
-  return launch_wide_linear(out, x, w, rows, outputs, k, act, plan.groups, stream);
+  if (plan.body == LVLLM_PROMPT_TILE) return launch_tile_linear(out, x, w_packed, bias, rows, outputs, k, act, limit, plan.nt, stream);
+  return launch_wide_linear(out, x, w, rows, outputs, k, act, limit, plan.groups, stream);
 }

@@ -11,7 +11,7 @@ import torch
 
 from .local_config import ClampedMlpConfig, ParallelHeadsConfig, RetentionConfig, RotaryConfig, RotaryHeadsConfig
 from .mixers import DECODE_ROWS, LayerCache, StepLayout, make_weight, pad_columns, project_to_residual, stack_rows
-from .model import Weight, linear
+from .model import Weight, linear, linear_act
 from .moe import MixtureOfExperts
 
 amd = torch.ops._C_amd
@@ -180,7 +180,8 @@ class ClampedMlp:
         if 0 < h.shape[0] <= DECODE_ROWS and self.up.packed is not None:
             a = amd.skinny_linear_packed_clamped_unit(h, self.up.packed, self.up.N, self.up.K, self.limit)
         else:
-            a = amd.clamped_unit(linear(h, self.up), self.limit)
+            a = linear_act(h, self.up, "clamped_unit", self.up.N // 2, self.limit)
+            a = amd.clamped_unit(linear(h, self.up), self.limit) if a is None else a
         return Branch(project_to_residual(a, self.down))
 
 

@@ -72,14 +72,14 @@ def linear(x: torch.Tensor, w: "Weight", bias: Optional[torch.Tensor] = None) ->
     return F.linear(x, w.w, bias)
 
 
-PROMPT_ACTS = {"gelu": 1, "silu_and_mul": 2, "relu_squared": 3}  # include/lvllm_hip.h LVLLM_ACT_*
+PROMPT_ACTS = {"gelu": 1, "silu_and_mul": 2, "relu_squared": 3, "clamped_unit": 4}  # include/lvllm_hip.h LVLLM_ACT_*
 
 
-def linear_act(x: torch.Tensor, w: "Weight", act: str, outputs: int) -> Optional[torch.Tensor]:
+def linear_act(x: torch.Tensor, w: "Weight", act: str, outputs: int, limit: float = 0.0) -> Optional[torch.Tensor]:
     """A prompt's projection with its activation in one launch; None where two are faster (csrc/prompt_linear.h)."""
     if not x.is_cuda or _CALIBRATING or w.w is None:
         return None
-    return torch.ops._C_amd.prompt_linear(x, w.w, w.packed, None, outputs, PROMPT_ACTS[act])
+    return torch.ops._C_amd.prompt_linear(x, w.w, w.packed, None, outputs, PROMPT_ACTS[act], limit)
 
 
 _CALIBRATING = False

@@ -17,7 +17,7 @@ extern "C" int plan(int rows, int outputs, int k, int act, int row_major, int pa
   return p.body;
 }
 """
-GELU, SILU, RELU2 = 1, 2, 3
+GELU, SILU, RELU2, CLAMPED = 1, 2, 3, 4
 NONE, WIDE, TILE = 0, 1, 2
 
 
@@ -36,10 +36,11 @@ def plan(tmp_path_factory):
 
 
 MEASURED = [  # rows, outputs, k, activation -> body, groups or blocks
-    (4875, 14336, 4096, SILU, WIDE, 4), (3000, 14336, 4096, SILU, WIDE, 3), (1000, 14336, 4096, SILU, NONE, 0), (700, 14336, 4096, SILU, WIDE, 3),
-    (300, 14336, 4096, SILU, WIDE, 3), (100, 14336, 4096, SILU, NONE, 0), (8192, 11264, 2048, SILU, WIDE, 4), (300, 5632, 2048, SILU, NONE, 0),
-    (4096, 8448, 2048, RELU2, WIDE, 3), (1000, 8448, 2048, RELU2, WIDE, 3), (700, 8448, 2048, RELU2, TILE, 4), (300, 8448, 2048, RELU2, TILE, 2),
-    (100, 8448, 2048, RELU2, NONE, 0), (16384, 4096, 1024, GELU, TILE, 4), (2000, 4096, 1024, GELU, TILE, 2), (100, 4096, 1024, GELU, NONE, 0)]
+    (4875, 14336, 4096, SILU, WIDE, 4), (3000, 14336, 4096, SILU, WIDE, 3), (1000, 14336, 4096, SILU, WIDE, 4), (700, 14336, 4096, SILU, WIDE, 3),
+    (300, 14336, 4096, SILU, WIDE, 3), (65, 14336, 4096, SILU, TILE, 2), (1000, 11264, 2048, SILU, TILE, 4), (128, 11264, 2048, SILU, TILE, 2),
+    (4096, 5632, 2048, CLAMPED, TILE, 4), (300, 5632, 2048, CLAMPED, TILE, 2), (100, 5632, 2048, CLAMPED, NONE, 0),
+    (4096, 8448, 2048, RELU2, WIDE, 3), (1000, 8448, 2048, RELU2, WIDE, 3), (300, 8448, 2048, RELU2, TILE, 2),
+    (100, 8448, 2048, RELU2, NONE, 0), (16384, 4096, 1024, GELU, TILE, 4), (1000, 4096, 1024, GELU, TILE, 2), (100, 4096, 1024, GELU, NONE, 0)]
 
 
 @pytest.mark.parametrize("rows,outputs,k,act,body,size", MEASURED)
@@ -52,11 +53,11 @@ def test_any_size(plan):
     rng = random.Random(0)
     for _ in range(20000):
         rows, outputs, k = rng.randint(1, 40000), rng.choice([8, 16]) * rng.randint(1, 2000), rng.choice([8, 32, 64]) * rng.randint(1, 128)
-        act, row_major, packed = rng.choice([GELU, SILU, RELU2]), rng.random() < 0.5, rng.random() < 0.5
+        act, row_major, packed = rng.choice([GELU, SILU, RELU2, CLAMPED]), rng.random() < 0.5, rng.random() < 0.5
         body, size = plan(rows, outputs, k, act, row_major, packed)
         if body == WIDE:
             assert row_major and act != GELU and k % 64 == 0 and outputs % 16 == 0 and 2 <= size <= 4
         elif body == TILE:
-            assert packed and act != SILU and k % 32 == 0 and outputs % 16 == 0 and size in (2, 4)
+            assert packed and k % 32 == 0 and outputs % 16 == 0 and size in (2, 4)
         if body != NONE:
-            assert rows > 64 and outputs * k * (2 if act == SILU else 1) * 2 < 2 ** 31
+            assert rows > 64 and outputs * k * (2 if act in (SILU, CLAMPED) else 1) * 2 < 2 ** 31

@@ -6,7 +6,8 @@ import torch.nn.functional as F
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-GELU, SILU, RELU2 = 1, 2, 3
+GELU, SILU, RELU2, CLAMPED = 1, 2, 3, 4
+LIMIT = 1.5
 
 
 @pytest.fixture(scope="module")
@@ -23,15 +24,15 @@ TILE = [(300, 4096, 64), (1000, 4112, 96), (129, 6160, 1024), (2500, 4096, 160),
 
 def check(amd, rows, outputs, k, act, row_major, pack):
     gen = torch.Generator().manual_seed(rows + outputs + k)
-    n = outputs * (2 if act == SILU else 1)
+    n = outputs * (2 if act in (SILU, CLAMPED) else 1)
     x = torch.randn(rows, k, generator=gen).bfloat16().to(DEV)
     w = (torch.randn(n, k, generator=gen) * 2 * k ** -0.5).bfloat16().to(DEV)
     bias = (0.2 * torch.randn(n, generator=gen)).bfloat16().to(DEV) if act == GELU else None
-    got = amd.prompt_linear(x, w if row_major else None, amd.pack_weight(w) if pack else None, bias, outputs, act)
+    got = amd.prompt_linear(x, w if row_major else None, amd.pack_weight(w) if pack else None, bias, outputs, act, LIMIT)
     assert got is not None and got.shape == (rows, outputs)
     z = x.double() @ w.double().T
     # sums of up to 2048 products of values around 1 in fp32, rounded to 8 bits behind the product (not GELU) and behind the activation,
-    # SwiGLU once more between
+    # SwiGLU once more between; the clamped unit of rounded gate and value grows with the gate at most 1.1 times as fast, its parts at most LIMIT
     sums, eps = 1e-5, 2.0 ** -8
     if act == GELU:
         z = z + bias.double()
@@ -40,26 +41,27 @@ def check(amd, rows, outputs, k, act, row_major, pack):
         g, u = z[:, :outputs], z[:, outputs:]
         want = F.silu(g) * u
         slack = eps * (2 * want.abs() + 1.1 * g.abs() * u.abs() + F.silu(g).abs() * u.abs()) + 4 * sums * (1 + g.abs() + u.abs())
+    elif act == CLAMPED:
+        g, u = z[:, :outputs].clamp(max=LIMIT), z[:, outputs:].clamp(-LIMIT, LIMIT)
+        want = g * torch.sigmoid(1.702 * g) * (u + 1)
+        slack = eps * (want.abs() + 1.13 * g.abs() * (u + 1).abs() + 1.5 * u.abs()) + 4 * sums * (1 + LIMIT) + 1e-6
     else:
         want = z.clamp(min=0).square()
         slack = eps * 3.1 * want + 2 * sums * (z.abs() + 1)
     assert ((got.double() - want).abs() <= slack).all(), ((got.double() - want).abs() - slack).max()
 
 
-@pytest.mark.parametrize("act", [SILU, RELU2])
+@pytest.mark.parametrize("act", [SILU, RELU2, CLAMPED])
 @pytest.mark.parametrize("rows,outputs,k", WIDE)
 def test_wide_tiles(amd, rows, outputs, k, act):
     check(amd, rows, outputs, k, act, True, False)
 
 
+@pytest.mark.parametrize("act", [GELU, SILU, RELU2, CLAMPED])
 @pytest.mark.parametrize("rows,outputs,k", TILE)
-def test_tiles(amd, rows, outputs, k):
-    check(amd, rows, outputs, k, GELU, False, True)
-
-
-@pytest.mark.parametrize("rows,outputs,k", [(200, 8448, 96), (129, 12304, 1024), (640, 8464, 160)])
-def test_tiles_of_squared_relu(amd, rows, outputs, k):
-    check(amd, rows, outputs, k, RELU2, False, True)
+def test_tiles(amd, rows, outputs, k, act):
+    outputs *= 1 if act in (GELU, CLAMPED) else 3
+    check(amd, rows, outputs, k, act, False, True)
 
 
 def test_activations_of_the_largest_and_smallest_values(amd):
