@@ -598,6 +598,22 @@ def test_add_layer_norm_matches_torch(ops, dtype, T, hidden, with_y):
     assert torch.equal(x2.view(torch.int16), out.view(torch.int16))
 
 
+@pytest.mark.parametrize("seqs", [1, 5, 11, 17, 33])
+@pytest.mark.parametrize("longest", [512, 513, 1300])
+def test_shares_by_the_batch(ops, seqs, longest):
+    """Contexts cut into as many shares as leave a CU to each workgroup (8 kv heads: 8 shares down to one), with slots for eight: what
+    shares longer and shorter than a sequence's leave empty, and the largest batch without a cut."""
+    lens = [max(1, longest - 37 * i) for i in range(seqs)]
+    inp = make_paged_inputs(seqs, 16, 8, 64, 16, lens, dtype=torch.bfloat16, seed=seqs)
+    d64 = dense_attention_fp64(inp)
+    d = to_dev(inp)
+    tmp = torch.full((seqs, 16, 8, 64), float("nan"), dtype=torch.bfloat16, device=DEV)
+    es, ml, out = torch.full((seqs, 16, 8), float("nan"), device=DEV), torch.full((seqs, 16, 8), float("nan"), device=DEV), torch.empty_like(d["query"])
+    ops.paged_attention_v2(out, es, ml, tmp, d["query"], d["key_cache"], d["value_cache"], 8, inp["scale"], d["block_tables"], d["seq_lens"],
+                           16, inp["max_seq_len"], None, "auto", 1.0, 1.0)
+    check_attention(out, d64, d64)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,hidden", [(1, 8), (5, 128), (33, 1000), (4, 1024), (3, 2048)])
 def test_embed_layer_norm(ops, dtype, T, hidden):
