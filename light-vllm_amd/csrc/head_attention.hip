@@ -117,7 +117,9 @@ static bool takes_mfma(int kpad, int vpad, int maps, int block_size, int dtype) 
 }
 
 // Shares the keys of a sequence are cut into: enough workgroups to fill the chip, none of under 256 keys, and none at all
-// beside large prompt portions
+// beside large prompt portions.  Nor for up to 512 keys, whose walk is shorter than the launch that shares meet in: 16 heads over 4 of 128 and 64,
+// us in two shares and now, 100 keys: 1 sequence 6.6, 4.4; 24 sequences 7.3, 4.8; 300: 9.5, 6.9; 500: 10.4, 8.8.  (Two maps meet in that launch
+// in any case.)
 static int decode_shares(int rows, int num_seqs, int heads, int kv_heads, int max_seq_len, const lvllm_head_options& o) {
   if (rows > 512) return 1;
   const int wgs = num_seqs * kv_heads * ((heads / kv_heads * o.maps + kDecodeCols - 1) / kDecodeCols);
@@ -125,7 +127,7 @@ static int decode_shares(int rows, int num_seqs, int heads, int kv_heads, int ma
   int64_t keys = max_seq_len;
   if (o.window > 0) keys = std::min<int64_t>(keys, (int64_t)o.window + o.keep_first + kDecodeCols);
   if (o.chunk > 0) keys = std::min<int64_t>(keys, (int64_t)o.chunk + o.keep_first + kDecodeCols);
-  const int most = (int)((keys + 255) / 256);
+  const int most = o.maps == 1 && keys <= 512 ? 1 : (int)((keys + 255) / 256);
   n = n < most ? n : most;
   return n < 1 ? 1 : n > 64 ? 64 : n;
 }

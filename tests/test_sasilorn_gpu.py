@@ -298,6 +298,14 @@ def test_softmax_heads(amd, dtype, name, heads, kv_heads, dim, vdim):
         at += n
 
 
+@pytest.mark.parametrize("longest", [511, 512, 513])
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(4, 1, 128, 64), (2, 2, 64, 256)])
+def test_single_tokens_by_the_longest(amd, monkeypatch, longest, heads, kv_heads, dim, vdim):
+    """Up to 512 keys one share, beyond several that meet in a launch of their own."""
+    monkeypatch.setitem(ATTENTION_LAYOUTS, "longest", [(1, longest - 1), (1, 255), (3, 300), (1, 0)])
+    test_softmax_heads(amd, BF16, "longest", heads, kv_heads, dim, vdim)
+
+
 def dense_rows(q, k, v, scale, first):
     """The restatement's softmax heads for rows first .. (its own loop takes every row)."""
     if first == 0 and q.shape[0] < 40:
