@@ -192,16 +192,20 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, con
   __shared__ __attribute__((aligned(16))) char ring[tile_steps(NT) / 2][kStageBytes];
   const TileWork t = tile_work<PRODUCT, kMoeTile, 4 * NT>(p, blocks_first, blocks_last);
   if (!t.any) return;
+  // a body per height in groups of 16 slots, from four on: where power bounds the launch, products with slots that are not there cost as
+  // much as others.  Up + down, us, with bodies of 4, 6 and 8 groups and with these: 4096 rows, 6 of 64 experts of 2816 (tiles of 96 to 112 slots)
+  // 900, 876; 8192 rows 1548, 1538; 1300 rows, 2 of 32 of 1408 and a shared one (up) 104, 97; others 1.00 to 1.02.
   const int groups = (t.s1 - t.s0 + 15) >> 4;
-  if (t.once) {
-    if (groups <= 4) tile_product<PRODUCT, true, NT, 4>(p, t, ring);
-    else if (groups <= 6) tile_product<PRODUCT, true, NT, 6>(p, t, ring);
-    else tile_product<PRODUCT, true, NT, 8>(p, t, ring);
-  } else {
-    if (groups <= 4) tile_product<PRODUCT, false, NT, 4>(p, t, ring);
-    else if (groups <= 6) tile_product<PRODUCT, false, NT, 6>(p, t, ring);
-    else tile_product<PRODUCT, false, NT, 8>(p, t, ring);
-  }
+  auto go = [&](auto once) __attribute__((always_inline)) {
+    constexpr bool O = decltype(once)::value;
+    if (groups <= 4) tile_product<PRODUCT, O, NT, 4>(p, t, ring);
+    else if (groups == 5) tile_product<PRODUCT, O, NT, 5>(p, t, ring);
+    else if (groups == 6) tile_product<PRODUCT, O, NT, 6>(p, t, ring);
+    else if (groups == 7) tile_product<PRODUCT, O, NT, 7>(p, t, ring);
+    else tile_product<PRODUCT, O, NT, 8>(p, t, ring);
+  };
+  if (t.once) go(std::true_type{});
+  else go(std::false_type{});
 }
 
 // The router's logits on packed weights (experts and the shared gate, up to a multiple of 16 rows): 16 rows of h and a share

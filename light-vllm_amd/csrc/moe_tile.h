@@ -85,7 +85,7 @@ constexpr int tile_steps(int NT) { return NT == 4 ? 4 : 8; }  // k-steps of weig
 template <bool ONCE, int NT, int MT, class ROW, class TILE>
 __device__ __forceinline__ void tile_sums(e_f32x4_t (&acc)[NT][MT], const uint16_t* x_rows, const int64_t ld, const uint16_t* w_tiles,
                                           const TileWork& t, char (*ring)[kStageBytes], ROW row_of, TILE tile_of) {
-  constexpr int S = tile_steps(NT), X = S / 2, kCopies = MT / 2;  // (MT groups of 16 slots)
+  constexpr int S = tile_steps(NT), X = S / 2, kCopies = (MT + 1) / 2;  // (MT groups of 16 slots)
   constexpr int kYounger = (X - 2) * kCopies + (X - 1) * 2 * NT;  // loads behind a stage's copies when it is needed
   constexpr int kBehind = (X - 1) * kCopies + (S - 1) * NT;       // ... behind a second k-step's weights
   const int s0 = t.s0, s1 = t.s1, block = t.block, steps = t.steps, ntiles = t.ntiles;

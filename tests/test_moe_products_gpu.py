@@ -78,6 +78,15 @@ def test_products_of_few_rows(amd, counts, full, width, act):
     test_products(amd, counts, [ff, 96, 1408, 352], width, act, True)
 
 
+@pytest.mark.parametrize("act", ["clamped", "relu_squared"])
+@pytest.mark.parametrize("ff", [160, 8320], ids=["half blocks", "whole blocks"])
+@pytest.mark.parametrize("tiles", [1, 2], ids=["single tiles", "two tiles"])
+def test_tiles_of_every_height(amd, tiles, ff, act):
+    """Tiles of 65 to 128 slots in groups of 16, at both ends of each height."""
+    heights = [65, 80, 81, 96, 97, 112, 113]
+    test_products(amd, [tiles * n for n in heights], [ff] * 6 + [ff + 32], 160, act, False)
+
+
 @pytest.mark.parametrize("act", [0, 2], ids=["clamped", "relu_squared"])
 @pytest.mark.parametrize("copies", [1, 70], ids=["half blocks", "whole blocks"])
 def test_blocks_of_weight_rows(amd, copies, act):
