@@ -46,7 +46,7 @@ extern "C" int lvllm_set_tuning(const char* key, int value) {
   } else if (k == "varlen_dense") {
     lvllm::tuning().varlen_dense = value != 0;
   } else if (k == "varlen_dense_waves") {
-    LV_CHECK(value == 0 || value == 4 || value == 8, "varlen_dense_waves must be 0 (by sequence length), 4 or 8");
+    LV_CHECK(value == 0 || value == 4 || value == 8, "varlen_dense_waves must be 0 (by the sizes), 4 or 8");
     lvllm::tuning().varlen_dense_waves = value;
   } else if (k == "attn_waves") {
     LV_CHECK(value == 4 || value == 8, "attn_waves must be 4 or 8");

@@ -119,6 +119,38 @@ def test_rows_read_in_place_equal_the_pack_pass_bit_for_bit(ops, dtype, causal, 
     assert torch.equal(out2[sl].cpu().view(torch.int16), outs[0][sl].view(torch.int16))
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("H,KVH", [(40, 1), (6, 3), (1, 1)])
+def test_rows_read_in_place_by_columns_of_a_workgroup(ops, causal, H, KVH):
+    """128 and 256 columns a workgroup at their edges, groups of query heads beyond 32 and of two, logits whose maxima grow from tile to
+    tile, and NaN in a last key and value that a causal query of an earlier tile must not see: the bits of the pack pass."""
+    D, seq_lens = 64, [300, 63, 257, 128, 1, 513]
+    T = sum(seq_lens)
+    g = torch.Generator().manual_seed(H)
+    qkv = torch.randn(T, (H + 2 * KVH) * D, generator=g).bfloat16()
+    qkv[:, H * D:(H + KVH) * D] *= torch.linspace(0.1, 6, T)[:, None].bfloat16()
+    if causal:
+        qkv[299, H * D:] = float("nan")
+    q, k, v = (x.unflatten(1, (-1, D)) for x in qkv.to(DEV).split([H * D, KVH * D, KVH * D], dim=1))
+    cu = torch.tensor([0] + list(np.cumsum(seq_lens)), dtype=torch.int32, device=DEV)
+    outs = []
+    for dense, waves in ((0, 0), (1, 4), (1, 8)):
+        torch.ops._C_amd.set_tuning("varlen_dense", dense)
+        torch.ops._C_amd.set_tuning("varlen_dense_waves", waves)
+        try:
+            outs.append(torch.empty(T, H, D, dtype=torch.bfloat16, device=DEV))
+            ops.varlen_attention(outs[-1], q, k, v, cu, max(seq_lens), D ** -0.5, causal)
+        finally:
+            torch.ops._C_amd.set_tuning("varlen_dense", 1)
+            torch.ops._C_amd.set_tuning("varlen_dense_waves", 0)
+    rows = torch.ones(T, dtype=torch.bool)
+    rows[256:300] = not causal  # (of the tile that holds it)
+    want, *got = (o.cpu()[rows] for o in outs)
+    assert torch.isfinite(want).all()
+    for o in got:
+        assert torch.equal(o.view(torch.int16), want.view(torch.int16))
+
+
 def test_rows_read_in_place_with_different_key_and_value_strides(ops):
     """K and V of different buffers, different token strides, V not at the start of its rows: the in-place launch
     takes each operand's own stride and base (bit-identical to the pack pass, as above)."""
