@@ -17,8 +17,12 @@
 //     takes three scores at a time.  The scale stays a product of its own, rounded ahead of the subtraction (6 to 10 % of such a
 //     launch): fused with it, other roundings moved tokens of a mixture behind the attention to other experts;
 //   * tiles of kept first keys come ahead of the window's.
-// One prompt of 4096, us, with tiles through registers and an instruction for each of these, and now: 16 heads over 4, 128 + 64,
-// 133, 111; 32 over 8, 128 + 128, 212, 193; two maps 190, 168.  4 prompts of 2048, 16 heads, 192 + 128 (two stages): 145, 133.
+// The longest walk is one wave a SIMD for much of a launch, so that what a tile's chain waits for counts as much as what it issues:
+// fragments are read eight ahead of their MFMAs, the first of V in front of the softmax; the maximum is four chains and one exchange
+// of halves in registers; pages become addresses once in 16 tiles, in the lanes, and a copy's address is scalar; a masked tile's
+// comparisons are taken four at a time (all at once, their results were kept in lanes: 64 writes and as many reads a tile).
+// us before these and now, same bits: one prompt of 4096, 16 heads over 4, 128 + 64, 104, 95; of 1000 29.4, 25.7; of 2000, 128 + 128, 59.5, 53.4; of
+// 300 18.8, 14.4; two maps of 64 + 128, 2000 tokens 65, 62; 4 prompts of 2048, 16 heads, 192 + 128 (two stages) 140, 127; 3 of 777 35, 35.
 #pragma once
 #include <float.h>
 
@@ -31,9 +35,13 @@ __device__ __forceinline__ h_f32x16_t mfma32(h_u32x4_t a, h_u32x4_t b, h_f32x16_
                                                  0, 0, 0);
 }
 
-__device__ __forceinline__ void to_lds(const uint16_t* src, char* dst) {  // 16 bytes a lane, 1 KiB a wave
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                   (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+// 16 bytes a lane, 1 KiB a wave, from lane offsets `at` and `skip` into a block's head slice.  (Addresses of a descriptor are the scalar
+// unit's work, and not 64-bit additions of the lanes.)
+__device__ __forceinline__ void to_lds(const uint16_t* slice, int bytes, int at, int skip, char* dst) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(slice), 0, bytes, 0x00020000),
+                                           (__attribute__((address_space(3))) void*)dst, 16, at, skip, 0, 0);
+#endif
 }
 // The largest of three; fmaxf takes three instructions of what might be a signalling NaN.  The compiler does not look into this
 // one: where b and c are results of MFMAs, `a` has to come from an instruction behind the same ones, which has waited for them.
@@ -59,7 +67,7 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
   const int kvh = blockIdx.x, seq = blockIdx.z;
   // The end of the chunk, which sees the most keys, first.  Where all workgroups run at once, two a CU, those that come second on
   // their CUs (behind p.fold tiles) come in the other order, the shortest walk beside the longest: one prompt of 4096, 16 heads over
-  // 4, 128 + 64, 111 us without, 105 with.
+  // 4, 128 + 64, 111 us without, 105 with (as the tiles were then).
   const int tile_q = (int)blockIdx.y < p.fold ? gridDim.y - 1 - blockIdx.y : blockIdx.y - p.fold;
   const int G = p.heads / p.kv_heads;
   const int qbeg = p.query_start_loc[seq], qlen = p.query_start_loc[seq + 1] - qbeg;
@@ -91,29 +99,32 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
   const int32_t* table = p.block_tables + (int64_t)seq * p.max_blocks;
   const uint16_t* kc = (const uint16_t*)p.k_cache + (int64_t)kvh * KP * 16;
   const uint16_t* vc = (const uint16_t*)p.v_cache + (int64_t)kvh * VP * 16;
-  int pages = 0, run = -1;  // of 16 tiles, a lane each
+  const int k_lane = lane * 16, v_lane = (lane & 31) * 32 + (lane >> 5) * 16;
+  // Where the pages of 16 tiles lie, a lane each (multiplied there: scalar 64-bit products are chains of their own).
+  uint64_t k_page = 0, v_page = 0;
+  int run = -1;
   auto copy = [&](int stage, int tile) __attribute__((always_inline)) {
     if (tile >> 4 != run) {
       run = tile >> 4;
-      pages = table[min(run * 64 + lane, p.max_blocks - 1)];
-      __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // (here, and not in front of every use)
+      const int page = min(max(table[min(run * 64 + lane, p.max_blocks - 1)], 0), p.max_block);
+      k_page = (uint64_t)kc + (uint64_t)((int64_t)page * p.k_block_stride) * 2;
+      v_page = (uint64_t)vc + (uint64_t)((int64_t)page * p.v_block_stride) * 2;
     }
     char* base = smem + stage * kStage;
-    int blk[4];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) blk[b] = min(max(__builtin_amdgcn_readlane(pages, (tile & 15) * 4 + b), 0), p.max_block);
+    auto of = [&](uint64_t page, int b) __attribute__((always_inline)) {
+      const int at = (tile & 15) * 4 + b;
+      return (const uint16_t*)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)page, at) |
+                               (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(page >> 32), at) << 32);
+    };
 #pragma unroll
     for (int j = 0; j < NK; ++j) {
       const int b = (wave + 4 * j) / NK, w = (wave + 4 * j) - b * NK;  // 64-chunk group w of block b
-      const int bk = b == 0 ? blk[0] : b == 1 ? blk[1] : b == 2 ? blk[2] : blk[3];
-      to_lds(kc + (int64_t)bk * p.k_block_stride + (w * 64 + lane) * 8, base + b * kKBlock + w * 1024);
+      to_lds(of(k_page, b), kKBlock, k_lane, w * 1024, base + b * kKBlock + w * 1024);
     }
 #pragma unroll
     for (int j = 0; j < NV; ++j) {  // of a 32-row group: the first tokens' chunks of all rows, then the second ones'
       const int b = (wave + 4 * j) / NV, w = (wave + 4 * j) - b * NV;
-      const int bk = b == 0 ? blk[0] : b == 1 ? blk[1] : b == 2 ? blk[2] : blk[3];
-      to_lds(vc + (int64_t)bk * p.v_block_stride + (w * 64 + (lane & 31) * 2 + (lane >> 5)) * 8,
-             base + kImageK + b * kVBlock + w * 1024);
+      to_lds(of(v_page, b), kVBlock, v_lane, w * 1024, base + kImageK + b * kVBlock + w * 1024);
     }
   };
 
@@ -129,6 +140,7 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
   const int vlds = kImageK + lane * 16;  // (hi * 32 + lc) * 16
 
   constexpr int kCopies = NK + NV;  // of a wave and tile
+  constexpr int kWinK = 2 * KS < 8 ? 2 * KS : 8, kWinV = 4 * NV < 8 ? 4 * NV : 8;  // fragments read ahead of their MFMAs
   __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // (the queries are here: what is on its way below are copies)
 #pragma unroll
   for (int t = 0; t < S - 1; ++t)
@@ -144,13 +156,25 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
     if (wave_ok && k0 <= wave_last && (k0 + 63 >= wave_low || k0 < p.keep_first)) {
       const char* base = smem + stage * kStage;
       h_f32x16_t s[2] = {h_f32x16_t{}, h_f32x16_t{}};
+      h_u32x4_t kw[kWinK], vw[kWinV];
+      auto key = [&](int i) __attribute__((always_inline)) {  // fragment i: keys of half i % 2, k-step i / 2
+        return *reinterpret_cast<const h_u32x4_t*>(base + klds + (i & 1) * 2 * kKBlock + (i >> 1) * 512);
+      };
+      auto value = [&](int i) __attribute__((always_inline)) {  // ... keys of step i / NV, rows of block i % NV
+        return *reinterpret_cast<const h_u32x4_t*>(base + vlds + (i / NV) * kVBlock + (i % NV) * 1024);
+      };
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const h_u32x4_t a0 = *reinterpret_cast<const h_u32x4_t*>(base + klds + ks * 512);
-        const h_u32x4_t a1 = *reinterpret_cast<const h_u32x4_t*>(base + klds + 2 * kKBlock + ks * 512);
-        s[0] = mfma32(a0, qf[ks], s[0]);
-        s[1] = mfma32(a1, qf[ks], s[1]);
+      for (int i = 0; i < kWinK; ++i) kw[i] = key(i);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 2 * KS; ++i) {
+        s[i & 1] = mfma32(kw[i % kWinK], qf[i >> 1], s[i & 1]);
+        if (i + kWinK < 2 * KS) kw[i % kWinK] = key(i + kWinK);
+        __builtin_amdgcn_sched_barrier(0);
       }
+#pragma unroll
+      for (int i = 0; i < kWinV; ++i) vw[i] = value(i);
+      __builtin_amdgcn_sched_barrier(0);
       if (score.cap > 0.f) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
@@ -169,12 +193,17 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
           for (int i = 0; i < 16; ++i) {
             const int key = k0 + 32 * h + 16 * (i >> 3) + 8 * hi + (i & 7);
             s[h][i] = sees(p, key, pos, low) ? s[h][i] : -INFINITY;
+            if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // (else all are compared first, and their masks kept in lanes)
           }
       }
-      float mx = fmaxf(s[0][0], s[1][0]);  // (behind this both products' results are there)
+      float part[4];
 #pragma unroll
-      for (int i = 1; i < 16; ++i) mx = max3(mx, s[0][i], s[1][i]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      for (int i = 0; i < 4; ++i) part[i] = fmaxf(s[0][i], s[1][i]);  // (behind this both products' results are there)
+#pragma unroll
+      for (int i = 4; i < 16; ++i) part[i & 3] = max3(part[i & 3], s[0][i], s[1][i]);
+      float mx = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+      const auto both = halves_apart(mx);
+      mx = fmaxf(both.a, both.b);
       if (__any(mx > m)) {
         const float mn = fmaxf(m, mx), corr = exp2f(m - mn);
         m = mn;
@@ -191,15 +220,18 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
           sum += s[h][i];
         }
       l += sum;
+      h_u32x4_t pf[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        h_u32x4_t pf;
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) pf[r] = pack_bf16(s[j >> 1][8 * (j & 1) + 2 * r], s[j >> 1][8 * (j & 1) + 2 * r + 1]);
+        for (int r = 0; r < 4; ++r) pf[j][r] = pack_bf16(s[j >> 1][8 * (j & 1) + 2 * r], s[j >> 1][8 * (j & 1) + 2 * r + 1]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < NV; ++i) {
-          const h_u32x4_t vf = *reinterpret_cast<const h_u32x4_t*>(base + vlds + j * kVBlock + i * 1024);
-          o[i] = mfma32(vf, pf, o[i]);
+      for (int i = 0; i < 4 * NV; ++i) {
+        o[i % NV] = mfma32(vw[i % kWinV], pf[i / NV], o[i % NV]);
+        if (i + kWinV < 4 * NV) {
+          vw[i % kWinV] = value(i + kWinV);
+          __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
