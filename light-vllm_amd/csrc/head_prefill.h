@@ -2,8 +2,8 @@
 //
 // A workgroup is 4 waves = 128 columns, a column being a (query token, head of the GQA group, map) triple; the waves share one
 // stream of 64-key tiles, copied straight to LDS: three stages where two workgroups a CU have room for them, else two, one
-// barrier per tile.  A portion's last columns walk all keys one tile after the other, and that walk is how long the launch
-// takes: pages are looked up 16 tiles at a time, and copies are one or two tiles ahead of their use.
+// barrier per tile (with three in front of the last products of the tile before).  A portion's last columns walk all keys one tile after the other, and that walk is how long the launch
+// takes: pages are looked up 16 tiles at a time, and copies are a tile ahead of their use.
 // With two maps, waves 0 and 1 take the first one, waves 2 and 3 the second one of the same 64 (token, head) pairs: each reads
 // its half of the keys, and the two results meet in LDS at the end.
 //   * S^T = K Q^T: a lane holds 32 keys of ONE column, so the column's maximum is in-lane plus one exchange of halves;
@@ -21,8 +21,10 @@
 // fragments are read eight ahead of their MFMAs, the first of V in front of the softmax; the maximum is four chains and one exchange
 // of halves in registers; pages become addresses once in 16 tiles, in the lanes, and a copy's address is scalar; a masked tile's
 // comparisons are taken four at a time (all at once, their results were kept in lanes: 64 writes and as many reads a tile).
-// us before these and now, same bits: one prompt of 4096, 16 heads over 4, 128 + 64, 104, 95; of 1000 29.4, 25.7; of 2000, 128 + 128, 59.5, 53.4; of
-// 300 18.8, 14.4; two maps of 64 + 128, 2000 tokens 65, 62; 4 prompts of 2048, 16 heads, 192 + 128 (two stages) 140, 127; 3 of 777 35, 35.
+// With three stages a tile's first fragments of K are read beside the last products of the one before.
+// us before these and now, same bits: one prompt of 4096, 16 heads over 4, 128 + 64, 104, 92 (95 with K's fragments read behind the barrier);
+// of 1000 29.4, 25.2; of 2000, 128 + 128, 59.5, 53.4; of 300 18.8, 14.4; two maps of 64 + 128, 2000 tokens 65, 61; 4 prompts of 2048, 16
+// heads, 192 + 128 (two stages) 140, 127; 3 of 777 35, 35.
 #pragma once
 #include <float.h>
 
@@ -145,31 +147,44 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
 #pragma unroll
   for (int t = 0; t < S - 1; ++t)
     if (t < ntiles) copy(t, tile_of(t));
+  constexpr bool kAhead = S == 3;  // a tile's first fragments of K are read beside the last products of the one before
+  h_u32x4_t kw[kWinK];
+  auto key = [&](int stage, int i) __attribute__((always_inline)) {  // fragment i: keys of half i % 2, k-step i / 2
+    return *reinterpret_cast<const h_u32x4_t*>(smem + stage * kStage + klds + (i & 1) * 2 * kKBlock + (i >> 1) * 512);
+  };
+  auto read_keys = [&](int stage) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kWinK; ++i) kw[i] = key(stage, i);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Tile t is in LDS, for every wave, and everyone is done with the stage that is filled next.
+  auto publish = [&](int t, int stage) __attribute__((always_inline)) {
+    // loads retire in order: with only the youngest tile's copies outstanding, this one's have landed
+    if (kAhead && t == 0 && ntiles > 1) __builtin_amdgcn_s_waitcnt(kCopies | (7 << 4) | (15 << 8));
+    else __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+    asm volatile("s_barrier" ::: "memory");
+    read_keys(stage);
+    const int next = kAhead ? t + 1 : t + S - 1;
+    if ((!kAhead || t > 0) && next < ntiles) copy(stage + 1 == S ? 0 : stage + 1, tile_of(next));
+  };
+  if (kAhead) publish(0, 0);
   int stage = 0;
   for (int t = 0; t < ntiles; ++t) {
-    // loads retire in order: with only the youngest tile's copies outstanding (two stages: none), this one's have landed
-    if (S == 3 && t + 1 < ntiles) __builtin_amdgcn_s_waitcnt(kCopies | (7 << 4) | (15 << 8));
-    else __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
-    asm volatile("s_barrier" ::: "memory");  // ... for every wave; and everyone is done with the stage that is filled next
-    if (t + S - 1 < ntiles) copy(stage == 0 ? S - 1 : stage - 1, tile_of(t + S - 1));
+    if (!kAhead) publish(t, stage);
+    const int after = stage + 1 == S ? 0 : stage + 1;
+    bool published = !kAhead || t + 1 == ntiles;
     const int k0 = tile_of(t) * 64;
     if (wave_ok && k0 <= wave_last && (k0 + 63 >= wave_low || k0 < p.keep_first)) {
       const char* base = smem + stage * kStage;
       h_f32x16_t s[2] = {h_f32x16_t{}, h_f32x16_t{}};
-      h_u32x4_t kw[kWinK], vw[kWinV];
-      auto key = [&](int i) __attribute__((always_inline)) {  // fragment i: keys of half i % 2, k-step i / 2
-        return *reinterpret_cast<const h_u32x4_t*>(base + klds + (i & 1) * 2 * kKBlock + (i >> 1) * 512);
-      };
+      h_u32x4_t vw[kWinV];
       auto value = [&](int i) __attribute__((always_inline)) {  // ... keys of step i / NV, rows of block i % NV
         return *reinterpret_cast<const h_u32x4_t*>(base + vlds + (i / NV) * kVBlock + (i % NV) * 1024);
       };
 #pragma unroll
-      for (int i = 0; i < kWinK; ++i) kw[i] = key(i);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
       for (int i = 0; i < 2 * KS; ++i) {
         s[i & 1] = mfma32(kw[i % kWinK], qf[i >> 1], s[i & 1]);
-        if (i + kWinK < 2 * KS) kw[i % kWinK] = key(i + kWinK);
+        if (i + kWinK < 2 * KS) kw[i % kWinK] = key(stage, i + kWinK);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -226,6 +241,8 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
 #pragma unroll
         for (int r = 0; r < 4; ++r) pf[j][r] = pack_bf16(s[j >> 1][8 * (j & 1) + 2 * r], s[j >> 1][8 * (j & 1) + 2 * r + 1]);
       __builtin_amdgcn_sched_barrier(0);
+      if (!published) publish(t + 1, after);
+      published = true;
 #pragma unroll
       for (int i = 0; i < 4 * NV; ++i) {
         o[i % NV] = mfma32(vw[i % kWinV], pf[i / NV], o[i % NV]);
@@ -235,7 +252,8 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
         }
       }
     }
-    stage = stage + 1 == S ? 0 : stage + 1;
+    if (!published) publish(t + 1, after);
+    stage = after;
   }
   if constexpr (MAPS == 2) __syncthreads();  // (the stages make room for the second map's results)
   l += __shfl_xor(l, 32);
