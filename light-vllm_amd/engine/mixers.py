@@ -158,8 +158,9 @@ class ParallelMixer:
         # softmax heads
         kc, vc = attn.split_kv_cache(cache.kv, self.kv_spec, step.block_size)
         q = amd.qk_norm_cache(lq, lk, lv, self.q_norm, self.k_norm, self.eps, a.heads, a.kv_heads, kc, vc, step.slot_mapping)
+        shortest = min(step.query_lens) if step.query_lens else 0  # (no short portions: no launch for them)
         amd.head_attention(both[:, :self.left_cols], q, kc, vc, step.block_tables, step.seq_lens, step.query_start_loc, lg,
-                           a.vdim, a.scale, self.cfg.left_scale, step.max_query_len, step.max_seq_len)
+                           a.vdim, a.scale, self.cfg.left_scale, step.max_query_len, step.max_seq_len, min_query_len=shortest)
         # gated linear attention
         self.recurrence(both[:, self.left_cols:cols], rq, rk, rv, u, rg, self.out_norm, self.cfg.right_scale,
                         r.dim ** -0.5, cache.state["matrix"], step)
