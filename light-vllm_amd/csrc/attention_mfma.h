@@ -711,8 +711,7 @@ __global__ __launch_bounds__((NWAVES + attn_extra_waves<ROPE, D>()) * 64,
       x[r] = y;
       m_loc = fmaxf(m_loc, y);
     }
-    m_loc = fmaxf(m_loc, __shfl_xor(m_loc, 16));
-    m_loc = fmaxf(m_loc, __shfl_xor(m_loc, 32));
+    m_loc = max_over_rows(m_loc);
     const float m_new = fmaxf(m_run, m_loc);
     const float alpha = __expf(m_run - m_new);
     m_run = m_new;

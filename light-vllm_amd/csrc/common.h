@@ -236,6 +236,12 @@ __device__ __forceinline__ LanePair<V> halves_apart(V v) {
   const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   return {__builtin_bit_cast(V, (unsigned)r[0]), __builtin_bit_cast(V, (unsigned)r[1])};
 }
+// The largest of lanes c, c + 16, c + 32 and c + 48, in registers: by way of LDS each of the two exchanges is a round trip.
+__device__ __forceinline__ float max_over_rows(float v) {
+  const auto h = halves_apart(v);
+  const auto r = rows_apart(fmaxf(h.a, h.b));
+  return fmaxf(r.a, r.b);
+}
 template <int L = 64, typename V, typename OP>
 __device__ __forceinline__ V over_lanes(V v, OP op) {  // over L = 16, 32 or 64 neighbouring lanes
   if constexpr (L == 64) {

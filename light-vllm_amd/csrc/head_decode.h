@@ -98,8 +98,7 @@ __global__ __launch_bounds__(256, 2) void head_decode_kernel(const HeadAttnParam
       s[r] = sees(p, key, pos, low) ? z : -FLT_MAX;
     }
     float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    mx = max_over_rows(mx);
     if (__any(mx > m)) {
       const float mn = fmaxf(m, mx), corr = exp2f(m - mn);
       m = mn;

@@ -135,8 +135,7 @@ __device__ __forceinline__ void latent_columns(const LatentAttnParams& p, const 
 #pragma unroll
     for (int r = 0; r < 4; ++r) s[r] = key0 + r <= pos && key0 + r >= low ? s[r] * sl : -FLT_MAX;
     float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    mx = max_over_rows(mx);
     if (g == 0) sm[ct][kg][c] = mx;
     lds_barrier();
     mx = fmaxf(fmaxf(sm[ct][0][c], sm[ct][1][c]), fmaxf(sm[ct][2][c], sm[ct][3][c]));
