@@ -375,7 +375,7 @@ __global__ void add_layer_norm_wave_kernel(typename T::store_t* out, const typen
 }
 
 // LayerNorm of the sum of an encoder's embeddings, T(T(word[id] + pos[position + shift]) + type), in one launch where the library takes six (two
-// gathers, three sums) and the norm one.  Bound by bytes: 16384 rows of 1024, 2 x 2 KiB gathered and 2 KiB written a row, 72 us before, 17
+// gathers, three sums) and the norm one.  Bound by bytes: 16384 rows of 1024, 2 x 2 KiB gathered and 2 KiB written a row, 72 us before, 20
 // now.  A row whose id or position is outside its table becomes NaN.
 template <typename T>
 __global__ void embed_layer_norm_kernel(typename T::store_t* __restrict__ out, const int64_t* __restrict__ ids,
