@@ -25,13 +25,14 @@ __device__ __forceinline__ void write_value_tile(char* smem, const int tile_of_r
   struct alignas(16) Eight { S e[8]; };
   constexpr int LD = kValueTile + 2;
   S* tile = reinterpret_cast<S*>(smem);  // [vdim][LD]
-  __shared__ int64_t slots[kValueTile];
+  __shared__ int64_t to[kValueTile];  // where a row's value of d = 0 goes (a 64-bit division is about 100 instructions: once a row)
   __shared__ int groups[kValueTile], num_groups;  // first row | length << 8
   const int row0 = tile_of_rows * kValueTile, nt = min(kValueTile, rows - row0), tid = threadIdx.x;
   if (tid < kValueTile) {
     int64_t s = tid < nt ? slot_mapping[row0 + tid] : -1;
     if (s >= num_slots) s = -1;
-    slots[tid] = s;
+    const int64_t blk = s / block_size;
+    to[tid] = blk * v_block_stride + (int64_t)head * vpad * block_size + (s - blk * block_size);
     const int64_t prev = (int64_t)__shfl_up((long long)s, 1);
     const bool first = s >= 0 && (tid == 0 || prev < 0 || s != prev + 1 || (s & 7) == 0);
     const uint64_t starts = __ballot(first), used = __ballot(s >= 0);
@@ -64,8 +65,7 @@ __device__ __forceinline__ void write_value_tile(char* smem, const int tile_of_r
   const int ng = num_groups;
   for (int i = tid; i < vpad * ng; i += 256) {
     const int d = i / ng, gr = groups[i - d * ng], t = gr & 0xff, len = gr >> 8;
-    const int64_t s = slots[t], b = s / block_size;
-    S* dst = value_cache + b * v_block_stride + ((int64_t)head * vpad + d) * block_size + (s - b * block_size);
+    S* dst = value_cache + to[t] + (int64_t)d * block_size;
     Eight e;
 #pragma unroll
     for (int j = 0; j < 8; ++j) e.e[j] = (d < vdim && j < len) ? tile[d * LD + t + j] : (S)0;
