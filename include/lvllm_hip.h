@@ -116,6 +116,11 @@ int lvllm_paged_attention_v2(
     int blocksparse_vert_stride, int blocksparse_block_size,
     int blocksparse_head_sliding_step, int64_t kv_cache_bytes, void* stream);
 
+/* Shares that paged_attention_v2 cuts each context into for these sizes (16-byte aligned operands, not block-sparse, "attn_splits" 0):
+ * slots 0 .. shares - 1 of the scratch are used, none with one share.  csrc/paged_shares.h is the rule. */
+int lvllm_paged_attention_v2_shares(int num_seqs, int num_heads, int num_kv_heads, int max_seq_len, int max_num_partitions, int dtype,
+                                    int kv_dtype);
+
 /* The two passes of paged_attention_v2 individually, for profiling and for the benchmark's
  * per-kernel timing: phases = 1 runs only the partition pass (writes tmp_out / exp_sums /
  * max_logits), 2 only the reduce pass (attention_kernels.cu:564-669), 3 both (== v2). */

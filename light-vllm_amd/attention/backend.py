@@ -296,19 +296,13 @@ class PagedAttnImpl:
 
     def make_v2_scratch(self, num_seqs: int, max_seq_len: int, dtype, device):
         """(exp_sums, max_logits, tmp_out) of paged_attn.py:156-166 for a caller that owns them."""
-        parts = self._v2_parts(max_seq_len)
+        parts = (max_seq_len + 511) // 512
         tmp = torch.empty(num_seqs, self.num_heads, parts, self.head_size, dtype=dtype, device=device)
         es = torch.empty(num_seqs, self.num_heads, parts, dtype=torch.float32, device=device)
         return es, torch.empty_like(es), tmp
 
-    @staticmethod
-    def _v2_parts(max_seq_len: int) -> int:
-        """Slots of a head: one per 512 tokens (what the operator asks for), and up to eight shares of 256 tokens, which a small
-        batch's contexts are cut into (csrc/attention.hip)."""
-        return max((max_seq_len + 511) // 512, min(max_seq_len // 256, 8))
-
     def _v2_scratch(self, num_seqs: int, max_seq_len: int, like: torch.Tensor):
-        parts = self._v2_parts(max_seq_len)
+        parts = (max_seq_len + 511) // 512
         # per stream: steps in flight on different streams (and the graphs captured on them)
         # must not share scratch
         key = (num_seqs, parts, torch.cuda.current_stream(like.device).cuda_stream)

@@ -6,6 +6,7 @@
 
 #include "attention_params.h"
 #include "common.h"
+#include "paged_shares.h"
 
 namespace lvllm {
 
@@ -374,25 +375,8 @@ static int paged_attention_v2_impl(
                       (q_stride * 2) % 16 == 0 && (kv_block_stride * kvb) % 16 == 0 &&
                       (kv_head_stride * kvb) % 16 == 0 && block_size >= 8;
   LV_CHECK(!p.kv_fp8 || vec_ok, "fp8 kv cache: operands must be 16-byte aligned");
-  // How many equal shares each context is cut into.  The reference always cuts at 512
-  // tokens; here the cut exists only to fill the GPU: as many shares as leave a CU to each workgroup, bounded by the
-  // caller's scratch (max_num_partitions slots per head) and by 256 tokens a share; no cut for up to 512 tokens, whose walk
-  // is shorter than the merge's launch.  More workgroups than CUs cost a second turn, which the last of them wait for.  One layer
-  // of 8 kv heads of 128, us, with as many shares as give 8 waves a CU and now: 1 sequence of 1024 13.1 (2 shares), 11.5 (4), of 4000 18.6 (4 of
-  // 512), 15.7 (8); 6 of 2000 16.9, 16.1; 12 of 1024 15.6, 15.6; 17 24.6, 17.2; 24 26.4, 19.6; 20 of 2000 39.0, 30.3; 300 tokens, 24 sequences,
-  // 512 in the table 17.3 with two shares, 10.0.
-  // Over an fp8 cache it is as many as give 8 waves a CU, one per 512 tokens at most (24 sequences of 1024 27.1, would be 24.2): what follows is rounded
-  // to 8 bits, which makes 0.11 of the logits (relative, four layers) of the last bit of a merge in other shares.
-  const int G = num_heads / num_kv_heads;
   const bool use_mfma = (dtype == LVLLM_BF16 || dtype == LVLLM_F16) && vec_ok && !bsparse;
-  const int64_t pairs = use_mfma ? (int64_t)num_seqs * num_kv_heads * ((G + 15) / 16)
-                                 : (int64_t)num_seqs * num_heads;
-  const int max_tiles = (max_seq_len + 15) / 16;
-  const bool by_cus = use_mfma && !p.kv_fp8;
-  const int64_t want = by_cus ? 256 / pairs : use_mfma ? (2048 + 8 * pairs - 1) / (8 * pairs) : (1024 + pairs - 1) / pairs;
-  const int slots = by_cus && max_seq_len > kPartitionSize ? max_num_partitions : (max_seq_len + kPartitionSize - 1) / kPartitionSize;
-  int nsplit = std::min((int)std::min<int64_t>(want, slots), max_tiles / (by_cus ? 16 : 4));
-  if (nsplit < 1) nsplit = 1;
+  int nsplit = paged_shares(num_seqs, num_heads, num_kv_heads, max_seq_len, max_num_partitions, use_mfma, p.kv_fp8);
   // lvllm_set_tuning("attn_splits", n): n >= 1 forces n shares (tests, experiments); -1 = the reference's
   // partitioning, 512 tokens per share whatever the batch, so that the scratch slots hold exactly what
   // attention_kernels.cu:349-357,483-495 stores in them
@@ -448,6 +432,13 @@ static int paged_attention_v2_impl(
 #undef LV_REDUCE
   LV_LAUNCH_CHECK();
   return 0;
+}
+
+extern "C" int lvllm_paged_attention_v2_shares(int num_seqs, int num_heads, int num_kv_heads, int max_seq_len, int max_num_partitions,
+                                               int dtype, int kv_dtype) {
+  if (num_seqs <= 0 || num_kv_heads <= 0 || num_heads < num_kv_heads) return 1;
+  return paged_shares(num_seqs, num_heads, num_kv_heads, max_seq_len, max_num_partitions, dtype == LVLLM_BF16 || dtype == LVLLM_F16,
+                      kv_dtype == LVLLM_KV_FP8_E4M3);
 }
 
 extern "C" int lvllm_paged_attention_v2_phases(

@@ -598,12 +598,13 @@ def test_add_layer_norm_matches_torch(ops, dtype, T, hidden, with_y):
     assert torch.equal(x2.view(torch.int16), out.view(torch.int16))
 
 
-@pytest.mark.parametrize("seqs", [1, 5, 11, 17, 33])
-@pytest.mark.parametrize("longest", [512, 513, 1300])
-def test_shares_by_the_batch(ops, seqs, longest):
-    """Contexts cut into as many shares as leave a CU to each workgroup (8 kv heads: 8 shares down to one), with slots for eight: what
-    shares longer and shorter than a sequence's leave empty, and the largest batch without a cut."""
-    lens = [max(1, longest - 37 * i) for i in range(seqs)]
+@pytest.mark.parametrize("seqs,longest,shares", [
+    (1, 512, 8), (5, 513, 7), (11, 512, 3), (16, 1024, 2), (17, 1024, 1), (31, 513, 1), (32, 1024, 1), (33, 513, 1),
+    (1, 1300, 8), (4, 2100, 8), (5, 2100, 7), (11, 1300, 3), (16, 1025, 2), (17, 1025, 2), (31, 1300, 2), (32, 1300, 1), (33, 1300, 1)])
+def test_shares_by_the_batch(ops, seqs, longest, shares):
+    """Contexts cut into eight shares down to one (8 kv heads, eight slots), with one short context that shares leave empty: the slots that a launch
+    fills are those of its shares, and none without a cut."""
+    lens = [longest] + [max(1, longest - 37 * i) for i in range(2, seqs)] + [17] * (seqs > 1)
     inp = make_paged_inputs(seqs, 16, 8, 64, 16, lens, dtype=torch.bfloat16, seed=seqs)
     d64 = dense_attention_fp64(inp)
     d = to_dev(inp)
@@ -612,6 +613,9 @@ def test_shares_by_the_batch(ops, seqs, longest):
     ops.paged_attention_v2(out, es, ml, tmp, d["query"], d["key_cache"], d["value_cache"], 8, inp["scale"], d["block_tables"], d["seq_lens"],
                            16, inp["max_seq_len"], None, "auto", 1.0, 1.0)
     check_attention(out, d64, d64)
+    filled = shares if shares > 1 else 0
+    assert torch.isfinite(es[0, :, :filled]).all() and es[0, :, filled:].isnan().all()
+    assert torch.isfinite(tmp[0, :, :filled].float()).all() and tmp[0, :, filled:].isnan().all()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
