@@ -213,10 +213,8 @@ def kernel_leg(engine, B, iters, seq_len=None):
     esz = 2
     algo_bytes = (2 * sum(lens) * KVH * D * (1 if kv_fp8 else esz) + 2 * len(seqs) * H * D * esz +
                   len(seqs) * ((max_len + BS - 1) // BS) * 4 + len(seqs) * 4)
-    # shares per context the library picks for this launch (attention.hip: want = ceil(2048 / (8 * pairs)),
-    # pairs = seqs * kv heads * ceil(G / 16)), for the label of the roofline object
-    pairs = len(seqs) * KVH * ((H // KVH + 15) // 16)
-    nsplit = max(1, min(P, (2048 + 8 * pairs - 1) // (8 * pairs), ((max_len + 15) // 16) // 4))
+    # shares per context the library picks for this launch, for the label of the roofline object
+    nsplit = lib.lvllm_paged_attention_v2_shares(len(seqs), H, KVH, max_len, P, dt, 1 if kv_fp8 else 0)
     return dict(avg_s=avg, min_s=min(ts), algo_bytes=algo_bytes, lens=lens, partitions=P, nsplit=nsplit)
 
 
