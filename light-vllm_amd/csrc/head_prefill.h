@@ -24,7 +24,9 @@
 // With three stages a tile's first fragments of K are read beside the last products of the one before.
 // us before these and now, same bits: one prompt of 4096, 16 heads over 4, 128 + 64, 104, 92 (95 with K's fragments read behind the barrier);
 // of 1000 29.4, 25.2; of 2000, 128 + 128, 59.5, 53.4; of 300 18.8, 14.4; two maps of 64 + 128, 2000 tokens 65, 61; 4 prompts of 2048, 16
-// heads, 192 + 128 (two stages) 140, 127; 3 of 777 35, 35.
+// heads, 192 + 128 (two stages) 140, 127; 3 of 777 35, 35.  Heads of up to 64 + 64 keep three workgroups a CU (64 + 32: four) by half as many
+// fragments of K ahead; 32 heads over 8 of 64 + 64, before, with two workgroups, now: 2300 tokens, a window of 256, 22.0, 23.6, 19.5; 3100, of
+// 1500, 54.9, 60.2, 51.1; 4096 101, 109, 97.
 #pragma once
 #include <float.h>
 
@@ -54,9 +56,11 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
 }
 
 constexpr int prefill_stages(int nk, int nv) { return 3 * 4 * (nk + nv) <= 80 ? 3 : 2; }
+// Workgroups a CU that LDS has room for, and registers with it.
+constexpr int prefill_workgroups(int nk, int nv) { return nk + nv <= 3 ? 4 : nk + nv <= 4 ? 3 : nk + nv <= 10 ? 2 : 1; }
 
 template <int NK, int NV, int MAPS>
-__global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kernel(const HeadAttnParams p) {
+__global__ __launch_bounds__(256, prefill_workgroups(NK, NV)) void head_prefill_kernel(const HeadAttnParams p) {
   constexpr int KP = 32 * NK, VP = 32 * NV, KS = 2 * NK / MAPS;  // KS: k-steps of a column
   constexpr int kPrefillCols = 128 / MAPS;                       // (token, head) pairs of a workgroup
   constexpr int kKBlock = KP * 16 * 2, kVBlock = VP * 16 * 2;  // bytes of a block's head slice
@@ -142,7 +146,8 @@ __global__ __launch_bounds__(256, NK + NV <= 10 ? 2 : 1) void head_prefill_kerne
   const int vlds = kImageK + lane * 16;  // (hi * 32 + lc) * 16
 
   constexpr int kCopies = NK + NV;  // of a wave and tile
-  constexpr int kWinK = 2 * KS < 8 ? 2 * KS : 8, kWinV = 4 * NV < 8 ? 4 * NV : 8;  // fragments read ahead of their MFMAs
+  // Fragments read ahead of their MFMAs; where more than two workgroups share a CU, which then have the registers of half of K's.
+  constexpr int kMostK = prefill_workgroups(NK, NV) > 2 ? 4 : 8, kWinK = 2 * KS < kMostK ? 2 * KS : kMostK, kWinV = 4 * NV < 8 ? 4 * NV : 8;
   __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // (the queries are here: what is on its way below are copies)
 #pragma unroll
   for (int t = 0; t < S - 1; ++t)
