@@ -15,7 +15,7 @@ Tuning& tuning() {
     if (const char* e = getenv("LVLLM_ATTN_WAVES")) v.attn_waves = atoi(e);
     if (const char* e = getenv("LVLLM_ATTN_SPLITS")) v.attn_splits = atoi(e);  // read once, at load
     if (const char* e = getenv("LVLLM_PREFILL_LDS")) v.prefill_lds = atoi(e);
-    if (const char* e = getenv("LVLLM_VARLEN_DENSE")) v.varlen_dense = atoi(e) != 0;
+    if (const char* e = getenv("LVLLM_VARLEN_DENSE")) v.varlen_dense = atoi(e) == 2 ? 2 : atoi(e) != 0;
     if (const char* e = getenv("LVLLM_VARLEN_DENSE_WAVES")) v.varlen_dense_waves = atoi(e) == 4 ? 4 : atoi(e) == 8 ? 8 : 0;
     if (const char* e = getenv("LVLLM_PREFILL_MFMA32_MIN_QUERY")) v.prefill_mfma32_min_query = atoi(e);
     if (const char* e = getenv("LVLLM_PREFILL_CHUNK_MAX_QUERY")) v.prefill_chunk_max_query = atoi(e);
@@ -44,7 +44,7 @@ extern "C" int lvllm_set_tuning(const char* key, int value) {
   } else if (k == "gemm_balance") {
     lvllm::tuning().gemm_balance = value != 0;
   } else if (k == "varlen_dense") {
-    lvllm::tuning().varlen_dense = value != 0;
+    lvllm::tuning().varlen_dense = value == 2 ? 2 : value != 0;
   } else if (k == "varlen_dense_waves") {
     LV_CHECK(value == 0 || value == 4 || value == 8, "varlen_dense_waves must be 0 (by the sizes), 4 or 8");
     lvllm::tuning().varlen_dense_waves = value;

@@ -1,5 +1,5 @@
 // Attention of whole sequences over the caller's row-major [token][KVH][64] rows (slices of a fused qkv projection), causal or not, without
-// a pack pass: heads of 64, 16-bit types (lvllm_varlen_attention; the paged kernels are prefill_mfma.h and prefill_mfma32.h).
+// a pack pass: heads of 64, 16-bit types (lvllm_varlen_attention, where lengths are alike or many: dense_rule.h).
 //
 // The arithmetic is that of prefill_mfma32.h, sum for sum: S^T = K Q^T and O^T += V^T P^T on 32x32x16 MFMAs, P never moving between lanes,
 // sums rescaled where a column's maximum grew by more than 2^6.  What differs is how a wave is kept busy:
@@ -20,7 +20,6 @@
 
 namespace lvllm {
 
-typedef short i16x4_t __attribute__((ext_vector_type(4)));
 constexpr int kDenseKeys = 64, kDenseHead = 64;       // keys of a tile, head size
 constexpr int kDenseRow = kDenseHead * 2;             // bytes of a row
 constexpr int kDenseImage = kDenseKeys * kDenseRow;   // of a tile's K or V
@@ -286,31 +285,18 @@ __global__ __launch_bounds__(256, CG == 2 ? 2 : 3) void dense_attention_kernel(c
   }
 }
 
-// Whether a launch of lvllm_varlen_attention can read the caller's rows directly ...
-inline bool dense_attention_takes(const PrefillParams& p, int head_size, int num_seqs, int max_query_len) {
-  return head_size == kDenseHead && !p.kv_fp8 && p.alibi_slopes == nullptr && p.softcap <= 0.f && p.sliding_window <= 0 &&
-         p.dense_k_bytes > 0 && p.dense_v_bytes > 0 && p.dense_k_bytes < ((int64_t)1 << 31) &&
-         p.dense_v_bytes < ((int64_t)1 << 31) && takes_mfma32(p, num_seqs, max_query_len);
-}
-// ... and the launch (block_tables = seq_lens = null: context == chunk)
+// What dense_mfma32_takes takes (block_tables = seq_lens = null: context == chunk), 128 or 256 columns a workgroup
 template <typename T>
-static int launch_dense_attention(const PrefillParams& p0, int num_seqs, int max_query_len, hipStream_t stream) {
+static int launch_dense_attention(const PrefillParams& p0, int num_seqs, int max_query_len, int columns, hipStream_t stream) {
   PrefillParams p = p0;
   const int G = p.num_heads / p.num_kv_heads, HG = (G + 31) / 32;
   p.gp_shift = G == 1 ? 0 : G == 2 ? 1 : G <= 4 ? 2 : G <= 8 ? 3 : G <= 16 ? 4 : 5;
-  // 256 columns a workgroup where walks are long and two workgroups a CU have work: 32 x 512 tokens 61.1 us for 62.1 with 128 columns, 8 x 2048
-  // 153 for 163, causal 93.3 for 94.2; but 24 x 400 37.4 for 35.9, 2 x 1024 (128 workgroups) 25.6 for 18.9, 32 x 512 causal 50.7 for 49.3.
   auto grid_of = [&](int columns) {
     const int tokens = columns >> p.gp_shift;
     return dim3(p.num_kv_heads * HG, num_seqs, (max_query_len + tokens - 1) / tokens);
   };
-  const dim3 wide = grid_of(256);
-  int columns = 32 * tuning().varlen_dense_waves;
-  if (columns == 0)
-    columns = max_query_len >= (p.causal ? 2048 : 512) && (int64_t)wide.x * wide.y * wide.z >= 512 ? 256 : 128;
-  const dim3 grid = columns == 256 ? wide : grid_of(128);
-  if (columns == 128) hipLaunchKernelGGL((dense_attention_kernel<T, 1>), grid, dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL((dense_attention_kernel<T, 2>), grid, dim3(256), 0, stream, p);
+  if (columns == 128) hipLaunchKernelGGL((dense_attention_kernel<T, 1>), grid_of(128), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((dense_attention_kernel<T, 2>), grid_of(256), dim3(256), 0, stream, p);
   return 0;
 }
 

@@ -4,6 +4,7 @@
 #include "../../include/lvllm_hip.h"
 #include "prefill_mfma32.h"
 #include "dense_attention.h"
+#include "dense_rule.h"
 #include "prefill_chunk.h"
 
 using namespace lvllm;
@@ -218,7 +219,7 @@ extern "C" int lvllm_varlen_attention(
            "workspace too small or misaligned (lvllm_varlen_attention_workspace_bytes)");
   hipStream_t s = (hipStream_t)stream;
   if (lvllm::tuning().varlen_dense) {
-    // long plain sequences: dense_attention.h reads the caller's rows itself: no pack pass
+    // long plain sequences: a body that reads the caller's rows itself (dense_rule.h): no pack pass
     PrefillParams p{};
     p.out = out; p.q = query; p.k_cache = key; p.v_cache = value; p.query_start_loc = cu_seqlens;
     p.num_heads = num_heads; p.num_kv_heads = num_kv_heads; p.max_num_blocks_per_seq = 1; p.max_block = 0;
@@ -228,11 +229,18 @@ extern "C" int lvllm_varlen_attention(
     p.dense_k_stride = k_stride; p.dense_v_stride = v_stride;
     p.dense_k_bytes = ((int64_t)(num_tokens - 1) * k_stride + (int64_t)num_kv_heads * head_size) * 2;
     p.dense_v_bytes = ((int64_t)(num_tokens - 1) * v_stride + (int64_t)num_kv_heads * head_size) * 2;
-    if (dense_attention_takes(p, head_size, num_seqs, max_seq_len)) {
+    if (dense_mfma32_takes(p, head_size, num_seqs, max_seq_len)) {
       LV_CHECK((((uintptr_t)query | (uintptr_t)out) & 15) == 0 && (q_stride * 2) % 16 == 0 && (out_stride * 2) % 8 == 0,
                "operands must be 16-byte aligned");
-      const int rc = dtype == LVLLM_BF16 ? launch_dense_attention<BF16>(p, num_seqs, max_seq_len, s)
-                                         : launch_dense_attention<F16>(p, num_seqs, max_seq_len, s);
+      const int waves = tuning().varlen_dense_waves;
+      const DenseBody body = tuning().varlen_dense == 2 ? kDenseWaves : waves ? waves == 8 ? kDense256 : kDense128
+                             : dense_body(num_seqs, num_tokens, max_seq_len, num_heads, num_kv_heads, causal != 0);
+      auto launch = [&](auto type) {
+        using T = decltype(type);
+        return body == kDenseWaves ? launch_prefill_mfma32_dense<T>(p, head_size, num_seqs, max_seq_len, s)
+                                   : launch_dense_attention<T>(p, num_seqs, max_seq_len, body == kDense256 ? 256 : 128, s);
+      };
+      const int rc = dtype == LVLLM_BF16 ? launch(BF16{}) : launch(F16{});
       if (rc) return rc;
       LV_LAUNCH_CHECK();
       return 0;

@@ -69,7 +69,7 @@ struct PrefillParams {
   int num_tokens;  // rows of `query` the caller states (0: unknown)
   void* workspace;
   int64_t workspace_bytes;
-  // the dense twin of the 32x32 body (dense_attention.h): k_cache / v_cache are row-major [token][KVH][D] rows
+  // the dense twins of the 32x32 body (dense_rule.h): k_cache / v_cache are row-major [token][KVH][D] rows
   // of the caller (token strides in elements), readable for dense_k_bytes / dense_v_bytes from their bases
   int64_t dense_k_stride, dense_v_stride, dense_k_bytes, dense_v_bytes;
 };

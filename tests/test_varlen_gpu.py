@@ -151,6 +151,34 @@ def test_rows_read_in_place_by_columns_of_a_workgroup(ops, causal, H, KVH):
         assert torch.equal(o.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("H,KVH", [(2, 2), (8, 1), (40, 1)])
+@pytest.mark.parametrize("seqs", [2, 65, 300])
+def test_long_sequences_among_short_ones(ops, causal, H, KVH, seqs):
+    """Every body that reads rows in place, and the one that the sizes choose, where long sequences stand first, last and between short and empty
+    ones: the bits of the pack pass, and no other rows."""
+    D, lens = 64, [(7 * i) % 6 for i in range(seqs)]
+    for i, n in ((0, 300), (seqs // 2, 129), (seqs - 1, 514)):
+        lens[i] = n
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32, device=DEV)
+    T = int(cu[-1])
+    qkv = torch.randn(T, (H + 2 * KVH) * D, generator=torch.Generator().manual_seed(seqs)).bfloat16().to(DEV)
+    q, k, v = (x.unflatten(1, (-1, D)) for x in qkv.split([H * D, KVH * D, KVH * D], dim=1))
+    outs = []
+    for dense, waves in ((0, 0), (1, 0), (1, 4), (1, 8), (2, 0), (2, 4), (2, 8)):
+        torch.ops._C_amd.set_tuning("varlen_dense", dense)
+        torch.ops._C_amd.set_tuning("varlen_dense_waves", waves)
+        try:
+            outs.append(torch.full((T + 1, H, D), 9., dtype=torch.bfloat16, device=DEV))
+            ops.varlen_attention(outs[-1][:T], q, k, v, cu, max(lens), D ** -0.5, causal)
+        finally:
+            torch.ops._C_amd.set_tuning("varlen_dense", 1)
+            torch.ops._C_amd.set_tuning("varlen_dense_waves", 0)
+    assert (outs[0][:T] != 9.).any(dim=2).all()
+    for o in outs[1:]:
+        assert torch.equal(o.view(torch.int16), outs[0].view(torch.int16))
+
+
 def test_rows_read_in_place_with_different_key_and_value_strides(ops):
     """K and V of different buffers, different token strides, V not at the start of its rows: the in-place launch
     takes each operand's own stride and base (bit-identical to the pack pass, as above)."""
