@@ -37,7 +37,13 @@ inline int64_t wide_time(int64_t units, int groups, int k, int act) {
 }
 
 // The shortest of these; `row_major`, `packed`: the orders of the weights that are there.  Nothing where the half tiles are too few to fill
-// half of the chip: the library cuts K then.  us, library and activation, then this:
+// half of the chip: the library cuts K then.  Nor where its products are the better ones, of 1750 random sizes of 65 to 9000 rows:
+//   * k > 5120: 0.71 to 1.23 of the library and the activation, whatever the rest.  (Up to 256 rows of k >= 8192 have a kernel of their own,
+//     stream_gemm_kernel, which is ahead of both: SwiGLU of 8192, 100 rows 68.5 us, here 92.5.)
+//   * 2048 < k: tiles that are filled to less than 0.6 of what MFMAs do in the time, but for half tiles that take most of the CUs once, 0.94 to
+//     1.22 (SwiGLU of 9728, 2560 wide, 214 rows 47.8, 52.4; of 18944, 3584 wide, 89 rows 80, 88; of 14336, 4096 wide, 129 rows 74, 82);
+//   * GELU from k = 1025 on, to less than 0.7, with the same exception: 0.8 to 1.12.
+// What is left takes 0.46 to 1.09 of the two (1000 other sizes, three above 1.03), mean 0.84.  us, the two launches, then this:
 //   * SwiGLU of 14336, 4096 wide: 65 rows 58, 45; 300 88, 84; 700 163, 144; 1000 206, 195; 2000 382, 376; 3000 575, 515; 4875 990, 855; 8192 1398,
 //     1346; of 11264, 2048 wide: 128 rows 32, 27; 700 99, 77; 1000 106, 85; 2000 193, 164; 4096 402, 320; 8192 634, 577;
 //   * the clamped unit of 5632, 2048 wide: 100 rows (88 half tiles) 21.1, 23.0; 200 30.6, 22.7; 300 32.6, 27.2; 512 39, 34; 1000 58, 55; 2000 99, 88;
@@ -45,11 +51,12 @@ inline int64_t wide_time(int64_t units, int groups, int k, int act) {
 //   * squared ReLU of 8448, 2048 wide: 100 rows (66) 19.4, 20.8; 300 27.9, 21.4; 700 37.7, 31.1; 1000 43.6, 40.4; 4096 141, 120; 8192 311, 223;
 //   * GELU of 4096, 1024 wide: 100 rows (32) 11.7, 12.3; 300 (96) 13.9, 12.6; 1000 20.8, 14.2; 3000 37.3, 31.8; 16384 164, 131.  Its
 //     instructions run beside another tile's MFMAs, where a wide tile (149) has nobody beside it.
+// (Cards differ: one measured 154 and 125 for the last, and 891 + 73 and 842 for 4875 rows of SwiGLU.)
 inline PromptLinearPlan prompt_linear_plan(int rows, int outputs, int k, int act, bool row_major, bool packed) {
   PromptLinearPlan plan{LVLLM_PROMPT_NONE, 0, 0};
   const int64_t wrows = (int64_t)outputs * (prompt_pairs(act) ? 2 : 1);
   const bool gelu = act == LVLLM_ACT_GELU;
-  if (rows <= 64 || outputs < 128 || outputs % 16 != 0 || wrows * k >= (int64_t)1 << 30) return plan;
+  if (rows <= 64 || outputs < 128 || outputs % 16 != 0 || k > 5120 || wrows * k >= (int64_t)1 << 30) return plan;
   const int64_t tiles = (rows + 127) / 128, half = tiles * ((wrows + 127) / 128);
   if (half < (gelu ? 96 : 128)) return plan;
   int64_t best = 0;
@@ -62,6 +69,10 @@ inline PromptLinearPlan prompt_linear_plan(int rows, int outputs, int k, int act
     take(LVLLM_PROMPT_TILE, 0, 4, tile_time(tiles * ((wrows + 255) / 256), 4, k));
     take(LVLLM_PROMPT_TILE, 0, 2, tile_time(half, 2, k));
   }
+  // What 2^23 products of rows with W rows, one whole tile a CU, take at the rate of full tiles is 80 of tile_time.
+  auto filled = [&](int most) { return best << 23 <= (int64_t)rows * wrows * most; };
+  const bool once = plan.body == LVLLM_PROMPT_TILE && plan.nt == 2 && half >= 160 && half <= 256;
+  if (!once && (gelu ? k > 1024 && !filled(114) : k > 2048 && !filled(132))) plan = {LVLLM_PROMPT_NONE, 0, 0};
   return plan;
 }
 

@@ -40,6 +40,10 @@ MEASURED = [  # rows, outputs, k, activation -> body, groups or blocks
     (300, 14336, 4096, SILU, WIDE, 3), (65, 14336, 4096, SILU, TILE, 2), (1000, 11264, 2048, SILU, TILE, 4), (128, 11264, 2048, SILU, TILE, 2),
     (4096, 5632, 2048, CLAMPED, TILE, 4), (300, 5632, 2048, CLAMPED, TILE, 2), (100, 5632, 2048, CLAMPED, NONE, 0),
     (4096, 8448, 2048, RELU2, WIDE, 3), (1000, 8448, 2048, RELU2, WIDE, 3), (300, 8448, 2048, RELU2, TILE, 2),
+    # where the library or the stream product is faster
+    (100, 8192, 8192, SILU, NONE, 0), (257, 8192, 8192, SILU, NONE, 0), (700, 4096, 12288, SILU, NONE, 0), (2000, 14336, 8192, CLAMPED, NONE, 0),
+    (129, 14336, 4096, SILU, NONE, 0), (89, 18944, 3584, SILU, NONE, 0), (214, 9728, 2560, SILU, NONE, 0), (916, 5136, 3776, RELU2, NONE, 0),
+    (128, 16384, 4096, RELU2, NONE, 0), (257, 16384, 4096, RELU2, NONE, 0), (221, 10064, 3456, CLAMPED, NONE, 0), (517, 17184, 1920, GELU, NONE, 0),
     (100, 8448, 2048, RELU2, NONE, 0), (16384, 4096, 1024, GELU, TILE, 4), (1000, 4096, 1024, GELU, TILE, 2), (100, 4096, 1024, GELU, NONE, 0)]
 
 
@@ -52,7 +56,7 @@ def test_measured_sizes(plan, rows, outputs, k, act, body, size):
 def test_any_size(plan):
     rng = random.Random(0)
     for _ in range(20000):
-        rows, outputs, k = rng.randint(1, 40000), rng.choice([8, 16]) * rng.randint(1, 2000), rng.choice([8, 32, 64]) * rng.randint(1, 128)
+        rows, outputs, k = rng.randint(1, 40000), rng.choice([8, 16]) * rng.randint(1, 2000), rng.choice([8, 32, 64, 65536]) * rng.randint(1, 128)
         act, row_major, packed = rng.choice([GELU, SILU, RELU2, CLAMPED]), rng.random() < 0.5, rng.random() < 0.5
         body, size = plan(rows, outputs, k, act, row_major, packed)
         if body == WIDE:
@@ -60,4 +64,4 @@ def test_any_size(plan):
         elif body == TILE:
             assert packed and k % 32 == 0 and outputs % 16 == 0 and size in (2, 4)
         if body != NONE:
-            assert rows > 64 and outputs * k * (2 if act in (SILU, CLAMPED) else 1) * 2 < 2 ** 31
+            assert rows > 64 and outputs * k * (2 if act in (SILU, CLAMPED) else 1) * 2 < 2 ** 31 and 256 * k * 2 < 2 ** 31
