@@ -3,8 +3,8 @@
 
 namespace lvllm {
 
-// x Phi(x): Phi as a sigmoid of an odd polynomial, which a least-maximum fit gave (largest error of the result 6.7e-8, where
-// 1 + erf(x / sqrt(2)) in 32 bits has 1.2e-7 by itself).  13 instructions; erff is 40.
+// x Phi(x): Phi as a sigmoid of an odd polynomial, which a least-maximum fit gave (largest error of the result 6.7e-8 before any rounding; with those of
+// 32 bits 1.0e-7 for x < 0, 4.9e-7 up to 4, 5.9e-7 up to 8, where x / 2 (1 + erf) has 0.8e-7, 2.9e-7 and 4.5e-7).  13 instructions; erff is 40.
 __device__ __forceinline__ float gelu_of(float x) {
   const float t = x * x;
   float p = 5.20991372e-09f;

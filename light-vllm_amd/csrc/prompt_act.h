@@ -5,16 +5,17 @@
 namespace lvllm {
 
 // x / (1 + e^-x) to the last bit or so: what the product with log2(e) loses goes into the power behind it, and a Newton step takes the
-// reciprocal's error.  The power is taken between +-87; below, the sigmoid is 0 to any bit that x could bring back.
+// reciprocal's error.  Below -88.72 e^-x has no place in 32 bits and x / (1 + expf(-x)) is -0, as here; above, a quarter of 1 + e^-x keeps the
+// reciprocal among the normal numbers, which the hardware's needs.
 __device__ __forceinline__ float prompt_silu(float x) {
-  const float y = -__builtin_amdgcn_fmed3f(x, -87.f, 87.f), t = y * 1.44269504f;
+  const float y = -__builtin_amdgcn_fmed3f(x, -88.72f, 87.f), t = y * 1.44269504f;
   const float lost = fmaf(y, 1.92596303e-08f, fmaf(y, 1.44269504f, -t));
   float e = __builtin_amdgcn_exp2f(t);
   e = fmaf(e, lost * 0.693147181f, e);
-  const float d = 1.f + e;
+  const float d = fmaf(e, 0.25f, 0.25f);
   float r = __builtin_amdgcn_rcpf(d);
   r = fmaf(fmaf(-d, r, 1.f), r, r);
-  return x * (x < -87.f ? 0.f : r);
+  return (x * 0.25f) * (x < -88.72f ? 0.f : r);
 }
 
 template <int ACT>
