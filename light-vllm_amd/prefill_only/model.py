@@ -116,9 +116,10 @@ class EncoderModel:
                 return h
             return F.gelu(h)
 
-        if fused and hid <= 2048 and input_ids.dtype == positions.dtype == torch.int64:  # (one launch: csrc/layernorm.hip)
+        if (fused and hid <= 2048 and input_ids.dtype == positions.dtype == torch.int64 and self.word_emb.is_contiguous()
+                and self.pos_emb.is_contiguous()):  # (one launch: csrc/layernorm.hip)
             x = torch.ops._C_amd.embed_layer_norm(input_ids.contiguous(), positions.contiguous(), shift, self.word_emb, self.pos_emb,
-                                                  self.type_emb, *self.emb_ln, eps)
+                                                  self.type_emb[0], *self.emb_ln, eps)
         else:
             x = F.embedding(input_ids, self.word_emb) + F.embedding(positions + shift, self.pos_emb) + self.type_emb[0]
             x = add_ln(x, None, self.emb_ln)

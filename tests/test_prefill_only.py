@@ -142,6 +142,27 @@ def encoder_prompts():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tables", ["two types", "strided"])
+def test_embedding_tables(tables):
+    """A table of two types, of which the first is taken, and tables that are parts of wider ones."""
+    from light_vllm_amd.attention.prefill_only import PrefillOnlyAttentionMetadata
+    from light_vllm_amd.prefill_only.model import EncoderConfig, EncoderModel
+    model = EncoderModel(EncoderConfig.tiny(), DEV, 0)
+    ids = torch.randint(2, 512, (100,), generator=torch.Generator().manual_seed(3)).to(DEV)
+    md = PrefillOnlyAttentionMetadata(100, [100], torch.tensor([0, 100], dtype=torch.int32, device=DEV))
+
+    def run():
+        with torch.inference_mode():
+            return model.forward(ids, torch.arange(100, device=DEV), md)
+    first = run()
+    if tables == "two types":
+        model.type_emb = torch.cat([model.type_emb, model.type_emb + 1])
+    else:
+        model.word_emb, model.pos_emb = (torch.cat([t, t], dim=1)[:, :128] for t in (model.word_emb, model.pos_emb))
+    assert torch.equal(run(), first)
+
+
+@pytest.mark.gpu
 def test_encoder_engine_matches_fp32_reference():
     eng = make_encoder(pooling="last_hidden_states")
     ps = encoder_prompts()
