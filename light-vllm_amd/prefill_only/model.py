@@ -9,7 +9,7 @@ exact GELU leaves the projection in front of it (csrc/tile_linear.hip) or is an 
 are library GEMMs (prompt batches are hundreds to thousands of rows).
 Weights are random-initialised: no checkpoint is available offline."""
 from dataclasses import dataclass
-from typing import List
+from typing import List, Optional
 
 import torch
 import torch.nn.functional as F
@@ -64,11 +64,24 @@ class EncoderLayerWeights:
         self.out_w, self.out_b = w(hid, hid), w(hid)
         self.attn_ln = ln()
         self.fc1_w, self.fc1_b = w(inter, hid), w(inter)
-        # once more in fragment order, for the kernel with GELU behind the product
-        pack = self.fc1_w.is_cuda and cfg.dtype == torch.bfloat16 and inter % 16 == 0 and hid % 32 == 0
-        self.fc1_packed = torch.ops._C_amd.pack_weight(self.fc1_w) if pack else None
         self.fc2_w, self.fc2_b = w(hid, inter), w(hid)
         self.out_ln = ln()
+        self._fused, self._fc1_packed = cfg.fused_layer_norm, None
+        self.fc1_packed  # (laid out now, and not in the first forward)
+
+    @property
+    def fc1_packed(self) -> Optional[torch.Tensor]:
+        """fc1_w once more in fragment order, for the kernel with GELU behind the product (None: what it does not take).  Laid out anew when
+        fc1_w has been replaced or written to since.  Writes that torch does not count (`fc1_w.data.copy_`, or to inference tensors) are not
+        seen: assign fc1_w behind those."""
+        w = self.fc1_w
+        if not (self._fused and w.is_cuda and w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[0] % 16 == 0 and w.shape[1] % 32 == 0):
+            return None
+        version = -1 if w.is_inference() else w._version
+        was = self._fc1_packed  # (fc1_w, its memory, which nothing else can have meanwhile, and its version then, the copy)
+        if was is None or was[0] is not w or was[1].data_ptr() != w.data_ptr() or was[2] != version:
+            was = self._fc1_packed = w, w.detach(), version, torch.ops._C_amd.pack_weight(w)
+        return was[3]
 
 
 class EncoderModel:
@@ -106,8 +119,9 @@ class EncoderModel:
             return F.layer_norm(a if b is None else a + b, (hid,), ln[0], ln[1], eps)
 
         def fc1_gelu(a, lw):
-            if fused and lw.fc1_packed is not None:
-                h = torch.ops._C_amd.prompt_linear(a, None, lw.fc1_packed, lw.fc1_b, cfg.intermediate_size, PROMPT_ACTS["gelu"])
+            packed = lw.fc1_packed if fused else None
+            if packed is not None:
+                h = torch.ops._C_amd.prompt_linear(a, None, packed, lw.fc1_b, cfg.intermediate_size, PROMPT_ACTS["gelu"])
                 if h is not None:
                     return h
             h = F.linear(a, lw.fc1_w, lw.fc1_b)

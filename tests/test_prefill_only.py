@@ -163,6 +163,41 @@ def test_embedding_tables(tables):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("how", ["assigned", "copied", "in a part", "by storage"])
+def test_weights_that_come_after_the_model(how):
+    """Weights assigned or written into a model that has been used are the ones that its next forward takes."""
+    from light_vllm_amd.attention.prefill_only import PrefillOnlyAttentionMetadata
+    from light_vllm_amd.prefill_only.model import EncoderConfig, EncoderModel
+    cfg = EncoderConfig(hidden_size=1024, intermediate_size=4096, num_hidden_layers=1, num_attention_heads=16, vocab_size=512,
+                        max_position_embeddings=1024)
+    lens = [500, 300, 400]  # (rows that the kernel with GELU behind the product takes)
+    model, other = (EncoderModel(cfg, DEV, seed) for seed in (0, 1))
+    ids = torch.randint(2, 512, (sum(lens),), generator=torch.Generator().manual_seed(3)).to(DEV)
+    pos = torch.cat([torch.arange(n) for n in lens]).to(DEV)
+    starts = torch.tensor([0, 500, 800, 1200], dtype=torch.int32, device=DEV)
+    md = PrefillOnlyAttentionMetadata(max(lens), lens, starts)
+
+    def run():
+        with torch.inference_mode():
+            return model.forward(ids, pos, md)
+    first, lw, new = run(), model.layers[0], other.layers[0].fc1_w
+    if how == "assigned":
+        lw.fc1_w = new
+    elif how == "copied":
+        lw.fc1_w.copy_(new)
+    elif how == "in a part":
+        lw.fc1_w[:2048].copy_(new[:2048])
+    else:
+        lw.fc1_w.data = new
+    got = run()
+    model.cfg.fused_layer_norm = False  # (the library's product and GELU)
+    want = run()
+    assert not torch.equal(got, first)
+    assert (got.float() - want.float()).norm() < 1e-2 * want.float().norm()
+    assert (first.float() - want.float()).norm() > 5e-2 * want.float().norm()
+
+
+@pytest.mark.gpu
 def test_encoder_engine_matches_fp32_reference():
     eng = make_encoder(pooling="last_hidden_states")
     ps = encoder_prompts()
