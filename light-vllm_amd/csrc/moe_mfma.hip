@@ -187,21 +187,20 @@ __device__ __forceinline__ void tile_product(const MoeParams& p, const TileWork&
                     });
 }
 
-template <int PRODUCT, int NT>
+// EVERY: a body per height in groups of 16 slots, from four on, for launches that power bounds, where products with slots that are not there cost as
+// much as others (takes_every_height, moe_turns.h); else bodies of 4, 6 and 8.
+template <int PRODUCT, int NT, bool EVERY>
 __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const MoeParams p, const int blocks_first, const int blocks_last) {
   __shared__ __attribute__((aligned(16))) char ring[tile_steps(NT) / 2][kStageBytes];
   const TileWork t = tile_work<PRODUCT, kMoeTile, 4 * NT>(p, blocks_first, blocks_last);
   if (!t.any) return;
-  // a body per height in groups of 16 slots, from four on: where power bounds the launch, products with slots that are not there cost as
-  // much as others.  Up + down, us, with bodies of 4, 6 and 8 groups and with these: 4096 rows, 6 of 64 experts of 2816 (tiles of 96 to 112 slots)
-  // 900, 876; 8192 rows 1548, 1538; 1300 rows, 2 of 32 of 1408 and a shared one (up) 104, 97; others 1.00 to 1.02.
   const int groups = (t.s1 - t.s0 + 15) >> 4;
   auto go = [&](auto once) __attribute__((always_inline)) {
     constexpr bool O = decltype(once)::value;
     if (groups <= 4) tile_product<PRODUCT, O, NT, 4>(p, t, ring);
-    else if (groups == 5) tile_product<PRODUCT, O, NT, 5>(p, t, ring);
-    else if (groups == 6) tile_product<PRODUCT, O, NT, 6>(p, t, ring);
-    else if (groups == 7) tile_product<PRODUCT, O, NT, 7>(p, t, ring);
+    else if (EVERY && groups == 5) tile_product<PRODUCT, O, NT, EVERY ? 5 : 6>(p, t, ring);
+    else if (groups <= 6) tile_product<PRODUCT, O, NT, 6>(p, t, ring);
+    else if (EVERY && groups == 7) tile_product<PRODUCT, O, NT, EVERY ? 7 : 8>(p, t, ring);
     else tile_product<PRODUCT, O, NT, 8>(p, t, ring);
   };
   if (t.once) go(std::true_type{});
@@ -419,14 +418,16 @@ static void go(const MoeParams& p, hipStream_t s) {
     const int64_t last_tiles = (p.rows + least - 1) / least;  // a token takes an expert once
     auto blocks = [&](int nt, int ff) { return ((GATED ? ff / 8 : (UP ? ff : p.width) / 16) + 4 * nt - 1) / (4 * nt); };
     const BlockCounts whole{blocks(4, p.ff_first), blocks(4, p.ff_last)}, half{blocks(2, p.ff_first), blocks(2, p.ff_last)};
-    auto launch = [&](auto nt, const BlockCounts& b) {
+    auto launch = [&](auto nt, auto every, const BlockCounts& b) {
       const unsigned grid = (unsigned)unit_workgroups(tiles * b.first, last_tiles * b.last);
-      hipLaunchKernelGGL((moe_tile_kernel<PRODUCT, decltype(nt)::value>), dim3(grid), dim3(256), 0, s, p, b.first, b.last);
+      hipLaunchKernelGGL((moe_tile_kernel<PRODUCT, decltype(nt)::value, decltype(every)::value>), dim3(grid), dim3(256), 0, s, p, b.first, b.last);
     };
     if (takes_half_blocks(p.rows, p.slots, p.experts, least, whole, half, UP, p.ff_last > p.ff_first))
-      launch(std::integral_constant<int, 2>{}, half);
+      launch(std::integral_constant<int, 2>{}, std::false_type{}, half);
+    else if (takes_every_height(p.rows, p.slots, p.experts, least, whole))
+      launch(std::integral_constant<int, 4>{}, std::true_type{}, whole);
     else
-      launch(std::integral_constant<int, 4>{}, whole);
+      launch(std::integral_constant<int, 4>{}, std::false_type{}, whole);
   }
 }
 

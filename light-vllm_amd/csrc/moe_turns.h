@@ -34,6 +34,20 @@ struct BlockCounts {
   int first, last;
 };
 
+// Workgroups that slots spread evenly over all experts make.
+inline int64_t even_workgroups(int rows, int64_t slots, int experts, int tile, const BlockCounts& b) {
+  const int64_t even = (slots + (int64_t)experts * tile - 1) / ((int64_t)experts * tile), last = ((int64_t)rows + tile - 1) / tile;
+  return experts * even * b.first + last * b.last;
+}
+
+// Whether whole blocks have a body for each height of a tile: more workgroups than two a CU, which power bounds.  With bodies of 4, 6 and 8 groups of 16
+// slots, then of every height, us going up: 4096 rows, 6 of 64 experts of 2816, 2048 wide 612, 594; 3000 rows, 6 of 64 of 1408 and a shared one of
+// 2816 312, 301; 8192 rows, 2 of 32 of 1408 and a shared one 294, 285.  Fewer workgroups wait for memory, and a launch with more code takes longer:
+// 2500 rows, 2 of 16 of 512, 1024 wide (192) 28.3, 30.0; 1300 rows, 2 of 8 of 1024 (192) 27.9, 29.5; 1500 rows, 4 of 32 of 512 (256) 31.1, 31.9.
+inline bool takes_every_height(int rows, int64_t slots, int experts, int tile, const BlockCounts& whole) {
+  return even_workgroups(rows, slots, experts, tile, whole) > 512;
+}
+
 // Whether a prompt's products take half blocks (128 W rows) or whole ones, by the workgroups with work that slots spread evenly over
 // the experts make.  `larger_last`: the last expert is larger, a shared one then, which has every row.  A half block's walk takes three
 // quarters of a whole one's where a workgroup has a CU to itself, and where two share one no less than a whole one that has none beside
@@ -55,8 +69,7 @@ inline bool takes_half_blocks(int rows, int64_t slots, int experts, int tile, co
     return unit_workgroups((experts - 1) * each * b.first, (shared ? last_tiles : each) * b.last);
   };
   if (workgroups(half, true) <= 256 || (!larger_last && workgroups(half, false) <= 256)) return true;
-  const int64_t even = (slots + (int64_t)experts * tile - 1) / ((int64_t)experts * tile);
-  if (experts * even * whole.first + last_tiles * whole.last > 384) return false;
+  if (even_workgroups(rows, slots, experts, tile, whole) > 384) return false;
   return (!up && larger_last) || workgroups(whole, larger_last) > 256;
 }
 

@@ -29,7 +29,7 @@ def test_products(amd, counts, ff, width, act, weigh):
     of_row = torch.repeat_interleave(torch.arange(experts), torch.tensor(counts))[torch.randperm(rows, generator=torch.Generator().manual_seed(1))]
     h = 0.5 * rand(rows, width, seed=2)
     h[:, :experts] = 0.25 * torch.nn.functional.one_hot(of_row, experts).bfloat16()
-    router = torch.zeros(16, width, dtype=torch.bfloat16)  # the expert of a row is the column that it marks
+    router = torch.zeros(-(-experts // 16) * 16, width, dtype=torch.bfloat16)  # the expert of a row is the column that it marks
     router[:experts, :experts] = 8 * torch.eye(experts)
     gate, up = ([rand(n, width, seed=s + i) * width ** -0.5 for i, n in enumerate(ff)] for s in (10, 30))
     down = [rand(width, n, seed=50 + i) * n ** -0.5 for i, n in enumerate(ff)]
@@ -79,12 +79,18 @@ def test_products_of_few_rows(amd, counts, full, width, act):
 
 
 @pytest.mark.parametrize("act", ["clamped", "relu_squared"])
-@pytest.mark.parametrize("ff", [160, 8320], ids=["half blocks", "whole blocks"])
+@pytest.mark.parametrize("ff", [160, 8320, 20480], ids=["half blocks", "whole blocks", "bodies of every height"])
 @pytest.mark.parametrize("tiles", [1, 2], ids=["single tiles", "two tiles"])
 def test_tiles_of_every_height(amd, tiles, ff, act):
     """Tiles of 65 to 128 slots in groups of 16, at both ends of each height."""
     heights = [65, 80, 81, 96, 97, 112, 113]
     test_products(amd, [tiles * n for n in heights], [ff] * 6 + [ff + 32], 160, act, False)
+
+
+@pytest.mark.parametrize("tiles", [1, 2], ids=["single tiles", "two tiles"])
+def test_tiles_of_every_height_going_down(amd, tiles):
+    """The same where the products going down have a body for each height (70 experts of 10 blocks)."""
+    test_products(amd, [tiles * n for n in [65, 80, 81, 96, 97, 112, 113]] * 10, [96] * 70, 2400, "clamped", False)
 
 
 @pytest.mark.parametrize("act", [0, 2], ids=["clamped", "relu_squared"])

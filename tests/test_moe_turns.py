@@ -28,6 +28,9 @@ extern "C" long single(long units_first, long units_last) { return unit_workgrou
 extern "C" int half(int rows, long slots, int experts, int first4, int last4, int first2, int last2, int up, int larger) {
   return takes_half_blocks(rows, slots, experts, 128, {first4, last4}, {first2, last2}, up, larger);
 }
+extern "C" int every(int rows, long slots, int experts, int first4, int last4) {
+  return takes_every_height(rows, slots, experts, 128, {first4, last4});
+}
 """
 
 
@@ -40,6 +43,7 @@ def lib(tmp_path_factory):
     t = ctypes.CDLL(str(d / "t.so"))
     t.single.restype = ctypes.c_long
     t.half.argtypes = [ctypes.c_int, ctypes.c_long] + [ctypes.c_int] * 7
+    t.every.argtypes = [ctypes.c_int, ctypes.c_long] + [ctypes.c_int] * 3
     t.single.argtypes = [ctypes.c_long] * 2
     return t
 
@@ -80,3 +84,13 @@ def test_half_blocks(lib, rows, top, experts, ff, shared, width, up, down):
         got = lib.half(rows, slots, all_experts, blocks(tiles(ff), 4), blocks(tiles(last), 4), blocks(tiles(ff), 2), blocks(tiles(last), 2),
                        is_up, last > ff)
         assert want is None or bool(got) == want
+
+
+@pytest.mark.parametrize("rows,top,experts,ff,shared,up", [
+    (4096, 6, 64, 2816, 0, True), (3000, 6, 64, 1408, 2816, True), (8192, 2, 32, 1408, 1408, True), (1943, 6, 64, 1408, 2816, True),
+    (2500, 2, 16, 512, 0, False), (1300, 2, 8, 1024, 0, False), (1500, 4, 32, 512, 0, False), (2000, 2, 8, 512, 0, False)])
+def test_bodies_of_every_height(lib, rows, top, experts, ff, shared, up):
+    """Products going up (gated experts) that power bounds, and those whose launch with more code is slower."""
+    blocks = lambda f: -(-f // 128)
+    all_experts, slots = experts + (shared > 0), rows * (top + (shared > 0))
+    assert bool(lib.every(rows, slots, all_experts, blocks(ff), blocks(shared or ff))) == up
