@@ -130,8 +130,8 @@ class EncoderModel:
                 return h
             return F.gelu(h)
 
-        if (fused and hid <= 2048 and input_ids.dtype == positions.dtype == torch.int64 and self.word_emb.is_contiguous()
-                and self.pos_emb.is_contiguous()):  # (one launch: csrc/layernorm.hip)
+        if (fused and hid <= 2048 and input_ids.dtype == positions.dtype == torch.int64
+                and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (self.word_emb, self.pos_emb, self.type_emb[0]))):  # (one launch)
             x = torch.ops._C_amd.embed_layer_norm(input_ids.contiguous(), positions.contiguous(), shift, self.word_emb, self.pos_emb,
                                                   self.type_emb[0], *self.emb_ln, eps)
         else:

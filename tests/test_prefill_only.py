@@ -142,9 +142,9 @@ def encoder_prompts():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tables", ["two types", "strided"])
+@pytest.mark.parametrize("tables", ["two types", "strided", "off 16 bytes"])
 def test_embedding_tables(tables):
-    """A table of two types, of which the first is taken, and tables that are parts of wider ones."""
+    """A table of two types, of which the first is taken, tables that are parts of wider ones, and some that begin anywhere."""
     from light_vllm_amd.attention.prefill_only import PrefillOnlyAttentionMetadata
     from light_vllm_amd.prefill_only.model import EncoderConfig, EncoderModel
     model = EncoderModel(EncoderConfig.tiny(), DEV, 0)
@@ -157,6 +157,10 @@ def test_embedding_tables(tables):
     first = run()
     if tables == "two types":
         model.type_emb = torch.cat([model.type_emb, model.type_emb + 1])
+    elif tables == "off 16 bytes":
+        for name in ("word_emb", "pos_emb", "type_emb"):
+            t = getattr(model, name)
+            setattr(model, name, torch.cat([t.new_zeros(3), t.flatten()])[3:].view(t.shape))
     else:
         model.word_emb, model.pos_emb = (torch.cat([t, t], dim=1)[:, :128] for t in (model.word_emb, model.pos_emb))
     assert torch.equal(run(), first)
