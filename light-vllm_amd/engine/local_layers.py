@@ -167,8 +167,9 @@ class ParallelHeads:
 
 class ClampedMlp:
 
-    def __init__(self, get, name: str, cfg: ClampedMlpConfig, pack: bool):
-        self.limit = cfg.limit
+    def __init__(self, get, name: str, cfg: ClampedMlpConfig, pack: bool, routed: bool = False):
+        """routed: the model has routers, and sums of prompts keep the library's order: in another one tokens go to other experts."""
+        self.limit, self.routed = cfg.limit, routed
         # zero rows of gate and up give zero activations: all sizes may be padded for the weight-streaming kernel
         self.up = make_weight(stack_rows([get(name + ".gate"), get(name + ".up")], 32)[0], pack)
         self.down = make_weight(pad_columns(get(name + ".down")), pack)
@@ -180,7 +181,7 @@ class ClampedMlp:
         if 0 < h.shape[0] <= DECODE_ROWS and self.up.packed is not None:
             a = amd.skinny_linear_packed_clamped_unit(h, self.up.packed, self.up.N, self.up.K, self.limit)
         else:
-            a = linear_act(h, self.up, "clamped_unit", self.up.N // 2, self.limit)
+            a = None if self.routed else linear_act(h, self.up, "clamped_unit", self.up.N // 2, self.limit)
             a = amd.clamped_unit(linear(h, self.up), self.limit) if a is None else a
         return Branch(project_to_residual(a, self.down))
 

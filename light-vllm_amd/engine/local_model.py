@@ -82,6 +82,7 @@ class LocalModel(LayeredModel):
         self.pairs = get("bigram").contiguous() if cfg.pairs is not None else None
         self.layers: List[tuple] = []
         before, norms = [], []  # the norms in front of the sublayers, those behind them
+        routed = any(isinstance(l.mlp, MixtureConfig) for l in cfg.layers)
         for i, l in enumerate(cfg.layers):
             p = f"l{i}"
             before.append(get(p + ".norm1").float().contiguous())
@@ -91,8 +92,9 @@ class LocalModel(LayeredModel):
             if l.mlp is not None:
                 before.append(get(p + ".norm2").float().contiguous())
                 norms.append(SandwichNorm(get, p + ".norm2b", eps))
-                kind = MixtureMlp if isinstance(l.mlp, MixtureConfig) else ClampedMlp
-                sub.append((kind(get, p + ".mlp", l.mlp, pack), norms[-1]))
+                mlp = (MixtureMlp(get, p + ".mlp", l.mlp, pack) if isinstance(l.mlp, MixtureConfig)
+                       else ClampedMlp(get, p + ".mlp", l.mlp, pack, routed))
+                sub.append((mlp, norms[-1]))
             self.layers.append(tuple(sub))
         before.append(get("final.norm").float().contiguous())
         self.first_norm = before[0]

@@ -216,7 +216,9 @@ class TimeMixer:
 class SiluMlp:
     """W_down (silu(W_gate h) * (W_up h))."""
 
-    def __init__(self, get, name: str, pack: bool):
+    def __init__(self, get, name: str, pack: bool, routed: bool = False):
+        """routed: the model has routers, and sums of prompts keep the library's order: in another one tokens go to other experts."""
+        self.routed = routed
         # zero rows of gate and up give zero activations: all sizes may be padded for the weight-streaming kernel
         self.up = make_weight(stack_rows([get(name + ".gate"), get(name + ".up")], 32)[0], pack)
         self.down = make_weight(pad_columns(get(name + ".down")), pack)
@@ -228,7 +230,7 @@ class SiluMlp:
         if 0 < h.shape[0] <= DECODE_ROWS and self.up.packed is not None:
             a = amd.skinny_linear_packed_swiglu(h, self.up.packed, None, self.up.N, self.up.K)
         else:
-            a = linear_act(h, self.up, "silu_and_mul", self.up.N // 2)
+            a = None if self.routed else linear_act(h, self.up, "silu_and_mul", self.up.N // 2)
             a = amd.silu_unit(linear(h, self.up)) if a is None else a
         return project_to_residual(a, self.down)
 

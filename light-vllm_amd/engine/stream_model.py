@@ -72,6 +72,7 @@ class StreamModel(LayeredModel):
         cfg, eps = self.cfg, self.cfg.norm_eps
         self.embed = get("embed").contiguous()
         layers: List[list] = []
+        routed = any(isinstance(l.mlp, MixtureConfig) for l in cfg.layers)
         for i, l in enumerate(cfg.layers):
             p = f"l{i}"
             kind = LatentAttention if isinstance(l.mixer, LatentAttentionConfig) else DeltaRule
@@ -81,7 +82,7 @@ class StreamModel(LayeredModel):
             if isinstance(l.mlp, MixtureConfig):
                 subs.append(MixtureOfExperts(get, p + ".mlp", l.mlp, pack))
             elif l.mlp is not None:
-                subs.append(SiluMlp(get, p + ".mlp", pack))
+                subs.append(SiluMlp(get, p + ".mlp", pack, routed))
             layers.append([(sub, StreamReader(get(f"{p}.hc{q}.in"), get(f"{p}.norm{q}")),
                             StreamWriter(get(f"{p}.hc{q}.mix"), get(f"{p}.hc{q}.out"))) for q, sub in enumerate(subs, 1)])
         self.layers = [layers[i] for i in cfg.runs]

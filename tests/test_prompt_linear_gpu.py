@@ -101,3 +101,35 @@ def test_what_is_refused(amd):
     assert amd.prompt_linear(flat[1:].view(2048, 512), w, None, None, 4096, SILU) is None   # not aligned
     with pytest.raises(RuntimeError):
         amd.prompt_linear(x, w, None, None, 8192, SILU)
+
+
+@pytest.mark.parametrize("mixture", [True, False])
+@pytest.mark.parametrize("kind", ["Lizazen", "Susalorn"])
+def test_dense_feed_forwards_beside_routers(amd, kind, mixture):
+    """In a model with routers the sums of prompts keep the library's order; in one without, the product takes its activation along."""
+    from light_vllm_amd.engine.mixers import SiluMlp, project_to_residual
+    from light_vllm_amd.engine.local_layers import ClampedMlp
+    from light_vllm_amd.engine.registry import model_entry
+    dense, moe = {"kind": "dense", "ff": 4096}, {"kind": "moe", "router": {"experts": 8, "top": 2}, "expert": {"ff": 128}}
+    if kind == "Lizazen":
+        dense["limit"], moe["shared"] = 7.0, {"ff": 128}
+        d = {"norm": {"eps": 1e-6}, "embedding": {}}
+        mixer = {"type": "attention", "mixer": {"heads": 4, "kv_heads": 2, "dim": 64, "vdim": 64, "scale": 0.125, "rot": {"dims": 64, "base": 1e4}, "softcap": 50.0,
+                                                "mask": {"size": 4096}}}
+    else:
+        moe["router"].update(groups={"count": 4, "keep": 2}, scale=2.5)
+        d = {"norm": {"eps": 1e-5}, "streams": 4, "loop": None}
+        mixer = {"type": "channel_delta", "mixer": {"heads": 4, "kv_heads": 4, "dim": 64, "vdim": 64, "conv": 4}}
+    d.update(architecture=kind, vocab=512, width=512, layers=[{**mixer, "mlp": dense}, {**mixer, "mlp": moe if mixture else dense}])
+    entry = model_entry(kind)
+    model = entry.model_cls()(entry.config_cls().from_dict(d), entry.backend_cls().get_impl_cls()(), DEV)
+    subs = [s[0] for layer in model.layers for s in layer]
+    mlp = next(s for s in subs if isinstance(s, (ClampedMlp, SiluMlp)))
+    assert mlp.routed == mixture
+    h = torch.randn(1500, 512, device=DEV).bfloat16()
+    both = F.linear(h, mlp.up.w)
+    want = project_to_residual(amd.clamped_unit(both, 7.0) if kind == "Lizazen" else amd.silu_unit(both), mlp.down)
+    y = mlp(h)
+    y = y.y if kind == "Lizazen" else y
+    assert y.dtype == want.dtype and (not mixture or torch.equal(y, want))
+    assert (y.float() - want.float()).norm() < 1e-2 * want.float().norm()
