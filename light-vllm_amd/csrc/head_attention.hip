@@ -117,18 +117,16 @@ static bool takes_mfma(int kpad, int vpad, int maps, int block_size, int dtype) 
 }
 
 // Shares the keys of a sequence are cut into: enough workgroups to fill the chip, none of under 256 keys, and none at all
-// beside large prompt portions.  Nor for up to 512 keys of at most 448 elements (key and value), whose walk is shorter than the launch that shares
-// meet in: 16 heads over 4 of 128 and 64, us in two shares and whole, 100 keys: 1 sequence 6.6, 4.4; 24 sequences 7.3, 4.8; 300: 9.5, 6.9;
-// 500: 10.4, 8.8; 8 over 2 of 192 and 256, 512: 13.8, 13.3.  16 over 1 of 256 and 256, 24 sequences: 300 16.6, 18.4; 512 18.8, 22.3.  (Two
-// maps meet in that launch in any case.)
-static int decode_shares(int rows, int num_seqs, int heads, int kv_heads, int kpad, int vpad, int max_seq_len, const lvllm_head_options& o) {
+// beside large prompt portions.  (No cut for up to 512 keys would be faster, 16 heads over 4 of 128 and 64, 24 sequences of 300 9.5 us, 6.9; but sums
+// of decode steps in another order ahead of a router move tokens to other experts.)
+static int decode_shares(int rows, int num_seqs, int heads, int kv_heads, int max_seq_len, const lvllm_head_options& o) {
   if (rows > 512) return 1;
   const int wgs = num_seqs * kv_heads * ((heads / kv_heads * o.maps + kDecodeCols - 1) / kDecodeCols);
   int n = (1024 + wgs - 1) / wgs;
   int64_t keys = max_seq_len;
   if (o.window > 0) keys = std::min<int64_t>(keys, (int64_t)o.window + o.keep_first + kDecodeCols);
   if (o.chunk > 0) keys = std::min<int64_t>(keys, (int64_t)o.chunk + o.keep_first + kDecodeCols);
-  const int most = o.maps == 1 && keys <= 512 && kpad + vpad <= 448 ? 1 : (int)((keys + 255) / 256);
+  const int most = (int)((keys + 255) / 256);
   n = n < most ? n : most;
   return n < 1 ? 1 : n > 64 ? 64 : n;
 }
@@ -142,7 +140,7 @@ extern "C" int64_t lvllm_head_attention_workspace_bytes(int rows, int num_seqs, 
                                                         int dtype) {
   const lvllm_head_options& o = *options;
   if (heads <= 0 || kv_heads <= 0 || rows <= 0 || num_seqs <= 0 || !takes_mfma(kpad, vpad, o.maps, block_size, dtype)) return 0;
-  return shares_bytes(rows, heads, vpad, o.maps, decode_shares(rows, num_seqs, heads, kv_heads, kpad, vpad, max_seq_len, o));
+  return shares_bytes(rows, heads, vpad, o.maps, decode_shares(rows, num_seqs, heads, kv_heads, max_seq_len, o));
 }
 
 extern "C" int lvllm_head_attention(void* out, int64_t out_stride, const void* q, const void* key_cache,
@@ -174,7 +172,7 @@ extern "C" int lvllm_head_attention(void* out, int64_t out_stride, const void* q
   p.softcap = o.softcap; p.sink = o.sink; p.map_weight = o.map_weight; p.map_eps = o.map_eps;
   hipStream_t s = (hipStream_t)stream;
   if (takes_mfma(kpad, vpad, o.maps, block_size, dtype)) {
-    p.nsplit = decode_shares(rows, num_seqs, heads, kv_heads, kpad, vpad, max_seq_len, o);
+    p.nsplit = decode_shares(rows, num_seqs, heads, kv_heads, max_seq_len, o);
     if (const int64_t need = shares_bytes(rows, heads, vpad, o.maps, p.nsplit)) {
       LV_CHECK(workspace != nullptr && workspace_bytes >= need, "workspace too small (see lvllm_head_attention_workspace_bytes)");
       p.part_o = (float*)workspace;

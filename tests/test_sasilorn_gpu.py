@@ -301,7 +301,7 @@ def test_softmax_heads(amd, dtype, name, heads, kv_heads, dim, vdim):
 @pytest.mark.parametrize("longest", [511, 512, 513])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(4, 1, 128, 64), (2, 2, 64, 256)])
 def test_single_tokens_by_the_longest(amd, monkeypatch, longest, heads, kv_heads, dim, vdim):
-    """Up to 512 keys one share, beyond several that meet in a launch of their own."""
+    """Where a third share begins: shares of unequal lengths, which meet in a launch of their own, and sequences that leave some empty."""
     monkeypatch.setitem(ATTENTION_LAYOUTS, "longest", [(1, longest - 1), (1, 255), (3, 300), (1, 0)])
     test_softmax_heads(amd, BF16, "longest", heads, kv_heads, dim, vdim)
 
