@@ -1,6 +1,6 @@
 // Projections of prompts with a gated unit or squared ReLU behind them, in the tiles of wide_tile.h over the library's row-major weights: what
 // they leave is the activation of what the projection would, in one launch and without its way through memory.  4875 rows of 4096, SwiGLU of
-// 14336: 842 us (1.36 PFLOP/s) for 891 and 73 in two launches; prompt_linear.h has more.
+// 14336: 842 us (1.36 PFLOP/s) for 891 and 73 in two launches, on another card 855 for 990; prompt_linear.h has more.
 #include <algorithm>
 #include <type_traits>
 

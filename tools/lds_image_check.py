@@ -1,7 +1,9 @@
 """Bank-conflict check of the row-major K / V LDS images of the dense twin of the 32x32-MFMA prefill body
 (prefill_mfma32.h, DENSE): the 16-byte row reads of the K fragments (ds_read_b128), the transposed reads of the V^T
 fragments (ds_read_b64_tr_b16) and the copy's 16-byte writes (ds_write_b128), with the banking rules of
-MI355X_MICROARCH.md 'LDS'.  Prints the worst multiplicity per instruction kind; 1 = conflict-free.  Host-only."""
+MI355X_MICROARCH.md 'LDS'.  Prints the worst multiplicity per instruction kind; 1 = conflict-free.  dense_attention.h has the
+same image of D = 64, copied straight to LDS, and makes the reads' addresses from one base by exclusive or: checked to be
+the same.  Host-only."""
 import sys
 
 B128_GROUPS = [
@@ -65,6 +67,16 @@ def main():
                 row = piece * (64 // cpr) + lane // cpr
                 addrs.append(off(D, row, lane % cpr))
             ww = max(ww, worst(addrs, [list(range(8 * i, 8 * i + 8)) for i in range(8)], 16, 8))
+        if D == 64:
+            for lane in range(64):
+                col, hi = lane & 31, lane >> 5
+                q, c, b = (lane & 15) >> 2, 2 * (col >> 4) + ((lane & 3) >> 1), 8 * (lane & 1)
+                k_at, v_at = off(D, krow(col), hi), off(D, 8 * hi + q, c) + b
+                for i in range(8):
+                    assert (k_at ^ ((i >> 1) << 5)) + (i & 1) * 32 * 128 == off(D, 32 * (i & 1) + krow(col), 2 * (i >> 1) + hi)
+                    at = (i >> 1) * 16 * 128
+                    assert at + (v_at ^ ((i & 1) << 6)) == off(D, 16 * (i >> 1) + 8 * hi + q, 4 * (i & 1) + c) + b
+                    assert at + (v_at ^ ((i & 1) << 6) ^ 16) + 4 * 128 == off(D, 16 * (i >> 1) + 8 * hi + 4 + q, 4 * (i & 1) + c) + b
         print(f"D {D}: K row reads {wk}-way, V transposed reads {wv}-way, copy writes {ww}-way")
     return 0
 
