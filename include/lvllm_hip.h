@@ -286,6 +286,10 @@ int lvllm_skinny_gemm_ex(void* y, const void* x, const void* w, const void* bias
  * LayerNorm).  16-bit element types, hidden_size % 8 == 0, contiguous rows, out may alias x. */
 int lvllm_add_layer_norm(void* out, const void* x, const void* y, const void* weight, const void* bias,
                          float epsilon, int num_tokens, int hidden_size, int dtype, void* stream);
+/* ... of x + T(y + y_bias), y the sum of fp32 slabs [num_slabs, num_tokens, hidden_size] (lvllm_prompt_product) and y_bias [hidden_size] or
+ * null; hidden_size up to 2048 */
+int lvllm_add_layer_norm_slabs(void* out, const void* x, const float* slabs, int num_slabs, const void* y_bias, const void* weight,
+                               const void* bias, float epsilon, int num_tokens, int hidden_size, int dtype, void* stream);
 /* LayerNorm(T(T(word[ids] + pos[positions + shift]) + type)) of an encoder's embeddings: word [words, hidden], pos [places, hidden], type
  * [hidden].  16-bit element types, hidden_size a multiple of 8 up to 2048; rows of an id or position outside its table become NaN. */
 int lvllm_embed_layer_norm(void* out, const int64_t* ids, const int64_t* positions, int64_t shift, const void* word, const void* pos,
@@ -706,6 +710,13 @@ int lvllm_prompt_linear_body(int rows, int outputs, int k, int act, int row_majo
  * bias [outputs]: GELU only; limit: CLAMPED_UNIT only.  bf16.  All but GELU round the product as the library's result is before they act. */
 int lvllm_prompt_linear(void* out, const void* x, const void* w, const void* w_packed, const void* bias, int rows, int outputs, int k,
                         int act, float limit, int dtype, void* stream);
+/* x w^T of prompts of some hundreds of rows, x [rows, k], w [n, k] packed (lvllm_pack_weight), bf16.  The plan (four numbers) holds for one
+ * device and these sizes; the call returns the shares that K is cut into, 0 where the library's product is the better one.  `slabs`: K may be
+ * cut, and the caller sums what leaves then. */
+int lvllm_prompt_product_plan(int rows, int n, int k, int gelu, int slabs, int* plan);
+/* one share: out [rows, n] = x w^T + bias (null: none), GELU behind it where asked for; more: slabs [shares, rows, n], plain sums */
+int lvllm_prompt_product(void* out, float* slabs, const void* x, const void* w_packed, const void* bias, int rows, int n, int k, int gelu,
+                         const int* plan, void* stream);
 /* ---- mixtures of experts (csrc/moe*.hip, moe.h) ---- */
 enum { LVLLM_MOE_SOFTMAX = 0, LVLLM_MOE_SIGMOID = 1 };  /* weights: softmax over the chosen logits, or each logit's sigmoid */
 enum { LVLLM_MOE_NO_SHARED = 0, LVLLM_MOE_GATED_SHARED = 1, LVLLM_MOE_PLAIN_SHARED = 2 };

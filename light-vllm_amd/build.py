@@ -33,7 +33,7 @@ ARCH = "gfx950"
 
 SOURCES = {
     "base": ["capi.hip", "cache.hip", "skinny_gemm.hip", "prepare_inputs.hip", "sampler.hip", "activation.hip",
-             "wide_linear.hip", "tile_linear.hip"],
+             "wide_linear.hip", "tile_linear.hip", "prompt_product.hip"],
     "heads": ["head_attention.hip", "head_attention_prefill.hip", "head_attention_decode.hip", "head_attention_maps.hip",
               "head_cache.hip"],
     "moe": ["moe.hip", "moe_mfma.hip"],

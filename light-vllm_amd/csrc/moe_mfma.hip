@@ -161,7 +161,7 @@ __device__ __forceinline__ TileWork tile_work(const MoeParams& p, const int bloc
   const int end = tile + 1 < min(tile0 + count, p.max_tiles) ? p.tiles[4 * tile + 5] : p.offsets[t.e + 1];
   t.s1 = min(min(end, t.s0 + TILE), p.slots);
   const int ff = p.ff[t.e];
-  t.steps = (UP ? p.width : ff) >> 5;
+  t.steps = t.all = (UP ? p.width : ff) >> 5;
   t.ntiles = GATED ? ff >> 3 : (UP ? ff : p.width) >> 4;
   t.any = t.block * TILEW < t.ntiles && t.s0 < t.s1;
   t.once = count == 1;

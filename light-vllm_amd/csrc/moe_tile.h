@@ -27,6 +27,7 @@ __device__ __forceinline__ e_u32x4_t load_weights(const uint16_t* p) {
 // W block `block` (4 NT tiles of 16 rows) of slots s0 .. s1 - 1 of expert e
 struct TileWork {
   int e, block, s0, s1, steps, ntiles;  // slots s0 .. s1 - 1, k-steps, W tiles of 16 rows of the expert
+  int all;  // k-steps that lie side by side in w: more than `steps` where a workgroup takes a share of them
   bool any, once;  // once: the expert's only tile
 };
 // A wave's results by way of 2 KiB of LDS of its own: W tiles nt0 .. of groups of 16 slots from slot0 on, a group at a time, so that a
@@ -97,7 +98,7 @@ __device__ __forceinline__ void tile_sums(e_f32x4_t (&acc)[NT][MT], const uint16
   const uint16_t *wsrc[NT], *xsrc[kCopies];
   const uint16_t* w = w_tiles + lane * 8;
 #pragma unroll
-  for (int j = 0; j < NT; ++j) wsrc[j] = w + (int64_t)tile_of(min(nt0 + j, ntiles - 1)) * steps * 512;
+  for (int j = 0; j < NT; ++j) wsrc[j] = w + (int64_t)tile_of(min(nt0 + j, ntiles - 1)) * t.all * 512;
   const int chunk = (lane & 7) ^ (lane >> 3);
 #pragma unroll
   for (int j = 0; j < kCopies; ++j) {

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(const TileLinear p)
   t.s0 = (strip * kSide + in - t.block * side) * size;
   t.s1 = min(t.s0 + size, p.rows);
   if (t.s0 >= t.s1) return;
-  t.steps = p.k >> 5;
+  t.steps = t.all = p.k >> 5;
   t.ntiles = (prompt_pairs(ACT) ? 2 : 1) * (p.outputs >> 4);
   const int groups = (t.s1 - t.s0 + 15) >> 4;
   if (groups <= 4) tile_linear<ACT, NT, 4>(p, t, ring);

@@ -144,6 +144,28 @@ void add_layer_norm(torch::Tensor& out, const torch::Tensor& x, const std::optio
                              dtype_code(x, "add_layer_norm"), current_stream(x)));
 }
 
+void add_layer_norm_slabs(torch::Tensor& out, const torch::Tensor& x, const torch::Tensor& slabs, const std::optional<torch::Tensor>& y_bias,
+                          const torch::Tensor& weight, const torch::Tensor& bias, double epsilon) {
+  const char* op = "add_layer_norm_slabs";
+  LV_CHECK_DEVICE(x);
+  TORCH_CHECK(x.dim() == 2 && x.is_contiguous() && out.is_contiguous() && out.sizes() == x.sizes() && out.scalar_type() == x.scalar_type(), op,
+              ": contiguous out and x [rows, hidden] of the same type");
+  TORCH_CHECK(slabs.device() == x.device() && slabs.dim() == 3 && slabs.is_contiguous() && slabs.scalar_type() == at::kFloat &&
+                  slabs.size(1) == x.size(0) && slabs.size(2) == x.size(1),
+              op, ": float32 slabs [s, rows, hidden]");
+  const int hidden = (int)x.size(1);
+  for (const auto* t : {&weight, &bias})
+    TORCH_CHECK(t->device() == x.device() && t->numel() == hidden && t->is_contiguous() && t->scalar_type() == x.scalar_type(), op,
+                ": weight and bias of [hidden] in x's type");
+  TORCH_CHECK(!y_bias || (y_bias->device() == x.device() && y_bias->numel() == hidden && y_bias->is_contiguous() &&
+                          y_bias->scalar_type() == x.scalar_type()),
+              op, ": y_bias of [hidden] in x's type");
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(x));
+  check(lvllm_add_layer_norm_slabs(out.data_ptr(), x.data_ptr(), slabs.data_ptr<float>(), (int)slabs.size(0),
+                                   y_bias ? y_bias->data_ptr() : nullptr, weight.data_ptr(), bias.data_ptr(), (float)epsilon, (int)x.size(0),
+                                   hidden, dtype_code(x, op), current_stream(x)));
+}
+
 torch::Tensor embed_layer_norm(const torch::Tensor& ids, const torch::Tensor& positions, int64_t shift, const torch::Tensor& word,
                                const torch::Tensor& pos, const torch::Tensor& type, const torch::Tensor& weight, const torch::Tensor& bias,
                                double epsilon) {
@@ -579,6 +601,8 @@ TORCH_LIBRARY_FRAGMENT(_C_amd, amd) {
   amd.impl("gelu", torch::kCUDA, &gelu);
   amd.def("add_layer_norm(Tensor! out, Tensor x, Tensor? y, Tensor weight, Tensor bias, float epsilon) -> ()");
   amd.impl("add_layer_norm", torch::kCUDA, &add_layer_norm);
+  amd.def("add_layer_norm_slabs(Tensor! out, Tensor x, Tensor slabs, Tensor? y_bias, Tensor weight, Tensor bias, float epsilon) -> ()");
+  amd.impl("add_layer_norm_slabs", torch::kCUDA, &add_layer_norm_slabs);
   amd.def("embed_layer_norm(Tensor ids, Tensor positions, int shift, Tensor word, Tensor pos, Tensor type, Tensor weight, Tensor bias, "
           "float epsilon) -> Tensor");
   amd.impl("embed_layer_norm", torch::kCUDA, &embed_layer_norm);

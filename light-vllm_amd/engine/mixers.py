@@ -11,7 +11,7 @@ import torch
 import torch.nn.functional as F
 
 from .hybrid_config import KVSpec, LinearHeadsConfig, ParallelMixerConfig, SoftmaxHeadsConfig, TimeMixerConfig
-from .model import Weight, linear, linear_act
+from .model import Weight, linear, linear_act, product
 
 amd = torch.ops._C_amd
 DECAY_LOGSIGMOID, DECAY_NEGEXP = 0, 1
@@ -70,11 +70,12 @@ def make_weight(w: torch.Tensor, pack: bool) -> Weight:
     return Weight(w.contiguous(), pack and w.dtype != torch.float32)
 
 
-def project_to_residual(x: torch.Tensor, w: Weight) -> torch.Tensor:
-    """A projection whose only reader is the next residual add: split-K slabs where that launch sums them."""
+def project_to_residual(x: torch.Tensor, w: Weight, routed: bool = True) -> torch.Tensor:
+    """A projection whose only reader is the next residual add: split-K slabs where that launch sums them.  `routed`: the model has routers, and
+    sums of prompts keep the library's order."""
     if 0 < x.shape[0] <= DECODE_ROWS and w.packed is not None:
         return amd.skinny_linear_packed_partials(x, w.packed, w.N, w.K, False)
-    return linear(x, w)
+    return linear(x, w) if routed else product(x, w, slabs=True)
 
 
 class DynTanhNorm:
@@ -150,7 +151,7 @@ class ParallelMixer:
     def __call__(self, x, y, norm: DynTanhNorm, cache: LayerCache, step: StepLayout, attn, dtype):
         a, r = self.cfg.left, self.cfg.right
         h = norm(x, y, dtype)
-        proj = linear(h, self.proj)
+        proj = product(h, self.proj)
         lq, lk, lv, rq, rk, rv, rg, lg, u = (proj[:, o:o + n] for o, n in zip(self.at, self.sizes))
         rows = proj.shape[0]
         cols = self.left_cols + self.right_cols
@@ -164,7 +165,7 @@ class ParallelMixer:
         # gated linear attention
         self.recurrence(both[:, self.left_cols:cols], rq, rk, rv, u, rg, self.out_norm, self.cfg.right_scale,
                         r.dim ** -0.5, cache.state["matrix"], step)
-        return x, project_to_residual(both, self.out)
+        return x, project_to_residual(both, self.out, False)
 
 
 class TimeMixer:
@@ -205,12 +206,12 @@ class TimeMixer:
                 r, k, v, g = (linear(mix[i], w) for i, w in enumerate(self.rkvg))
             else:
                 r, k, v, g = torch.bmm(mix[:4], self.rkvg_t)
-            u = linear(mix[4], self.w1)
+            u = product(mix[4], self.w1)
         u = u[:, :self.rank]
         cols = self.cfg.heads * self.cfg.dim
         out = (torch.empty if self.out.K == cols else torch.zeros)(rows, self.out.K, dtype=dtype, device=x.device)
         self.recurrence(out[:, :cols], r, k, v, u, g, self.norm, 1.0, 1.0, cache.state["matrix"], step)
-        return x, project_to_residual(out, self.out)
+        return x, project_to_residual(out, self.out, False)
 
 
 class SiluMlp:
@@ -249,6 +250,6 @@ class SquaredReluMlp:
         else:
             a = linear_act(h, self.up, "relu_squared", self.up.N)
             if a is None:
-                a = linear(h, self.up)
+                a = product(h, self.up)
                 amd.relu_squared(a, a)
-        return project_to_residual(a, self.down)
+        return project_to_residual(a, self.down, False)

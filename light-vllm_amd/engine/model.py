@@ -72,6 +72,16 @@ def linear(x: torch.Tensor, w: "Weight", bias: Optional[torch.Tensor] = None) ->
     return F.linear(x, w.w, bias)
 
 
+def product(x: torch.Tensor, w: "Weight", bias: Optional[torch.Tensor] = None, slabs: bool = False) -> torch.Tensor:
+    """linear(), for models without routers: its sums go another way for prompts of some hundreds of rows (csrc/prompt_product.h), and ahead of a
+    router the last bits decide which expert a token takes.  `slabs`: or fp32 [s, rows, N], whose sum the next launch takes, without the bias."""
+    if x.shape[0] > 64 and x.is_cuda and w.packed is not None and not _CALIBRATING:
+        y = torch.ops._C_amd.prompt_product(x, w.packed, bias, w.N, False, slabs)
+        if y is not None:
+            return y
+    return linear(x, w, bias)
+
+
 PROMPT_ACTS = {"gelu": 1, "silu_and_mul": 2, "relu_squared": 3, "clamped_unit": 4}  # include/lvllm_hip.h LVLLM_ACT_*
 
 
@@ -265,7 +275,7 @@ class DecoderModel:
                         else:
                             qkv_roped = True
                 if qkv is None:
-                    qkv = linear(hidden, lw.qkv, lw.qkv_bias)
+                    qkv = product(hidden, lw.qkv, lw.qkv_bias)
             q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)  # strided views
             fused = False
             attn_out = None
@@ -309,7 +319,7 @@ class DecoderModel:
                 hidden = torch.ops._C_amd.skinny_linear_w8a8_q(attn8, lw.o.w8_packed, lw.o.w_scale, lw.o.x_scale, lw.o.N,
                                                                lw.o.K, None, cfg.dtype)
             else:
-                hidden = linear(attn_out, lw.o)
+                hidden = product(attn_out, lw.o, slabs=True)
             if q_once:
                 g, d = lw.gate_up, lw.down
                 h8 = self._norm_fp8(hidden, residual, lw.post_norm, g.x_scale)
@@ -350,7 +360,7 @@ class DecoderModel:
                 if part.numel() > 0:
                     hidden = (part, d.x_scale, d.w_scale)
             if hidden is None:
-                hidden = linear(act, lw.down)
+                hidden = product(act, lw.down, slabs=True)
         return self._add_norm(hidden, residual, self.final_norm)
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:

@@ -54,7 +54,8 @@ class EncoderLayerWeights:
         hid, inter = cfg.hidden_size, cfg.intermediate_size
 
         def w(*shape, std=0.02):
-            return (torch.randn(*shape, generator=gen, device=device, dtype=torch.float32) * std).to(cfg.dtype)
+            with torch.inference_mode(False):  # (torch counts writes to these, wherever the model is made)
+                return (torch.randn(*shape, generator=gen, device=device, dtype=torch.float32) * std).to(cfg.dtype)
 
         def ln():
             return ((1.0 + 0.05 * torch.randn(hid, generator=gen, device=device)).to(cfg.dtype),
@@ -66,22 +67,32 @@ class EncoderLayerWeights:
         self.fc1_w, self.fc1_b = w(inter, hid), w(inter)
         self.fc2_w, self.fc2_b = w(hid, inter), w(hid)
         self.out_ln = ln()
-        self._fused, self._fc1_packed = cfg.fused_layer_norm, None
-        self.fc1_packed  # (laid out now, and not in the first forward)
+        self._fused, self._packed = cfg.fused_layer_norm, {}
+        for name in self.WEIGHTS:
+            self.packed(name)  # (laid out now, and not in the first forward)
 
-    @property
-    def fc1_packed(self) -> Optional[torch.Tensor]:
-        """fc1_w once more in fragment order, for the kernel with GELU behind the product (None: what it does not take).  Laid out anew when
-        fc1_w has been replaced or written to since.  Writes that torch does not count (`fc1_w.data.copy_`, or to inference tensors) are not
-        seen: assign fc1_w behind those."""
-        w = self.fc1_w
+    WEIGHTS = "qkv_w", "out_w", "fc1_w", "fc2_w"
+
+    def packed(self, name: str) -> Optional[torch.Tensor]:
+        """A weight once more in fragment order, for this package's kernels (None: what they do not take).  Laid out anew when the weight has been
+        replaced or written to since.  Writes that torch does not count (`fc1_w.data.copy_`, or to inference tensors) are not seen: assign the
+        weight behind those."""
+        w = getattr(self, name)
         if not (self._fused and w.is_cuda and w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[0] % 16 == 0 and w.shape[1] % 32 == 0):
             return None
         version = -1 if w.is_inference() else w._version
-        was = self._fc1_packed  # (fc1_w, its memory, which nothing else can have meanwhile, and its version then, the copy)
+        was = self._packed.get(name)  # (the weight, its memory, which nothing else can have meanwhile, and its version then, the copy)
         if was is None or was[0] is not w or was[1].data_ptr() != w.data_ptr() or was[2] != version:
-            was = self._fc1_packed = w, w.detach(), version, torch.ops._C_amd.pack_weight(w)
+            if torch.cuda.is_current_stream_capturing():  # (a copy that only the graph would write)
+                return None
+            was = w, w.detach(), version, torch.ops._C_amd.pack_weight(w)
+            torch.cuda.current_stream(w.device).synchronize()  # (the next forward may come on another stream)
+            self._packed[name] = was
         return was[3]
+
+    @property
+    def fc1_packed(self) -> Optional[torch.Tensor]:
+        return self.packed("fc1_w")
 
 
 class EncoderModel:
@@ -111,19 +122,32 @@ class EncoderModel:
         emb, shift = self.word_emb, cfg.pad_token_id + 1  # xlm_roberta.py: position ids start after the padding index
         fused = emb.is_cuda and hid % 8 == 0 and emb.dtype in (torch.bfloat16, torch.float16) and self.cfg.fused_layer_norm
 
-        def add_ln(a, b, ln):  # LayerNorm(a + b), b optional
+        def add_ln(a, b, ln, b_bias=None):  # LayerNorm(a + b), b optional; slabs: without their bias
+            if b is not None and b.dim() == 3:
+                out = torch.empty_like(a)
+                torch.ops._C_amd.add_layer_norm_slabs(out, a, b, b_bias, ln[0], ln[1], eps)
+                return out
             if fused:
                 out = torch.empty_like(a)
                 torch.ops._C_amd.add_layer_norm(out, a, b, ln[0], ln[1], eps)
                 return out
             return F.layer_norm(a if b is None else a + b, (hid,), ln[0], ln[1], eps)
 
+        def product(a, lw, name, bias, slabs=False, gelu=False):
+            """This package's kernels where they are the better ones (csrc/prompt_product.h)."""
+            packed = lw.packed(name) if fused and a.shape[0] > 64 else None
+            y = None
+            if packed is not None:
+                y = torch.ops._C_amd.prompt_product(a, packed, bias, packed.numel() // a.shape[1], gelu, slabs and hid <= 2048)
+            return F.linear(a, getattr(lw, name), bias) if y is None and not gelu else y
+
         def fc1_gelu(a, lw):
-            packed = lw.fc1_packed if fused else None
+            h = product(a, lw, "fc1_w", lw.fc1_b, gelu=True)
+            packed = lw.fc1_packed if fused and h is None else None
             if packed is not None:
                 h = torch.ops._C_amd.prompt_linear(a, None, packed, lw.fc1_b, cfg.intermediate_size, PROMPT_ACTS["gelu"])
-                if h is not None:
-                    return h
+            if h is not None:
+                return h
             h = F.linear(a, lw.fc1_w, lw.fc1_b)
             if fused and h.numel() % 8 == 0:
                 torch.ops._C_amd.gelu(h, h)  # exact GELU in place
@@ -138,10 +162,10 @@ class EncoderModel:
             x = F.embedding(input_ids, self.word_emb) + F.embedding(positions + shift, self.pos_emb) + self.type_emb[0]
             x = add_ln(x, None, self.emb_ln)
         for lw in self.layers:
-            qkv = F.linear(x, lw.qkv_w, lw.qkv_b)
+            qkv = product(x, lw, "qkv_w", lw.qkv_b)
             q, k, v = qkv.split([hid, hid, hid], dim=-1)  # strided views of the fused projection
             a = self.attn.forward(q, k, v, None, attn_metadata, attn_type=AttentionType.ENCODER)
-            x = add_ln(x, F.linear(a, lw.out_w, lw.out_b), lw.attn_ln)
+            x = add_ln(x, product(a, lw, "out_w", lw.out_b, slabs=True), lw.attn_ln, lw.out_b)
             blk = cfg.mlp_block_tokens
             if blk > 0 and x.shape[0] > blk:
                 y = torch.empty_like(x)
@@ -149,6 +173,6 @@ class EncoderModel:
                     hb = fc1_gelu(x[r0:r0 + blk], lw)
                     torch.addmm(lw.fc2_b, hb, lw.fc2_w.t(), out=y[r0:r0 + blk])
             else:
-                y = F.linear(fc1_gelu(x, lw), lw.fc2_w, lw.fc2_b)
-            x = add_ln(x, y, lw.out_ln)
+                y = product(fc1_gelu(x, lw), lw, "fc2_w", lw.fc2_b, slabs=True)
+            x = add_ln(x, y, lw.out_ln, lw.fc2_b)
         return x

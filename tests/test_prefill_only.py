@@ -202,6 +202,46 @@ def test_weights_that_come_after_the_model(how):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name", ["qkv_w", "out_w", "fc1_w", "fc2_w"])
+@pytest.mark.parametrize("how", ["assigned", "copied", "captured"])
+def test_each_weight_that_comes_after_the_model(name, how):
+    """... each of them, in prompts of few rows; first seen in a capture: taken there and afterwards."""
+    from light_vllm_amd.attention.prefill_only import PrefillOnlyAttentionMetadata
+    from light_vllm_amd.prefill_only.model import EncoderConfig, EncoderModel
+    cfg = EncoderConfig(hidden_size=1024, intermediate_size=4096, num_hidden_layers=1, num_attention_heads=16, vocab_size=512,
+                        max_position_embeddings=1024)
+    with torch.inference_mode():  # (as users make one)
+        model, other = (EncoderModel(cfg, DEV, seed) for seed in (0, 1))
+    lens = [50, 70]
+    ids = torch.randint(2, 512, (sum(lens),), generator=torch.Generator().manual_seed(3)).to(DEV)
+    pos = torch.cat([torch.arange(n) for n in lens]).to(DEV)
+    md = PrefillOnlyAttentionMetadata(max(lens), lens, torch.tensor([0, 50, 120], dtype=torch.int32, device=DEV))
+
+    def run():
+        with torch.inference_mode():
+            return model.forward(ids, pos, md)
+    first, lw, new = run().clone(), model.layers[0], getattr(other.layers[0], name) * 2
+    if how == "assigned":
+        setattr(lw, name, new)
+    else:
+        getattr(lw, name).copy_(new)
+    if how == "captured":
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = run()
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.allclose(got.float(), run().float(), atol=0.1, rtol=0.02)
+    got = run()
+    model.cfg.fused_layer_norm = False  # (the library's)
+    want = run()
+    assert (got.float() - want.float()).norm() < 1e-2 * want.float().norm()
+    assert (first.float() - want.float()).norm() > 5e-2 * want.float().norm()
+
+
+@pytest.mark.gpu
 def test_encoder_engine_matches_fp32_reference():
     eng = make_encoder(pooling="last_hidden_states")
     ps = encoder_prompts()

@@ -1,0 +1,118 @@
+"""Products of prompts over packed weights (csrc/prompt_product.hip): each body at the edges of its tiles and shares, against 64 bits."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+SHORT, TILE = 1, 2
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from light_vllm_amd import _native
+    _native.load_torch_ops()
+    return _native.load_hip_library()
+
+
+def operands(rows, n, k):
+    g = torch.Generator(device=DEV).manual_seed(rows * 31 + n + k)
+    x = torch.randn(rows, k, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).bfloat16()
+    b = torch.randn(n, generator=g, device=DEV).bfloat16()
+    return x, w, torch.ops._C_amd.pack_weight(w), b
+
+
+def bound(x, w, k):  # k additions in 32 bits, in any order
+    return (k + 8) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+
+
+SIZES = [(16, 128), (17, 144), (65, 16), (100, 272), (129, 240), (300, 304)]  # rows, n: remainders of tiles of rows, and of blocks of weights
+PLANS = [(SHORT, 16, 4), (SHORT, 32, 4), (SHORT, 48, 4), (SHORT, 64, 4), (SHORT, 32, 8), (TILE, 64, 2), (TILE, 80, 4), (TILE, 96, 2),
+         (TILE, 112, 4), (TILE, 128, 2), (TILE, 128, 4)]
+
+
+@pytest.mark.parametrize("rows,n", SIZES)
+@pytest.mark.parametrize("body,size,nt", PLANS)
+@pytest.mark.parametrize("k", [256, 896, 2560])
+def test_bodies(lib, rows, n, body, size, nt, k):
+    x, w, packed, b = operands(rows, n, k)
+    want, err = x.double() @ w.double().t(), bound(x, w, k)
+    p = lambda t: ctypes.c_void_p(0 if t is None else t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for shares in (1, 2, 3, 8):
+        batch = 4 if (body, size) == (SHORT, 16) else 2
+        if -(-(k // 32 // batch) // shares) * batch * (shares - 1) >= k // 32:
+            continue  # (a share without steps: refused)
+        plan = (ctypes.c_int * 4)(body, size, nt, shares)
+        for gelu in (False, True) if shares == 1 and body == SHORT else (False,):
+            out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)  # (a row behind the last: not written)
+            slabs = torch.full((shares * rows + 1, n), 7.0, device=DEV) if shares > 1 else None
+            bias = b if shares == 1 else None
+            print(rows, n, k, body, size, nt, shares, gelu, flush=True)
+            rc = lib.lvllm_prompt_product(p(out if shares == 1 else None), p(slabs), p(x), p(packed), p(bias), rows, n, k, int(gelu), plan, stream)
+            assert rc == 0, lib.lvllm_last_error()
+            if shares > 1:
+                got = slabs[:-1].view(shares, rows, n).double().sum(0)
+                assert bool(((got - want).abs() <= err).all()) and bool((slabs[-1] == 7).all())
+                continue
+            z = want + b.double()
+            ref = torch.nn.functional.gelu(z) if gelu else z
+            # half a step of bfloat16; GELU's slope is below 1.13, and its own error in 32 bits below 1e-6
+            most = 2.0 ** -8 * ref.abs() + 1.13 * (err + 2.0 ** -23 * z.abs()) + (1e-6 if gelu else 0)
+            assert bool(((out[:-1].double() - ref).abs() <= most).all()) and bool((out[-1] == 7).all())
+
+
+@pytest.mark.parametrize("rows,n,k", [(65, 1024, 1024), (100, 4096, 4096), (300, 2048, 8448), (1000, 1024, 4096)])
+def test_op(lib, rows, n, k):
+    x, w, packed, b = operands(rows, n, k)
+    want, err = x.double() @ w.double().t(), bound(x, w, k)
+    y = torch.ops._C_amd.prompt_product(x, packed, None, n, False, True)
+    assert y is not None
+    got = y.double() if y.dim() == 2 else y.double().sum(0)
+    assert bool(((got - want).abs() <= err + (2.0 ** -8 * want.abs() if y.dim() == 2 else 0)).all())
+    z = torch.ops._C_amd.prompt_product(x, packed, b, n)
+    if z is not None:
+        assert bool(((z.double() - want - b.double()).abs() <= err + 2.0 ** -8 * (want + b.double()).abs() + 2.0 ** -23 * want.abs()).all())
+
+
+def test_operands_that_the_library_takes(lib):
+    x, w, packed, b = operands(130, 1024, 1024)
+    op = torch.ops._C_amd.prompt_product
+    assert op(x, packed, b, 1024) is not None
+    wide = torch.zeros(130, 1025, dtype=torch.bfloat16, device=DEV)
+    shifted = torch.zeros(130 * 1024 + 1, dtype=torch.bfloat16, device=DEV)[1:].view(130, 1024)
+    odd_bias = torch.zeros(1025, dtype=torch.bfloat16, device=DEV)[1:]
+    assert op(wide[:, :1024], packed, b, 1024) is None and op(shifted, packed, b, 1024) is None
+    assert op(x.half(), packed, b, 1024) is None and op(x, packed.half(), b, 1024) is None
+    assert op(x, packed, odd_bias, 1024) is None and op(x, packed, b.float(), 1024) is None
+    assert op(x[:64], packed, b, 1024) is None and op(x[:0], packed, b, 1024) is None
+    with pytest.raises(RuntimeError):
+        op(x, packed, b, 1040)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,hidden", [(1, 8), (7, 1000), (33, 1024), (130, 2048)])
+@pytest.mark.parametrize("shares", [1, 2, 4, 5, 8])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_add_layer_norm_slabs(lib, dtype, rows, hidden, shares, with_bias):
+    """The sum and its bias rounded first, and then added and normed: the bits of that but for the order of the norm's sums."""
+    g = torch.Generator(device=DEV).manual_seed(rows + hidden + shares)
+    x = torch.randn(rows, hidden, generator=g, device=DEV).to(dtype)
+    slabs = torch.randn(shares, rows, hidden, generator=g, device=DEV)
+    w, b, yb = ((i + 0.1 * torch.randn(hidden, generator=g, device=DEV)).to(dtype) for i in (1, 0, 0))
+    total = torch.zeros_like(slabs[0])
+    for s in slabs:
+        total = total + s
+    y = (total + yb.float() if with_bias else total).to(dtype)
+    want, got = torch.empty_like(x), x.clone()
+    torch.ops._C_amd.add_layer_norm(want, x, y, w, b, 1e-5)
+    torch.ops._C_amd.add_layer_norm_slabs(got, got, slabs, yb if with_bias else None, w, b, 1e-5)
+    ref = torch.nn.functional.layer_norm((x + y).double(), (hidden,), w.double(), b.double(), 1e-5)
+    # half a step of the result; mean and variance of `hidden` terms in 32 bits
+    most = 2.0 ** (-8 if dtype == torch.bfloat16 else -11) * ref.abs() + hidden * 2.0 ** -23 * (ref.abs() + 1)
+    assert bool(((got.double() - ref).abs() <= most).all()) and bool(((want.double() - ref).abs() <= most).all())
+    for bad in (slabs.half(), slabs[:, :, ::2] if hidden > 8 else slabs[0], slabs[0]):
+        with pytest.raises(RuntimeError):
+            torch.ops._C_amd.add_layer_norm_slabs(got, got, bad, None, w, b, 1e-5)
