@@ -60,3 +60,14 @@ def test_values_without_parts(amd, where, value, kind):
     want = reference(t["u"], t["a"], t["b"], kind)
     want[~nan & ~z.isfinite()] = -torch.exp(torch.tensor(9.0, dtype=torch.float64))
     torch.testing.assert_close(got[~nan], want[~nan], rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("rows", [350, 353, 1888, 1889, 1904, 1905, 2100])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_tiles(amd, rows, kind):
+    """The same bits from each size of tile: of rows by themselves, whose tiles are the smallest, and of all of them."""
+    u, a, b = (t.to(DEV) for t in tensors(rows, 72, 2000, torch.bfloat16, 72))
+    got = amd.log_decay(u, a, b, kind, 1 / 16)
+    want = torch.cat([amd.log_decay(part, a, b, kind, 1 / 16) for part in u.split(40)])
+    assert torch.equal(got, want)
+    assert ((got.double() - reference(u, a, b, kind)).abs() <= 1e-4 * (1 + got.double().abs())).all()
