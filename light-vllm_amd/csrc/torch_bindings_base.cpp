@@ -280,25 +280,26 @@ std::optional<torch::Tensor> prompt_linear(const torch::Tensor& x, const std::op
 }
 
 // x w^T + bias of a prompt of some hundreds of rows, GELU behind it where asked for; `slabs`: or fp32 sums of shares of K, [shares, rows, n],
-// without the bias.  Nothing where the library's product is faster, or the operands are none that the kernels take
+// without the bias; `ordered`: sums one k after the other.  Nothing where the library's product is faster, or the operands are none that the kernels take
 std::optional<torch::Tensor> prompt_product(const torch::Tensor& x, const torch::Tensor& w_packed, const std::optional<torch::Tensor>& bias,
-                                            int64_t n, bool gelu, bool slabs) {
+                                            int64_t n, bool gelu, bool slabs, bool ordered) {
   const char* op = "prompt_product";
   LV_CHECK_DEVICE(x);
   TORCH_CHECK(x.dim() == 2 && w_packed.numel() == n * x.size(1) && w_packed.device() == x.device(), op, ": x [rows, k] and weights [n, k] packed");
   TORCH_CHECK(!bias || (bias->numel() == n && bias->device() == x.device()), op, ": a bias [n]");
   const int64_t rows = x.size(0), k = x.size(1);
   auto aligned = [](const torch::Tensor& t) { return ((uintptr_t)t.data_ptr() & 15) == 0; };
-  if (x.scalar_type() != at::kBFloat16 || w_packed.scalar_type() != at::kBFloat16 || !x.is_contiguous() || !w_packed.is_contiguous() ||
-      !aligned(x) || !aligned(w_packed) || rows > 8192 || n >= (1 << 24) || k >= (1 << 24) ||
+  if (x.scalar_type() != at::kBFloat16 || w_packed.scalar_type() != at::kBFloat16 || x.stride(1) != 1 || x.stride(0) < k ||
+      x.stride(0) % 8 != 0 || !w_packed.is_contiguous() || !aligned(x) || !aligned(w_packed) || rows > 8192 || n >= (1 << 24) || k >= (1 << 24) ||
       (bias && (bias->scalar_type() != at::kBFloat16 || !bias->is_contiguous() || !aligned(*bias))))
     return std::nullopt;
-  int plan[4];
-  const int shares = lvllm_prompt_product_plan((int)rows, (int)n, (int)k, gelu, slabs && !gelu, plan);
+  int plan[3];
+  const int sums = gelu ? LVLLM_SUMS_ANY : ordered ? LVLLM_SUMS_ORDERED : slabs ? LVLLM_SUMS_SLABS : LVLLM_SUMS_ANY;
+  const int shares = lvllm_prompt_product_plan((int)rows, (int)n, (int)k, gelu, sums, plan);
   if (shares == 0) return std::nullopt;
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(x));
   auto out = shares > 1 ? torch::empty({shares, rows, n}, x.options().dtype(at::kFloat)) : torch::empty({rows, n}, x.options());
-  check(lvllm_prompt_product(shares > 1 ? nullptr : out.data_ptr(), shares > 1 ? out.data_ptr<float>() : nullptr, x.data_ptr(),
+  check(lvllm_prompt_product(shares > 1 ? nullptr : out.data_ptr(), shares > 1 ? out.data_ptr<float>() : nullptr, x.data_ptr(), x.stride(0),
                              w_packed.data_ptr(), bias && shares == 1 ? bias->data_ptr() : nullptr, (int)rows, (int)n, (int)k, gelu, plan,
                              current_stream(x)));
   return out;
@@ -742,7 +743,7 @@ TORCH_LIBRARY_FRAGMENT(_C_amd, amd) {
   amd.impl("clamped_unit", torch::kCUDA, &clamped_unit);
   amd.def("prompt_linear(Tensor x, Tensor? w, Tensor? w_packed, Tensor? bias, int outputs, int act, float limit=0.) -> Tensor?");
   amd.impl("prompt_linear", torch::kCUDA, &prompt_linear);
-  amd.def("prompt_product(Tensor x, Tensor w_packed, Tensor? bias, int n, bool gelu=False, bool slabs=False) -> Tensor?");
+  amd.def("prompt_product(Tensor x, Tensor w_packed, Tensor? bias, int n, bool gelu=False, bool slabs=False, bool ordered=False) -> Tensor?");
   amd.impl("prompt_product", torch::kCUDA, &prompt_product);
   amd.def("silu_unit(Tensor x) -> Tensor");
   amd.impl("silu_unit", torch::kCUDA, &silu_unit);

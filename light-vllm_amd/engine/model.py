@@ -69,11 +69,16 @@ def linear(x: torch.Tensor, w: "Weight", bias: Optional[torch.Tensor] = None) ->
         # 65..256 rows: X through LDS, one pass over the packed weights -- where it beats the library
         # (tools/bench_stream_gemm.py, M = 128: down 37 vs 76 us, o 21 vs 24, qkv 26 vs 27; not gate_up: 59 vs 55)
         return torch.ops._C_amd.stream_linear_packed(x, w.packed, bias, w.N, w.K)
+    elif x.is_cuda and w.packed is not None and not _CALIBRATING:
+        # prompts of some hundreds of rows: sums one k after the other, as the library's are but where it cuts K (csrc/prompt_product.h)
+        y = torch.ops._C_amd.prompt_product(x, w.packed, bias, w.N, ordered=True)
+        if y is not None:
+            return y
     return F.linear(x, w.w, bias)
 
 
 def product(x: torch.Tensor, w: "Weight", bias: Optional[torch.Tensor] = None, slabs: bool = False) -> torch.Tensor:
-    """linear(), for models without routers: its sums go another way for prompts of some hundreds of rows (csrc/prompt_product.h), and ahead of a
+    """linear(), for models without routers: its sums go any way for prompts of some hundreds of rows (csrc/prompt_product.h), where ahead of a
     router the last bits decide which expert a token takes.  `slabs`: or fp32 [s, rows, N], whose sum the next launch takes, without the bias."""
     if x.shape[0] > 64 and x.is_cuda and w.packed is not None and not _CALIBRATING:
         y = torch.ops._C_amd.prompt_product(x, w.packed, bias, w.N, False, slabs)

@@ -6,7 +6,6 @@ import torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-SHORT, TILE = 1, 2
 
 
 @pytest.fixture(scope="module")
@@ -29,29 +28,29 @@ def bound(x, w, k):  # k additions in 32 bits, in any order
 
 
 SIZES = [(16, 128), (17, 144), (65, 16), (100, 272), (129, 240), (300, 304)]  # rows, n: remainders of tiles of rows, and of blocks of weights
-PLANS = [(SHORT, 16, 4), (SHORT, 32, 4), (SHORT, 48, 4), (SHORT, 64, 4), (SHORT, 32, 8), (TILE, 64, 2), (TILE, 80, 4), (TILE, 96, 2),
-         (TILE, 112, 4), (TILE, 128, 2), (TILE, 128, 4)]
+PLANS = [(16, 1), (32, 1), (48, 1), (64, 1), (80, 1), (96, 1), (64, 2), (80, 2), (96, 2), (112, 2), (128, 2), (80, 4), (112, 4), (128, 4)]
 
 
 @pytest.mark.parametrize("rows,n", SIZES)
-@pytest.mark.parametrize("body,size,nt", PLANS)
+@pytest.mark.parametrize("size,nt", PLANS)
 @pytest.mark.parametrize("k", [256, 896, 2560])
-def test_bodies(lib, rows, n, body, size, nt, k):
+def test_bodies(lib, rows, n, size, nt, k):
     x, w, packed, b = operands(rows, n, k)
+    ld = k + 8 if size % 32 else k  # rows of x beside others
+    x = torch.nn.functional.pad(x, (0, ld - k))[:, :k]
     want, err = x.double() @ w.double().t(), bound(x, w, k)
     p = lambda t: ctypes.c_void_p(0 if t is None else t.data_ptr())
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     for shares in (1, 2, 3, 8):
-        batch = 4 if (body, size) == (SHORT, 16) else 2
-        if -(-(k // 32 // batch) // shares) * batch * (shares - 1) >= k // 32:
+        if -(-(k // 64) // shares) * 2 * (shares - 1) >= k // 32:
             continue  # (a share without steps: refused)
-        plan = (ctypes.c_int * 4)(body, size, nt, shares)
-        for gelu in (False, True) if shares == 1 and body == SHORT else (False,):
+        plan = (ctypes.c_int * 3)(size, nt, shares)
+        for gelu in (False, True) if shares == 1 and nt < 4 else (False,):
             out = torch.full((rows + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)  # (a row behind the last: not written)
             slabs = torch.full((shares * rows + 1, n), 7.0, device=DEV) if shares > 1 else None
             bias = b if shares == 1 else None
-            print(rows, n, k, body, size, nt, shares, gelu, flush=True)
-            rc = lib.lvllm_prompt_product(p(out if shares == 1 else None), p(slabs), p(x), p(packed), p(bias), rows, n, k, int(gelu), plan, stream)
+            print(rows, n, k, size, nt, shares, gelu, flush=True)
+            rc = lib.lvllm_prompt_product(p(out if shares == 1 else None), p(slabs), p(x), ctypes.c_int64(ld), p(packed), p(bias), rows, n, k, int(gelu), plan, stream)
             assert rc == 0, lib.lvllm_last_error()
             if shares > 1:
                 got = slabs[:-1].view(shares, rows, n).double().sum(0)
@@ -75,6 +74,24 @@ def test_op(lib, rows, n, k):
     z = torch.ops._C_amd.prompt_product(x, packed, b, n)
     if z is not None:
         assert bool(((z.double() - want - b.double()).abs() <= err + 2.0 ** -8 * (want + b.double()).abs() + 2.0 ** -23 * want.abs()).all())
+
+
+@pytest.mark.parametrize("rows,n,k", [(65, 2048, 2048), (100, 1024, 512), (257, 7680, 2048), (300, 2048, 5632), (520, 3072, 1536), (800, 2048, 3072)])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_sums_in_order(lib, rows, n, k, with_bias):
+    """Every tile adds one k-step of 32 behind the other: the same bits, whichever takes a product (ahead of routers, the last ones matter)."""
+    x, w, packed, b = operands(rows, n, k)
+    bias = b if with_bias else None
+    y = torch.ops._C_amd.prompt_product(x, packed, bias, n, ordered=True)
+    assert y is not None and y.shape == (rows, n)
+    p = lambda t: ctypes.c_void_p(0 if t is None else t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for size, nt in PLANS:
+        out = torch.empty_like(y)
+        plan = (ctypes.c_int * 3)(size, nt, 1)
+        print(rows, n, k, size, nt, flush=True)
+        rc = lib.lvllm_prompt_product(p(out), None, p(x), ctypes.c_int64(k), p(packed), p(bias), rows, n, k, 0, plan, stream)
+        assert rc == 0 and torch.equal(out, y), (size, nt)
 
 
 def test_operands_that_the_library_takes(lib):
