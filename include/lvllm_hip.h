@@ -712,13 +712,14 @@ int lvllm_prompt_linear(void* out, const void* x, const void* w, const void* w_p
                         int act, float limit, int dtype, void* stream);
 /* x w^T of prompts of some hundreds of rows, x [rows, k], w [n, k] packed (lvllm_pack_weight), bf16.  The plan (three numbers) holds for one
  * device and these sizes; the call returns the shares that K is cut into, 0 where the library's product is the better one.  `sums`: how those of K
- * are taken, in any order (ANY), as slabs that the caller sums where K is cut (SLABS), or one k after the other (ORDERED: without GELU). */
+ * are taken, in any order (ANY), as slabs that the caller sums where K is cut (SLABS), or one k after the other (ORDERED: without GELU).  `batch`: so
+ * many products of these sizes, 1 to 64, in one launch. */
 enum { LVLLM_SUMS_ANY = 0, LVLLM_SUMS_SLABS = 1, LVLLM_SUMS_ORDERED = 2 };
-int lvllm_prompt_product_plan(int rows, int n, int k, int gelu, int sums, int* plan);
-/* one share: out [rows, n] = x w^T + bias (null: none), GELU behind it where asked for; more: slabs [shares, rows, n], plain sums.  x_stride:
- * of x's rows, in elements, a multiple of 8 */
-int lvllm_prompt_product(void* out, float* slabs, const void* x, int64_t x_stride, const void* w_packed, const void* bias, int rows, int n,
-                         int k, int gelu, const int* plan, void* stream);
+int lvllm_prompt_product_plan(int rows, int n, int k, int gelu, int sums, int batch, int* plan);
+/* one share: out [rows, n] = x w^T + bias (null: none), GELU behind it where asked for; more: slabs [shares, rows, n], plain sums.
+ * batch > 1: out [batch, rows, n], w_packed back to back, no bias.  x_stride, x_batch_stride: of x's rows and batches, in elements, multiples of 8 */
+int lvllm_prompt_product(void* out, float* slabs, const void* x, int64_t x_stride, int64_t x_batch_stride, const void* w_packed,
+                         const void* bias, int rows, int n, int k, int gelu, int batch, const int* plan, void* stream);
 /* ---- mixtures of experts (csrc/moe*.hip, moe.h) ---- */
 enum { LVLLM_MOE_SOFTMAX = 0, LVLLM_MOE_SIGMOID = 1 };  /* weights: softmax over the chosen logits, or each logit's sigmoid */
 enum { LVLLM_MOE_NO_SHARED = 0, LVLLM_MOE_GATED_SHARED = 1, LVLLM_MOE_PLAIN_SHARED = 2 };

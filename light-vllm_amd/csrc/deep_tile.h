@@ -2,9 +2,9 @@
 // (moe_tile.h).  There a workgroup's waves are on their own: what one of them waits for, no other covers.  A wave issues in order, 16 cycles
 // a MFMA, and a load of 1 KiB keeps the CU's one address unit for as long, so that four waves whose loads stand together wait 64 cycles for each:
 // loads and MFMAs took turns (80 rows x 128: 356 cycles a k-step, 160 of MFMAs and 224 of loads).  Here the loads are dealt
-// among the MFMAs, and fragments are read a k-step ahead.  us of 32 such k-steps of two, a workgroup a CU: 64 rows x 64 9.4, 8.0; 96 x 128 14.6, 11.2;
-// 128 x 128 18.3, 13.3.  Two workgroups a CU: 112 x 128 29.5, 27.7; 64 x 128 37.4, 39.0.  More stages than these were slower, so that it is
-// not memory's latency that is left (64 x 64, 16 and 24 k-steps under way 9.8 and 11.0 us for 9.4).
+// among the MFMAs, and fragments are read a k-step ahead.  us of 64 k-steps, weights in the last cache, a workgroup a CU: 64 rows x 64 9.4, 8.0; 96 x
+// 128 14.6, 11.2; 128 x 128 18.3, 13.3; two a CU: 112 x 128 29.5, 27.7; 64 x 128 37.4, 39.0.  From memory, 4096 x 4096, 300 rows 25.9 (the
+// library's), 19.8.
 #pragma once
 #include <type_traits>
 
@@ -12,16 +12,17 @@
 
 namespace lvllm {
 
-// stages of two k-steps under way: as many as leave two workgroups a CU (80 KiB each) and, for NT = 2, registers for their weights
-constexpr int deep_stages(int NT, int MT) { return MT <= 4 ? 8 : MT <= 6 ? 6 : 5; }
+// stages of two k-steps under way: as many as leave two workgroups a CU (80 KiB each) and registers for their weights.  Three are slower (2048 x 2048,
+// 300 rows from memory 11.3 us, 8.8), four to eight alike
+constexpr int deep_stages(int MT) { return MT <= 6 ? 6 : 5; }
 constexpr int deep_stage_bytes(int MT) { return 4096 * ((MT + 1) / 2); }
-constexpr int deep_lds_bytes(int NT, int MT) { return deep_stages(NT, MT) * deep_stage_bytes(MT); }
+constexpr int deep_lds_bytes(int MT) { return deep_stages(MT) * deep_stage_bytes(MT); }
 
-// t.steps: even.  `ring`: deep_lds_bytes.  Ends with LDS free, for every wave.
-template <int NT, int MT>
+// t.steps: even.  `ring`: deep_lds_bytes.  tile_of: where in w a W tile lies.  Ends with LDS free, for every wave.
+template <int NT, int MT, class TILE>
 __device__ __forceinline__ void deep_sums(e_f32x4_t (&acc)[NT][MT], const uint16_t* x_rows, const int64_t ld, const uint16_t* w_tiles,
-                                          const TileWork& t, char* ring) {
-  constexpr int X = deep_stages(NT, MT), S = 2 * X, kCopies = (MT + 1) / 2, kStage = deep_stage_bytes(MT);
+                                          const TileWork& t, char* ring, TILE tile_of) {
+  constexpr int X = deep_stages(MT), S = 2 * X, kCopies = (MT + 1) / 2, kStage = deep_stage_bytes(MT);
   constexpr int kNow = (kCopies + 1) / 2, kLater = kCopies - kNow;  // of a stage's copies: with its first k-step's weights, with its second's
   constexpr int kYounger = NT + (X - 2) * (2 * NT + kCopies);       // loads behind the copies of the next stage
   constexpr int kFirst = kYounger + NT + kNow;
@@ -32,7 +33,7 @@ __device__ __forceinline__ void deep_sums(e_f32x4_t (&acc)[NT][MT], const uint16
   // this wave's W tiles, and the rows it copies: lane l moves chunk l % 8, exchanged by the row, of row l / 8 of eight
   const uint16_t *wsrc[NT], *xsrc[kCopies];
 #pragma unroll
-  for (int n = 0; n < NT; ++n) wsrc[n] = w_tiles + (int64_t)min(nt0 + n, t.ntiles - 1) * t.all * 512 + lane * 8;
+  for (int n = 0; n < NT; ++n) wsrc[n] = w_tiles + (int64_t)tile_of(min(nt0 + n, t.ntiles - 1)) * t.all * 512 + lane * 8;
 #pragma unroll
   for (int i = 0; i < kCopies; ++i)
     xsrc[i] = x_rows + min(t.s0 + (wave * kCopies + i) * 8 + (lane >> 3), t.s1 - 1) * ld + ((lane & 7) ^ (lane >> 3)) * 8;

@@ -23,35 +23,36 @@ inline int64_t product_units(const ProductPlan& p, int rows, int n) {
 }
 
 // us of a launch: a workgroup's way in and out, its k-steps, and the megabytes that leave; of workgroups that have a CU each, and of up to two a
-// CU.  Least squares over 4086 products of 65 to 2200 rows, n 768 to 11264, k 512 to 14336, all plans of up to 512 workgroups: 4 to 10 %
-// (root mean square) off; what it chooses takes 0.4 % longer than the best plan with K whole, 1.0 % where it may be cut.
+// CU.  Least squares over 3702 products of 65 to 2200 rows, n 768 to 11264, k 512 to 14336, all plans of up to 512 workgroups, weights that
+// no cache holds (as in a model whose layers take turns): 5 to 12 % (root mean square) off; what it chooses takes 1.4 % longer than the best plan
+// with K whole, 1.8 % where it may be cut.
 struct ProductTimes {
   float fixed, step, out;
 };
-inline double product_time(const ProductPlan& p, int rows, int n, int k) {
+inline double product_time(const ProductPlan& p, int rows, int n, int k, int batch = 1) {
   static const ProductTimes kOne[6][2] = {
-      {{2.723f, 0.05187f, 0.3175f}, {3.247f, 0.1022f, 0.1113f}},
-      {{2.477f, 0.06026f, 0.445f}, {3.039f, 0.1207f, 0.2109f}},
-      {{2.723f, 0.07458f, 0.3617f}, {3.276f, 0.1522f, 0.2328f}},
-      {{2.586f, 0.08304f, 0.4016f}, {3.141f, 0.1714f, 0.2446f}},
-      {{2.732f, 0.09542f, 0.3601f}, {3.265f, 0.1932f, 0.2565f}},
-      {{2.691f, 0.1032f, 0.3742f}, {3.199f, 0.2142f, 0.2505f}}};  // nt = 1; 16, 32 .. 96 rows
+      {{2.623f, 0.0794f, 0.3561f}, {2.06f, 0.1357f, 0.8835f}},
+      {{2.772f, 0.08631f, 0.334f}, {2.592f, 0.1521f, 0.4529f}},
+      {{2.892f, 0.09792f, 0.3492f}, {2.551f, 0.1767f, 0.4665f}},
+      {{2.874f, 0.1034f, 0.3875f}, {2.606f, 0.2003f, 0.3941f}},
+      {{3.187f, 0.1175f, 0.3382f}, {2.689f, 0.2247f, 0.3988f}},
+      {{3.315f, 0.1258f, 0.3171f}, {2.524f, 0.2421f, 0.4105f}}};  // nt = 1; 16, 32 .. 96 rows
   static const ProductTimes kTwo[5][2] = {
-      {{3.063f, 0.123f, 0.3697f}, {4.133f, 0.2644f, 0.2241f}},
-      {{3.205f, 0.1376f, 0.3229f}, {3.97f, 0.2876f, 0.2283f}},
-      {{3.213f, 0.1513f, 0.3139f}, {4.039f, 0.3143f, 0.2192f}},
-      {{3.326f, 0.1653f, 0.3002f}, {3.992f, 0.3487f, 0.2052f}},
-      {{3.582f, 0.1753f, 0.2888f}, {4.465f, 0.3727f, 0.1884f}}};  // nt = 2; up to 64, 80, 96, 112, 128 rows
+      {{3.552f, 0.1735f, 0.269f}, {3.288f, 0.3065f, 0.3384f}},
+      {{4.268f, 0.1862f, 0.2083f}, {2.794f, 0.331f, 0.3679f}},
+      {{4.584f, 0.1957f, 0.1974f}, {2.819f, 0.3559f, 0.3446f}},
+      {{4.603f, 0.2101f, 0.2022f}, {2.893f, 0.3802f, 0.309f}},
+      {{4.731f, 0.2273f, 0.2055f}, {3.128f, 0.4086f, 0.2885f}}};  // nt = 2; up to 64, 80, 96, 112, 128 rows
   static const ProductTimes kFour[5][2] = {
-      {{3.328f, 0.2258f, 0.2683f}, {5.358f, 0.418f, 0.1452f}},
-      {{4.188f, 0.2516f, 0.2239f}, {5.208f, 0.4717f, 0.1583f}},
-      {{4.902f, 0.2954f, 0.1948f}, {5.888f, 0.5416f, 0.1476f}},
-      {{5.479f, 0.3346f, 0.1796f}, {6.677f, 0.6068f, 0.136f}},
-      {{5.987f, 0.3597f, 0.1672f}, {6.839f, 0.656f, 0.1376f}}};  // nt = 4
-  const bool two = product_units(p, rows, n) > 256;
+      {{3.798f, 0.2844f, 0.2426f}, {4.425f, 0.4436f, 0.2531f}},
+      {{4.429f, 0.2968f, 0.2107f}, {2.732f, 0.4958f, 0.2947f}},
+      {{4.823f, 0.3157f, 0.2116f}, {3.968f, 0.5675f, 0.2346f}},
+      {{5.339f, 0.3472f, 0.1954f}, {4.613f, 0.6315f, 0.2096f}},
+      {{5.629f, 0.3732f, 0.1902f}, {4.f, 0.6884f, 0.2167f}}};  // nt = 4
+  const bool two = product_units(p, rows, n) * batch > 256;
   const int at = p.size <= 64 ? 0 : p.size / 16 - 4;
   const ProductTimes& t = p.nt == 1 ? kOne[p.size / 16 - 1][two] : p.nt == 2 ? kTwo[at][two] : kFour[at][two];
-  const double mb = (double)rows * n * 1e-6;
+  const double mb = (double)rows * n * batch * 1e-6;
   double us = t.fixed + t.step * product_share(p, k) + t.out * mb * (p.shares > 1 ? 4 * p.shares : 2);
   if (p.shares > 1) us += .2 * mb * (4 * p.shares - 2);  // the slabs' way into the launch that sums them
   return us;
@@ -59,24 +60,24 @@ inline double product_time(const ProductPlan& p, int rows, int n, int k) {
 
 enum { kSumsAny = 0, kSumsSlabs = 1, kSumsOrdered = 2 };  // include/lvllm_hip.h LVLLM_SUMS_*
 
-// The shortest of the plans, and the library where its products are the better ones, by the rate that the plan reaches, TFLOP/s (of those 4086, own
+// The shortest of the plans, and the library where its products are the better ones, by the rate that the plan reaches, TFLOP/s (of those 3702, own
 // time of the library's; host time, 3 us for 20, not counted):
-//   * up to 900; above k = 5120 1050, and above k = 9000, where the library has too few tiles for too long, 1400.  From there on the library's,
-//     both of whose operands go through LDS, take less power: 0.94 to 1.2 of its time;
-//   * one share, whose sums are in the library's order but where that cuts K: 0.76 of its time in the mean up to k = 2048, 0.81 up to 5120, 0.88 above
-//     (us, before and after: 300 rows of 2048 for 2048 11.2, 7.8; for 7680 19.8, 13.8; 300 rows of 5632 for 2048 20.7, 17.1; 1000 rows of 1024 for
-//     3072 14.4, 10.3).  With few tiles of long K the library cuts it and is faster: 0.96 to 1.4 below 100 for k > 2048, 200 for k > 5120, 300
-//     for k > 9000;
-//   * K may be cut into slabs: 0.74, 0.75 and 0.70, what the slabs cost the next launch included (300 rows of 14336 for 4096 75, 51; 100 rows 48,
-//     29; 300 rows of 4096 for 1024 13.8, 7.7).
-inline ProductPlan prompt_product_plan(int rows, int n, int k, bool gelu, int sums) {
+//   * up to 900; above k = 5120 1000, and above k = 9000, where the library has too few tiles for too long, 1150.  From there on the library's,
+//     both of whose operands go through LDS, take less power: 0.95 to 1.2 of its time;
+//   * one share, whose sums are in the library's order but where that cuts K: 0.64 of its time in the mean up to k = 1024, 0.79 up to 2048, 0.86 up to
+//     5120, 0.90 above (us, before and after: 300 rows of 2048 for 2048 12.9, 8.8; for 7680 25.4, 19.0; 300 rows of 5632 for 2048 25.7, 20.8).  With
+//     few tiles of long K the library cuts it and is faster: 0.99 to 1.6 below 100 for k > 2048, below 200 for k > 5120;
+//   * K may be cut into slabs: 0.64, 0.75, 0.77 and 0.70, what the slabs cost the next launch included (300 rows of 14336 for 4096 75, 50; 100 rows 48,
+//     29; 300 rows of 4096 for 1024 14.6, 8.7).
+// `batch` products of one size in a launch (K whole): as one of so many times the tiles.
+inline ProductPlan prompt_product_plan(int rows, int n, int k, bool gelu, int sums, int batch = 1) {
   ProductPlan best{0, 0, 0};
-  if (rows <= 64 || rows > 8192 || n < 16 || n % 16 != 0 || k < 256 || k % 64 != 0 || (int64_t)n * k >= (int64_t)1 << 30) return best;
-  const bool slabs = sums == kSumsSlabs && !gelu;
+  if (rows <= 64 || rows > 8192 || n < 16 || n % 16 != 0 || k < 256 || k % 64 != 0 || (int64_t)n * k >= (int64_t)1 << 30 || batch < 1 || batch > 64) return best;
+  const bool slabs = sums == kSumsSlabs && !gelu && batch == 1;
   double least = 0;
   auto take = [&](const ProductPlan& p) {
-    if (!product_plan_valid(p, k) || product_units(p, rows, n) > 512 || (p.shares > 1 && k / 32 / p.shares < 8)) return;
-    const double us = product_time(p, rows, n, k);
+    if (!product_plan_valid(p, k) || product_units(p, rows, n) * batch > 512 || (p.shares > 1 && k / 32 / p.shares < 8)) return;
+    const double us = product_time(p, rows, n, k, batch);
     if (best.size == 0 || us < least) best = p, least = us;
   };
   for (int shares = 1; shares <= (slabs ? kProductShares : 1); ++shares) {
@@ -92,8 +93,8 @@ inline ProductPlan prompt_product_plan(int rows, int n, int k, bool gelu, int su
     }
   }
   if (best.size == 0) return best;
-  const double rate = 2e-6 * rows * n * k / least;
-  const double fewest = slabs || k <= 2048 ? 0 : k <= 5120 ? 100 : k <= 9000 ? 200 : 300, most = k <= 5120 ? 900 : k <= 9000 ? 1050 : 1400;
+  const double rate = 2e-6 * rows * n * k * batch / least;
+  const double fewest = slabs || k <= 2048 ? 0 : k <= 5120 ? 100 : 200, most = k <= 5120 ? 900 : k <= 9000 ? 1000 : 1150;
   return rate >= fewest && rate <= most ? best : ProductPlan{0, 0, 0};
 }
 

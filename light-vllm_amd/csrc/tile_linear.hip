@@ -3,8 +3,8 @@
 // 4096: 125 us for 105 and 49 in two launches (one workgroup a CU 149), on another card 143 for 162; prompt_linear.h has more.
 #include <type_traits>
 
+#include "deep_tile.h"
 #include "gelu.h"
-#include "moe_tile.h"
 #include "prompt_act.h"
 #include "prompt_linear.h"
 
@@ -17,19 +17,20 @@ struct TileLinear {
   float limit;                    // CLAMPED_UNIT
 };
 
-template <int ACT, int NT, int MT>
-__device__ __forceinline__ void tile_linear(const TileLinear& p, const TileWork& t, char (*ring)[kStageBytes]) {
+template <int ACT, int NT, int MT, bool DEEP>
+__device__ __forceinline__ void tile_linear(const TileLinear& p, const TileWork& t, char* lds) {
   constexpr bool GELU = ACT == LVLLM_ACT_GELU, PAIRS = prompt_pairs(ACT);
   e_f32x4_t acc[NT][MT];
   // PAIRS: 16 gate rows, the 16 value rows that belong to them, ...
-  tile_sums<false>(acc, p.x, p.k, p.w, t, ring, [](int slot) { return slot; },
-                   [&](int tile) { return PAIRS ? (tile & 1) * (p.outputs >> 4) + (tile >> 1) : tile; });
+  auto tile_of = [&](int tile) { return PAIRS ? (tile & 1) * (p.outputs >> 4) + (tile >> 1) : tile; };
+  if constexpr (DEEP) deep_sums(acc, p.x, p.k, p.w, t, lds, tile_of);
+  else tile_sums<false>(acc, p.x, p.k, p.w, t, reinterpret_cast<char(*)[kStageBytes]>(lds), [](int slot) { return slot; }, tile_of);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nt0 = (t.block * 4 + wave) * NT, g = (threadIdx.x & 63) >> 4;
   float z[NT][4];
   if constexpr (GELU)
 #pragma unroll
     for (int n = 0; n < NT; ++n) load4<BF16>(p.bias + min(nt0 + n, t.ntiles - 1) * 16 + 4 * g, z[n]);
-  tile_store<PAIRS>(p.out, p.outputs, acc, ring[0] + wave * 2048, nt0, t.ntiles, t.s0, t.s1, [](int) { return 1.f; },
+  tile_store<PAIRS>(p.out, p.outputs, acc, lds + wave * 2048, nt0, t.ntiles, t.s0, t.s1, [](int) { return 1.f; },
                     [&](float, int n, const e_f32x4_t& a, const e_f32x4_t& b, float (&v)[4]) {
 #pragma unroll
                       for (int r = 0; r < 4; ++r) {
@@ -39,10 +40,12 @@ __device__ __forceinline__ void tile_linear(const TileLinear& p, const TileWork&
                     });
 }
 
-// An eighth of the tiles to each XCD, 1024 rows side by side, W block after W block.
-template <int ACT, int NT>
+// An eighth of the tiles to each XCD, 1024 rows side by side, W block after W block.  DEEP: half tiles by deep_tile.h, k a multiple of 64.  us, weights
+// from memory: squared ReLU of 8448, 2048 wide, 300 rows (198 half tiles) 22.5, 19.9; 500 (264) 32.9, 29.4; 700 (396) 33.5, 32.6; the clamped unit
+// of 5632, 200 rows (176) 23.0, 21.7.  Not GELU, whose instructions take the loads' place: 4096, 1024 wide, 1000 rows (256) 14.8, 15.1.
+template <int ACT, int NT, bool DEEP>
 __global__ __launch_bounds__(256, 2) void tile_linear_kernel(const TileLinear p) {
-  __shared__ __attribute__((aligned(16))) char ring[tile_steps(NT) / 2][kStageBytes];
+  __shared__ __attribute__((aligned(16))) char ring[DEEP ? deep_lds_bytes(8) : tile_steps(NT) / 2 * kStageBytes];
   constexpr int kSide = 1024 / kMoeTile;
   const int units = p.tiles * p.blocks, per = (units + 7) >> 3, mine = blockIdx.x >> 3, unit = (blockIdx.x & 7) * per + mine;
   if (mine >= per || unit >= units) return;
@@ -56,9 +59,11 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(const TileLinear p)
   t.steps = t.all = p.k >> 5;
   t.ntiles = (prompt_pairs(ACT) ? 2 : 1) * (p.outputs >> 4);
   const int groups = (t.s1 - t.s0 + 15) >> 4;
-  if (groups <= 4) tile_linear<ACT, NT, 4>(p, t, ring);
-  else if (groups <= 6) tile_linear<ACT, NT, 6>(p, t, ring);
-  else tile_linear<ACT, NT, 8>(p, t, ring);
+  if (groups <= 4) tile_linear<ACT, NT, 4, DEEP>(p, t, ring);
+  else if (DEEP && groups <= 5) tile_linear<ACT, NT, DEEP ? 5 : 6, DEEP>(p, t, ring);
+  else if (groups <= 6) tile_linear<ACT, NT, 6, DEEP>(p, t, ring);
+  else if (DEEP && groups <= 7) tile_linear<ACT, NT, DEEP ? 7 : 8, DEEP>(p, t, ring);
+  else tile_linear<ACT, NT, 8, DEEP>(p, t, ring);
 }
 
 int launch_tile_linear(void* out, const void* x, const void* w, const void* bias, int rows, int outputs, int k, int act, float limit,
@@ -67,14 +72,16 @@ int launch_tile_linear(void* out, const void* x, const void* w, const void* bias
   p.out = (uint16_t*)out; p.x = (const uint16_t*)x; p.w = (const uint16_t*)w; p.bias = (const uint16_t*)bias;
   p.rows = rows; p.outputs = outputs; p.k = k; p.limit = limit;
   p.tiles = (rows + kMoeTile - 1) / kMoeTile;
-  auto launch = [&](auto act, auto nt) {
+  auto launch = [&](auto act, auto nt, auto deep) {
     constexpr int ACT = decltype(act)::value, NT = decltype(nt)::value;
     p.blocks = ((prompt_pairs(ACT) ? 2 : 1) * outputs + 64 * NT - 1) / (64 * NT);
-    hipLaunchKernelGGL((tile_linear_kernel<ACT, NT>), dim3((p.tiles * p.blocks + 7) / 8 * 8), dim3(256), 0, (hipStream_t)stream, p);
+    hipLaunchKernelGGL((tile_linear_kernel<ACT, NT, decltype(deep)::value>), dim3((p.tiles * p.blocks + 7) / 8 * 8), dim3(256), 0, (hipStream_t)stream, p);
   };
   auto with = [&](auto act) {
-    if (nt == 4) launch(act, std::integral_constant<int, 4>{});
-    else launch(act, std::integral_constant<int, 2>{});
+    constexpr std::integral_constant<int, 2> two{};
+    if (nt == 4) launch(act, std::integral_constant<int, 4>{}, std::false_type{});
+    else if (k % 64 == 0 && act != LVLLM_ACT_GELU) launch(act, two, std::integral_constant<bool, decltype(act)::value != LVLLM_ACT_GELU>{});
+    else launch(act, two, std::false_type{});
   };
   if (act == LVLLM_ACT_GELU) with(std::integral_constant<int, LVLLM_ACT_GELU>{});
   else if (act == LVLLM_ACT_RELU_SQUARED) with(std::integral_constant<int, LVLLM_ACT_RELU_SQUARED>{});

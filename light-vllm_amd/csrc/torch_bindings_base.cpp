@@ -295,13 +295,33 @@ std::optional<torch::Tensor> prompt_product(const torch::Tensor& x, const torch:
     return std::nullopt;
   int plan[3];
   const int sums = gelu ? LVLLM_SUMS_ANY : ordered ? LVLLM_SUMS_ORDERED : slabs ? LVLLM_SUMS_SLABS : LVLLM_SUMS_ANY;
-  const int shares = lvllm_prompt_product_plan((int)rows, (int)n, (int)k, gelu, sums, plan);
+  const int shares = lvllm_prompt_product_plan((int)rows, (int)n, (int)k, gelu, sums, 1, plan);
   if (shares == 0) return std::nullopt;
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(x));
   auto out = shares > 1 ? torch::empty({shares, rows, n}, x.options().dtype(at::kFloat)) : torch::empty({rows, n}, x.options());
   check(lvllm_prompt_product(shares > 1 ? nullptr : out.data_ptr(), shares > 1 ? out.data_ptr<float>() : nullptr, x.data_ptr(), x.stride(0),
-                             w_packed.data_ptr(), bias && shares == 1 ? bias->data_ptr() : nullptr, (int)rows, (int)n, (int)k, gelu, plan,
+                             0, w_packed.data_ptr(), bias && shares == 1 ? bias->data_ptr() : nullptr, (int)rows, (int)n, (int)k, gelu, 1, plan,
                              current_stream(x)));
+  return out;
+}
+
+// x[b] w[b]^T of prompts of some hundreds of rows, x [batch, rows, k], the packed weights back to back; nothing as above
+std::optional<torch::Tensor> prompt_products(const torch::Tensor& x, const torch::Tensor& w_packed, int64_t n) {
+  const char* op = "prompt_products";
+  LV_CHECK_DEVICE(x);
+  TORCH_CHECK(x.dim() == 3 && x.size(0) >= 1 && w_packed.numel() == x.size(0) * n * x.size(2) && w_packed.device() == x.device(), op,
+              ": x [batch, rows, k] and weights [batch, n, k] packed");
+  const int64_t batch = x.size(0), rows = x.size(1), k = x.size(2);
+  if (x.scalar_type() != at::kBFloat16 || w_packed.scalar_type() != at::kBFloat16 || x.stride(2) != 1 || x.stride(1) < k || x.stride(1) % 8 != 0 ||
+      x.stride(0) % 8 != 0 || !w_packed.is_contiguous() || (((uintptr_t)x.data_ptr() | (uintptr_t)w_packed.data_ptr()) & 15) != 0 || rows > 8192 ||
+      batch > 64 || n >= (1 << 24) || k >= (1 << 24))
+    return std::nullopt;
+  int plan[3];
+  if (lvllm_prompt_product_plan((int)rows, (int)n, (int)k, 0, LVLLM_SUMS_ANY, (int)batch, plan) == 0) return std::nullopt;
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(x));
+  auto out = torch::empty({batch, rows, n}, x.options());
+  check(lvllm_prompt_product(out.data_ptr(), nullptr, x.data_ptr(), x.stride(1), x.stride(0), w_packed.data_ptr(), nullptr, (int)rows, (int)n,
+                             (int)k, 0, (int)batch, plan, current_stream(x)));
   return out;
 }
 
@@ -745,6 +765,8 @@ TORCH_LIBRARY_FRAGMENT(_C_amd, amd) {
   amd.impl("prompt_linear", torch::kCUDA, &prompt_linear);
   amd.def("prompt_product(Tensor x, Tensor w_packed, Tensor? bias, int n, bool gelu=False, bool slabs=False, bool ordered=False) -> Tensor?");
   amd.impl("prompt_product", torch::kCUDA, &prompt_product);
+  amd.def("prompt_products(Tensor x, Tensor w_packed, int n) -> Tensor?");
+  amd.impl("prompt_products", torch::kCUDA, &prompt_products);
   amd.def("silu_unit(Tensor x) -> Tensor");
   amd.impl("silu_unit", torch::kCUDA, &silu_unit);
   amd.def("skinny_linear_packed_relu_squared(Tensor x, Tensor w_packed, int N, int K) -> Tensor");

@@ -205,7 +205,9 @@ class TimeMixer:
             if 0 < rows <= DECODE_ROWS and self.rkvg[0].packed is not None:
                 r, k, v, g = (linear(mix[i], w) for i, w in enumerate(self.rkvg))
             else:
-                r, k, v, g = torch.bmm(mix[:4], self.rkvg_t)
+                n, packed = self.rkvg[0].N, self.all_packed
+                some = amd.prompt_products(mix[:4], packed[:4 * n * self.w1.K], n) if packed is not None and rows > DECODE_ROWS else None
+                r, k, v, g = torch.bmm(mix[:4], self.rkvg_t) if some is None else some
             u = product(mix[4], self.w1)
         u = u[:, :self.rank]
         cols = self.cfg.heads * self.cfg.dim

@@ -50,7 +50,7 @@ def test_bodies(lib, rows, n, size, nt, k):
             slabs = torch.full((shares * rows + 1, n), 7.0, device=DEV) if shares > 1 else None
             bias = b if shares == 1 else None
             print(rows, n, k, size, nt, shares, gelu, flush=True)
-            rc = lib.lvllm_prompt_product(p(out if shares == 1 else None), p(slabs), p(x), ctypes.c_int64(ld), p(packed), p(bias), rows, n, k, int(gelu), plan, stream)
+            rc = lib.lvllm_prompt_product(p(out if shares == 1 else None), p(slabs), p(x), ctypes.c_int64(ld), ctypes.c_int64(0), p(packed), p(bias), rows, n, k, int(gelu), 1, plan, stream)
             assert rc == 0, lib.lvllm_last_error()
             if shares > 1:
                 got = slabs[:-1].view(shares, rows, n).double().sum(0)
@@ -90,8 +90,22 @@ def test_sums_in_order(lib, rows, n, k, with_bias):
         out = torch.empty_like(y)
         plan = (ctypes.c_int * 3)(size, nt, 1)
         print(rows, n, k, size, nt, flush=True)
-        rc = lib.lvllm_prompt_product(p(out), None, p(x), ctypes.c_int64(k), p(packed), p(bias), rows, n, k, 0, plan, stream)
+        rc = lib.lvllm_prompt_product(p(out), None, p(x), ctypes.c_int64(k), ctypes.c_int64(0), p(packed), p(bias), rows, n, k, 0, 1, plan, stream)
         assert rc == 0 and torch.equal(out, y), (size, nt)
+
+
+@pytest.mark.parametrize("batch,rows,n,k", [(4, 100, 2048, 2048), (4, 300, 2048, 2048), (4, 700, 512, 512), (3, 65, 1040, 320), (5, 129, 64, 256)])
+def test_batches(lib, batch, rows, n, k):
+    """Several products in a launch: what each is by itself."""
+    g = torch.Generator(device=DEV).manual_seed(batch)
+    x = torch.randn(batch + 1, rows, k, generator=g, device=DEV).bfloat16()[:batch]
+    ws = [(torch.randn(n, k, generator=g, device=DEV) * k ** -0.5).bfloat16() for _ in range(batch)]
+    packed = torch.cat([torch.ops._C_amd.pack_weight(w).reshape(-1) for w in ws])
+    y = torch.ops._C_amd.prompt_products(x, packed, n)
+    assert y is not None and y.shape == (batch, rows, n)
+    for b in range(batch):
+        want = x[b].double() @ ws[b].double().t()
+        assert bool(((y[b].double() - want).abs() <= bound(x[b], ws[b], k) + 2.0 ** -8 * want.abs()).all()), b
 
 
 def test_operands_that_the_library_takes(lib):
