@@ -10,7 +10,7 @@ import numpy as np
 import torch
 
 from .local_config import ClampedMlpConfig, ParallelHeadsConfig, RetentionConfig, RotaryConfig, RotaryHeadsConfig
-from .mixers import DECODE_ROWS, LayerCache, StepLayout, make_weight, pad_columns, project_to_residual, stack_rows
+from .mixers import DECODE_ROWS, ORDERED_ROWS, LayerCache, StepLayout, make_weight, pad_columns, project_to_residual, stack_rows
 from .model import Weight, linear, linear_act
 from .moe import MixtureOfExperts
 
@@ -168,7 +168,7 @@ class ParallelHeads:
 class ClampedMlp:
 
     def __init__(self, get, name: str, cfg: ClampedMlpConfig, pack: bool, routed: bool = False):
-        """routed: the model has routers, and sums of prompts keep the library's order: in another one tokens go to other experts."""
+        """routed: the model has routers, and sums of prompts keep the library's order (ORDERED_ROWS): in another one tokens go to other experts."""
         self.limit, self.routed = cfg.limit, routed
         # zero rows of gate and up give zero activations: all sizes may be padded for the weight-streaming kernel
         self.up = make_weight(stack_rows([get(name + ".gate"), get(name + ".up")], 32)[0], pack)
@@ -181,7 +181,8 @@ class ClampedMlp:
         if 0 < h.shape[0] <= DECODE_ROWS and self.up.packed is not None:
             a = amd.skinny_linear_packed_clamped_unit(h, self.up.packed, self.up.N, self.up.K, self.limit)
         else:
-            a = None if self.routed else linear_act(h, self.up, "clamped_unit", self.up.N // 2, self.limit)
+            fused = not self.routed or h.shape[0] <= ORDERED_ROWS
+            a = linear_act(h, self.up, "clamped_unit", self.up.N // 2, self.limit) if fused else None
             a = amd.clamped_unit(linear(h, self.up), self.limit) if a is None else a
         return Branch(project_to_residual(a, self.down))
 
