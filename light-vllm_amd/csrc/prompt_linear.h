@@ -21,7 +21,8 @@ struct PromptLinearPlan {
 // 11264, 2048 wide, 65 to 8192 rows):
 //   * whole tiles: a CU's second one beside the first 0.50 to 0.81 (0.65 to 0.81 from k = 3072 on); from the third on a round of both at 1.58
 //     (1.64), and 0.70 of ends;
-//   * half tiles (nt = 2): 0.71 alone, 0.85 to 1.19 two, then 1.05 a round and 0.45;
+//   * half tiles (nt = 2): 0.71 alone, 0.85 to 1.19 two, then 1.05 a round and 0.45 (0.9 to 1.0 of that where k is a multiple of 64, deep_tile.h; no
+//     choice between them and the others turned on it);
 //   * wide ones take turns, 256 tiles at a time, of 0.97, 1.28 and 1.64 with 2, 3 and 4 groups; of 0.88, 1.17, 1.50 from k = 3072 on, where
 //     their way in and out counts less.  Nothing covers their activations: 4 % more with SwiGLU, 10 % with the clamped unit, whose
 //     exponential and division are the mathematical library's.
