@@ -279,10 +279,20 @@ std::optional<torch::Tensor> prompt_linear(const torch::Tensor& x, const std::op
   return out;
 }
 
+torch::Tensor pack_weight(const torch::Tensor& w) {
+  TORCH_CHECK(w.is_cuda() && w.dim() == 2 && w.is_contiguous(), "pack_weight: contiguous [N,K] GPU tensor");
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(w));
+  auto out = torch::empty_like(w);
+  check(lvllm_pack_weight(out.data_ptr(), w.data_ptr(), (int)w.size(0), (int)w.size(1),
+                          dtype_code(w, "pack_weight"), current_stream(w)));
+  return out;
+}
+
 // x w^T + bias of a prompt of some hundreds of rows, GELU behind it where asked for; `slabs`: or fp32 sums of shares of K, [shares, rows, n],
-// without the bias; `ordered`: sums one k after the other.  Nothing where the library's product is faster, or the operands are none that the kernels take
+// without the bias; `ordered`: sums one k after the other.  Nothing where the library's product is faster, or the operands are none that the kernels take.
+// `row_major`: w_packed is the weights as they are, [n, k]; a launch ahead of the product packs them.
 std::optional<torch::Tensor> prompt_product(const torch::Tensor& x, const torch::Tensor& w_packed, const std::optional<torch::Tensor>& bias,
-                                            int64_t n, bool gelu, bool slabs, bool ordered) {
+                                            int64_t n, bool gelu, bool slabs, bool ordered, bool row_major) {
   const char* op = "prompt_product";
   LV_CHECK_DEVICE(x);
   TORCH_CHECK(x.dim() == 2 && w_packed.numel() == n * x.size(1) && w_packed.device() == x.device(), op, ": x [rows, k] and weights [n, k] packed");
@@ -298,9 +308,10 @@ std::optional<torch::Tensor> prompt_product(const torch::Tensor& x, const torch:
   const int shares = lvllm_prompt_product_plan((int)rows, (int)n, (int)k, gelu, sums, 1, plan);
   if (shares == 0) return std::nullopt;
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(x));
+  const auto w = row_major ? pack_weight(w_packed) : w_packed;
   auto out = shares > 1 ? torch::empty({shares, rows, n}, x.options().dtype(at::kFloat)) : torch::empty({rows, n}, x.options());
   check(lvllm_prompt_product(shares > 1 ? nullptr : out.data_ptr(), shares > 1 ? out.data_ptr<float>() : nullptr, x.data_ptr(), x.stride(0),
-                             0, w_packed.data_ptr(), bias && shares == 1 ? bias->data_ptr() : nullptr, (int)rows, (int)n, (int)k, gelu, 1, plan,
+                             0, w.data_ptr(), bias && shares == 1 ? bias->data_ptr() : nullptr, (int)rows, (int)n, (int)k, gelu, 1, plan,
                              current_stream(x)));
   return out;
 }
@@ -686,15 +697,6 @@ torch::Tensor skinny_linear_w8a8_argmax(const torch::Tensor& x, const torch::Ten
   return tokens;
 }
 
-torch::Tensor pack_weight(const torch::Tensor& w) {
-  TORCH_CHECK(w.is_cuda() && w.dim() == 2 && w.is_contiguous(), "pack_weight: contiguous [N,K] GPU tensor");
-  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(w));
-  auto out = torch::empty_like(w);
-  check(lvllm_pack_weight(out.data_ptr(), w.data_ptr(), (int)w.size(0), (int)w.size(1),
-                          dtype_code(w, "pack_weight"), current_stream(w)));
-  return out;
-}
-
 int64_t get_device_attribute(int64_t attribute, int64_t device_id) {
   return lvllm_get_device_attribute(attribute, device_id);
 }
@@ -763,7 +765,8 @@ TORCH_LIBRARY_FRAGMENT(_C_amd, amd) {
   amd.impl("clamped_unit", torch::kCUDA, &clamped_unit);
   amd.def("prompt_linear(Tensor x, Tensor? w, Tensor? w_packed, Tensor? bias, int outputs, int act, float limit=0.) -> Tensor?");
   amd.impl("prompt_linear", torch::kCUDA, &prompt_linear);
-  amd.def("prompt_product(Tensor x, Tensor w_packed, Tensor? bias, int n, bool gelu=False, bool slabs=False, bool ordered=False) -> Tensor?");
+  amd.def("prompt_product(Tensor x, Tensor w_packed, Tensor? bias, int n, bool gelu=False, bool slabs=False, bool ordered=False, "
+          "bool row_major=False) -> Tensor?");
   amd.impl("prompt_product", torch::kCUDA, &prompt_product);
   amd.def("prompt_products(Tensor x, Tensor w_packed, int n) -> Tensor?");
   amd.impl("prompt_products", torch::kCUDA, &prompt_products);

@@ -50,6 +50,16 @@ class EncoderConfig:
 
 
 class EncoderLayerWeights:
+    """A layer's weights: attributes that may be read, written to and assigned at any time.
+
+    Prompts of some hundreds of rows take this package's kernels, which read a weight in fragment order, from a copy that is made with the layer.
+    It is read only as long as nobody but the model has the weight: who reads or assigns an attribute may write to the tensor from then on, also in
+    ways that torch does not count (`lw.qkv_w.data.copy_`), so that the model takes the weight itself.  lay_out() behind the last write lays the
+    copies out anew; prompts are as fast as before it.  A captured forward runs the same kernels as others (what it has not run before, the library
+    cannot load under capture) over copies that the graph makes at each replay, which so sees every write: 20 us a layer of 1024 x 4096."""
+
+    WEIGHTS = "qkv_w", "out_w", "fc1_w", "fc2_w"
+
     def __init__(self, cfg: EncoderConfig, device, gen: torch.Generator):
         hid, inter = cfg.hidden_size, cfg.intermediate_size
 
@@ -67,32 +77,77 @@ class EncoderLayerWeights:
         self.fc1_w, self.fc1_b = w(inter, hid), w(inter)
         self.fc2_w, self.fc2_b = w(hid, inter), w(hid)
         self.out_ln = ln()
-        self._fused, self._packed = cfg.fused_layer_norm, {}
-        for name in self.WEIGHTS:
-            self.packed(name)  # (laid out now, and not in the first forward)
+        self._fused, self._kept, self._copies = cfg.fused_layer_norm, {}, {}  # _kept: weights that only the model has
+        self.lay_out()
 
-    WEIGHTS = "qkv_w", "out_w", "fc1_w", "fc2_w"
+    def __getattr__(self, name: str):
+        """A weight that only the model had: from now on it is an attribute as any other."""
+        kept = self.__dict__.get("_kept", {})
+        if name not in kept:
+            raise AttributeError(name)
+        self.__dict__.setdefault(name, kept[name])
+        return self.__dict__[name]
+
+    def weight(self, name: str) -> torch.Tensor:
+        w = self.__dict__.get(name)
+        if w is None:
+            return self._kept[name]
+        if self._kept.get(name, w) is not w:  # (assigned: what was there before goes)
+            self._kept.pop(name, None)
+            self._copies.pop(name, None)
+        return w
+
+    def lay_out(self) -> None:
+        """The weights stay as they are now: prompts may take copies of them in fragment order.  Writes that torch counts, and new assignments,
+        are seen after it as well; behind others it is called again.  As with a write, no forward may be under way."""
+        kept = {name: self.weight(name) for name in self.WEIGHTS}
+        self._copies = {name: self._copy(w) for name, w in kept.items() if self._takes(w)}
+        self._kept = kept
+        for name in self.WEIGHTS:
+            self.__dict__.pop(name, None)
+
+    def _takes(self, w: torch.Tensor) -> bool:
+        return (self._fused and w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous() and w.shape[0] % 16 == 0
+                and w.shape[1] % 32 == 0)
+
+    @staticmethod
+    def _version(w: torch.Tensor) -> int:
+        return -1 if w.is_inference() else w._version
+
+    def _copy(self, w: torch.Tensor):
+        """(the weight, its memory, which nothing else can have meanwhile, its version, the weight in fragment order)"""
+        copy = w, w.detach(), self._version(w), torch.ops._C_amd.pack_weight(w)
+        torch.cuda.synchronize(w.device)  # (the next forward may come on another stream, and one may still read the copy before)
+        return copy
+
+    def _current(self, name: str, w: torch.Tensor) -> Optional[torch.Tensor]:
+        was = self._copies.get(name)
+        if was is None or was[0] is not w or was[1].data_ptr() != w.data_ptr() or was[2] != self._version(w):
+            return None
+        return was[3]
 
     def packed(self, name: str) -> Optional[torch.Tensor]:
-        """A weight once more in fragment order, for this package's kernels (None: what they do not take).  Laid out anew when the weight has been
-        replaced or written to since.  Writes that torch does not count (`fc1_w.data.copy_`, or to inference tensors) are not seen: assign the
-        weight behind those."""
-        w = getattr(self, name)
-        if not (self._fused and w.is_cuda and w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[0] % 16 == 0 and w.shape[1] % 32 == 0):
-            return None
-        version = -1 if w.is_inference() else w._version
-        was = self._packed.get(name)  # (the weight, its memory, which nothing else can have meanwhile, and its version then, the copy)
-        if was is None or was[0] is not w or was[1].data_ptr() != w.data_ptr() or was[2] != version:
-            if torch.cuda.is_current_stream_capturing():  # (a copy that only the graph would write)
-                return None
-            was = w, w.detach(), version, torch.ops._C_amd.pack_weight(w)
-            torch.cuda.current_stream(w.device).synchronize()  # (the next forward may come on another stream)
-            self._packed[name] = was
-        return was[3]
+        """A weight in fragment order, None where somebody else has it."""
+        return None if name in self.__dict__ else self._current(name, self._kept[name])
 
     @property
     def fc1_packed(self) -> Optional[torch.Tensor]:
-        return self.packed("fc1_w")
+        """fc1_w in fragment order for the kernel with GELU behind the product of long prompts (None: what it does not take), laid out anew when
+        fc1_w has been replaced or written to since.  Writes that torch does not count (`fc1_w.data.copy_`, or to inference tensors) are not
+        seen: assign fc1_w or lay_out() behind those."""
+        w = self.weight("fc1_w")
+        if not self._takes(w):
+            return None
+        packed = self._current("fc1_w", w)
+        if packed is None:
+            self._copies["fc1_w"] = self._copy(w)
+            packed = self._copies["fc1_w"][3]
+        return packed
+
+    def fc1_packed_in_graph(self) -> Optional[torch.Tensor]:
+        """... a copy that the graph under capture makes at each replay."""
+        w = self.weight("fc1_w")
+        return torch.ops._C_amd.pack_weight(w) if self._takes(w) else None
 
 
 class EncoderModel:
@@ -121,6 +176,7 @@ class EncoderModel:
         hid = cfg.hidden_size
         emb, shift = self.word_emb, cfg.pad_token_id + 1  # xlm_roberta.py: position ids start after the padding index
         fused = emb.is_cuda and hid % 8 == 0 and emb.dtype in (torch.bfloat16, torch.float16) and self.cfg.fused_layer_norm
+        captured = emb.is_cuda and torch.cuda.is_current_stream_capturing()
 
         def add_ln(a, b, ln, b_bias=None):  # LayerNorm(a + b), b optional; slabs: without their bias
             if b is not None and b.dim() == 3:
@@ -135,20 +191,21 @@ class EncoderModel:
 
         def product(a, lw, name, bias, slabs=False, gelu=False):
             """This package's kernels where they are the better ones (csrc/prompt_product.h)."""
-            packed = lw.packed(name) if fused and a.shape[0] > 64 else None
-            y = None
-            if packed is not None:
-                y = torch.ops._C_amd.prompt_product(a, packed, bias, packed.numel() // a.shape[1], gelu, slabs and hid <= 2048)
-            return F.linear(a, getattr(lw, name), bias) if y is None and not gelu else y
+            w, y = lw.weight(name), None
+            if fused and a.shape[0] > 64:
+                packed = w if captured else lw.packed(name)
+                if packed is not None:
+                    y = torch.ops._C_amd.prompt_product(a, packed, bias, packed.numel() // a.shape[1], gelu, slabs and hid <= 2048, False, captured)
+            return F.linear(a, w, bias) if y is None and not gelu else y
 
         def fc1_gelu(a, lw):
             h = product(a, lw, "fc1_w", lw.fc1_b, gelu=True)
-            packed = lw.fc1_packed if fused and h is None else None
+            packed = (lw.fc1_packed_in_graph() if captured else lw.fc1_packed) if fused and h is None and a.shape[0] > 64 else None
             if packed is not None:
                 h = torch.ops._C_amd.prompt_linear(a, None, packed, lw.fc1_b, cfg.intermediate_size, PROMPT_ACTS["gelu"])
             if h is not None:
                 return h
-            h = F.linear(a, lw.fc1_w, lw.fc1_b)
+            h = F.linear(a, lw.weight("fc1_w"), lw.fc1_b)
             if fused and h.numel() % 8 == 0:
                 torch.ops._C_amd.gelu(h, h)  # exact GELU in place
                 return h
@@ -171,7 +228,7 @@ class EncoderModel:
                 y = torch.empty_like(x)
                 for r0 in range(0, x.shape[0], blk):
                     hb = fc1_gelu(x[r0:r0 + blk], lw)
-                    torch.addmm(lw.fc2_b, hb, lw.fc2_w.t(), out=y[r0:r0 + blk])
+                    torch.addmm(lw.fc2_b, hb, lw.weight("fc2_w").t(), out=y[r0:r0 + blk])
             else:
                 y = product(fc1_gelu(x, lw), lw, "fc2_w", lw.fc2_b, slabs=True)
             x = add_ln(x, y, lw.out_ln, lw.fc2_b)

@@ -241,6 +241,123 @@ def test_each_weight_that_comes_after_the_model(name, how):
     assert (first.float() - want.float()).norm() > 5e-2 * want.float().norm()
 
 
+WEIGHTS = ["qkv_w", "out_w", "fc1_w", "fc2_w"]
+
+
+def one_layer(lens):
+    """Two encoders of a layer, and a forward over sequences of these lengths."""
+    from light_vllm_amd.attention.prefill_only import PrefillOnlyAttentionMetadata
+    from light_vllm_amd.prefill_only.model import EncoderConfig, EncoderModel
+    cfg = EncoderConfig(hidden_size=1024, intermediate_size=4096, num_hidden_layers=1, num_attention_heads=16, vocab_size=512,
+                        max_position_embeddings=2048)
+    model, other = (EncoderModel(cfg, DEV, seed) for seed in (0, 1))
+    ids = torch.randint(2, 512, (sum(lens),), generator=torch.Generator().manual_seed(3)).to(DEV)
+    pos = torch.cat([torch.arange(n) for n in lens]).to(DEV)
+    starts = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32, device=DEV)
+    md = PrefillOnlyAttentionMetadata(max(lens), lens, starts)
+
+    @torch.inference_mode()
+    def run(m=model):
+        return m.forward(ids, pos, md)
+    return model, other, run
+
+
+def close(a, b):
+    return float((a.float() - b.float()).norm()) < 1e-2 * float(b.float().norm())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", WEIGHTS)
+@pytest.mark.parametrize("how", ["data.copy_", "data.copy_ by who had it before", "from_dlpack", "vars"])
+def test_writes_that_torch_does_not_count(name, how):
+    """Short prompts: whoever has a weight may write to it in any way, and the next forward takes what is there."""
+    model, other, run = one_layer([50, 70])
+    lw, new = model.layers[0], getattr(other.layers[0], name) * 2
+    first = run().clone()
+    if how == "data.copy_":
+        getattr(lw, name).data.copy_(new)
+    elif how == "data.copy_ by who had it before":
+        had = getattr(lw, name)
+        run()
+        had.data.copy_(new)
+    elif how == "from_dlpack":
+        torch.from_dlpack(torch.utils.dlpack.to_dlpack(getattr(lw, name))).copy_(new)
+    else:
+        vars(lw).update({name: new})
+    got = run()
+    model.cfg.fused_layer_norm = False  # (the library's products, of the weights themselves)
+    want = run()
+    assert close(got, want) and not close(first, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", WEIGHTS)
+@pytest.mark.parametrize("lens", [[50, 70], [900, 700, 800]])  # (own products; GELU behind a copy that the graph makes)
+def test_weights_that_come_after_a_capture(name, lens):
+    """Replays take the weight as it is, before the next forward outside of the graph and after it; so do those behind an assignment, which
+    leaves the graph the tensor that it was captured with."""
+    model, other, run = one_layer(lens)
+    lw = model.layers[0]
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run()
+
+    def replay():
+        graph.replay()
+        torch.cuda.synchronize()
+        return out.clone()
+
+    def library():
+        model.cfg.fused_layer_norm = False
+        y = run().clone()
+        model.cfg.fused_layer_norm = True
+        return y
+    first = replay()
+    assert close(first, library())
+    w = getattr(lw, name)
+    w.copy_(getattr(other.layers[0], name) * 2)
+    second = replay()
+    want = library()
+    assert close(second, want) and not close(first, want)
+    for _ in range(3):
+        assert close(run(), want)
+        torch.full((3 * 1024, 1024), 9.0, dtype=torch.bfloat16, device=DEV)  # (memory that a copy might have left)
+        assert torch.equal(replay(), second)
+    setattr(lw, name, getattr(other.layers[0], name).clone())
+    assert close(run(), library()) and torch.equal(replay(), second)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", ["data.copy_", "assigned"])
+def test_weights_laid_out_anew(how):
+    """Behind lay_out() a model is what one that was made with the weights is: the same kernels, the same bits; and what is written then is seen."""
+    model, other, run = one_layer([50, 70])
+    lw, theirs = model.layers[0], other.layers[0]
+    made_with = run(other).clone()
+    for name in ("word_emb", "pos_emb", "type_emb", "emb_ln"):
+        setattr(model, name, getattr(other, name))
+    for name in vars(theirs):
+        if name.endswith(("_b", "_ln")):
+            setattr(lw, name, getattr(theirs, name))
+    for name in WEIGHTS:
+        new = theirs.weight(name).clone()
+        if how == "assigned":
+            setattr(lw, name, new)
+        else:
+            getattr(lw, name).data.copy_(new)
+    assert close(run(), made_with) and all(lw.packed(name) is None for name in WEIGHTS)
+    lw.lay_out()
+    assert torch.equal(run(), made_with) and all(lw.packed(name) is not None for name in WEIGHTS)
+    w = lw.qkv_w
+    lw.lay_out()
+    w.mul_(2)  # (by one who had it before)
+    got = run()
+    model.cfg.fused_layer_norm = False
+    assert close(got, run()) and not close(got, made_with)
+
+
 @pytest.mark.gpu
 def test_encoder_engine_matches_fp32_reference():
     eng = make_encoder(pooling="last_hidden_states")
