@@ -133,6 +133,7 @@ extern "C" int lvllm_prompt_product_plan(int rows, int n, int k, int gelu, int s
 extern "C" int lvllm_prompt_product(void* out, float* slabs, const void* x, int64_t x_stride, int64_t x_batch_stride,
                                     const void* w_packed, const void* bias, int rows, int n, int k, int gelu, int batch, const int* plan, void* stream) {
   if (rows == 0) return 0;
+  LV_CHECK(plan != nullptr && x != nullptr && w_packed != nullptr, "a plan, x and weights");
   const ProductPlan p{plan[0], plan[1], plan[2]};
   LV_CHECK(rows > 0 && n > 0 && k > 0 && n % 16 == 0 && k % 64 == 0, "n a multiple of 16 and k of 64");
   LV_CHECK(x_stride >= k && x_stride % 8 == 0, "rows of x 16-byte aligned, one after the other");

@@ -288,6 +288,8 @@ torch::Tensor pack_weight(const torch::Tensor& w) {
   return out;
 }
 
+bool differentiated(const torch::Tensor& t) { return at::GradMode::is_enabled() && t.requires_grad(); }
+
 // x w^T + bias of a prompt of some hundreds of rows, GELU behind it where asked for; `slabs`: or fp32 sums of shares of K, [shares, rows, n],
 // without the bias; `ordered`: sums one k after the other.  Nothing where the library's product is faster, or the operands are none that the kernels take.
 // `row_major`: w_packed is the weights as they are, [n, k]; a launch ahead of the product packs them.
@@ -295,8 +297,10 @@ std::optional<torch::Tensor> prompt_product(const torch::Tensor& x, const torch:
                                             int64_t n, bool gelu, bool slabs, bool ordered, bool row_major) {
   const char* op = "prompt_product";
   LV_CHECK_DEVICE(x);
-  TORCH_CHECK(x.dim() == 2 && w_packed.numel() == n * x.size(1) && w_packed.device() == x.device(), op, ": x [rows, k] and weights [n, k] packed");
-  TORCH_CHECK(!bias || (bias->numel() == n && bias->device() == x.device()), op, ": a bias [n]");
+  if (x.dim() != 2) return std::nullopt;
+  TORCH_CHECK(w_packed.numel() == n * x.size(1) && w_packed.device() == x.device(), op, ": x [rows, k] and weights [n, k] packed");
+  TORCH_CHECK(!bias || bias->device() == x.device(), op, ": a bias on x's device");
+  if (differentiated(x) || differentiated(w_packed) || (bias && (differentiated(*bias) || bias->numel() != n))) return std::nullopt;
   const int64_t rows = x.size(0), k = x.size(1);
   auto aligned = [](const torch::Tensor& t) { return ((uintptr_t)t.data_ptr() & 15) == 0; };
   if (x.scalar_type() != at::kBFloat16 || w_packed.scalar_type() != at::kBFloat16 || x.stride(1) != 1 || x.stride(0) < k ||

@@ -195,14 +195,14 @@ class EncoderModel:
             if fused and a.shape[0] > 64:
                 packed = w if captured else lw.packed(name)
                 if packed is not None:
-                    y = torch.ops._C_amd.prompt_product(a, packed, bias, packed.numel() // a.shape[1], gelu, slabs and hid <= 2048, False, captured)
+                    y = torch.ops._C_amd.prompt_product(a, packed, bias, w.shape[0], gelu, slabs and hid <= 2048, False, captured)
             return F.linear(a, w, bias) if y is None and not gelu else y
 
         def fc1_gelu(a, lw):
             h = product(a, lw, "fc1_w", lw.fc1_b, gelu=True)
             packed = (lw.fc1_packed_in_graph() if captured else lw.fc1_packed) if fused and h is None and a.shape[0] > 64 else None
             if packed is not None:
-                h = torch.ops._C_amd.prompt_linear(a, None, packed, lw.fc1_b, cfg.intermediate_size, PROMPT_ACTS["gelu"])
+                h = torch.ops._C_amd.prompt_linear(a, None, packed, lw.fc1_b, packed.shape[0], PROMPT_ACTS["gelu"])
             if h is not None:
                 return h
             h = F.linear(a, lw.weight("fc1_w"), lw.fc1_b)

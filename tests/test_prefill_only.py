@@ -330,6 +330,21 @@ def test_weights_that_come_after_a_capture(name, lens):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("name", WEIGHTS)
+@pytest.mark.parametrize("rows", [100, 1200])
+def test_weights_of_another_shape(name, rows):
+    """A weight that is turned round is refused, laid out or not."""
+    model, other, run = one_layer([rows])
+    lw = model.layers[0]
+    w = getattr(lw, name)
+    setattr(lw, name, w.t().contiguous() if name != "out_w" else w[:, :512].reshape(512, 1024).contiguous())
+    for _ in range(2):
+        with pytest.raises(RuntimeError):
+            run()
+        lw.lay_out()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("how", ["data.copy_", "assigned"])
 def test_weights_laid_out_anew(how):
     """Behind lay_out() a model is what one that was made with the weights is: the same kernels, the same bits; and what is written then is seen."""

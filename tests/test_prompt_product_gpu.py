@@ -119,8 +119,32 @@ def test_operands_that_the_library_takes(lib):
     assert op(x.half(), packed, b, 1024) is None and op(x, packed.half(), b, 1024) is None
     assert op(x, packed, odd_bias, 1024) is None and op(x, packed, b.float(), 1024) is None
     assert op(x[:64], packed, b, 1024) is None and op(x[:0], packed, b, 1024) is None
+    assert op(x, packed, b[:1], 1024) is None and op(x[None], packed, b, 1024) is None  # (what the library makes of these)
     with pytest.raises(RuntimeError):
         op(x, packed, b, 1040)
+
+
+@pytest.mark.parametrize("which", ["x", "bias"])
+def test_gradients(lib, which):
+    """Products that are differentiated are the library's."""
+    from light_vllm_amd.engine.model import Weight, linear, product
+    x, w, _, b = operands(300, 1024, 1024)
+    x.requires_grad_(which == "x")
+    b.requires_grad_(which == "bias")
+    for f in (linear, product):
+        y = f(x, Weight(w), b)
+        g, = torch.autograd.grad(y.float().sum(), x if which == "x" else b)
+        assert torch.isfinite(g).all() and g.abs().max() > 0
+    with torch.no_grad():
+        assert torch.ops._C_amd.prompt_product(x, torch.ops._C_amd.pack_weight(w), b, 1024) is not None
+
+
+@pytest.mark.parametrize("rows", [100, 300])
+def test_linear_of_several_dimensions(lib, rows):
+    from light_vllm_amd.engine.model import Weight, linear
+    x, w, _, b = operands(rows, 1024, 1024)
+    x = torch.stack([x, 2 * x], 1)  # [rows, 2, k]
+    assert torch.equal(linear(x, Weight(w), b), torch.nn.functional.linear(x, w, b))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
