@@ -204,10 +204,12 @@ class DecoderModel:
             torch.ops._C_amd.fused_add_rms_norm_splitk_scaled(out, residual, x[0], weight, self.cfg.rms_norm_eps,
                                                               x[1], x[2])
             return out
-        if x.dim() == 3:
+        if x.dim() == 3 and weight.data_ptr() % 16 == 0:
             out = torch.empty_like(residual)
             torch.ops._C_amd.fused_add_rms_norm_splitk(out, residual, x, weight, self.cfg.rms_norm_eps)
             return out
+        if x.dim() == 3:
+            x = x.sum(0).to(residual.dtype)
         ops.fused_add_rms_norm(x, residual, weight, self.cfg.rms_norm_eps)
         return x
 

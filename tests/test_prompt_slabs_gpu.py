@@ -117,6 +117,18 @@ def test_prompts_of_a_dense_decoder(amd, monkeypatch, rows):
     assert not torch.equal(got, library) and float(off) < 1.25 * float(theirs) and float(theirs) < 0.03 * float(want.norm())
 
 
+@pytest.mark.parametrize("rows", [100, 300])
+def test_norm_weights_off_16_bytes(amd, rows):
+    model = decoder(hidden_size=1024, intermediate_size=4096, num_attention_heads=8, num_key_value_heads=2)
+    tokens = torch.randint(0, 512, (rows,), generator=torch.Generator().manual_seed(rows)).to(DEV)
+    want = run(model, tokens).float()
+    for lw in model.layers:
+        lw.post_norm, lw.input_norm = (torch.cat([w[:1], w])[1:] for w in (lw.post_norm, lw.input_norm))
+    assert model.layers[0].post_norm.data_ptr() % 16
+    got = run(model, tokens).float()
+    assert (got - want).norm() < 1e-2 * want.norm()
+
+
 @pytest.mark.parametrize("rows", [100, 300, 700])
 def test_feed_forward_of_a_hybrid_decoder(amd, rows):
     """Slabs out of the feed-forward, into the norm behind it: the sum of both in 64 bits, and the norm's bits."""
