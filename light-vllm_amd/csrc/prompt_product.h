@@ -1,6 +1,6 @@
 // Products of prompts of some hundreds of rows: which tiles take which, in plain numbers.
 #pragma once
-#include <stdint.h>
+#include "prompt_linear.h"
 
 namespace lvllm {
 
@@ -58,7 +58,13 @@ inline double product_time(const ProductPlan& p, int rows, int n, int k, int bat
   return us;
 }
 
-enum { kSumsAny = 0, kSumsSlabs = 1, kSumsOrdered = 2 };  // include/lvllm_hip.h LVLLM_SUMS_*
+// us of GELU behind a product in tiles of 128 rows (prompt_linear.h), where that takes it and every tile has a CU: 5.9 + .255 a k-step of 32 for half
+// tiles, 8.5 + .42 for whole ones, of 69 such products of 384 to 2048 wide, 5 % off (root mean square).  0: it does not, or tiles take turns.
+inline double tile_gelu_time(int rows, int n, int k) {
+  const PromptLinearPlan t = prompt_linear_plan(rows, n, k, LVLLM_ACT_GELU, false, true);
+  if (t.body != LVLLM_PROMPT_TILE || (int64_t)((rows + 127) / 128) * ((n + 64 * t.nt - 1) / (64 * t.nt)) > 256) return 0;
+  return t.nt == 2 ? 5.9 + .255 * (k / 32) : 8.5 + .42 * (k / 32);
+}
 
 // The shortest of the plans, and the library where its products are the better ones, by the rate that the plan reaches, TFLOP/s (of those 3702, own
 // time of the library's; host time, 3 us for 20, not counted):
@@ -68,12 +74,15 @@ enum { kSumsAny = 0, kSumsSlabs = 1, kSumsOrdered = 2 };  // include/lvllm_hip.h
 //     5120, 0.90 above (us, before and after: 300 rows of 2048 for 2048 12.9, 8.8; for 7680 25.4, 19.0; 300 rows of 5632 for 2048 25.7, 20.8).  With
 //     few tiles of long K the library cuts it and is faster: 0.99 to 1.6 below 100 for k > 2048, below 200 for k > 5120;
 //   * K may be cut into slabs: 0.64, 0.75, 0.77 and 0.70, what the slabs cost the next launch included (300 rows of 14336 for 4096 75, 50; 100 rows 48,
-//     29; 300 rows of 4096 for 1024 14.6, 8.7).
+//     29; 300 rows of 4096 for 1024 14.6, 8.7);
+//   * GELU behind a product makes it 1.15 times as long (1.11 to 1.16 in the mean by tiles and rounds, of 1100).  The tiles of prompt_linear.h keep
+//     what takes them less: 4096 of 1024, 65 to 600 rows 0.41 to 0.85 of theirs or the library's; 800 rows 16.1 us for 14.1, 1000 rows 15.7 for
+//     14.9, 2000 rows 23.8 for 23.3.  Of 31 other sizes it leaves two slower, 1.04; by plain products' times 18 were, up to 1.19.
 // `batch` products of one size in a launch (K whole): as one of so many times the tiles.
 inline ProductPlan prompt_product_plan(int rows, int n, int k, bool gelu, int sums, int batch = 1) {
   ProductPlan best{0, 0, 0};
   if (rows <= 64 || rows > 8192 || n < 16 || n % 16 != 0 || k < 256 || k % 64 != 0 || (int64_t)n * k >= (int64_t)1 << 30 || batch < 1 || batch > 64) return best;
-  const bool slabs = sums == kSumsSlabs && !gelu && batch == 1;
+  const bool slabs = sums == LVLLM_SUMS_SLABS && !gelu && batch == 1;
   double least = 0;
   auto take = [&](const ProductPlan& p) {
     if (!product_plan_valid(p, k) || product_units(p, rows, n) * batch > 512 || (p.shares > 1 && k / 32 / p.shares < 8)) return;
@@ -94,6 +103,10 @@ inline ProductPlan prompt_product_plan(int rows, int n, int k, bool gelu, int su
   }
   if (best.size == 0) return best;
   const double rate = 2e-6 * rows * n * k * batch / least;
+  if (gelu) {
+    const double tile = tile_gelu_time(rows, n, k);
+    if (tile > 0 && 1.15 * least > tile) return ProductPlan{0, 0, 0};
+  }
   const double fewest = slabs || k <= 2048 ? 0 : k <= 5120 ? 100 : 200, most = k <= 5120 ? 900 : k <= 9000 ? 1000 : 1150;
   return rate >= fewest && rate <= most ? best : ProductPlan{0, 0, 0};
 }

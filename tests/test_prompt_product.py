@@ -51,6 +51,17 @@ def test_measured_sizes(plan, rows, n, k, sums, own):
     assert (plan(rows, n, k, sums=sums)[0] != 0) == own
 
 
+GELU = [  # rows, n, k -> this kernel's, or tiles with GELU behind them and the library's
+    (65, 4096, 1024, True), (300, 4096, 1024, True), (600, 4096, 1024, True), (1200, 4096, 1024, True), (1500, 4096, 1024, True),
+    (800, 4096, 1024, False), (1000, 4096, 1024, False), (2000, 4096, 1024, False), (1000, 3072, 768, False), (1500, 5120, 1280, False),
+    (500, 8192, 2048, False), (600, 8192, 2048, True), (1171, 3072, 896, False), (716, 5248, 320, False), (1978, 896, 384, True)]
+
+
+@pytest.mark.parametrize("rows,n,k,own", GELU)
+def test_measured_sizes_with_gelu(plan, rows, n, k, own):
+    assert (plan(rows, n, k, gelu=True)[0] != 0) == own
+
+
 def test_any_size(plan):
     rng = random.Random(0)
     taken = set()
