@@ -77,6 +77,21 @@ inline PromptLinearPlan prompt_linear_plan(int rows, int outputs, int k, int act
   return plan;
 }
 
+// Rows of a launch's tiles of up to 128, in 16s.
+inline int tile_groups(int rows) { return ((rows + (rows + 127) / 128 - 1) / ((rows + 127) / 128) + 15) / 16; }
+
+// Half tiles whose loads are dealt among their MFMAs (deep_tile.h), k a multiple of 64.  What they take of the others' time, of 114 products, weights
+// from memory, by groups of 16 rows in a tile: 0.97 with 8 and 0.96 with 7 (0.88 to 1.02) where up to 256 tiles have a CU each, 0.96 and 0.94
+// beyond; 0.99 with 5 up to 256 tiles, 1.02 beyond; with 6, which the others have a body of, 1.02 and 1.05 (SwiGLU of 5632, 2048 wide, 288 rows
+// 26.3 us, 28.0).  GELU, 0.94 with 7 and 0.97 with 8 but 0.86 to 1.18, is left to the others.  us: squared ReLU of 8448, 2048 wide, 300 rows
+// (198 tiles) 20.8, 20.2; 500 (264) 31.9, 29.2; the clamped unit of 5632, 200 rows (176) 22.9, 21.8; 400 (352) 34.8, 31.9; SwiGLU of 14336,
+// 4096 wide, 65 to 128 rows level.
+inline bool dealt_half_tiles(int rows, int wrows, int k, int act) {
+  const int groups = tile_groups(rows);
+  const int64_t units = (int64_t)((rows + 127) / 128) * ((wrows + 127) / 128);
+  return k % 64 == 0 && act != LVLLM_ACT_GELU && (groups > 6 || (groups < 6 && units <= 256));
+}
+
 int launch_wide_linear(void* out, const void* x, const void* w, int rows, int outputs, int k, int act, float limit, int groups,
                        void* stream);
 int launch_tile_linear(void* out, const void* x, const void* w, const void* bias, int rows, int outputs, int k, int act, float limit,

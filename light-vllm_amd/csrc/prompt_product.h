@@ -77,7 +77,7 @@ inline double tile_gelu_time(int rows, int n, int k) {
 //     29; 300 rows of 4096 for 1024 14.6, 8.7);
 //   * GELU behind a product makes it 1.15 times as long (1.11 to 1.16 in the mean by tiles and rounds, of 1100).  The tiles of prompt_linear.h keep
 //     what takes them less: 4096 of 1024, 65 to 600 rows 0.41 to 0.85 of theirs or the library's; 800 rows 16.1 us for 14.1, 1000 rows 15.7 for
-//     14.9, 2000 rows 23.8 for 23.3.  Of 31 other sizes it leaves two slower, 1.04; by plain products' times 18 were, up to 1.19.
+//     14.9, 2000 rows 23.8 for 23.3.  Of 29 other sizes it leaves two slower, 1.04; by plain products' times 18 were, up to 1.19.
 // `batch` products of one size in a launch (K whole): as one of so many times the tiles.
 inline ProductPlan prompt_product_plan(int rows, int n, int k, bool gelu, int sums, int batch = 1) {
   ProductPlan best{0, 0, 0};

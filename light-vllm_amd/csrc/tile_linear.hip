@@ -13,7 +13,7 @@ namespace lvllm {
 struct TileLinear {
   uint16_t* out;                  // [rows, outputs]
   const uint16_t *x, *w, *bias;   // x [rows, k], w packed [n, k] (pairs: [gate rows | value rows]), bias [n] (GELU)
-  int rows, outputs, k, tiles, blocks;  // tiles of 128 rows, blocks of W rows
+  int rows, outputs, k, tiles, size, blocks;  // tiles of `size` rows, up to 128, blocks of W rows
   float limit;                    // CLAMPED_UNIT
 };
 
@@ -40,9 +40,7 @@ __device__ __forceinline__ void tile_linear(const TileLinear& p, const TileWork&
                     });
 }
 
-// An eighth of the tiles to each XCD, 1024 rows side by side, W block after W block.  DEEP: half tiles by deep_tile.h, k a multiple of 64.  us, weights
-// from memory: squared ReLU of 8448, 2048 wide, 300 rows (198 half tiles) 22.5, 19.9; 500 (264) 32.9, 29.4; 700 (396) 33.5, 32.6; the clamped unit
-// of 5632, 200 rows (176) 23.0, 21.7.  Not GELU, whose instructions take the loads' place: 4096, 1024 wide, 1000 rows (256) 14.8, 15.1.
+// An eighth of the tiles to each XCD, 1024 rows side by side, W block after W block.  DEEP: half tiles by deep_tile.h (dealt_half_tiles).
 template <int ACT, int NT, bool DEEP>
 __global__ __launch_bounds__(256, 2) void tile_linear_kernel(const TileLinear p) {
   __shared__ __attribute__((aligned(16))) char ring[DEEP ? deep_lds_bytes(8) : tile_steps(NT) / 2 * kStageBytes];
@@ -52,7 +50,7 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(const TileLinear p)
   const int strip = unit / (kSide * p.blocks), side = min(kSide, p.tiles - strip * kSide), in = unit - strip * kSide * p.blocks;
   TileWork t{};
   t.block = in / side;
-  const int size = ((p.rows + p.tiles - 1) / p.tiles + 15) / 16 * 16;
+  const int size = p.size;
   t.s0 = (strip * kSide + in - t.block * side) * size;
   t.s1 = min(t.s0 + size, p.rows);
   if (t.s0 >= t.s1) return;
@@ -72,6 +70,8 @@ int launch_tile_linear(void* out, const void* x, const void* w, const void* bias
   p.out = (uint16_t*)out; p.x = (const uint16_t*)x; p.w = (const uint16_t*)w; p.bias = (const uint16_t*)bias;
   p.rows = rows; p.outputs = outputs; p.k = k; p.limit = limit;
   p.tiles = (rows + kMoeTile - 1) / kMoeTile;
+  p.size = 16 * tile_groups(rows);
+  const bool dealt = dealt_half_tiles(rows, (prompt_pairs(act) ? 2 : 1) * outputs, k, act);
   auto launch = [&](auto act, auto nt, auto deep) {
     constexpr int ACT = decltype(act)::value, NT = decltype(nt)::value;
     p.blocks = ((prompt_pairs(ACT) ? 2 : 1) * outputs + 64 * NT - 1) / (64 * NT);
@@ -80,7 +80,7 @@ int launch_tile_linear(void* out, const void* x, const void* w, const void* bias
   auto with = [&](auto act) {
     constexpr std::integral_constant<int, 2> two{};
     if (nt == 4) launch(act, std::integral_constant<int, 4>{}, std::false_type{});
-    else if (k % 64 == 0 && act != LVLLM_ACT_GELU) launch(act, two, std::integral_constant<bool, decltype(act)::value != LVLLM_ACT_GELU>{});
+    else if (dealt) launch(act, two, std::integral_constant<bool, decltype(act)::value != LVLLM_ACT_GELU>{});
     else launch(act, two, std::false_type{});
   };
   if (act == LVLLM_ACT_GELU) with(std::integral_constant<int, LVLLM_ACT_GELU>{});

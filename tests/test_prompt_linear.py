@@ -7,6 +7,8 @@ import subprocess
 
 import pytest
 
+from test_prompt_linear_gpu import HALF_TILES
+
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "light-vllm_amd", "csrc")
 SOURCE = r"""
 #include "prompt_linear.h"
@@ -15,6 +17,10 @@ extern "C" int plan(int rows, int outputs, int k, int act, int row_major, int pa
   *groups = p.groups;
   *nt = p.nt;
   return p.body;
+}
+extern "C" int dealt(int rows, int wrows, int k, int act, int* groups) {
+  *groups = lvllm::tile_groups(rows);
+  return lvllm::dealt_half_tiles(rows, wrows, k, act);
 }
 """
 GELU, SILU, RELU2, CLAMPED = 1, 2, 3, 4
@@ -32,6 +38,7 @@ def plan(tmp_path_factory):
         g, n = ctypes.c_int(), ctypes.c_int()
         body = lib.plan(rows, outputs, k, act, row_major, packed, ctypes.byref(g), ctypes.byref(n))
         return body, g.value if body == WIDE else n.value
+    f.lib = lib
     return f
 
 
@@ -51,6 +58,15 @@ MEASURED = [  # rows, outputs, k, activation -> body, groups or blocks
 def test_measured_sizes(plan, rows, outputs, k, act, body, size):
     got = plan(rows, outputs, k, act)
     assert got[0] == body and (body == NONE or got[1] == size)
+
+
+@pytest.mark.parametrize("rows,wrows,k,groups,dealt", HALF_TILES)
+@pytest.mark.parametrize("act", [GELU, SILU, RELU2, CLAMPED])
+def test_half_tiles(plan, rows, wrows, k, act, groups, dealt):
+    """The sizes at which test_prompt_linear_gpu.py runs the bodies of half tiles lead there."""
+    g = ctypes.c_int()
+    assert plan(rows, wrows // 2 if act in (SILU, CLAMPED) else wrows, k, act, False) == (TILE, 2)
+    assert bool(plan.lib.dealt(rows, wrows, k, act, ctypes.byref(g))) == (dealt and act != GELU) and g.value == groups
 
 
 def test_any_size(plan):

@@ -22,6 +22,12 @@ WIDE = [(769, 8464, 512), (1100, 5904, 576), (1500, 4096, 512), (3000, 2832, 640
 TILE = [(300, 4096, 64), (1000, 4112, 96), (129, 6160, 1024), (2500, 4096, 160), (4097, 784, 32), (513, 4224, 2048)]
 
 
+# rows, W rows, k of half tiles, the groups of 16 rows in one, and whether their loads are dealt: one tile a CU and more
+HALF_TILES = [(130, 8224, 256, 5, True), (180, 8224, 256, 6, False), (220, 8224, 320, 7, True), (250, 8224, 576, 8, True), (280, 8224, 256, 6, False),
+              (300, 8224, 256, 7, True), (130, 16544, 256, 5, False), (180, 16544, 256, 6, False), (400, 8736, 256, 7, True),
+              (512, 8736, 320, 8, True), (220, 8224, 288, 7, False)]
+
+
 def check(amd, rows, outputs, k, act, row_major, pack):
     gen = torch.Generator().manual_seed(rows + outputs + k)
     n = outputs * (2 if act in (SILU, CLAMPED) else 1)
@@ -62,6 +68,12 @@ def test_wide_tiles(amd, rows, outputs, k, act):
 def test_tiles(amd, rows, outputs, k, act):
     outputs *= 1 if act in (GELU, CLAMPED) else 3
     check(amd, rows, outputs, k, act, False, True)
+
+
+@pytest.mark.parametrize("act", [GELU, SILU, RELU2, CLAMPED])
+@pytest.mark.parametrize("rows,wrows,k", [h[:3] for h in HALF_TILES])
+def test_half_tiles(amd, rows, wrows, k, act):
+    check(amd, rows, wrows // 2 if act in (SILU, CLAMPED) else wrows, k, act, False, True)
 
 
 def test_activations_of_the_largest_and_smallest_values(amd):
