@@ -148,8 +148,7 @@ class LatentAttention:
         self.pages = KVSpec(H, cfg.dim + cfg.rot_dim, cfg.vdim)  # of expanded keys and values
         # long portions take the expanded way where head_attention has a matrix-core body
         self.expands = uk.dtype == torch.bfloat16 and uk.is_cuda and self.pages.kpad <= 256 and self.pages.vpad <= 256
-        self.expand = F.pad(torch.cat([uk, uv]), (0, cpad - cfg.kv_rank)).contiguous() if self.expands else None
-        self.expand_packed = amd.pack_weight(self.expand) if self.expands and self.expand.shape[0] % 16 == 0 and cpad % 32 == 0 else None
+        self.expand = make_weight(F.pad(torch.cat([uk, uv]), (0, cpad - cfg.kv_rank)), pack) if self.expands else None
         self.out_cols = H * cfg.vdim
         self.out = make_weight(pad_columns(get(name + ".o")), pack)
 
@@ -191,9 +190,9 @@ class LatentAttention:
     def _long(self, out, q, gate, cache, layer: int, plan: LongPortions, step: LatentStep) -> None:
         c, l, spec, p = self.cfg, step.layout, self.spec, self.pages
         lat = step.gathered(layer, c.window, cache, plan)
-        lat_c = lat[:, :spec.cpad]
-        kv = amd.prompt_product(lat_c, self.expand_packed, None, self.expand.shape[0], ordered=True) if self.expand_packed is not None else None
-        kv = F.linear(lat_c, self.expand) if kv is None else kv
+        lat_c, w = lat[:, :spec.cpad], self.expand
+        kv = amd.prompt_product(lat_c, w.packed, None, w.N, ordered=True) if w.packed is not None else None
+        kv = F.linear(lat_c, w.w) if kv is None else kv
         keys, values = amd.latent_expand(kv, lat, spec.cpad, c.heads, c.dim, c.rot_dim, c.vdim, p.kpad, p.vpad)
         qr = amd.latent_rotate_query(q, c.heads, c.dim, p.kpad, l.positions, self.rotation.turns,
                                      self.rotation.grow)

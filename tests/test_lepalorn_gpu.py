@@ -455,3 +455,21 @@ def test_programs(folders, tmp_path):
     for step, places in ((0, [3, 24]), (2, [29, 27])):
         got = torch.frombuffer(bytearray((tmp_path / f"{step}.f32").read_bytes()), dtype=F32).view(len(places), -1)
         check_rows(got, want[places], F32, step)
+
+
+@pytest.mark.parametrize("pack", [True, False])
+def test_weights_are_packed_where_that_is_asked_for(pack):
+    """Without, prompts take the library's products, those of expanded latents too: the same keys and values to a rounding."""
+    from light_vllm_amd.engine.latent_layers import LatentAttention
+    from light_vllm_amd.engine.model import Weight
+    from light_vllm_amd.engine.registry import model_entry
+    entry = model_entry("Lepalorn")
+    cfg = entry.config_cls().from_dict(lc.CONFIGS["large"])
+    cfg.pack_weights = pack
+    model = entry.model_cls()(cfg, entry.backend_cls().get_impl_cls()(), DEV)
+    mixers = [s for layer in model.layers for s in layer if isinstance(s, LatentAttention)]
+    assert len(mixers) == 2 and all(m.expands for m in mixers)
+    for m in mixers:
+        weights = [v for v in vars(m).values() if isinstance(v, Weight)]
+        assert m.expand in weights and all((w.packed is not None) == pack for w in weights)
+        assert not [k for k, v in vars(m).items() if torch.is_tensor(v) and "packed" in k]
