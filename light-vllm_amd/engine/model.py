@@ -17,10 +17,14 @@ from .config import ModelConfig
 
 
 class Weight:
-    """A projection weight [N, K] kept in two orders: row-major for the library GEMM (prompt
-    batches) and, for decode batches, packed into MFMA-fragment order so that the
-    weight-streaming kernel reads one contiguous KiB per wave load (csrc/skinny_gemm.hip).
-    Twice the bytes; sized for 288 GB of HBM."""
+    """A projection weight [N, K] kept in two orders: row-major for the library GEMM (long
+    prompts) and, for decode batches and prompts of up to some thousand rows, packed into
+    MFMA-fragment order so that a wave load reads one contiguous KiB (csrc/skinny_gemm.hip,
+    csrc/prompt_product.h).  Twice the bytes; sized for 288 GB of HBM.
+
+    Which of the two a step reads goes by its rows, and nothing looks whether they agree: `w`
+    does not change once it is packed, except with lay_out() behind the write.  (Models keep
+    stacks and transposes of some weights beside them: those are made once.)"""
 
     __slots__ = ("w", "packed", "N", "K", "w8_t", "w8_packed", "w_scale", "x_scale", "x_absmax")
 
@@ -34,6 +38,11 @@ class Weight:
 
     def numel(self) -> int:
         return self.N * self.K
+
+    def lay_out(self) -> None:
+        """Packs `w` as it is now, in the memory that captured steps read."""
+        if self.packed is not None:
+            self.packed.copy_(torch.ops._C_amd.pack_weight(self.w))
 
     def quantize_fp8(self) -> None:
         """Per-tensor e4m3 weights + the calibrated static activation scale; the 16-bit copies are

@@ -117,6 +117,30 @@ def test_prompts_of_a_dense_decoder(amd, monkeypatch, rows):
     assert not torch.equal(got, library) and float(off) < 1.25 * float(theirs) and float(theirs) < 0.03 * float(want.norm())
 
 
+def test_weights_laid_out_anew(amd):
+    """One weight for steps of every length, and for those that were captured before."""
+    from light_vllm_amd.engine.model import Weight, linear, product
+    w, b = rand(2048, 1024, seed=1).bfloat16(), rand(2048, 1024, seed=2).bfloat16()
+    weight, xs = Weight(w.clone()), [rand(n, 1024, seed=n).bfloat16() for n in (1, 64, 100, 300, 700, 6000)]
+    outs = [linear(x, weight) for x in xs]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = linear(xs[1], weight)
+    packed = weight.packed
+    weight.w.copy_(b)
+    weight.lay_out()
+    assert weight.packed is packed
+    for x, before in zip(xs, outs):
+        want = x.double() @ b.double().t()
+        for y in (linear(x, weight), product(x, weight)):
+            assert (y.double() - want).norm() < 1e-2 * want.norm() and (before.double() - want).norm() > want.norm()
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, linear(xs[1], weight))
+
+
 @pytest.mark.parametrize("rows", [100, 300])
 def test_norm_weights_off_16_bytes(amd, rows):
     model = decoder(hidden_size=1024, intermediate_size=4096, num_attention_heads=8, num_key_value_heads=2)
