@@ -1,5 +1,5 @@
-"""Decays from a low-rank projection at the edges of their tiles (64 rows, 128 channels, 128 and 32 of the rank) and with values that have no
-parts of 16 bits."""
+"""Decays from a low-rank projection at the edges of their tiles (16 rows x 64 channels, 32 x 64 and 64 x 128 by how many there are, 64 and 32 of the
+rank) and with values that have no parts of 16 bits."""
 import pytest
 import torch
 
@@ -25,6 +25,19 @@ def tensors(rows, rank, channels, dtype, stride):
     return u, torch.randn(rank, channels, generator=g) * 3 * rank ** -0.5, torch.randn(channels, generator=g)
 
 
+# rows, channels of the larger tiles: the last ones end inside a wave's part, with channels that are no multiple of 4 and those that are
+TILES_32 = [(2003, 387), (705, 1092)]     # 882 and 810 tiles of 16 x 64, of which 700 and fewer are taken as they are
+TILES_64 = [(8003, 515), (4097, 1028)]    # 4509 and 4369, more than 3800
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("rows,channels", TILES_32 + TILES_64)
+@pytest.mark.parametrize("rank,stride", [(1, 1), (31, 37), (33, 40), (63, 64), (65, 65), (129, 131)])
+def test_decays_of_many_rows(amd, rows, channels, rank, stride, kind, dtype):
+    test_decays(amd, rows, rank, channels, stride, kind, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("rows,rank,channels,stride", [(1, 1, 1, 1), (63, 31, 127, 37), (64, 32, 128, 32), (65, 33, 129, 33),
@@ -44,9 +57,9 @@ def test_decays(amd, rows, rank, channels, stride, kind, dtype):
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("where,value", [("u", float("inf")), ("u", float("-inf")), ("u", float("nan")), ("a", float("inf")),
                                          ("a", float("nan")), ("a", 3.4028e38), ("b", float("-inf"))])
-def test_values_without_parts(amd, where, value, kind):
-    t = dict(zip("uab", tensors(130, 40, 140, torch.bfloat16, 40)))
-    at = {"u": (65, 3), "a": (3, 5), "b": (5,)}[where]
+def test_values_without_parts(amd, where, value, kind, rows=130, channels=140, rank=40):
+    t = dict(zip("uab", tensors(rows, rank, channels, torch.bfloat16, rank)))
+    at = {"u": (rows // 2, 3), "a": (3, 5), "b": (5,)}[where]
     t[where][at] = value
     if where == "a" and value < float("inf"):
         t["u"][:, 3] = 2.0 ** -100  # (finite products)
@@ -60,6 +73,14 @@ def test_values_without_parts(amd, where, value, kind):
     want = reference(t["u"], t["a"], t["b"], kind)
     want[~nan & ~z.isfinite()] = -torch.exp(torch.tensor(9.0, dtype=torch.float64))
     torch.testing.assert_close(got[~nan], want[~nan], rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("rows,channels", TILES_32[:1] + TILES_64[:1])
+@pytest.mark.parametrize("rank", [40, 129])
+@pytest.mark.parametrize("where,value", [("u", float("inf")), ("u", float("nan")), ("a", float("inf")), ("a", 3.4028e38), ("b", float("-inf"))])
+def test_values_without_parts_among_many_rows(amd, where, value, rank, rows, channels, kind):
+    test_values_without_parts(amd, where, value, kind, rows, channels, rank)
 
 
 @pytest.mark.parametrize("rows", [350, 353, 1888, 1889, 1904, 1905, 2100])
