@@ -94,6 +94,26 @@ def test_sums_in_order(lib, rows, n, k, with_bias):
         assert rc == 0 and torch.equal(out, y), (size, nt)
 
 
+@pytest.mark.parametrize("rows,n,k", [(300, 2048, 2048), (300, 7680, 2048), (300, 2048, 5632), (257, 2048, 2816), (700, 3072, 2048), (500, 4096, 512)])
+def test_sums_in_the_library_s_order(lib, rows, n, k):
+    """Sizes of models with routers at which the library takes K in one piece: the same bits, so that tokens go to the same experts."""
+    x, w, packed, _ = operands(rows, n, k)
+    y = torch.ops._C_amd.prompt_product(x, packed, None, n, ordered=True)
+    assert y is not None and torch.equal(y, torch.nn.functional.linear(x, w))
+
+
+@pytest.mark.parametrize("rows,outputs,k,act", [(300, 5632, 2048, "clamped_unit"), (700, 5632, 2048, "clamped_unit"), (1000, 11264, 2048, "silu_and_mul"),
+                                                (1536, 4096, 2048, "silu_and_mul")])
+def test_activations_behind_sums_in_the_library_s_order(lib, rows, outputs, k, act):
+    from light_vllm_amd.engine.mixers import ORDERED_ROWS
+    from light_vllm_amd.engine.model import Weight, linear_act
+    assert rows <= ORDERED_ROWS
+    x, w, _, _ = operands(rows, 2 * outputs, k)
+    y, both = linear_act(x, Weight(w), act, outputs, 7.0), torch.nn.functional.linear(x, w)
+    want = torch.ops._C_amd.clamped_unit(both, 7.0) if act == "clamped_unit" else torch.ops._C_amd.silu_unit(both)
+    assert y is not None and torch.equal(y, want)
+
+
 @pytest.mark.parametrize("batch,rows,n,k", [(4, 100, 2048, 2048), (4, 300, 2048, 2048), (4, 700, 512, 512), (3, 65, 1040, 320), (5, 129, 64, 256)])
 def test_batches(lib, batch, rows, n, k):
     """Several products in a launch: what each is by itself."""
