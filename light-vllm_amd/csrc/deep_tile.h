@@ -3,9 +3,9 @@
 // a MFMA, and a load of 1 KiB keeps the CU's one address unit for as long, so that four waves whose loads stand together wait 64 cycles for each:
 // loads and MFMAs took turns (80 rows x 128: 356 cycles a k-step, 160 of MFMAs and 224 of loads).  Here the loads are dealt
 // among the MFMAs, and fragments are read a k-step ahead.  us of 64 k-steps, weights in the last cache, a workgroup a CU: 64 rows x 64 9.4, 8.0; 96 x
-// 128 14.6, 11.2; 128 x 128 18.3, 13.3; two a CU: 112 x 128 29.5, 27.7, but 64 x 128 37.4, 39.0 (products have 64 x 64
-// instead; prompt_linear.h says which half tiles with an activation are others).  From memory, 4096 x 4096, 300 rows 25.9 (the
-// library's), 19.8.
+// 128 14.6, 11.2; 128 x 128 18.3, 13.3; two a CU: 112 x 128 29.5, 27.7, but 64 x 128 37.4, 39.0: a plan of
+// products counts with that (prompt_product.h), and half tiles with an activation are dealt where they gain (prompt_linear.h).  From memory,
+// 4096 x 4096, 300 rows 25.9 (the library's), 19.8.
 #pragma once
 #include <type_traits>
 

@@ -54,7 +54,10 @@ inline double product_time(const ProductPlan& p, int rows, int n, int k, int bat
   const ProductTimes& t = p.nt == 1 ? kOne[p.size / 16 - 1][two] : p.nt == 2 ? kTwo[at][two] : kFour[at][two];
   const double mb = (double)rows * n * batch * 1e-6;
   double us = t.fixed + t.step * product_share(p, k) + t.out * mb * (p.shares > 1 ? 4 * p.shares : 2);
-  if (p.shares > 1) us += .2 * mb * (4 * p.shares - 2);  // the slabs' way into the launch that sums them
+  // The slabs' way into the launch that sums them.  Launches of Dynamic Tanh take more (300 rows of 2048 in two slabs 1.7 us, not .7), and those with
+  // the token shift behind it, which sum a row and the one before it, 2.8: 300 rows of 2048 for 2048 and such a launch 18.2, K whole 16.0;
+  // 200 rows 15.0, 14.3.  Ahead of the token shift stand the products of feed-forwards, 8448 for 2048: 300 rows 29.9, 34.7; 900 49.4, 59.7.
+  if (p.shares > 1) us += .2 * mb * (4 * p.shares - 2);
   return us;
 }
 

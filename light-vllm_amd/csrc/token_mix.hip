@@ -8,8 +8,8 @@
 
 namespace lvllm {
 
-// value i of a projection result: T values, or the fp32 split-K slabs of a decode GEMM, summed in slab order and rounded
-// to T (the value the GEMM's own reduce pass would have stored)
+// value i of a projection result: T values, or the fp32 slabs of shares of K (of a decode GEMM, or of prompt_product.hip for prompts of some
+// hundreds of rows), summed in slab order and rounded to T (the value that a reduce pass of the product's own would have stored)
 template <typename T>
 struct ProjOut {
   const typename T::store_t* y;  // null: no addend

@@ -2,8 +2,8 @@
 (softmax heads beside gated linear attention; token-shift time mixing) and the squared-ReLU feed-forward.
 
 The residual stream is fp32 and travels as (x, y): x the stream, y the projection result of the sublayer before, which the
-next norm's launch adds.  y is [rows, width] in the compute dtype or, for decode-size steps, the fp32 split-K slabs of a
-weight-streaming GEMM.  Constants come from the configuration; nothing here knows a model's sizes."""
+next norm's launch adds.  y is [rows, width] in the compute dtype or fp32 slabs of shares of K, [shares, rows, width]: of the
+weight-streaming GEMM for decode-size steps, of prompt_product.hip for prompts of some hundreds of rows.  Constants come from the configuration; nothing here knows a model's sizes."""
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Tuple
 
@@ -68,7 +68,7 @@ def pad_columns(w: torch.Tensor, align: int = 32) -> torch.Tensor:
 
 # Products with an activation behind them add one k behind the other.  So does the library up to some rows: of 174 gated products of 65 to 8192 rows it
 # cut K in 25, all of more than 1600 rows, where up to 2200 of their 50 million results differ; of 253 others of up to these rows in one.  us of a
-# pass of four layers: stream (one dense) 1000 rows 1926, 1893; 1400 2290, 2235; local (two) 700 890, 878; 1200 1160, 1145.
+# pass of four layers: stream (one dense) 1000 rows 1926, 1893; 1400 2290, 2235; local (two) 700 890, 878; 1200 1160, 1145.  What another library does, tests/test_prompt_product_gpu.py says of some sizes.
 ORDERED_ROWS = 1536
 
 

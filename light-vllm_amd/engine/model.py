@@ -4,8 +4,8 @@ Follows light_vllm/decode_only/modelzoo/qwen2.py:144-292: per layer
   fused_add_rms_norm -> qkv GEMM -> rotary_embedding -> attention (reshape_and_cache +
   paged attention) -> o_proj GEMM -> fused_add_rms_norm -> gate_up GEMM -> silu_and_mul ->
   down GEMM; then the final norm and the lm_head GEMM.
-Dense projections are plain torch GEMMs (hipBLASLt / MFMA); everything else is a gfx950
-kernel of this package.  Weights are random-initialised: no checkpoint is available offline.
+Dense projections of long prompts are plain torch GEMMs (hipBLASLt / MFMA) where those are
+the better ones; everything else is a gfx950 kernel of this package.  Weights are random-initialised: no checkpoint is available offline.
 """
 from typing import List, Optional
 
@@ -59,7 +59,8 @@ class Weight:
 
 def linear(x: torch.Tensor, w: "Weight", bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Dense projection.  Decode batches (<= 64 rows) stream the weights through the gfx950
-    weight-streaming kernel; larger batches use the library GEMM (hipBLASLt)."""
+    weight-streaming kernel; prompts of up to some thousand rows take this package's products
+    where they are faster (csrc/prompt_product.h), others the library GEMM (hipBLASLt)."""
     if x.shape[0] == 0:  # a step of unfinished prompt chunks samples nothing
         return x.new_empty((0, w.N))
     if w.w8_t is not None:  # W8A8

@@ -5,8 +5,8 @@ attention -> output projection -> add & LayerNorm -> GELU MLP -> add & LayerNorm
 
 Attention is this package's HIP varlen kernel (AttentionType.ENCODER); the residual add and the LayerNorm
 behind it are one launch (`_C_amd.add_layer_norm`; the reference leaves both to torch),
-exact GELU leaves the projection in front of it (csrc/tile_linear.hip) or is an in-place kernel of this package; the other projections
-are library GEMMs (prompt batches are hundreds to thousands of rows).
+exact GELU leaves the projection in front of it (csrc/tile_linear.hip, csrc/prompt_product.hip) or is an in-place kernel of this package; batches
+of up to some thousand rows take this package's products where those are faster (csrc/prompt_product.h), the rest library GEMMs.
 Weights are random-initialised: no checkpoint is available offline."""
 from dataclasses import dataclass
 from typing import List, Optional
