@@ -120,29 +120,25 @@ class EncoderLayerWeights:
         torch.cuda.synchronize(w.device)  # (the next forward may come on another stream, and one may still read the copy before)
         return copy
 
-    def _current(self, name: str, w: torch.Tensor) -> Optional[torch.Tensor]:
+    def _renewed(self, name: str, w: torch.Tensor) -> Optional[torch.Tensor]:
+        """`w` in fragment order (None: what the kernels do not take), laid out anew when it is another tensor or has been written to since, as far
+        as torch counts that."""
+        if not self._takes(w):
+            return None
         was = self._copies.get(name)
         if was is None or was[0] is not w or was[1].data_ptr() != w.data_ptr() or was[2] != self._version(w):
-            return None
+            was = self._copies[name] = self._copy(w)
         return was[3]
 
     def packed(self, name: str) -> Optional[torch.Tensor]:
         """A weight in fragment order, None where somebody else has it."""
-        return None if name in self.__dict__ else self._current(name, self._kept[name])
+        return None if name in self.__dict__ else self._renewed(name, self._kept[name])
 
     @property
     def fc1_packed(self) -> Optional[torch.Tensor]:
-        """fc1_w in fragment order for the kernel with GELU behind the product of long prompts (None: what it does not take), laid out anew when
-        fc1_w has been replaced or written to since.  Writes that torch does not count (`fc1_w.data.copy_`, or to inference tensors) are not
-        seen: assign fc1_w or lay_out() behind those."""
-        w = self.weight("fc1_w")
-        if not self._takes(w):
-            return None
-        packed = self._current("fc1_w", w)
-        if packed is None:
-            self._copies["fc1_w"] = self._copy(w)
-            packed = self._copies["fc1_w"][3]
-        return packed
+        """fc1_w in fragment order for the kernel with GELU behind the product of long prompts.  Writes that torch does not count
+        (`fc1_w.data.copy_`, or to inference tensors) are not seen: assign fc1_w or lay_out() behind those."""
+        return self._renewed("fc1_w", self.weight("fc1_w"))
 
     def fc1_packed_in_graph(self) -> Optional[torch.Tensor]:
         """... a copy that the graph under capture makes at each replay."""

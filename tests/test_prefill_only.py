@@ -345,6 +345,19 @@ def test_weights_of_another_shape(name, rows):
 
 
 @pytest.mark.gpu
+def test_copies_of_a_model():
+    """A copy of an encoder takes the kernels that the encoder takes."""
+    import copy
+    model, _, run = one_layer([50, 70])
+    first = run().clone()
+    other = copy.deepcopy(model)
+    assert torch.equal(run(other), first) and all(other.layers[0].packed(name) is not None for name in WEIGHTS)
+    assert all(other.layers[0].packed(name) is not model.layers[0].packed(name) for name in WEIGHTS)
+    other.layers[0].qkv_w.zero_()
+    assert not close(run(other), first) and torch.equal(run(), first)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("how", ["data.copy_", "assigned"])
 def test_weights_laid_out_anew(how):
     """Behind lay_out() a model is what one that was made with the weights is: the same kernels, the same bits; and what is written then is seen."""
